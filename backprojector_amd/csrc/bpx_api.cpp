@@ -359,7 +359,7 @@ bpx_status bpx_plan_row_storage(bpx_plan plan, uint32_t* storage) {
     return guarded([&] {
         if (!plan || !storage) fail(BPX_ERR_INVALID_ARGUMENT, "NULL argument");
         const int f = staged_format(*plan->impl);
-        *storage = f == kF16 ? BPX_STORAGE_F16 : f == kBF16 ? BPX_STORAGE_BF16 : BPX_STORAGE_F32;
+        *storage = f == kF16 || f == kCount ? BPX_STORAGE_F16 : f == kBF16 ? BPX_STORAGE_BF16 : BPX_STORAGE_F32;
     });
 }
 
@@ -368,7 +368,11 @@ bpx_status bpx_plan_kernel_name(bpx_plan plan, char* out, uint64_t capacity) {
         if (!plan || !out || capacity == 0) fail(BPX_ERR_INVALID_ARGUMENT, "NULL argument");
         const PlanImpl& pl = *plan->impl;
         std::string name;
-        if (pl.lds_tiles) {
+        if (pl.poly.kz && staged_format(pl) == kCount) {
+            name = "confocal_lds_kernel_poly<KZ=" + std::to_string(pl.poly.kz) + ", degree=" +
+                   std::to_string(pl.poly.deg) + "> (16x16x" + std::to_string(pl.poly.kz) + " tiles, " +
+                   std::to_string(pl.poly_parts) + (pl.poly_parts > 1 ? " pair parts)" : " pair part)");
+        } else if (pl.lds_tiles) {
             const LdsShape sh = lds_shape(pl.variant, pl.format);
             name = "confocal_lds_kernel<KZ=" + std::to_string(sh.kz) + ", waves=" + std::to_string(sh.nw) +
                    "> (16x16x" + std::to_string(sh.depth()) + " tiles)";
@@ -425,13 +429,16 @@ bpx_status bpx_plan_tune(bpx_plan plan, int32_t reps, int32_t* variant) {
                 fail(BPX_ERR_DEVICE, "hipEventCreate failed");
             }
             const int initial = pl.variant;
+            const bool initial_auto = pl.auto_variant;
             int best = initial;
             float best_ms = INFINITY;
             try {
+                pl.auto_variant = false;   // each variant as asked for
                 for (int v = 3; v < variant_count(); ++v) {
                     set_fused_variant(pl, v);
-                    if (v >= kLdsVariant && !pl.lds_tiles) continue;   // would run as a texture-path shape
+                    if (v >= kLdsVariant && !pl.lds_tiles && !pl.poly.kz) continue;   // a texture-path shape
                     pl.execute(pl.stream);                             // warm-up
+                    if (v >= kLdsVariant && !pl.lds_tiles && staged_format(pl) != kCount) continue;
                     hip_check(hipEventRecord(t0, pl.stream), "hipEventRecord");
                     for (int r = 0; r < reps; ++r) pl.execute(pl.stream);
                     hip_check(hipEventRecord(t1, pl.stream), "hipEventRecord");
@@ -447,6 +454,7 @@ bpx_status bpx_plan_tune(bpx_plan plan, int32_t reps, int32_t* variant) {
             } catch (...) {
                 (void)hipEventDestroy(t0);
                 (void)hipEventDestroy(t1);
+                pl.auto_variant = initial_auto;
                 set_fused_variant(pl, initial);
                 throw;
             }

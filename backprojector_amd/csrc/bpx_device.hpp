@@ -10,6 +10,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "bpx_internal.hpp"
+
 namespace bpx {
 
 // ------------------------------------------------------------------ exact arithmetic
@@ -28,6 +30,23 @@ __device__ __forceinline__ float sq3(float a, float b, float c) {
 // round((total - t0) / deltaT), total = ((lw + d1) + d2) + cw (:45).
 __device__ __forceinline__ float tap_round(float total, float t0, float dT) {
     return round_away(exact_div(total - t0, dT));
+}
+
+// A.1 voxel position, backproject_cuda.cu:144-148.
+__device__ __forceinline__ void voxel_position(const Grid& g, uint32_t x, uint32_t y, uint32_t z,
+                                               float v[3]) {
+    const float fx = (float)x, fy = (float)y, fz = (float)z;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        float a = g.zero[k] + g.inc[k] * fx;
+        a = a + g.inc[3 + k] * fy;
+        v[k] = a + g.inc[6 + k] * fz;
+    }
+}
+
+// Whether the rows of this execution are in the format a kernel reads (ConfocalArgs::fmt_flag).
+__device__ __forceinline__ bool rows_wanted(const ConfocalArgs& a) {
+    return !a.fmt_flag || (__builtin_amdgcn_readfirstlane(*a.fmt_flag) & a.fmt_mask) == a.fmt_want;
 }
 
 // ------------------------------------------------------------------ ordered float keys

@@ -80,6 +80,12 @@ struct OctreeState {
     uint32_t P_sub = 0, sub_stride = 0;   // subset size and the stride it was built for (0: none)
     uint32_t coarse_P = 0;                // pairs the coarse levels used in the last execution
     std::vector<uint32_t> fallback_voxels;  // fine voxels added by the fallback, per level
+    // Captures of counts: the fine voxels of well-filled 16 x 16 x kz tiles are gathered tile by
+    // tile with integer sums (LdsPolyShape; kz 0: never), from count rows beside the fp32 ones
+    LdsPolyShape poly;
+    DeviceBuffer count_rows, count_job, count_flag;
+    DeviceBuffer tile_mask, tile_fill, tile_counts, tile_list, tile_parts;
+    uint32_t* host_flag = nullptr;        // pinned copy of count_flag
     DeviceBuffer bound_part_u, bound_part_v;  // pair-segment partial bounds (kBoundPartCapacity floats)
     static constexpr uint64_t kBoundPartCapacity = 1ull << 20;
     uint32_t* host_total = nullptr;
@@ -111,6 +117,13 @@ struct PlanImpl {
     // integer of magnitude <= 2048; fmt_flag (one word) = 0 then, 1 otherwise
     bool rows16 = false;
     bool keep_f32 = false;               // BPX_FLAG_KEEP_F32_ROWS: rows16 never applies
+    // rows of counts (integers 0 .. 2048) gathered with integer sums by the polynomial-quotient
+    // kernel whenever every sample of the execution is one; poly.kz = 0: never
+    LdsPolyShape poly;
+    bool auto_variant = false;           // the variant was not asked for: poly applies whatever it is
+    uint32_t poly_parts = 1, poly_part_pairs = 0;
+    DeviceBuffer parts;                  // integer partial sums [poly_parts][voxels] when split
+    double tap_bound = 0, max_path = 0;  // of the approximate quotient; longest total path
     DeviceBuffer fmt_flag;
     float lz = 0;
     uint32_t kahan_block = 32;

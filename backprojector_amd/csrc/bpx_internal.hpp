@@ -10,12 +10,13 @@ namespace bpx {
 enum SampleFormat : int {
     kF32 = 0, kF16 = 1, kBF16 = 2,     // real
     kC64 = 3, kCF16 = 4, kCBF16 = 5,   // complex (interleaved re, im)
+    kCount = 6,                        // real integers 0 .. 2048 as 16-bit integers (fused rows only)
 };
-__host__ __device__ inline bool format_complex(int f) { return f >= kC64; }
+__host__ __device__ inline bool format_complex(int f) { return f >= kC64 && f <= kCBF16; }
 inline int format_bytes(int f) {
     switch (f) {
         case kF32: return 4;
-        case kF16: case kBF16: return 2;
+        case kF16: case kBF16: case kCount: return 2;
         case kC64: return 8;
         default: return 4;
     }
@@ -50,9 +51,37 @@ struct ConfocalArgs {
     float lz;              // common wall z when every pair shares it
     uint32_t kahan_block;
     // rows whose format is decided on the device at each execution: the kernel runs only when
-    // *fmt_flag == fmt_want (nullptr: always)
+    // (*fmt_flag & fmt_mask) == fmt_want (nullptr: always)
     const uint32_t* fmt_flag;
-    uint32_t fmt_want;
+    uint32_t fmt_mask, fmt_want;
+};
+
+// The LDS-staged gather with polynomial quotients (bpx_lds.hip).
+struct LdsPolyShape {
+    int kz = 0;          // voxels per lane along z, 8 or 16 (0: the kernel does not apply)
+    int deg = 0;         // 2: cubic term folded into the linear one; 3
+    uint32_t seg = 0;    // staged elements per pair, a multiple of 128
+};
+struct LdsPolyArgs {
+    ConfocalArgs c;
+    uint32_t seg;
+    uint32_t part_pairs; // pairs per work-group (a multiple of 4; >= P when not split)
+    uint32_t* parts;     // [parts][voxels] integer partial sums, or nullptr: straight to c.out
+    // the tiles of a list (its length on the device; partial sums [work-groups][256 kz]); nullptr:
+    // every tile of the grid
+    const uint32_t* tiles;
+    const uint32_t* n_tiles;
+    float k1, k2, k3;    // Taylor coefficients' constants: -inv2 step, inv2 step^2 / 2, inv2 step^3 / 2
+};
+// Fine-voxel lists sorted into tiles of that kernel (octree): the voxels of well-filled tiles are
+// computed tile by tile, the others one by one.
+struct TileListArgs {
+    Grid g;
+    uint32_t* mask;      // 16 bits per tile column, [tiles][256] (cleared by the caller)
+    uint32_t* fill;      // listed voxels per tile (cleared)
+    uint32_t* counts;    // [0] listed tiles, [1] other voxels (cleared)
+    uint32_t* tiles;     // the well-filled tiles
+    uint32_t* rest;      // packed voxels of the others
 };
 
 // Factorised exhaustive-grid kernel parameters (threshold table in path-length space).
@@ -147,6 +176,7 @@ struct OctFineArgs {
     const float4* pairs;
     const uint32_t* voxels;  // packed fine voxel coordinates
     uint32_t n;
+    const uint32_t* n_dev;   // their number on the device (<= n; count rows only)
     float* out;
     uint32_t P, Tc, lde, e_bytes, kahan_block;
     Grid g;
@@ -177,6 +207,7 @@ hipError_t launch_oct_bound(const OctBoundArgs& a, uint32_t segments, hipStream_
 hipError_t launch_oct_reduce(const float* U, const float* V, uint32_t n, double* partial,
                              uint32_t max_parts, double* stats, double tau, hipStream_t s);
 hipError_t launch_oct_fine(const OctFineArgs& a, hipStream_t s);
+hipError_t launch_oct_fine_counts(const OctFineArgs& a, hipStream_t s);
 hipError_t launch_fill(float* p, uint64_t n, float v, hipStream_t s);
 hipError_t launch_oct_all_blocks(uint32_t nx, uint32_t ny, uint32_t nz, uint32_t* out, hipStream_t s);
 // Children (8 per block, flags[8 b + c]) whose flag equals want, compacted in block order.
@@ -227,7 +258,9 @@ struct StageJob {
     void* dst;            // fused rows [rows][lde] elements
     const float* pair8;   // pair table, 8 floats per pair
     float* Z;             // [Tc + 1] path-length thresholds (written by the first pass)
-    const uint32_t* fmt_flag;   // non-null: rows written in alt_format while *fmt_flag == 0
+    // non-null: rows written as kCount while *fmt_flag == 0 (if count_rows), else in alt_format
+    // while bit 0 of *fmt_flag is clear, else in `format`
+    const uint32_t* fmt_flag;
     // non-null: [rows][2] element windows [lo, hi) of each row that the gathers can read;
     // only those elements are staged (the others keep the zeros the plan wrote once)
     const uint32_t* win;
@@ -235,7 +268,8 @@ struct StageJob {
     int32_t format;
     float inv_scale, t0, dT;
     uint32_t z_first, s_first;
-    int32_t alt_format;
+    int32_t alt_format, count_rows;
+    uint32_t skip_mask;         // nothing is staged while *fmt_flag has one of these bits
 };
 // raw[r][c] = src[map[r]][from + c - cfrom] for c in [cfrom, cfrom + ncopy), else 0
 // (r < rows, c < Tc; src rows have pitch src_T; map NULL = identity).
@@ -260,6 +294,18 @@ hipError_t launch_phasor_fir(const float* src, uint32_t rows, uint32_t Tc, const
                              int format, float inv_scale, hipStream_t stream);
 hipError_t launch_confocal(const ConfocalArgs& a, int format, int variant, bool sep, bool flat,
                            hipStream_t stream);
+// Shape of the polynomial kernel for a separable grid and a flat wall (kz = 0: does not apply):
+// bound = the host's bound on the approximate quotient's error, max_path = longest total path.
+constexpr uint32_t kPolySegMax = 1024;
+LdsPolyShape lds_poly_shape(const Grid& g, float inv2, float lz, double bound, double max_path, int max_kz);
+uint32_t lds_poly_parts(const Grid& g, const LdsPolyShape& sh, uint32_t P, uint32_t* part_pairs);
+LdsPolyArgs lds_poly_args(const ConfocalArgs& c, const LdsPolyShape& sh);
+hipError_t launch_lds_counts(const LdsPolyArgs& a, const LdsPolyShape& sh, uint32_t parts, hipStream_t s);
+uint64_t lds_tile_count(const Grid& g, const LdsPolyShape& sh);
+hipError_t launch_tile_lists(const TileListArgs& a, const LdsPolyShape& sh, const uint32_t* const lists[2],
+                             const uint32_t n[2], uint32_t dense, hipStream_t s);
+hipError_t launch_lds_counts_tiles(LdsPolyArgs a, const LdsPolyShape& sh, const TileListArgs& t, uint32_t max_tiles,
+                                   uint32_t groups, hipStream_t s);
 hipError_t launch_grid(const GridArgs& a, int format, int variant, hipStream_t stream);
 hipError_t launch_pairs(const PairsArgs& a, int format, int variant, hipStream_t stream);
 // fp32 samples read straight from unpadded rows [P][Tc] (ldh = Tc); no padded copy needed.
@@ -285,8 +331,8 @@ bool batch_lds_applies(const Grid& g, float inv2, int format, bool sep, bool fla
 uint32_t batch_lds_tiles(const Grid& g, int kz);
 hipError_t launch_window(const WindowArgs& a, int complex_samples, hipStream_t stream);
 hipError_t launch_abs_max(const float* src, uint64_t n, float* result_dev, hipStream_t stream);
-// *flag |= 1 unless every one of n samples is an integer of magnitude <= 2048 (exact in fp16);
-// the caller clears *flag first.
+// *flag |= 1 unless every one of n samples is an integer of magnitude <= 2048 (exact in fp16),
+// *flag |= 2 unless every one is an integer in [0, 2048] (a count); the caller clears *flag first.
 hipError_t launch_exact16_check(const float* src, uint64_t n, uint32_t* flag, hipStream_t stream);
 // |v| and atan2(im, re) of n interleaved complex values (either output may be null).
 hipError_t launch_complex_post(const void* complex_volume, uint64_t n, float* mag, float* phase,

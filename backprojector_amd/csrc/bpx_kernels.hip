@@ -205,6 +205,8 @@ __device__ __forceinline__ void write_fused(void* dst, uint64_t e, const float v
     const uint32_t sb = __float_as_uint(S);
     if constexpr (F == kF32) {
         static_cast<float2*>(dst)[e] = make_float2(v[0], S);
+    } else if constexpr (F == kCount) {   // integers 0 .. 2048
+        static_cast<uint2*>(dst)[e] = make_uint2(sb, (uint32_t)v[0] | ((uint32_t)v[1] << 16));
     } else if constexpr (F == kF16 || F == kBF16) {
         const uint32_t ha = F == kF16 ? f32_to_f16(v[0]) : f32_to_bf16_rne(v[0]);
         const uint32_t hb = F == kF16 ? f32_to_f16(v[1]) : f32_to_bf16_rne(v[1]);
@@ -276,8 +278,14 @@ __device__ __forceinline__ void stage_row_elements(const StageJob& jb, uint32_t 
 
 __device__ __forceinline__ void stage_row_block(const StageJob& jb, uint32_t p) {
     // rows of a plan whose samples are checked per execution: fp16 while the check allows it
-    const int format = __builtin_amdgcn_readfirstlane(jb.fmt_flag && *jb.fmt_flag == 0u ? jb.alt_format : jb.format);
+    // (integer counts while they all are, where the plan's kernel takes those)
+    const uint32_t flag = jb.fmt_flag ? __builtin_amdgcn_readfirstlane(*jb.fmt_flag) : 1u;
+    if (flag & jb.skip_mask) return;
+    const int format = __builtin_amdgcn_readfirstlane(flag == 0u && jb.count_rows ? (int)kCount
+                                                      : !(flag & 1u)              ? jb.alt_format
+                                                                                  : jb.format);
     switch (format) {
+        case kCount: stage_row_elements<kCount>(jb, p); break;
         case kF32: stage_row_elements<kF32>(jb, p); break;
         case kF16: stage_row_elements<kF16>(jb, p); break;
         case kBF16: stage_row_elements<kBF16>(jb, p); break;
@@ -526,26 +534,31 @@ hipError_t launch_complex_post(const void* complex_volume, uint64_t n, float* ma
     return hipGetLastError();
 }
 
-// Whether every sample is an integer that fp16 holds exactly (|x| <= 2048): one flag word,
-// set by any wave that finds a sample that is not (NaN and infinities included).
-__device__ __forceinline__ bool exact16_sample(float x) {
-    return __builtin_fabsf(x) <= 2048.0f && x == __builtin_rintf(x);
+// What a sample is not: bit 0 set unless it is an integer that fp16 holds exactly (|x| <= 2048),
+// bit 1 unless it is a count (an integer in [0, 2048]); NaN and infinities set both.
+__device__ __forceinline__ uint32_t sample_flags(float x) {
+    const bool integer = __builtin_fabsf(x) <= 2048.0f && x == __builtin_rintf(x);
+    return integer ? (x >= 0.0f ? 0u : 2u) : 3u;
 }
 
-// Sets *flag when a sample is not an integer of magnitude <= 2048: 16-byte loads over the
-// aligned body (src 16-byte aligned), single samples for the tail.
+// Sets the bits of *flag that any sample sets: 16-byte loads over the aligned body (src 16-byte
+// aligned), single samples for the tail.
 __global__ __launch_bounds__(256) void exact16_check_kernel(const float* __restrict__ src, uint64_t n,
                                                             uint32_t* flag) {
-    bool bad = false;
+    uint32_t bad = 0u;
     const uint64_t n4 = n / 4u, stride = (uint64_t)gridDim.x * blockDim.x;
     const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const float4* s4 = reinterpret_cast<const float4*>(src);
     for (uint64_t i = tid; i < n4; i += stride) {
         const float4 v = s4[i];
-        bad = bad || !(exact16_sample(v.x) && exact16_sample(v.y) && exact16_sample(v.z) && exact16_sample(v.w));
+        bad |= (sample_flags(v.x) | sample_flags(v.y)) | (sample_flags(v.z) | sample_flags(v.w));
     }
-    for (uint64_t i = 4u * n4 + tid; i < n; i += stride) bad = bad || !exact16_sample(src[i]);
-    if (__ballot(bad) != 0ull && (threadIdx.x & 63u) == 0u) atomicOr(flag, 1u);
+    for (uint64_t i = 4u * n4 + tid; i < n; i += stride) bad |= sample_flags(src[i]);
+    const uint32_t wave = (__ballot(bad & 1u) != 0ull ? 1u : 0u) | (__ballot(bad & 2u) != 0ull ? 2u : 0u);
+    // one atomic per wave that adds a bit: waves that find theirs set already write nothing
+    if (wave && (threadIdx.x & 63u) == 0u &&
+        (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & wave) != wave)
+        atomicOr(flag, wave);
 }
 
 hipError_t launch_exact16_check(const float* src, uint64_t n, uint32_t* flag, hipStream_t stream) {
@@ -583,18 +596,6 @@ __device__ __forceinline__ LaneVoxels lane_voxels_of(const Tiles& t, int K, uint
 }
 __device__ __forceinline__ LaneVoxels lane_voxels(const Tiles& t, int K) {
     return lane_voxels_of(t, K, xcd_remap(blockIdx.x, gridDim.x), threadIdx.x >> 6);
-}
-
-// A.1 voxel position, backproject_cuda.cu:144-148.
-__device__ __forceinline__ void voxel_position(const Grid& g, uint32_t x, uint32_t y, uint32_t z,
-                                               float v[3]) {
-    const float fx = (float)x, fy = (float)y, fz = (float)z;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        float a = g.zero[k] + g.inc[k] * fx;
-        a = a + g.inc[3 + k] * fy;
-        v[k] = a + g.inc[6 + k] * fz;
-    }
 }
 
 template <class T>
@@ -740,6 +741,7 @@ __device__ __forceinline__ void confocal_tile(const ConfocalArgs& a, uint32_t ti
 
 template <class Src, int K, bool SEP, bool FLAT>
 __global__ __launch_bounds__(256) void confocal_kernel(ConfocalArgs a) {
+    if (!rows_wanted(a)) return;
     confocal_tile<Src, K, SEP, FLAT>(a, xcd_remap(blockIdx.x, gridDim.x), threadIdx.x >> 6);
 }
 
@@ -983,7 +985,7 @@ __device__ __forceinline__ void lds_tile(const ConfocalArgs& a, uint32_t tile) {
 template <class Fz, int KZ, int NW>
 __global__ __launch_bounds__(NW * 64) void confocal_lds_kernel(ConfocalArgs a) {
     // rows staged in the other format this execution: the other instantiation runs instead
-    if (a.fmt_flag && __builtin_amdgcn_readfirstlane(*a.fmt_flag) != a.fmt_want) return;
+    if (!rows_wanted(a)) return;
     lds_tile<Fz, KZ, NW>(a, xcd_remap(blockIdx.x, gridDim.x));
 }
 
@@ -1556,7 +1558,7 @@ bool variant_fused(int variant) { return variant >= 3; }
 int variant_count() { return 9; }
 int fused_elem_bytes(int format) {
     switch (format) {
-        case kF32: case kF16: case kBF16: return 8;
+        case kF32: case kF16: case kBF16: case kCount: return 8;
         default: return 16;
     }
 }

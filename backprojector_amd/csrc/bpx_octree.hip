@@ -573,6 +573,64 @@ __global__ __launch_bounds__(256) void oct_fine_kernel(OctFineArgs a) {
         if (base + r < a.n) a.out[ids[r]] = kahan_result(sum[r], comp[r]);
 }
 
+// The same for count rows (elements (S, lo | hi << 16), flat wall): integer sums, added to the
+// zeroed volume as 32-bit integers, so the pairs of a voxel may be split over lanes in any way.  The
+// list's length is on the device; the launch's work-groups are shared out over (256 voxels, part of
+// the pairs), at most 16 parts.  A lane's scattered gathers are bound by their latency: 100,000
+// voxels and 16,384 pairs filled a fifth of the wavefront slots with one lane per voxel and took
+// 3.1 ms however few they were.
+__global__ __launch_bounds__(256) void oct_fine_count_kernel(OctFineArgs a) {
+    const uint32_t n = __builtin_amdgcn_readfirstlane(*a.n_dev), blocks = (n + 255u) / 256u;
+    if (n == 0u) return;
+    const uint32_t parts = max(1u, min(min(gridDim.x / blocks, 16u), a.P / 64u));
+    const uint32_t part = blockIdx.x / blocks, per = (a.P + parts - 1u) / parts;
+    const uint32_t first = part * per, end = min(first + per, a.P);
+    if (part >= parts || first >= end) return;
+    const uint32_t i = (blockIdx.x % blocks) * 256u + threadIdx.x;
+    uint32_t x, y, z;
+    unpack_block(a.voxels[min(i, n - 1u)], x, y, z);
+    float v[3];
+    voxel_position(a.g, x, y, z, v);
+    const float cz = a.lz - v[2], vz2 = cz * cz;
+    const auto er = make_rsrc(a.E, a.e_bytes);
+    using Off = ElemOffset<8>;
+    const float top = Off::kBias + (float)a.Tc;
+    auto tap = [&](uint32_t q) {
+        const float4 pr = a.pairs[q];
+        const float dx = pr.x - v[0], dy = pr.y - v[1];
+        const float s = (dx * dx + dy * dy) + vz2;
+        const float yq = __builtin_fmaf(__builtin_amdgcn_sqrtf(s), a.inv2, pr.w + Off::kBias);
+        const auto e = __builtin_amdgcn_raw_buffer_load_b64(er, (int)Off::clamped(yq, top), (int)(q * a.lde * 8u), 0);
+        return s >= __uint_as_float(e[0]) ? e[1] >> 16 : e[1] & 0xffffu;
+    };
+    uint32_t acc = 0, p = first;
+    constexpr uint32_t kUnroll = 8;
+    for (; p + kUnroll <= end; p += kUnroll) {
+        uint32_t t[kUnroll];
+#pragma unroll
+        for (uint32_t u = 0; u < kUnroll; ++u) t[u] = tap(p + u);
+#pragma unroll
+        for (uint32_t u = 0; u < kUnroll; ++u) acc += t[u];
+    }
+    for (; p < end; ++p) acc += tap(p);
+    if (i < n) atomicAdd(reinterpret_cast<uint32_t*>(a.out) + ((x * a.g.n[1] + y) * a.g.n[2] + z), acc);
+}
+__global__ __launch_bounds__(256) void oct_count_values_kernel(OctFineArgs a) {
+    const uint32_t n = *a.n_dev, i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    uint32_t x, y, z;
+    unpack_block(a.voxels[i], x, y, z);
+    float* o = a.out + ((x * a.g.n[1] + y) * a.g.n[2] + z);
+    *o = (float)__float_as_uint(*o);
+}
+hipError_t launch_oct_fine_counts(const OctFineArgs& a, hipStream_t s) {
+    const uint32_t blocks = (a.n + 255u) / 256u;
+    if (blocks == 0u) return hipSuccess;
+    hipLaunchKernelGGL(oct_fine_count_kernel, dim3(std::max(blocks, 4096u)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(oct_count_values_kernel, dim3(blocks), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
 // One voxel per lane up to 4M voxels (more lanes hide the gather latency of these sparse
 // lists), two beyond (measured on 256^3 x 16384-pair captures: 1.1M voxels 10.8 ms with one
 // per lane against 17.9 ms with two; 9.0M voxels 63 ms with two).

@@ -432,7 +432,9 @@ PlanImpl* make_plan_single_tap(const CaptureIn& c, const uint32_t n[3], const fl
     // exactness precondition of the table lookup
     double corners[8][3];
     grid_corners(n, zero, inc, corners);
-    const double bound = tap_error_bound(max_total_path(pr.data(), pr.size(), corners), c.t0, c.dT, c.T);
+    pl->max_path = max_total_path(pr.data(), pr.size(), corners);
+    const double bound = tap_error_bound(pl->max_path, c.t0, c.dT, c.T);
+    pl->tap_bound = bound;
     if (bound >= 0.25)
         fail(BPX_ERR_UNSUPPORTED,
              "path lengths / t0 too large relative to deltaT for the exact bin lookup (bound " +
@@ -519,6 +521,7 @@ PlanImpl* make_plan_single_tap(const CaptureIn& c, const uint32_t n[3], const fl
             else if (t8 >= kLdsMinTiles && fits8) pl->variant = kLdsVariant + 1;
         }
         pl->keep_f32 = (o.flags & BPX_FLAG_KEEP_F32_ROWS) != 0;
+        pl->auto_variant = o.variant < 0;
         if (pl->fused) {
             set_fused_variant(*pl, pl->variant);
         } else {
@@ -561,11 +564,11 @@ PlanImpl* make_plan_single_tap(const CaptureIn& c, const uint32_t n[3], const fl
 }
 
 int staged_format(const PlanImpl& pl) {
-    if (!pl.rows16) return pl.format;
+    if (!pl.rows16 && !pl.poly.kz) return pl.format;
     plan_wait(pl);
-    uint32_t flag = 1;
+    uint32_t flag = 3;
     hip_check(hipMemcpy(&flag, pl.fmt_flag.ptr, 4, hipMemcpyDeviceToHost), "hipMemcpy(row format)");
-    return flag == 0u ? kF16 : pl.format;
+    return flag == 0u && pl.poly.kz ? kCount : pl.rows16 && !(flag & 1u) ? kF16 : pl.format;
 }
 
 StageJob stage_job(const PlanImpl& pl) {
@@ -578,9 +581,10 @@ StageJob stage_job(const PlanImpl& pl) {
     j.Tc = pl.T;
     j.lde = pl.ldh;
     j.format = pl.format;
-    j.fmt_flag = pl.rows16 ? static_cast<const uint32_t*>(pl.fmt_flag.ptr) : nullptr;
+    j.fmt_flag = pl.rows16 || pl.poly.kz ? static_cast<const uint32_t*>(pl.fmt_flag.ptr) : nullptr;
     j.win = static_cast<const uint32_t*>(pl.win.ptr);
-    j.alt_format = kF16;
+    j.alt_format = pl.rows16 ? kF16 : pl.format;
+    j.count_rows = pl.poly.kz ? 1 : 0;
     j.inv_scale = 1.0f / pl.scale;
     j.t0 = pl.t0;
     j.dT = pl.dT;
@@ -603,7 +607,7 @@ void set_fused_variant(PlanImpl& pl, int variant) {
     // 91.7 -> 89.7); the 16-per-lane shape, bound by its arithmetic and the default where
     // it applies (256^3), measured slower with fp16 rows (84.5 -> 86.4), so it keeps fp32.
     pl.rows16 = pl.lds_tiles && pl.format == kF32 && lds_shape(variant, pl.format).kz == 8 && !pl.keep_f32;
-    if (pl.rows16 && !pl.fmt_flag.ptr) {
+    if ((pl.rows16 || pl.poly.kz) && !pl.fmt_flag.ptr) {
         pl.fmt_flag.alloc(4);
         hip_check(hipMemset(pl.fmt_flag.ptr, 0xff, 4), "hipMemset(row format)");   // fp32 until run
     }
@@ -671,7 +675,7 @@ void PlanImpl::execute(hipStream_t s) {
     hip_check(hipEventRecord(ev[1], s), "hipEventRecord");
     if (path == kPathConfocal) {
         if (fused) {
-            if (rows16) {
+            if (rows16 || poly.kz) {
                 hip_check(launch_fill(static_cast<float*>(fmt_flag.ptr), 1, 0.0f, s), "fill kernel");
                 hip_check(launch_exact16_check(static_cast<const float*>(raw.ptr), (uint64_t)P * T,
                                                static_cast<uint32_t*>(fmt_flag.ptr), s),
@@ -703,13 +707,24 @@ void PlanImpl::execute(hipStream_t s) {
         a.scale = scale;
         a.lz = lz;
         a.kahan_block = kahan_block;
-        if (rows16) {
-            // both instantiations launched; the one the device check did not pick returns at once
+        if (rows16 || poly.kz) {
+            // every instantiation launched; those the device check did not pick return at once
             a.fmt_flag = static_cast<const uint32_t*>(fmt_flag.ptr);
-            a.fmt_want = 1u;
+            if (poly.kz) {
+                LdsPolyArgs pa = lds_poly_args(a, poly);
+                pa.c.fmt_mask = 3u;
+                pa.c.fmt_want = 0u;
+                pa.part_pairs = poly_part_pairs;
+                pa.parts = poly_parts > 1 ? static_cast<uint32_t*>(parts.ptr) : nullptr;
+                hip_check(launch_lds_counts(pa, poly, poly_parts, s), "confocal gather kernel (count rows)");
+            }
+            if (rows16) {
+                a.fmt_mask = poly.kz ? 3u : 1u;
+                a.fmt_want = poly.kz ? 2u : 0u;
+                hip_check(launch_confocal(a, kF16, variant, sep, flat, s), "confocal gather kernel (fp16 rows)");
+            }
+            a.fmt_mask = a.fmt_want = rows16 ? 1u : 2u;
             hip_check(launch_confocal(a, format, variant, sep, flat, s), "confocal gather kernel");
-            a.fmt_want = 0u;
-            hip_check(launch_confocal(a, kF16, variant, sep, flat, s), "confocal gather kernel (fp16 rows)");
         } else {
             hip_check(launch_confocal(a, format, variant, sep, flat, s), "confocal gather kernel");
         }
