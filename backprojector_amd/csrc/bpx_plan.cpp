@@ -607,6 +607,19 @@ void set_fused_variant(PlanImpl& pl, int variant) {
     // 91.7 -> 89.7); the 16-per-lane shape, bound by its arithmetic and the default where
     // it applies (256^3), measured slower with fp16 rows (84.5 -> 86.4), so it keeps fp32.
     pl.rows16 = pl.lds_tiles && pl.format == kF32 && lds_shape(variant, pl.format).kz == 8 && !pl.keep_f32;
+    // Rows of counts: integer sums need no order and no compensation, so any split of the pairs
+    // gives the volume of the fp32 rows bit for bit while a block of kahan_block counts stays
+    // below 2^24 and the whole sum below 2^32.  For variants 7 and 8 (as the exact fp16 rows), and for
+    // every confocal plan whose variant was left to the library.
+    pl.poly = LdsPolyShape{};
+    if (pl.format == kF32 && !pl.keep_f32 && pl.sep && pl.flat && (pl.auto_variant || variant > kLdsVariant) &&
+        pl.kahan_block <= 4096u && pl.P <= (1u << 20))
+        pl.poly = lds_poly_shape(pl.g, pl.inv2, pl.lz, pl.tap_bound, pl.max_path, 16);
+    if (pl.poly.kz) {
+        pl.poly_parts = lds_poly_parts(pl.g, pl.poly, pl.P, &pl.poly_part_pairs);
+        const size_t bytes = pl.poly_parts > 1 ? (size_t)pl.poly_parts * pl.g.n[0] * pl.g.n[1] * pl.g.n[2] * 4u : 0;
+        if (bytes > pl.parts.bytes) pl.parts.alloc(bytes);
+    }
     if ((pl.rows16 || pl.poly.kz) && !pl.fmt_flag.ptr) {
         pl.fmt_flag.alloc(4);
         hip_check(hipMemset(pl.fmt_flag.ptr, 0xff, 4), "hipMemset(row format)");   // fp32 until run
