@@ -23,6 +23,7 @@ ARCH = "gfx950"
 SOURCES = [
     "bpx_kernels.hip",
     "bpx_lds.hip",
+    "bpx_window.hip",
     "bpx_plan.cpp",
     "bpx_api.cpp",
     "bpx_pipeline.cpp",

@@ -150,6 +150,27 @@ struct WindowArgs {
     Tiles t;
 };
 
+// The LDS-staged window kernel (bpx_window.hip): confocal pairs, flat wall.
+struct WindowLdsArgs {
+    const double* PS;      // exclusive prefix sums [P][ldp], the last one repeated past bin T - 1
+    const double* Slo;     // [P][pitch] smallest squared distance whose window starts at bin >= j
+    const double* Shi;     // ... ends
+    const float* Zlo;      // thresholds [T] in path-length space (window_table_kernel)
+    const float* Zhi;
+    const float* pair8;
+    const float4* pairs;   // (x, y, z, q): q ~ (lw + cw - w/2 - t0)/dT + 1
+    float* out;
+    double* parts;         // [parts][voxels] partial sums, or nullptr
+    uint32_t P, T, ldp, pitch, part_pairs;
+    uint32_t seg, seg_sums;    // staged thresholds and sums per pair, multiples of 128
+    uint32_t shift;        // even number of bins between the staged start and end thresholds
+    Grid g;
+    float inv2, lz;
+    float width_bins;      // window width in bins
+    float hi_offset;       // width_bins - shift + seg: from a start's biased quotient to the end's
+    float k1, k2, k3;      // as LdsPolyArgs
+};
+
 // Octree level bound: one lane per block (packed x | y << 10 | z << 20).
 struct OctBoundArgs {
     const float* M;         // window-max table of the level [P][ldm]
@@ -297,8 +318,9 @@ hipError_t launch_confocal(const ConfocalArgs& a, int format, int variant, bool 
 // Shape of the polynomial kernel for a separable grid and a flat wall (kz = 0: does not apply):
 // bound = the host's bound on the approximate quotient's error, max_path = longest total path.
 constexpr uint32_t kPolySegMax = 1024;
-LdsPolyShape lds_poly_shape(const Grid& g, float inv2, float lz, double bound, double max_path, int max_kz);
-uint32_t lds_poly_parts(const Grid& g, const LdsPolyShape& sh, uint32_t P, uint32_t* part_pairs);
+constexpr double kPolyBudget = 0.24, kWindowPolyBudget = 0.18;
+LdsPolyShape lds_poly_shape(const Grid& g, float inv2, float lz, double bound, double max_path, double budget);
+uint32_t lds_poly_parts(const Grid& g, const LdsPolyShape& sh, uint32_t P, uint32_t sum_bytes, uint32_t* part_pairs);
 LdsPolyArgs lds_poly_args(const ConfocalArgs& c, const LdsPolyShape& sh);
 hipError_t launch_lds_counts(const LdsPolyArgs& a, const LdsPolyShape& sh, uint32_t parts, hipStream_t s);
 uint64_t lds_tile_count(const Grid& g, const LdsPolyShape& sh);
@@ -330,6 +352,9 @@ hipError_t launch_batch_prologue(const StageJob* jobs, uint32_t n_jobs, uint32_t
 bool batch_lds_applies(const Grid& g, float inv2, int format, bool sep, bool flat, int kz);
 uint32_t batch_lds_tiles(const Grid& g, int kz);
 hipError_t launch_window(const WindowArgs& a, int complex_samples, hipStream_t stream);
+hipError_t launch_window_tables(const WindowLdsArgs& a, double* Slo, double* Shi, hipStream_t s);
+hipError_t launch_window_lds(const WindowLdsArgs& a, const LdsPolyShape& sh, uint32_t parts, hipStream_t s);
+size_t window_lds_bytes(const WindowLdsArgs& a);
 hipError_t launch_abs_max(const float* src, uint64_t n, float* result_dev, hipStream_t stream);
 // *flag |= 1 unless every one of n samples is an integer of magnitude <= 2048 (exact in fp16),
 // *flag |= 2 unless every one is an integer in [0, 2048] (a count); the caller clears *flag first.

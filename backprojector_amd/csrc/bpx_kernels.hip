@@ -372,13 +372,14 @@ hipError_t launch_pad_rows(const float* src, uint32_t rows, uint32_t Tc, uint32_
     return hipGetLastError();
 }
 
-// Exclusive prefix sums in double, one wave per row: PS[p][k] = sum_{i<k} H[p][i], k < T.
+// Exclusive prefix sums in double, one wave per row: PS[p][k] = sum_{i<k} H[p][i], k < T; entries
+// T .. ldp - 1 repeat PS[p][T - 1].
 __global__ __launch_bounds__(256) void prefix_kernel(const float* __restrict__ src, uint32_t rows,
                                                      uint32_t T, int cplx, void* dst, uint32_t ldp) {
     const uint32_t row = blockIdx.x * 4u + (threadIdx.x >> 6);
     const uint32_t lane = threadIdx.x & 63u;
     if (row >= rows) return;
-    double carry_re = 0.0, carry_im = 0.0;
+    double carry_re = 0.0, carry_im = 0.0, end_re = 0.0, end_im = 0.0;
     for (uint32_t c0 = 0; c0 < T; c0 += 64u) {
         const uint32_t i = c0 + lane;
         double xr = 0.0, xi = 0.0;
@@ -400,13 +401,21 @@ __global__ __launch_bounds__(256) void prefix_kernel(const float* __restrict__ s
                 si += ui;
             }
         }
+        const double er = carry_re + sr - xr, ei = carry_im + si - xi;
+        if (c0 + 64u >= T) {
+            end_re = __shfl(er, (T - 1u) & 63u, 64);
+            end_im = __shfl(ei, (T - 1u) & 63u, 64);
+        }
         if (i < T) {
-            const double er = carry_re + sr - xr, ei = carry_im + si - xi;
             if (cplx) static_cast<double2*>(dst)[(size_t)row * ldp + i] = make_double2(er, ei);
             else static_cast<double*>(dst)[(size_t)row * ldp + i] = er;
         }
         carry_re += __shfl(sr, 63, 64);
         carry_im += __shfl(si, 63, 64);
+    }
+    for (uint32_t i = T + lane; i < ldp; i += 64u) {
+        if (cplx) static_cast<double2*>(dst)[(size_t)row * ldp + i] = make_double2(end_re, end_im);
+        else static_cast<double*>(dst)[(size_t)row * ldp + i] = end_re;
     }
 }
 

@@ -15,8 +15,7 @@
 #include <algorithm>
 #include <cmath>
 
-#include "bpx_device.hpp"
-#include "bpx_internal.hpp"
+#include "bpx_lds.hpp"
 
 // dst = VCC ? high half of src : low half of src, zero-extended
 #define SEL16(dst, src)                                                                         \
@@ -27,29 +26,9 @@ namespace bpx {
 
 namespace {
 
-typedef __attribute__((address_space(3))) void lds_void;
-
-__device__ __forceinline__ uint32_t lds_offset(const void* p) { return (uint32_t)(uintptr_t)(lds_void*)p; }
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint2 lds_read8(uint32_t off) {
-    const u32x2 v = *(const __attribute__((address_space(3))) u32x2*)(uintptr_t)off;
-    return make_uint2(v[0], v[1]);
-}
-
-// 16 bytes per lane from the buffer at byte offset `off` (0 past its end) to LDS at
-// lds_base + 16 lane.  The load has no register output; its issuer waits for vmcnt before the
-// barrier that publishes the data.  (Written out because the compiler orders the builtin's load
-// before every later LDS read it cannot tell apart, which would drain the loads of the next stage
-// before the current stage's gathers.)
-__device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, uint32_t lds_base, int off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                 :: "s"(lds_base), "v"(off), "s"(r) : "memory");
-}
-__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
 // Count rows: samples are integers 0 .. 2048 (16 bits each), summed as integers: exact in any
-// order, one register per voxel and no compensation.  column() adds KZ updates: element e[r] =
-// (S, lo | hi << 16) gives lo where s < S and hi elsewhere, s = axy + dz2[r].  Each update is a
+// order, one register per voxel and no compensation.  column() adds KZ updates: element e[i] =
+// (S, lo | hi << 16) of voxel r = column_order(i) gives lo where s < S and hi elsewhere, s = axy + dz2[r].  Each update is a
 // compare, a select whose SDWA word selects move the chosen half into place, an add, and the add
 // that makes the next update's s; written in one chain so that the two wait states the select
 // needs after the compare (and the one the add needs after the select) hold the neighbours' adds.
@@ -57,23 +36,23 @@ struct CountRows {
     using acc_t = uint32_t;
     template <int KZ>
     __device__ static __forceinline__ void column(acc_t (&acc)[KZ], const uint2 (&e)[KZ], float axy,
-                                                  const float (&dz2)[KZ], const int (&order)[KZ]) {
-        float s = axy + dz2[order[0]];
+                                                  const float (&dz2)[KZ]) {
+        float s = axy + dz2[column_order<KZ>(0)];
         uint32_t h;
         asm("v_cmp_ge_f32_e32 vcc, %1, %2\n\ts_nop 1\n\t" SEL16("%0", "%3")
-            : "=v"(h) : "v"(s), "v"(e[order[0]].x), "v"(e[order[0]].y) : "vcc");
+            : "=v"(h) : "v"(s), "v"(e[0].x), "v"(e[0].y) : "vcc");
 #pragma unroll
         for (int i = 1; i < KZ; ++i) {
-            const int r = order[i], prev = order[i - 1];
+            const int r = column_order<KZ>(i), prev = column_order<KZ>(i - 1);
             s = axy + dz2[r];
             uint32_t hn;
             asm("v_cmp_ge_f32_e32 vcc, %2, %3\n\t"
                 "v_add_u32_e32 %0, %0, %5\n\t"
                 "s_nop 0\n\t" SEL16("%1", "%4")
-                : "+&v"(acc[prev]), "=v"(hn) : "v"(s), "v"(e[r].x), "v"(e[r].y), "v"(h) : "vcc");
+                : "+&v"(acc[prev]), "=v"(hn) : "v"(s), "v"(e[i].x), "v"(e[i].y), "v"(h) : "vcc");
             h = hn;
         }
-        acc[order[KZ - 1]] += h;
+        acc[column_order<KZ>(KZ - 1)] += h;
     }
 };
 
@@ -97,9 +76,7 @@ __global__ __launch_bounds__(256, 4) void confocal_lds_kernel_poly(LdsPolyArgs a
     float4* const meta = reinterpret_cast<float4*>(smem + 2u * PS * slot_bytes);
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
     const Grid& g = a.c.g;
-    const uint32_t n0 = g.n[0], n1 = g.n[1], n2 = g.n[2];
-    const uint32_t ntz = (n2 + KZ - 1u) / KZ, nty = (n1 + 15u) / 16u, ntx = (n0 + 15u) / 16u;
-    const uint32_t tiles = ntx * nty * ntz;
+    const uint32_t n0 = g.n[0], n1 = g.n[1], n2 = g.n[2], tiles = poly_tiles(g, KZ);
     // every tile of the grid, or those of a list whose length is on the device (then the launch is
     // fixed and its work-groups are shared out here)
     const uint32_t count = TILES ? __builtin_amdgcn_readfirstlane(*a.n_tiles) : tiles;
@@ -108,44 +85,17 @@ __global__ __launch_bounds__(256, 4) void confocal_lds_kernel_poly(LdsPolyArgs a
     if (TILES && (count == 0u || part * part_pairs >= a.c.P)) return;
     const uint32_t tile = TILES ? __builtin_amdgcn_readfirstlane(a.tiles[index]) : xcd_remap(index, tiles);
     const uint32_t p0 = part * part_pairs, p1 = min(p0 + part_pairs, a.c.P);
-    const uint32_t tz = tile % ntz, txy = tile / ntz, ty = txy % nty, tx = txy / nty;
-    const uint32_t ix = tx * 16u + (w & 1u) * 8u + (lane & 7u);
-    const uint32_t iy = ty * 16u + (w >> 1) * 8u + (lane >> 3);
-    const uint32_t iz0 = min(tz * KZ, n2 - KZ);   // the last slab reaches back over its neighbour
-    const uint32_t cx = min(ix, n0 - 1u), cy = min(iy, n1 - 1u);
-    float vx = 0.0f, vy = 0.0f, dz2[KZ];
+    const ColumnTile<KZ> t(g, tile, w, lane);
+    float dz2[KZ];   // uniform
 #pragma unroll
     for (int r = 0; r < KZ; ++r) {
         float v[3];
-        voxel_position(g, cx, cy, iz0 + r, v);
-        if (r == 0) {
-            vx = v[0];
-            vy = v[1];
-        }
+        voxel_position(g, t.cx, t.cy, t.iz0 + r, v);
         const float dz = a.c.lz - v[2];
-        dz2[r] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(dz * dz)));
+        dz2[r] = uniform_f32(dz * dz);
     }
-    // column centre: z = zero + inc (iz0 + (KZ - 1) / 2), uniform
-    const float u = a.c.lz - (g.zero[2] + g.inc[8] * ((float)iz0 + 0.5f * (float)(KZ - 1)));
-    const float u2 = u * u;
-    // bounding box of the tile (coordinates are monotone in each index: extremes at the corners)
-    const uint32_t x0 = min(tx * 16u, n0 - 1u), x1 = min(tx * 16u + 15u, n0 - 1u);
-    const uint32_t y0 = min(ty * 16u, n1 - 1u), y1 = min(ty * 16u + 15u, n1 - 1u);
-    float bmin[3] = {__builtin_inff(), __builtin_inff(), __builtin_inff()};
-    float bmax[3] = {-__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        float v[3];
-        voxel_position(g, (c & 1) ? x1 : x0, (c & 2) ? y1 : y0, (c & 4) ? iz0 + KZ - 1u : iz0, v);
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            bmin[k] = fminf(bmin[k], v[k]);
-            bmax[k] = fmaxf(bmax[k], v[k]);
-        }
-    }
-    const float ez = a.c.lz - fminf(fmaxf(a.c.lz, bmin[2]), bmax[2]);
-    const float fz = fmaxf(fabsf(a.c.lz - bmin[2]), fabsf(a.c.lz - bmax[2]));
-    const float ez2 = ez * ez, fz2 = fz * fz;
+    const float u = t.centre(g, a.c.lz), u2 = u * u;
+    const TileBox<KZ> box(g, t, a.c.lz);
     const uint32_t row_bytes = a.c.ldh * 8u;
     const uint32_t nstage = (p1 - p0 + PS - 1u) / PS;
 
@@ -159,12 +109,8 @@ __global__ __launch_bounds__(256, 4) void confocal_lds_kernel_poly(LdsPolyArgs a
         mjl = 0;
         if (p < p1) {
             const float4 pr = a.c.pairs[p];
-            const float ex = pr.x - fminf(fmaxf(pr.x, bmin[0]), bmax[0]);
-            const float ey = pr.y - fminf(fmaxf(pr.y, bmin[1]), bmax[1]);
-            const float fx = fmaxf(fabsf(pr.x - bmin[0]), fabsf(pr.x - bmax[0]));
-            const float fy = fmaxf(fabsf(pr.y - bmin[1]), fabsf(pr.y - bmax[1]));
-            const float smin = (ex * ex + ey * ey) + ez2;
-            const float smax = (fx * fx + fy * fy) + fz2;
+            float smin, smax;
+            box.distances(pr.x, pr.y, smin, smax);
             // 2 elements of margin each way; the start even, so that a 16-byte load never
             // straddles a row end
             const int jl = ((int)__builtin_fmaf(__builtin_amdgcn_sqrtf(smin), a.c.inv2, pr.w) - 2) & ~1;
@@ -192,35 +138,15 @@ __global__ __launch_bounds__(256, 4) void confocal_lds_kernel_poly(LdsPolyArgs a
     acc_t acc[KZ];
 #pragma unroll
     for (int r = 0; r < KZ; ++r) acc[r] = 0;
-    const float k1 = a.k1, k2 = a.k2, k3 = a.k3;
     auto pair_step = [&](const float4 m) {
-        const float dx = m.x - vx, dy = m.y - vy;
+        const float dx = m.x - t.vx, dy = m.y - t.vy;
         const float axy = dx * dx + dy * dy;
-        const float s0 = axy + u2;
-        const float gi = __builtin_amdgcn_rsqf(s0);
-        const float t = u * gi;                    // cosine to the wall normal
-        const float q = gi - (t * t) * gi;         // (1 - t^2) / d
-        const float c0 = __builtin_fmaf(s0 * gi, a.c.inv2, m.z);
-        const float c2 = q * k2;
-        const float c3 = (q * t) * (gi * k3);
-        float c1 = t * k1;
-        constexpr float kTop = 0.5f * (float)(KZ - 1);
-        if (DEG == 2) c1 = __builtin_fmaf(c3, 0.75f * kTop * kTop, c1);   // best linear part of c3 rho^3
+        const ColumnQuotient<KZ, DEG> q(axy, u, u2, a.c.inv2, a.k1, a.k2, a.k3, m.z);
         uint2 e[KZ];
-        int order[KZ];   // as the reads are issued
 #pragma unroll
-        for (int h = 0; h < KZ / 2; ++h) {
-            order[2 * h] = KZ / 2 + h;
-            order[2 * h + 1] = KZ / 2 - 1 - h;
-            const float rho = 0.5f + (float)h;
-            const float ev = __builtin_fmaf(c2, rho * rho, c0);
-            const float od = DEG == 3 ? __builtin_fmaf(c3, rho * rho, c1) : c1;
-            const float yp = __builtin_fmaf(od, rho, ev), ym = __builtin_fmaf(od, -rho, ev);
-            e[KZ / 2 + h] = lds_read8(Off::of(yp));
-            e[KZ / 2 - 1 - h] = lds_read8(Off::of(ym));
-        }
+        for (int i = 0; i < KZ; ++i) e[i] = lds_read8(Off::of(q.at(i)));
         __builtin_amdgcn_sched_barrier(0);
-        Fz::template column<KZ>(acc, e, axy, dz2, order);
+        Fz::template column<KZ>(acc, e, axy, dz2);
     };
     if (nstage) stage(0u);
     wait_loads();
@@ -243,8 +169,8 @@ __global__ __launch_bounds__(256, 4) void confocal_lds_kernel_poly(LdsPolyArgs a
         uint32_t* o = a.parts + (size_t)blockIdx.x * (256u * KZ) + threadIdx.x;
 #pragma unroll
         for (int r = 0; r < KZ; ++r) o[256u * r] = acc[r];
-    } else if (ix < n0 && iy < n1) {
-        const size_t id = ((size_t)ix * n1 + iy) * n2 + iz0;
+    } else if (t.ix < n0 && t.iy < n1) {
+        const size_t id = t.id(g);
         if (a.parts) {
             uint32_t* o = a.parts + (size_t)part * n0 * n1 * n2 + id;
 #pragma unroll
@@ -349,10 +275,6 @@ __global__ __launch_bounds__(256) void tile_store_kernel(TileListArgs a, LdsPoly
         }
 }
 
-static uint64_t poly_tiles(const Grid& g, int kz) {
-    return (uint64_t)((g.n[0] + 15u) / 16u) * ((g.n[1] + 15u) / 16u) * ((g.n[2] + (uint32_t)kz - 1u) / (uint32_t)kz);
-}
-
 template <int KZ, int DEG, bool TILES>
 static hipError_t poly_launch(const LdsPolyArgs& a, uint32_t groups, hipStream_t s) {
     const auto fn = confocal_lds_kernel_poly<CountRows, KZ, DEG, TILES>;
@@ -426,8 +348,8 @@ hipError_t launch_lds_counts_tiles(LdsPolyArgs a, const LdsPolyShape& sh, const 
 // its best linear approximation adds c3 h^3 / 4.  In use the polynomial's value rounds to 1/8 four
 // times (w, c0, the even part, the sum: 1/16 each), so the bound on the approximate quotient
 // (`bound`, which covers the arithmetic of its terms) and the polynomial's error must stay below
-// 1/4 together.
-LdsPolyShape lds_poly_shape(const Grid& g, float inv2, float lz, double bound, double max_path, int max_kz) {
+// 1/4 together (`budget`; the window kernel's end edge rounds a fifth time: 3/16).
+LdsPolyShape lds_poly_shape(const Grid& g, float inv2, float lz, double bound, double max_path, double budget) {
     LdsPolyShape none;
     // column along z alone; coordinates whose squares and reciprocals stay normal floats
     if (g.inc[2] != 0.0f || g.inc[5] != 0.0f || g.inc[6] != 0.0f || g.inc[7] != 0.0f) return none;
@@ -436,11 +358,11 @@ LdsPolyShape lds_poly_shape(const Grid& g, float inv2, float lz, double bound, d
     const double zmin = std::min(std::fabs(za), std::fabs(zb)) * (1.0 - 1e-5);
     if (!(za * zb > 0.0) || !(zmin > 1e-12) || !(max_path < 1e12) || !(step > 0.0)) return none;
     for (int kz : {16, 8}) {
-        if (kz > max_kz || g.n[2] < (uint32_t)kz) continue;
+        if (g.n[2] < (uint32_t)kz) continue;
         const double h = 0.5 * (kz - 1) * step;
         const double e3 = A * 0.0559 * h * h * h * h / (zmin * zmin * zmin);
         const double e2 = e3 + A * 0.0930 * h * h * h / (4.0 * zmin * zmin);
-        const double limit = 0.24 - bound;
+        const double limit = budget - bound;
         const int deg = e2 <= limit ? 2 : e3 <= limit ? 3 : 0;
         if (!deg) continue;
         double d2 = 0.0;
@@ -467,11 +389,11 @@ LdsPolyShape lds_poly_shape(const Grid& g, float inv2, float lz, double bound, d
 // tiles) 8.65 ms in 1 part, 6.85 in 2, 6.42 in 4, 6.08 in 8, 6.11 in 16 -- more rounds of resident
 // work-groups even out the last one; 1,961 pairs into 45 x 61 x 38 (60 tiles) 0.107 ms in 9 parts,
 // 0.082 in 18, 0.087 in 61.
-uint32_t lds_poly_parts(const Grid& g, const LdsPolyShape& sh, uint32_t P, uint32_t* part_pairs) {
+uint32_t lds_poly_parts(const Grid& g, const LdsPolyShape& sh, uint32_t P, uint32_t sum_bytes, uint32_t* part_pairs) {
     const uint64_t tiles = poly_tiles(g, sh.kz), vox = (uint64_t)g.n[0] * g.n[1] * g.n[2];
     uint64_t parts = std::max(std::min<uint64_t>((4096u + tiles - 1u) / tiles, P / 128u),
                               std::min<uint64_t>((1024u + tiles - 1u) / tiles, P / 32u));
-    parts = std::max<uint64_t>(1u, std::min<uint64_t>(parts, (64ull << 20) / (4u * vox)));
+    parts = std::max<uint64_t>(1u, std::min<uint64_t>(parts, (64ull << 20) / (sum_bytes * vox)));
     *part_pairs = (uint32_t)(((P + parts - 1u) / parts + 3u) / 4u * 4u);
     return std::max(1u, (P + *part_pairs - 1u) / *part_pairs);
 }

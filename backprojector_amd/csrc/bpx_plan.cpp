@@ -564,7 +564,7 @@ PlanImpl* make_plan_single_tap(const CaptureIn& c, const uint32_t n[3], const fl
 }
 
 int staged_format(const PlanImpl& pl) {
-    if (!pl.rows16 && !pl.poly.kz) return pl.format;
+    if (!pl.fmt_flag.ptr || (!pl.rows16 && !pl.poly.kz)) return pl.format;
     plan_wait(pl);
     uint32_t flag = 3;
     hip_check(hipMemcpy(&flag, pl.fmt_flag.ptr, 4, hipMemcpyDeviceToHost), "hipMemcpy(row format)");
@@ -614,9 +614,9 @@ void set_fused_variant(PlanImpl& pl, int variant) {
     pl.poly = LdsPolyShape{};
     if (pl.format == kF32 && !pl.keep_f32 && pl.sep && pl.flat && (pl.auto_variant || variant > kLdsVariant) &&
         pl.kahan_block <= 4096u && pl.P <= (1u << 20))
-        pl.poly = lds_poly_shape(pl.g, pl.inv2, pl.lz, pl.tap_bound, pl.max_path, 16);
+        pl.poly = lds_poly_shape(pl.g, pl.inv2, pl.lz, pl.tap_bound, pl.max_path, kPolyBudget);
     if (pl.poly.kz) {
-        pl.poly_parts = lds_poly_parts(pl.g, pl.poly, pl.P, &pl.poly_part_pairs);
+        pl.poly_parts = lds_poly_parts(pl.g, pl.poly, pl.P, 4u, &pl.poly_part_pairs);
         const size_t bytes = pl.poly_parts > 1 ? (size_t)pl.poly_parts * pl.g.n[0] * pl.g.n[1] * pl.g.n[2] * 4u : 0;
         if (bytes > pl.parts.bytes) pl.parts.alloc(bytes);
     }
@@ -652,6 +652,24 @@ void PlanImpl::execute(hipStream_t s) {
         hip_check(hipEventRecord(ev[1], s), "hipEventRecord");
         hip_check(launch_ztable(1, t0, dT, half_width, T, static_cast<float*>(Z.ptr), s), "window table (start)");
         hip_check(launch_ztable(2, t0, dT, half_width, T, static_cast<float*>(Z2.ptr), s), "window table (end)");
+        if (poly.kz) {
+            WindowLdsArgs a = wlds;
+            a.PS = static_cast<const double*>(H.ptr);
+            a.Slo = static_cast<const double*>(win_lo.ptr);
+            a.Shi = static_cast<const double*>(win_hi.ptr);
+            a.Zlo = static_cast<const float*>(Z.ptr);
+            a.Zhi = static_cast<const float*>(Z2.ptr);
+            a.pair8 = static_cast<const float*>(pair8.ptr);
+            a.pairs = static_cast<const float4*>(pair4.ptr);
+            a.out = static_cast<float*>(vol.ptr);
+            a.parts = poly_parts > 1 ? static_cast<double*>(parts.ptr) : nullptr;
+            hip_check(launch_window_tables(a, static_cast<double*>(win_lo.ptr), static_cast<double*>(win_hi.ptr), s),
+                      "window threshold kernel");
+            hip_check(hipEventRecord(ev[2], s), "hipEventRecord");
+            hip_check(launch_window_lds(a, poly, poly_parts, s), "window gather kernel (LDS-staged)");
+            hip_check(hipEventRecord(ev[3], s), "hipEventRecord");
+            return;
+        }
         hip_check(hipEventRecord(ev[2], s), "hipEventRecord");
         WindowArgs a{};
         a.PS = H.ptr;
@@ -786,6 +804,60 @@ void PlanImpl::execute(hipStream_t s) {
     hip_check(hipEventRecord(ev[3], s), "hipEventRecord");
 }
 
+// The LDS-staged window kernel where it applies: real samples, confocal pairs on a flat wall, bin
+// windows and threshold tables that fit.  Sets the row pitch of the prefix sums.
+static void window_lds_setup(PlanImpl& pl, const std::vector<bpx_pair>& pr, float width) {
+    bool flat = true;
+    for (const auto& p : pr) flat = flat && p.laser_point[2] == pr[0].laser_point[2];
+    if (pl.cplx || !pl.all_confocal || !flat) return;
+    for (int k = 0; k < 3; ++k) {
+        pl.g.zero[k] = pl.wzero[k];
+        pl.g.inc[4 * k] = pl.wvs[k];
+    }
+    pl.lz = pr[0].laser_point[2];
+    pl.inv2 = (float)(2.0 / (double)pl.dT);
+    const LdsPolyShape sh = lds_poly_shape(pl.g, pl.inv2, pl.lz, pl.tap_bound, pl.max_path, kWindowPolyBudget);
+    const double bins = (double)width / (double)pl.dT;
+    if (!sh.kz || !(bins < 1024.0)) return;
+    WindowLdsArgs& a = pl.wlds;
+    a.P = pl.P;
+    a.T = pl.T;
+    a.seg = sh.seg;
+    a.shift = (uint32_t)bins & ~1u;
+    a.seg_sums = round_up((uint64_t)sh.seg + a.shift + 6u, 128);
+    a.ldp = round_up((uint64_t)pl.T + a.seg_sums, 32);
+    a.pitch = round_up(pl.T, 32);
+    if (window_lds_bytes(a) > 160u * 1024u) return;
+    // tables beside the sums: 16 more bytes a bin, at most 16 GiB in all
+    if ((uint64_t)pl.P * (2u * a.pitch + a.ldp) * 8u > (16ull << 30)) return;
+    a.g = pl.g;
+    a.inv2 = pl.inv2;
+    a.lz = pl.lz;
+    a.width_bins = (float)bins;
+    a.hi_offset = (float)(bins - (double)a.shift + (double)a.seg);
+    const LdsPolyArgs k = lds_poly_args(ConfocalArgs{.g = pl.g, .inv2 = pl.inv2}, sh);
+    a.k1 = k.k1;
+    a.k2 = k.k2;
+    a.k3 = k.k3;
+    std::vector<float> p4((size_t)pl.P * 4);
+    for (uint32_t p = 0; p < pl.P; ++p) {
+        p4[4 * p + 0] = pr[p].laser_point[0];
+        p4[4 * p + 1] = pr[p].laser_point[1];
+        p4[4 * p + 2] = pr[p].laser_point[2];
+        p4[4 * p + 3] = (float)(((double)pr[p].laser_wall + (double)pr[p].camera_wall - (double)pl.half_width -
+                                 (double)pl.t0) / (double)pl.dT + 1.0);
+    }
+    pl.pair4.alloc(sizeof(float) * p4.size());
+    hip_check(hipMemcpy(pl.pair4.ptr, p4.data(), sizeof(float) * p4.size(), hipMemcpyHostToDevice), "hipMemcpy(pairs)");
+    pl.win_lo.alloc((size_t)pl.P * a.pitch * 8u);
+    pl.win_hi.alloc((size_t)pl.P * a.pitch * 8u);
+    pl.ldh = a.ldp;
+    // double sums: a split changes their last bits only; half the parts of the integer kernel
+    pl.poly = sh;
+    pl.poly_parts = lds_poly_parts(pl.g, sh, pl.P, 8u, &a.part_pairs);
+    if (pl.poly_parts > 1) pl.parts.alloc((size_t)pl.poly_parts * pl.g.n[0] * pl.g.n[1] * pl.g.n[2] * 8u);
+}
+
 PlanImpl* make_plan_window(const CaptureIn& c, const uint32_t n[3], const float vpos[3],
                            const float vsize[3]) {
     validate_common(c, n);
@@ -827,7 +899,9 @@ PlanImpl* make_plan_window(const CaptureIn& c, const uint32_t n[3], const float 
                              (m & 1) ? (double)(n[2] - 1) : 0.0};
         for (int k = 0; k < 3; ++k) corners[m][k] = (double)pl->wzero[k] + (double)pl->wvs[k] * i[k];
     }
-    const double bound = tap_error_bound(max_total_path(pr.data(), pr.size(), corners) + width, c.t0, c.dT, c.T);
+    pl->max_path = max_total_path(pr.data(), pr.size(), corners);
+    const double bound = tap_error_bound(pl->max_path + width, c.t0, c.dT, c.T);
+    pl->tap_bound = bound;
     if (bound >= 0.25)
         fail(BPX_ERR_UNSUPPORTED, "path lengths / t0 too large relative to deltaT for the exact bin lookup");
     pl->inv = (float)(1.0 / (double)c.dT);
@@ -836,6 +910,7 @@ PlanImpl* make_plan_window(const CaptureIn& c, const uint32_t n[3], const float 
     if (pl->P == 0 || c.T < 2) return pl.release();
     stage_raw(*pl, c, idx);
     pl->ldh = round_up(c.T, 32);
+    window_lds_setup(*pl, pr, width);
     pl->H.alloc((size_t)pl->P * pl->ldh * (c.cplx ? 16 : 8));
     pl->Z.alloc(sizeof(float) * c.T);
     pl->Z2.alloc(sizeof(float) * c.T);
