@@ -24,6 +24,7 @@ SOURCES = [
     "bpx_kernels.hip",
     "bpx_lds.hip",
     "bpx_window.hip",
+    "bpx_paths.hip",
     "bpx_plan.cpp",
     "bpx_api.cpp",
     "bpx_pipeline.cpp",

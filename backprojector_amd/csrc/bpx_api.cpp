@@ -372,6 +372,9 @@ bpx_status bpx_plan_kernel_name(bpx_plan plan, char* out, uint64_t capacity) {
             name = "confocal_lds_kernel_poly<KZ=" + std::to_string(pl.poly.kz) + ", degree=" +
                    std::to_string(pl.poly.deg) + "> (16x16x" + std::to_string(pl.poly.kz) + " tiles, " +
                    std::to_string(pl.poly_parts) + (pl.poly_parts > 1 ? " pair parts)" : " pair part)");
+        } else if (pl.paths.seg) {
+            name = std::string("paths_lds_kernel<") + (pl.paths.L ? "grid" : "pairs") + "> (16x16x8 tiles, " +
+                   std::to_string(pl.paths_parts) + (pl.paths_parts > 1 ? " parts)" : " part)");
         } else if (pl.lds_tiles) {
             const LdsShape sh = lds_shape(pl.variant, pl.format);
             name = "confocal_lds_kernel<KZ=" + std::to_string(sh.kz) + ", waves=" + std::to_string(sh.nw) +

@@ -134,6 +134,22 @@ struct PairsArgs {
     uint32_t kahan_block;
 };
 
+// The LDS-staged gather of exhaustive grids and pair lists (bpx_paths.hip).
+struct PathsLdsArgs {
+    const float* rows;      // unpadded fp32 rows [P][Tc]
+    const float4* lasers;   // exhaustive grid (L != 0): as GridArgs
+    const float4* spads;
+    const float* pairs;     // pair list: as PairsArgs
+    const float* Z;
+    float* out;
+    double* parts;          // [parts][voxels] partial sums, or nullptr
+    uint32_t L, C, P, Tc, seg;
+    uint32_t part_units;    // lasers (grid) or pairs of a part
+    uint32_t kahan_block;
+    Grid g;
+    float inv, c1, scale;
+};
+
 // Window (reference CPU path) kernel parameters.
 struct WindowArgs {
     const void* PS;         // exclusive prefix sums in double [P][ldp] (complex: double2)
@@ -330,6 +346,11 @@ hipError_t launch_lds_counts_tiles(LdsPolyArgs a, const LdsPolyShape& sh, const 
                                    uint32_t groups, hipStream_t s);
 hipError_t launch_grid(const GridArgs& a, int format, int variant, hipStream_t stream);
 hipError_t launch_pairs(const PairsArgs& a, int format, int variant, hipStream_t stream);
+// The LDS-staged kernel: arguments with seg a multiple of 256 and at least 256, every leg's squared
+// length in [2^-100, 2^100].
+hipError_t launch_paths_lds(const PathsLdsArgs& a, uint32_t parts, hipStream_t s);
+size_t paths_lds_bytes(const PathsLdsArgs& a);
+hipError_t launch_quantise_rows(const float* src, uint64_t n, int format, float inv_scale, float* dst, hipStream_t s);
 // fp32 samples read straight from unpadded rows [P][Tc] (ldh = Tc); no padded copy needed.
 hipError_t launch_pairs_raw(const PairsArgs& a, hipStream_t stream);
 // The batch queue kernel (K voxels per lane on the texture path, LDS tile depth kz, storage

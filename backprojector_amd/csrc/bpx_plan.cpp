@@ -385,6 +385,66 @@ static uint32_t grid_structure(const std::vector<bpx_pair>& pr) {
     return C;
 }
 
+// The LDS-staged kernel of non-confocal captures where it applies: real samples, voxels of a column
+// sharing x and y, points clear of the volume (its roots' range), windows that fit beside the
+// threshold table.  Tiles are 16 x 16 x 8.
+static void paths_lds_setup(PlanImpl& pl, const std::vector<bpx_pair>& pr, const double corners[8][3]) {
+    const Grid& g = pl.g;
+    if (pl.cplx || g.inc[6] != 0.0f || g.inc[7] != 0.0f || g.n[2] < 8u || pl.T + 1u > 16384u) return;
+    double lo[3], hi[3];
+    for (int k = 0; k < 3; ++k) {
+        lo[k] = hi[k] = corners[0][k];
+        for (int m = 1; m < 8; ++m) {
+            lo[k] = std::min(lo[k], corners[m][k]);
+            hi[k] = std::max(hi[k], corners[m][k]);
+        }
+        const double slack = 1e-5 * std::max(std::fabs(lo[k]), std::fabs(hi[k]));
+        lo[k] -= slack;
+        hi[k] += slack;
+    }
+    // distance of a point from the volume's box; a point inside it may be at distance 0 of a voxel
+    const auto clear = [&](const float* p) {
+        double d = 0.0;
+        for (int k = 0; k < 3; ++k) {
+            const double e = std::max({lo[k] - (double)p[k], (double)p[k] - hi[k], 0.0});
+            d = std::max(d, e);
+        }
+        return d > 1e-9;
+    };
+    for (const auto& p : pr)
+        if (!clear(p.laser_point) || !clear(p.camera_point)) return;
+    if (!(pl.max_path < 1e9)) return;
+    double d2 = 0.0;
+    for (int k = 0; k < 3; ++k) {
+        const double r = 15.0 * (std::fabs((double)g.inc[k]) + std::fabs((double)g.inc[3 + k])) + 7.0 * std::fabs((double)g.inc[6 + k]);
+        d2 += r * r;
+    }
+    const double need = std::ceil(2.0 * std::sqrt(d2) / (double)pl.dT * (1.0 + 1e-6)) + 14.0;
+    if (!(need <= 2048.0)) return;
+    PathsLdsArgs a{};
+    a.seg = round_up((uint64_t)need, 256);
+    a.Tc = pl.T;
+    if (paths_lds_bytes(a) > 160u * 1024u) return;
+    a.L = pl.L;
+    a.C = pl.C;
+    a.P = pl.P;
+    a.g = g;
+    // blocks of 8 pairs (a stage) between compensated adds: the order of the sums differs from the
+    // general kernels', and no sum should come out further from the exact one than theirs
+    a.kahan_block = std::min<uint32_t>(pl.kahan_block, 8u);
+    a.scale = pl.scale;
+    // parts towards 2,048 work-groups of at least 8 lasers or 64 pairs, 64 MiB of partial sums
+    const uint64_t tiles = (uint64_t)((g.n[0] + 15u) / 16u) * ((g.n[1] + 15u) / 16u) * ((g.n[2] + 7u) / 8u);
+    const uint64_t vox = (uint64_t)g.n[0] * g.n[1] * g.n[2];
+    const uint32_t units = pl.L ? pl.L : pl.P;
+    uint64_t parts = std::min<uint64_t>((2048u + tiles - 1u) / tiles, units / (pl.L ? 8u : 64u));
+    parts = std::max<uint64_t>(1u, std::min<uint64_t>(parts, (64ull << 20) / (8u * vox)));
+    a.part_units = (uint32_t)((units + parts - 1u) / parts);
+    pl.paths_parts = (units + a.part_units - 1u) / a.part_units;
+    if (pl.paths_parts > 1) pl.parts.alloc((size_t)pl.paths_parts * vox * 8u);
+    pl.paths = a;
+}
+
 PlanImpl* make_plan_single_tap(const CaptureIn& c, const uint32_t n[3], const float zero[3],
                                const float inc[9], const bpx_options* opt) {
     validate_common(c, n);
@@ -457,7 +517,9 @@ PlanImpl* make_plan_single_tap(const CaptureIn& c, const uint32_t n[3], const fl
     const uint64_t hbytes = (uint64_t)pl->P * pl->ldh *
                             (pl->fused ? fused_elem_bytes(pl->format) : format_bytes(pl->format));
     if (hbytes >= (1ull << 32)) fail(BPX_ERR_UNSUPPORTED, "transient rows above 4 GiB per plan");
-    pl->H.alloc(hbytes);
+    if (pl->path != kPathConfocal && o.variant < 0) paths_lds_setup(*pl, pr, corners);
+    if (!pl->paths.seg) pl->H.alloc(hbytes);
+    else if (pl->format != kF32) pl->H.alloc((size_t)pl->P * c.T * 4u);
     // fused rows staged over per-pair windows keep zeros outside them (written here only)
     if (pl->fused) hip_check(hipMemset(pl->H.ptr, 0, hbytes), "hipMemset(fused rows)");
 
@@ -699,7 +761,12 @@ void PlanImpl::execute(hipStream_t s) {
     // events: ev[0] | split-layout row padding | ev[1] | tables (fused: all staging) | ev[2] |
     // gather | ev[3]
     hip_check(hipEventRecord(ev[0], s), "hipEventRecord");
-    if (!fused)
+    if (paths.seg) {
+        if (format != kF32)
+            hip_check(launch_quantise_rows(static_cast<const float*>(raw.ptr), (uint64_t)P * T, format, 1.0f / scale,
+                                           static_cast<float*>(H.ptr), s),
+                      "row quantisation kernel");
+    } else if (!fused)
         hip_check(launch_pad_rows(static_cast<const float*>(raw.ptr), P, T, T, H.ptr, ldh, format,
                                   1.0f / scale, s),
                   "row staging kernel");
@@ -763,7 +830,19 @@ void PlanImpl::execute(hipStream_t s) {
         hip_check(launch_ztable(0, t0, dT, 0.0f, T + 1, static_cast<float*>(Z.ptr), s),
                   "threshold table kernel");
         hip_check(hipEventRecord(ev[2], s), "hipEventRecord");
-        if (path == kPathGrid) {
+        if (paths.seg) {
+            PathsLdsArgs a = paths;
+            a.rows = static_cast<const float*>(format == kF32 ? raw.ptr : H.ptr);
+            a.lasers = static_cast<const float4*>(lasers.ptr);
+            a.spads = static_cast<const float4*>(spads.ptr);
+            a.pairs = static_cast<const float*>(pair8.ptr);
+            a.Z = static_cast<const float*>(Z.ptr);
+            a.out = static_cast<float*>(vol.ptr);
+            a.parts = paths_parts > 1 ? static_cast<double*>(parts.ptr) : nullptr;
+            a.inv = inv;
+            a.c1 = c1;
+            hip_check(launch_paths_lds(a, paths_parts, s), "gather kernel (LDS-staged paths)");
+        } else if (path == kPathGrid) {
             GridArgs a{};
             a.H = H.ptr;
             a.lasers = static_cast<const float4*>(lasers.ptr);
