@@ -77,10 +77,7 @@ void run_plan_to_host(PlanImpl* raw, float* out) {
     std::unique_ptr<PlanImpl> pl(raw);
     pl->execute(pl->stream);
     const size_t nvox = (size_t)pl->g.n[0] * pl->g.n[1] * pl->g.n[2];
-    hip_check(hipMemcpyAsync(out, pl->vol.ptr, nvox * (pl->cplx ? 8 : 4), hipMemcpyDeviceToHost,
-                             pl->stream),
-              "hipMemcpyAsync(volume)");
-    hip_check(hipStreamSynchronize(pl->stream), "hipStreamSynchronize");
+    download_host(out, pl->vol.ptr, nvox * (pl->cplx ? 8 : 4), pl->stream);
 }
 
 }  // namespace bpx
@@ -212,9 +209,7 @@ bpx_status bpx_octree_backprojection(const float* transient_chunk, uint64_t tran
         std::unique_ptr<PlanImpl> pl(make_plan_octree(c, voxels_per_side, volume_zero_pos, voxel_inc, options));
         pl->execute(pl->stream);
         const size_t nvox = (size_t)pl->g.n[0] * pl->g.n[1] * pl->g.n[2];
-        hip_check(hipMemcpyAsync(voxel_volume, pl->vol.ptr, nvox * 4, hipMemcpyDeviceToHost, pl->stream),
-                  "hipMemcpyAsync(volume)");
-        hip_check(hipStreamSynchronize(pl->stream), "hipStreamSynchronize");
+        download_host(voxel_volume, pl->vol.ptr, nvox * 4, pl->stream);
         if (stats) fill_octree_stats(*pl, stats);
     });
 }
@@ -283,8 +278,8 @@ bpx_status bpx_plan_read_volume(bpx_plan plan, float* voxel_volume) {
         PlanImpl& pl = *plan->impl;
         const size_t nvox = (size_t)pl.g.n[0] * pl.g.n[1] * pl.g.n[2];
         plan_wait(pl);
-        hip_check(hipMemcpy(voxel_volume, pl.vol.ptr, nvox * (pl.cplx ? 8 : 4), hipMemcpyDeviceToHost),
-                  "hipMemcpy(volume)");
+        // on the null stream: after replays of a captured execution on blocking streams too
+        download_host(voxel_volume, pl.vol.ptr, nvox * (pl.cplx ? 8 : 4), nullptr);
     });
 }
 

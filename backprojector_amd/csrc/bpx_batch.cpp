@@ -515,7 +515,7 @@ bpx_status bpx_batch_read_volume(bpx_batch batch, uint32_t index, float* voxel_v
         b.wait();
         const PlanImpl& pl = *b.plans[index];
         const size_t nvox = (size_t)pl.g.n[0] * pl.g.n[1] * pl.g.n[2];
-        hip_check(hipMemcpy(voxel_volume, pl.vol.ptr, (b.cplx ? 8u : 4u) * nvox, hipMemcpyDeviceToHost), "hipMemcpy");
+        download_host(voxel_volume, pl.vol.ptr, (b.cplx ? 8u : 4u) * nvox, nullptr);
     });
 }
 

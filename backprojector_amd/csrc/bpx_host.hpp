@@ -36,13 +36,31 @@ std::vector<uint32_t> confocal_row_windows(const bpx_pair* pairs, uint32_t P, co
 // ------------------------------------------------------------------ plan
 enum Path : int { kPathConfocal = 0, kPathGrid = 1, kPathPairs = 2, kPathWindow = 3, kPathOctree = 4 };
 
+// Device memory.  Released blocks are kept for later allocations of about their size (hipMalloc of
+// 16 MB takes 47 us, hipFree of a plan's buffers up to 300): kPooledBytes in all at most, none larger
+// than half of that, none for longer than kPooledTicks allocations; when the device's memory runs out
+// all of them are given back before an allocation fails.  A release waits for the device, as hipFree
+// does, so no work queued on any stream still uses a block that is handed out again.
+constexpr size_t kPooledBytes = 512u << 20;
+constexpr uint64_t kPooledTicks = 256;
 struct DeviceBuffer {
     void* ptr = nullptr;
-    size_t bytes = 0;
+    size_t bytes = 0;   // as asked for
+    size_t cap = 0;     // of the block
+    int device = -1;
     DeviceBuffer() = default;
     DeviceBuffer(const DeviceBuffer&) = delete;
     DeviceBuffer& operator=(const DeviceBuffer&) = delete;
-    DeviceBuffer(DeviceBuffer&& o) noexcept : ptr(o.ptr), bytes(o.bytes) { o.ptr = nullptr; o.bytes = 0; }
+    DeviceBuffer(DeviceBuffer&& o) noexcept : ptr(o.ptr), bytes(o.bytes), cap(o.cap), device(o.device) {
+        o.ptr = nullptr;
+        o.bytes = o.cap = 0;
+    }
+    void swap(DeviceBuffer& o) noexcept {
+        std::swap(ptr, o.ptr);
+        std::swap(bytes, o.bytes);
+        std::swap(cap, o.cap);
+        std::swap(device, o.device);
+    }
     void alloc(size_t n);
     void release();
     ~DeviceBuffer() { release(); }
@@ -228,6 +246,31 @@ void plan_replace_rows(PlanImpl& pl, DeviceBuffer& rows);
 // Host -> device copy of a (possibly pageable) host array, enqueued on s and complete when
 // this returns; large arrays are pipelined through pinned staging buffers.
 void upload_host(void* dst, const void* src, size_t bytes, hipStream_t s);
+
+// Device -> host copy, ordered on s and complete when this returns; large arrays go through pinned
+// staging buffers, their host side written by several threads.
+void download_host(void* dst, const void* src, size_t bytes, hipStream_t s);
+// Small host tables -> device in one batch of copies from a pinned slab (a pageable hipMemcpy takes 13
+// to 65 us each).  They are in place after finish().
+class TableUploads {
+public:
+    explicit TableUploads(hipStream_t s) : stream(s) {}
+    TableUploads(const TableUploads&) = delete;
+    TableUploads& operator=(const TableUploads&) = delete;
+    ~TableUploads();
+    void add(void* dst, const void* src, size_t bytes);
+    void finish();
+
+private:
+    hipStream_t stream;
+    char* slab = nullptr;
+    size_t used = 0;
+    bool open = true;
+};
+// A stream for one plan (default priority, non-blocking); streams of destroyed plans are kept, at
+// most 8, for the next ones.
+hipStream_t take_stream();
+void give_stream(hipStream_t s);
 
 // Executes a plan, copies its volume to host memory and destroys the plan.
 void run_plan_to_host(PlanImpl* plan, float* out);

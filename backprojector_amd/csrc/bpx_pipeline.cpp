@@ -323,12 +323,12 @@ void phasor_filter_host(const float* in, uint64_t rows, uint32_t T, const std::v
     if (rows * T >= (1ull << 38)) fail(BPX_ERR_UNSUPPORTED, "phasor input too large");
     din.alloc(sizeof(float) * rows * T);
     dout.alloc(sizeof(float) * 2 * rows * T);
-    hip_check(hipMemcpy(din.ptr, in, sizeof(float) * rows * T, hipMemcpyHostToDevice), "hipMemcpy");
+    upload_host(din.ptr, in, sizeof(float) * rows * T, nullptr);
     hip_check(launch_phasor_fir(static_cast<const float*>(din.ptr), (uint32_t)rows, T,
                                 static_cast<const float*>(dc.ptr), static_cast<const float*>(ds.ptr),
                                 (int)c.size(), dout.ptr, T, 0u, kC64, 1.0f, nullptr),
               "phasor FIR kernel");
-    hip_check(hipMemcpy(out, dout.ptr, sizeof(float) * 2 * rows * T, hipMemcpyDeviceToHost), "hipMemcpy(phasor)");
+    download_host(out, dout.ptr, sizeof(float) * 2 * rows * T, nullptr);
 }
 
 // The chunk on the device: the source rows in one copy, the chunk window cropped
@@ -655,10 +655,7 @@ bpx_status bpx_nlos_phasor_output(const float* transient_data, const int64_t* da
                           "complex post-processing kernel");
                 src = post.ptr;
             }
-            hip_check(hipMemcpyAsync(volumes_out + per * nvox * i, src, 4 * per * nvox, hipMemcpyDeviceToHost,
-                                     plan->stream),
-                      "hipMemcpyAsync(volume)");
-            hip_check(hipStreamSynchronize(plan->stream), "hipStreamSynchronize");
+            download_host(volumes_out + per * nvox * i, src, 4 * per * nvox, plan->stream);
         }
         return BPX_OK;
     } catch (const Failure& e) {

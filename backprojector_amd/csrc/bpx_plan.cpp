@@ -1,10 +1,12 @@
 // Plans: validation, structure detection, device staging and execution of one capture.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <limits>
 #include <memory>
 #include <mutex>
+#include <system_error>
 #include <thread>
 
 #include "bpx_host.hpp"
@@ -12,21 +14,150 @@
 namespace bpx {
 
 // ------------------------------------------------------------------ device buffers
+namespace {
+struct PooledBlock {
+    void* ptr;
+    size_t cap;
+    int device;
+    uint64_t tick;   // of its release
+};
+// Never destroyed: plans may outlive this library's static objects.
+struct Pool {
+    std::mutex mutex;
+    std::vector<PooledBlock> blocks;   // oldest release first
+    size_t bytes = 0;
+    uint64_t ticks = 0;                // allocations so far
+    std::vector<std::pair<int, hipStream_t>> streams;
+    std::vector<char*> slabs;
+};
+Pool& pool() {
+    static Pool* p = new Pool;
+    return *p;
+}
+int current_device() {
+    int d = -1;
+    return hipGetDevice(&d) == hipSuccess ? d : -1;
+}
+
+// Block sizes: multiples of 256 bytes up to 64 KiB, then of an eighth of the power of two below.
+size_t block_size(size_t n) {
+    size_t step = 256;
+    if (n > (64u << 10)) {
+        size_t p = 64u << 10;
+        while (p <= n / 2) p *= 2;
+        step = p / 8;
+    }
+    return (n + step - 1) / step * step;
+}
+// Takes the oldest blocks out until at most `room` bytes are kept and none has lain unused for
+// kPooledTicks allocations; the caller frees them outside the lock.
+std::vector<void*> evict(Pool& p, size_t room) {
+    std::vector<void*> out;
+    size_t n = 0;
+    while (n < p.blocks.size() && (p.bytes > room || p.ticks - p.blocks[n].tick > kPooledTicks)) {
+        out.push_back(p.blocks[n].ptr);
+        p.bytes -= p.blocks[n].cap;
+        ++n;
+    }
+    p.blocks.erase(p.blocks.begin(), p.blocks.begin() + (ptrdiff_t)n);
+    return out;
+}
+}  // namespace
+
 void DeviceBuffer::alloc(size_t n) {
     release();
     if (n == 0) n = 256;
-    const hipError_t e = hipMalloc(&ptr, n);
-    if (e != hipSuccess) {
-        ptr = nullptr;
-        fail(BPX_ERR_OUT_OF_MEMORY, "hipMalloc(" + std::to_string(n) + " bytes) failed: " +
-                                        hipGetErrorString(e));
+    const size_t want = block_size(n);
+    Pool& p = pool();
+    device = current_device();
+    {
+        std::lock_guard<std::mutex> lock(p.mutex);
+        ++p.ticks;
+        size_t best = p.blocks.size();
+        for (size_t i = 0; i < p.blocks.size(); ++i)
+            if (p.blocks[i].device == device && p.blocks[i].cap >= want && p.blocks[i].cap <= want + want / 4 &&
+                (best == p.blocks.size() || p.blocks[i].cap < p.blocks[best].cap))
+                best = i;
+        if (best < p.blocks.size()) {
+            ptr = p.blocks[best].ptr;
+            cap = p.blocks[best].cap;
+            p.bytes -= cap;
+            p.blocks.erase(p.blocks.begin() + (ptrdiff_t)best);
+        }
+    }
+    if (!ptr) {
+        hipError_t e = hipMalloc(&ptr, want);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            std::vector<void*> all;
+            {
+                std::lock_guard<std::mutex> lock(p.mutex);
+                all = evict(p, 0);
+            }
+            for (void* b : all) (void)hipFree(b);
+            e = hipMalloc(&ptr, want);
+        }
+        if (e != hipSuccess) {
+            ptr = nullptr;
+            fail(BPX_ERR_OUT_OF_MEMORY, "hipMalloc(" + std::to_string(n) + " bytes) failed: " +
+                                            hipGetErrorString(e));
+        }
+        cap = want;
     }
     bytes = n;
 }
 void DeviceBuffer::release() {
-    if (ptr) (void)hipFree(ptr);
+    if (ptr) {
+        bool kept = false;
+        std::vector<void*> drop;
+        if (cap <= kPooledBytes / 2 && device >= 0 && current_device() == device && hipDeviceSynchronize() == hipSuccess) {
+            try {
+                Pool& p = pool();
+                std::lock_guard<std::mutex> lock(p.mutex);
+                drop = evict(p, kPooledBytes - cap);
+                p.blocks.push_back({ptr, cap, device, p.ticks});
+                p.bytes += cap;
+                kept = true;
+            } catch (const std::bad_alloc&) {   // no host memory for the list: free it below
+            }
+        }
+        if (!kept) (void)hipFree(ptr);
+        for (void* d : drop) (void)hipFree(d);
+    }
     ptr = nullptr;
-    bytes = 0;
+    bytes = cap = 0;
+}
+
+hipStream_t take_stream() {
+    const int device = current_device();
+    {
+        Pool& p = pool();
+        std::lock_guard<std::mutex> lock(p.mutex);
+        for (size_t i = p.streams.size(); i-- > 0;)
+            if (p.streams[i].first == device) {
+                const hipStream_t s = p.streams[i].second;
+                p.streams.erase(p.streams.begin() + (ptrdiff_t)i);
+                return s;
+            }
+    }
+    hipStream_t s = nullptr;
+    hip_check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreate");
+    return s;
+}
+void give_stream(hipStream_t s) {
+    hipDevice_t device = -1;
+    if (hipStreamGetDevice(s, &device) == hipSuccess && hipStreamSynchronize(s) == hipSuccess) {
+        Pool& p = pool();
+        std::lock_guard<std::mutex> lock(p.mutex);
+        if (p.streams.size() < 8) {
+            try {
+                p.streams.emplace_back((int)device, s);
+                return;
+            } catch (const std::bad_alloc&) {
+            }
+        }
+    }
+    (void)hipStreamDestroy(s);
 }
 
 PlanImpl::~PlanImpl() {
@@ -34,7 +165,7 @@ PlanImpl::~PlanImpl() {
         if (e) (void)hipEventDestroy(e);
     if (done) (void)hipEventDestroy(done);
     if (ready) (void)hipEventDestroy(ready);
-    if (stream) (void)hipStreamDestroy(stream);
+    if (stream) give_stream(stream);
 }
 
 static uint32_t round_up(uint64_t x, uint32_t m) { return (uint32_t)((x + m - 1) / m * m); }
@@ -224,53 +355,165 @@ static std::vector<uint32_t> used_pairs(const CaptureIn& c, uint32_t flags) {
 }
 
 // ------------------------------------------------------------------ host -> device uploads
-// Large pageable host arrays go through two pinned staging buffers (allocated once per
-// process): host threads copy chunk k + 1 into one buffer while the DMA engine copies chunk k
-// from the other.  Measured on MI355X: pageable hipMemcpy ~30 GB/s, pinned ~57 GB/s, 4-thread
-// host copies into pinned memory ~60 GB/s.
+// Large pageable host arrays go through pinned chunks (allocated once per process): host threads
+// copy chunks in or out while the DMA engine works on others.  Measured on MI355X: pageable
+// hipMemcpy ~30 GB/s in and, into fresh pages, 4 to 9 GB/s out; pinned ~57 GB/s; 4 host threads
+// copy into pinned memory at ~60 GB/s, 8 write fresh pages at 16 (one: 3.6).
 namespace {
-constexpr size_t kStageChunk = 32u << 20;
-constexpr int kCopyThreads = 4;
-std::mutex g_upload_mutex;
-void* g_pinned[2] = {nullptr, nullptr};
-hipEvent_t g_pinned_ev[2] = {nullptr, nullptr};
+constexpr size_t kRingChunk = 2u << 20;
+constexpr size_t kRingBytes = 32u << 20;
+constexpr size_t kStagedDown = 16u << 20;   // from here on an array goes through the ring
+constexpr size_t kStagedUp = 64u << 20;
+std::mutex g_ring_mutex;
+char* g_ring = nullptr;
+hipEvent_t g_ring_ev[kRingBytes / kRingChunk] = {};
 
-void parallel_copy(void* dst, const void* src, size_t bytes) {
-    std::thread th[kCopyThreads - 1];
-    const size_t part = (bytes / kCopyThreads + 63) & ~size_t(63);
-    auto piece = [&](int t) {
-        const size_t a = std::min(bytes, part * (size_t)t), b = std::min(bytes, part * (size_t)(t + 1));
-        if (b > a) std::memcpy(static_cast<char*>(dst) + a, static_cast<const char*>(src) + a, b - a);
+void ensure_ring() {
+    if (!g_ring) {
+        void* p = nullptr;
+        hip_check(hipHostMalloc(&p, kRingBytes, hipHostMallocDefault), "hipHostMalloc");
+        g_ring = static_cast<char*>(p);
+    }
+    for (auto& e : g_ring_ev)
+        if (!e) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+}
+
+// f(chunk, offset, bytes) for every chunk of an array, on up to `most` threads that take the chunks
+// in turn; the first error any of them met.
+template <class F>
+hipError_t for_chunks(size_t bytes, uint32_t most, F&& f) {
+    const uint32_t chunks = (uint32_t)((bytes + kRingChunk - 1) / kRingChunk);
+    const uint32_t n = std::min({most, (chunks + 1u) / 2u, std::max(1u, std::thread::hardware_concurrency() / 2u)});
+    const int device = current_device();
+    std::atomic<uint32_t> next{0};
+    std::atomic<int> error{(int)hipSuccess};
+    auto work = [&](bool own) {
+        if (!own && device >= 0) (void)hipSetDevice(device);
+        for (;;) {
+            const uint32_t k = next.fetch_add(1);
+            if (k >= chunks || error.load() != (int)hipSuccess) break;
+            const size_t off = (size_t)k * kRingChunk;
+            const hipError_t e = f(k, off, std::min(kRingChunk, bytes - off));
+            if (e != hipSuccess) error.store((int)e);
+        }
     };
-    for (int t = 1; t < kCopyThreads; ++t) th[t - 1] = std::thread(piece, t);
-    piece(0);
+    std::vector<std::thread> th;
+    th.reserve(n);
+    try {
+        for (uint32_t t = 1; t < n; ++t) th.emplace_back(work, false);
+    } catch (const std::exception&) {   // no further thread to be had: those that started, and this one
+    }
+    work(true);
     for (auto& x : th) x.join();
+    return (hipError_t)error.load();
 }
 }  // namespace
 
 void upload_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
-    if (bytes < 2 * kStageChunk) {
+    if (bytes < kStagedUp) {
         hip_check(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice), "hipMemcpy(upload)");
         return;
     }
-    std::lock_guard<std::mutex> lock(g_upload_mutex);
-    for (int b = 0; b < 2; ++b) {
-        if (!g_pinned[b]) hip_check(hipHostMalloc(&g_pinned[b], kStageChunk, hipHostMallocDefault), "hipHostMalloc");
-        if (!g_pinned_ev[b]) hip_check(hipEventCreateWithFlags(&g_pinned_ev[b], hipEventDisableTiming), "hipEventCreate");
+    std::lock_guard<std::mutex> lock(g_ring_mutex);
+    ensure_ring();
+    // The ring in two halves: threads fill one while the other one's copies run.
+    constexpr size_t half = kRingBytes / 2;
+    hipError_t e = hipSuccess;
+    uint32_t round = 0;
+    for (size_t base = 0; base < bytes && e == hipSuccess; base += half, ++round) {
+        char* at = g_ring + (round & 1u) * half;
+        hipEvent_t ev = g_ring_ev[round & 1u];
+        if (round >= 2) e = hipEventSynchronize(ev);   // this half's previous copies are done
+        if (e == hipSuccess)
+            e = for_chunks(std::min(half, bytes - base), 4, [&](uint32_t, size_t off, size_t n) {
+                std::memcpy(at + off, static_cast<const char*>(src) + base + off, n);
+                return hipMemcpyAsync(static_cast<char*>(dst) + base + off, at + off, n, hipMemcpyHostToDevice, s);
+            });
+        if (e == hipSuccess) e = hipEventRecord(ev, s);
     }
-    size_t off = 0;
-    for (int k = 0; off < bytes; ++k, off += kStageChunk) {
-        const int b = k & 1;
-        const size_t n = std::min(kStageChunk, bytes - off);
-        hip_check(hipEventSynchronize(g_pinned_ev[b]), "hipEventSynchronize");   // its previous DMA is done
-        parallel_copy(g_pinned[b], static_cast<const char*>(src) + off, n);
-        hip_check(hipMemcpyAsync(static_cast<char*>(dst) + off, g_pinned[b], n, hipMemcpyHostToDevice, s),
-                  "hipMemcpyAsync(upload)");
-        hip_check(hipEventRecord(g_pinned_ev[b], s), "hipEventRecord");
+    const hipError_t done = hipStreamSynchronize(s);   // the ring may be reused as soon as this returns
+    hip_check(e, "upload");
+    hip_check(done, "hipStreamSynchronize");
+}
+
+void download_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
+    if (bytes < kStagedDown) {
+        hip_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s), "hipMemcpyAsync(download)");
+        hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
+        return;
     }
-    // the buffers may be reused as soon as this returns
-    hip_check(hipEventSynchronize(g_pinned_ev[0]), "hipEventSynchronize");
-    hip_check(hipEventSynchronize(g_pinned_ev[1]), "hipEventSynchronize");
+    hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");   // other transfers may use the ring meanwhile
+    std::lock_guard<std::mutex> lock(g_ring_mutex);
+    ensure_ring();
+    for (size_t base = 0; base < bytes; base += kRingBytes) {
+        const size_t part = std::min(bytes - base, kRingBytes);
+        const char* from = static_cast<const char*>(src) + base;
+        char* to = static_cast<char*>(dst) + base;
+        hipError_t e = hipSuccess;
+        for (size_t off = 0, b = 0; off < part && e == hipSuccess; off += kRingChunk, ++b) {
+            e = hipMemcpyAsync(g_ring + off, from + off, std::min(kRingChunk, part - off), hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess) e = hipEventRecord(g_ring_ev[b], s);
+        }
+        if (e == hipSuccess)
+            e = for_chunks(part, 8, [&](uint32_t k, size_t off, size_t n) {
+                const hipError_t w = hipEventSynchronize(g_ring_ev[k]);
+                if (w == hipSuccess) std::memcpy(to + off, g_ring + off, n);
+                return w;
+            });
+        const hipError_t done = hipStreamSynchronize(s);
+        hip_check(e, "download");
+        hip_check(done, "hipStreamSynchronize");
+    }
+}
+
+namespace {
+constexpr size_t kSlabBytes = 1u << 20;
+}
+void TableUploads::add(void* dst, const void* src, size_t bytes) {
+    if (bytes == 0) return;
+    if (bytes > kSlabBytes) {
+        hip_check(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice), "hipMemcpy(table)");
+        return;
+    }
+    if (!slab) {
+        Pool& p = pool();
+        std::lock_guard<std::mutex> lock(p.mutex);
+        if (!p.slabs.empty()) {
+            slab = p.slabs.back();
+            p.slabs.pop_back();
+        }
+    }
+    if (!slab) {
+        void* m = nullptr;
+        hip_check(hipHostMalloc(&m, kSlabBytes, hipHostMallocDefault), "hipHostMalloc");
+        slab = static_cast<char*>(m);
+    }
+    if (used + bytes > kSlabBytes) {
+        hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+        used = 0;
+    }
+    std::memcpy(slab + used, src, bytes);
+    hip_check(hipMemcpyAsync(dst, slab + used, bytes, hipMemcpyHostToDevice, stream), "hipMemcpyAsync(table)");
+    used += (bytes + 255u) & ~(size_t)255u;
+}
+void TableUploads::finish() {
+    const hipError_t e = hipStreamSynchronize(stream);
+    open = false;
+    hip_check(e, "hipStreamSynchronize");
+}
+TableUploads::~TableUploads() {
+    if (open) (void)hipStreamSynchronize(stream);   // left by an exception
+    if (!slab) return;
+    try {
+        Pool& p = pool();
+        std::lock_guard<std::mutex> lock(p.mutex);
+        if (p.slabs.size() < 4) {
+            p.slabs.push_back(slab);
+            return;
+        }
+    } catch (const std::bad_alloc&) {
+    }
+    (void)hipHostFree(slab);
 }
 
 // Stages the raw rows of the used pairs on the device (compacting when pairs were dropped).
@@ -280,8 +523,7 @@ static void adopt_device_rows(PlanImpl& pl, DeviceBuffer& rows, uint32_t rows_in
                               const std::vector<uint32_t>& idx) {
     if (idx.size() == rows_in && rows_in) {
         pl.raw.release();
-        std::swap(pl.raw.ptr, rows.ptr);
-        std::swap(pl.raw.bytes, rows.bytes);
+        pl.raw.swap(rows);
         return;
     }
     pl.raw.alloc(sizeof(float) * row * std::max<size_t>(idx.size(), 1));
@@ -461,7 +703,7 @@ PlanImpl* make_plan_single_tap(const CaptureIn& c, const uint32_t n[3], const fl
     if (o.variant >= variant_count()) fail(BPX_ERR_INVALID_ARGUMENT, "unknown kernel variant");
 
     auto pl = std::make_unique<PlanImpl>();
-    hip_check(hipStreamCreateWithFlags(&pl->stream, hipStreamNonBlocking), "hipStreamCreate");
+    pl->stream = take_stream();
     make_events(*pl);
     pl->cplx = c.cplx;
     pl->format = c.cplx ? (o.storage == BPX_STORAGE_F16 ? kCF16 : o.storage == BPX_STORAGE_BF16 ? kCBF16 : kC64)
@@ -521,13 +763,13 @@ PlanImpl* make_plan_single_tap(const CaptureIn& c, const uint32_t n[3], const fl
     if (!pl->paths.seg) pl->H.alloc(hbytes);
     else if (pl->format != kF32) pl->H.alloc((size_t)pl->P * c.T * 4u);
     // fused rows staged over per-pair windows keep zeros outside them (written here only)
-    if (pl->fused) hip_check(hipMemset(pl->H.ptr, 0, hbytes), "hipMemset(fused rows)");
+    if (pl->fused) hip_check(hipMemsetAsync(pl->H.ptr, 0, hbytes, pl->stream), "hipMemsetAsync(fused rows)");
+    TableUploads tables(pl->stream);
 
     std::vector<float> p8((size_t)pl->P * 8);
     std::memcpy(p8.data(), pr.data(), sizeof(float) * p8.size());
     pl->pair8.alloc(sizeof(float) * p8.size());
-    hip_check(hipMemcpy(pl->pair8.ptr, p8.data(), sizeof(float) * p8.size(), hipMemcpyHostToDevice),
-              "hipMemcpy(pairs)");
+    tables.add(pl->pair8.ptr, p8.data(), sizeof(float) * p8.size());
 
     if (pl->path == kPathConfocal) {
         pl->Z.alloc(sizeof(float) * ((size_t)c.T + 1));
@@ -539,15 +781,11 @@ PlanImpl* make_plan_single_tap(const CaptureIn& c, const uint32_t n[3], const fl
         } else {
             pl->win_host = row_windows(pr, corners, c.t0, c.dT, c.T, pl->ldh);
             pl->win.alloc(sizeof(uint32_t) * pl->win_host.size());
-            hip_check(hipMemcpy(pl->win.ptr, pl->win_host.data(), sizeof(uint32_t) * pl->win_host.size(),
-                                hipMemcpyHostToDevice),
-                      "hipMemcpy(row windows)");
+            tables.add(pl->win.ptr, pl->win_host.data(), sizeof(uint32_t) * pl->win_host.size());
             const StageJob job = stage_job(*pl);
             pl->stage_zb = stage_z_blocks(job);
             pl->stage_sb = stage_row_blocks(job);
-            pl->stage.alloc(sizeof(StageJob));
-            hip_check(hipMemcpy(pl->stage.ptr, &job, sizeof(StageJob), hipMemcpyHostToDevice),
-                      "hipMemcpy(staging job)");
+            pl->stage.alloc(sizeof(StageJob));   // written by set_fused_variant
         }
         pl->inv2 = (float)(2.0 / (double)c.dT);
         std::vector<float> p4((size_t)pl->P * 4);
@@ -591,8 +829,7 @@ PlanImpl* make_plan_single_tap(const CaptureIn& c, const uint32_t n[3], const fl
             pl->rows16 = false;
         }
         pl->pair4.alloc(sizeof(float) * p4.size());
-        hip_check(hipMemcpy(pl->pair4.ptr, p4.data(), sizeof(float) * p4.size(), hipMemcpyHostToDevice),
-                  "hipMemcpy(pair table)");
+        tables.add(pl->pair4.ptr, p4.data(), sizeof(float) * p4.size());
     } else {
         if ((uint64_t)(c.T + 1) * 4 > 64 * 1024)
             fail(BPX_ERR_UNSUPPORTED, "non-confocal captures need T <= 16383 after cropping");
@@ -616,12 +853,11 @@ PlanImpl* make_plan_single_tap(const CaptureIn& c, const uint32_t n[3], const fl
             }
             pl->lasers.alloc(sizeof(float) * las.size());
             pl->spads.alloc(sizeof(float) * spd.size());
-            hip_check(hipMemcpy(pl->lasers.ptr, las.data(), sizeof(float) * las.size(), hipMemcpyHostToDevice),
-                      "hipMemcpy(lasers)");
-            hip_check(hipMemcpy(pl->spads.ptr, spd.data(), sizeof(float) * spd.size(), hipMemcpyHostToDevice),
-                      "hipMemcpy(spads)");
+            tables.add(pl->lasers.ptr, las.data(), sizeof(float) * las.size());
+            tables.add(pl->spads.ptr, spd.data(), sizeof(float) * spd.size());
         }
     }
+    tables.finish();
     return pl.release();
 }
 
@@ -684,7 +920,8 @@ void set_fused_variant(PlanImpl& pl, int variant) {
     }
     if ((pl.rows16 || pl.poly.kz) && !pl.fmt_flag.ptr) {
         pl.fmt_flag.alloc(4);
-        hip_check(hipMemset(pl.fmt_flag.ptr, 0xff, 4), "hipMemset(row format)");   // fp32 until run
+        // fp32 until run
+        hip_check(hipMemsetAsync(pl.fmt_flag.ptr, 0xff, 4, pl.stream), "hipMemsetAsync(row format)");
     }
     if (pl.stage.ptr) {   // the staging descriptor names the format flag (or none)
         const StageJob job = stage_job(pl);
@@ -945,7 +1182,7 @@ PlanImpl* make_plan_window(const CaptureIn& c, const uint32_t n[3], const float 
             fail(BPX_ERR_INVALID_ARGUMENT, "volume position/size must be finite");
     if (!device_ready()) fail(BPX_ERR_NO_DEVICE, "no gfx950 device available");
     auto pl = std::make_unique<PlanImpl>();
-    hip_check(hipStreamCreateWithFlags(&pl->stream, hipStreamNonBlocking), "hipStreamCreate");
+    pl->stream = take_stream();
     make_events(*pl);
     pl->path = kPathWindow;
     pl->cplx = c.cplx;
