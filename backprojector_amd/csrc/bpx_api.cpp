@@ -310,8 +310,9 @@ bpx_status bpx_plan_read_thresholds(bpx_plan plan, float* out, uint64_t capacity
         plan_wait(pl);
         const DeviceBuffer& src = pl.fused ? pl.H : pl.S;
         const int fmt = staged_format(pl);
-        const size_t stride = pl.fused ? (size_t)fused_elem_bytes(fmt) / 4 : 1;
-        const size_t pitch = pl.fused ? (size_t)pl.ldh * stride : pl.lds;
+        const bool apart = format_split(fmt);   // a row's thresholds first, then its samples
+        const size_t stride = pl.fused && !apart ? (size_t)fused_elem_bytes(fmt) / 4 : 1;
+        const size_t pitch = !pl.fused ? pl.lds : apart ? (size_t)pl.ldh * (fmt == kC64Split ? 3 : 2) : (size_t)pl.ldh * stride;
         const size_t off = pl.fused ? (size_t)fused_s_offset(fmt) : 0;
         std::vector<float> host(src.bytes / 4);
         hip_check(hipMemcpy(host.data(), src.ptr, host.size() * 4, hipMemcpyDeviceToHost), "hipMemcpy(thresholds)");
@@ -363,10 +364,12 @@ bpx_status bpx_plan_kernel_name(bpx_plan plan, char* out, uint64_t capacity) {
         if (!plan || !out || capacity == 0) fail(BPX_ERR_INVALID_ARGUMENT, "NULL argument");
         const PlanImpl& pl = *plan->impl;
         std::string name;
-        if (pl.poly.kz && staged_format(pl) == kCount) {
-            name = "confocal_lds_kernel_poly<KZ=" + std::to_string(pl.poly.kz) + ", degree=" +
-                   std::to_string(pl.poly.deg) + "> (16x16x" + std::to_string(pl.poly.kz) + " tiles, " +
-                   std::to_string(pl.poly_parts) + (pl.poly_parts > 1 ? " pair parts)" : " pair part)");
+        const bool counts = pl.poly_counts && staged_format(pl) == kCount;
+        if (counts || pl.poly_real) {
+            const uint32_t parts = counts ? pl.poly_parts : pl.real_parts;
+            name = (counts ? "confocal_lds_kernel_poly<KZ=" : "confocal_lds_kernel<KZ=") + std::to_string(pl.poly.kz) +
+                   ", degree=" + std::to_string(pl.poly.deg) + "> (16x16x" + std::to_string(pl.poly.kz) + " tiles, " +
+                   std::to_string(parts) + (parts > 1 ? " pair parts)" : " pair part)");
         } else if (pl.paths.seg) {
             name = std::string("paths_lds_kernel<") + (pl.paths.L ? "grid" : "pairs") + "> (16x16x8 tiles, " +
                    std::to_string(pl.paths_parts) + (pl.paths_parts > 1 ? " parts)" : " part)");
@@ -431,11 +434,21 @@ bpx_status bpx_plan_tune(bpx_plan plan, int32_t reps, int32_t* variant) {
             int best = initial;
             float best_ms = INFINITY;
             try {
-                pl.auto_variant = false;   // each variant as asked for
-                for (int v = 3; v < variant_count(); ++v) {
-                    set_fused_variant(pl, v);
-                    if (v >= kLdsVariant && !pl.lds_tiles && !pl.poly.kz) continue;   // a texture-path shape
+                // the plan as it is (its default kernel, which no variant names), then each variant
+                const bool own = initial_auto && pl.poly_real;
+                bool keep = own;
+                for (int v = own ? 2 : 3; v < variant_count(); ++v) {
+                    if (v > 2) {
+                        pl.auto_variant = false;
+                        set_fused_variant(pl, v);
+                        if (v >= kLdsVariant && !pl.lds_tiles && !pl.poly_counts) continue;   // a texture-path shape
+                    }
                     pl.execute(pl.stream);                             // warm-up
+                    // count rows: the kernel is variant 7's and 8's too
+                    if (v == 2 && staged_format(pl) == kCount) {
+                        keep = false;
+                        continue;
+                    }
                     if (v >= kLdsVariant && !pl.lds_tiles && staged_format(pl) != kCount) continue;
                     hip_check(hipEventRecord(t0, pl.stream), "hipEventRecord");
                     for (int r = 0; r < reps; ++r) pl.execute(pl.stream);
@@ -445,9 +458,11 @@ bpx_status bpx_plan_tune(bpx_plan plan, int32_t reps, int32_t* variant) {
                     hip_check(hipEventElapsedTime(&ms, t0, t1), "hipEventElapsedTime");
                     if (ms < best_ms) {
                         best_ms = ms;
-                        best = v;
+                        keep = v == 2;
+                        best = keep ? initial : v;
                     }
                 }
+                pl.auto_variant = keep;
                 set_fused_variant(pl, best);
             } catch (...) {
                 (void)hipEventDestroy(t0);

@@ -1,5 +1,12 @@
-// Batched uneven confocal captures: one device-resident plan per capture and one persistent
-// launch over a single work queue of staging items (fused rows and thresholds), LDS-staged
+// Batched uneven confocal captures, one device-resident plan per capture.
+//
+// Captures that the polynomial-quotient kernel takes (flat wall, columns along its normal; the
+// plans' rule) are gathered by it, as a plan of their own gathers them: their rows are staged
+// first (counts where a capture's samples all are), then one launch per depth and window class
+// covers the (capture, part of the pairs, tile) items of all of them.  Every item is computed
+// alike whatever the configuration below.
+//
+// The others: one persistent launch over a single work queue of staging items (fused rows and thresholds), LDS-staged
 // tiles (captures whose bin windows fit the LDS segment) and texture-path tiles (the rest),
 // after a prologue launch that builds every capture's path-length table and resets the queue.
 // The queue holds every staging item first and then the gather items; a capture's gathers wait
@@ -28,7 +35,25 @@ struct BatchImpl {
     hipEvent_t done = nullptr, ready = nullptr;   // as PlanImpl::done / ready
     DeviceBuffer caps, flags, items, items_tex, items_wide, jobs, init, next, staged, remaining, error;
     DeviceBuffer stamps;   // uint64 [1 + captures]: batch start, then each capture's completion
-    DeviceBuffer zjobs;    // StageJob per capture with pairs (path-length tables, prologue)
+    DeviceBuffer zjobs;    // StageJob per capture with pairs, those of poly_caps first (prologue)
+    // the captures of the polynomial-quotient kernel (shape kz != 0)
+    struct PolyCapture {
+        LdsPolyShape shape;
+        uint32_t parts = 1, part_pairs = 0;
+        bool counts = false;
+        size_t parts_offset = 0;   // bytes in poly_parts
+    };
+    struct PolyGroup {             // one launch per row format
+        LdsPolyShape shape;
+        uint32_t first = 0, n = 0;
+        bool counts = false;       // some capture of it may hold counts
+    };
+    std::vector<PolyCapture> poly;
+    std::vector<PolyGroup> poly_groups;
+    uint32_t n_poly = 0, poly_row_blocks = 0;
+    int poly_format = kF32Split;
+    DeviceBuffer poly_args, poly_items, poly_left, poly_first, poly_parts, fmt_flags;
+    bool foreign = false;          // executed on a caller's stream (`done` says when it ends)
     uint32_t n_zjobs = 0, z_blocks = 0, row_blocks = 0;
     uint32_t n_items = 0, n_tex_items = 0, n_wide_items = 0;
     uint32_t tex_groups = 0, wide_groups = 0;
@@ -58,17 +83,84 @@ struct BatchImpl {
         if (side2) (void)hipStreamDestroy(side2);
         if (stream) (void)hipStreamDestroy(stream);
     }
+    void choose_poly();
     void build(const bpx_batch_config& c);
     // Waits for the batch's own stream and for its last execution on a caller's stream, then
     // checks the queue's error word.
     void wait() const {
         hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
-        hip_check(hipEventSynchronize(done), "hipEventSynchronize");
+        if (foreign) hip_check(hipEventSynchronize(done), "hipEventSynchronize");
         uint32_t e = 0;
         hip_check(hipMemcpy(&e, error.ptr, 4, hipMemcpyDeviceToHost), "hipMemcpy(error word)");
         if (e) fail(BPX_ERR_DEVICE, "batch queue: a capture's staging did not finish in time");
     }
 };
+
+// Shapes, parts and items of the polynomial-quotient kernel: they depend on the captures alone.
+// Parts as a plan of its own has them, so that the sums are the plan's.
+void BatchImpl::choose_poly() {
+    const uint32_t n = (uint32_t)plans.size();
+    poly.assign(std::max<uint32_t>(n, 1u), PolyCapture{});
+    fmt_flags.alloc(4u * std::max<uint32_t>(n, 1u));
+    if (format == kCF16 || format == kCBF16) return;
+    poly_format = format == kC64 ? (int)kC64Split : format == kF32 ? (int)kF32Split : format;
+    const uint32_t bytes = lds_poly_part_bytes(poly_format);
+    size_t total = 0, tiles = 0;
+    std::vector<uint32_t> left, first(std::max<uint32_t>(n, 1u), 0u);
+    for (uint32_t i = 0; i < n; ++i) {
+        const PlanImpl& pl = *plans[i];
+        PolyCapture& pc = poly[i];
+        if (!pl.P || !pl.sep || !pl.flat) continue;
+        pc.shape = lds_poly_shape(pl.g, pl.inv2, pl.lz, pl.tap_bound, pl.max_path, kPolyBudget, poly_format);
+        if (!pc.shape.kz) continue;
+        ++n_poly;
+        pc.counts = format == kF32 && pl.kahan_block <= 4096u && pl.P <= (1u << 20);
+        pc.parts = lds_poly_parts(pl.g, pc.shape, pl.P, bytes, &pc.part_pairs);
+        const uint64_t t = lds_tile_count(pl.g, pc.shape);
+        if (t * pc.parts >= (1ull << 31)) fail(BPX_ERR_UNSUPPORTED, "batch capture too large");
+        pc.parts_offset = total;
+        if (pc.parts > 1)
+            total += ((size_t)pc.parts * pl.g.n[0] * pl.g.n[1] * pl.g.n[2] * bytes + 255u) / 256u * 256u;
+        first[i] = (uint32_t)tiles;
+        tiles += t;
+        left.insert(left.end(), t, pc.parts);
+    }
+    if (!n_poly) return;
+    if (tiles >= (1ull << 31)) fail(BPX_ERR_UNSUPPORTED, "batch too large");
+    poly_parts.alloc(total);
+    poly_left.alloc(4u * tiles);
+    poly_first.alloc(4u * first.size());
+    hip_check(hipMemcpy(poly_left.ptr, left.data(), 4u * tiles, hipMemcpyHostToDevice), "hipMemcpy");
+    hip_check(hipMemcpy(poly_first.ptr, first.data(), 4u * first.size(), hipMemcpyHostToDevice), "hipMemcpy");
+    // a launch per depth and window class (LDS decides how many work-groups a CU holds), its items
+    // by falling length: the short ones fill the end
+    std::vector<uint32_t> order(n);
+    std::iota(order.begin(), order.end(), 0u);
+    std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return poly[x].part_pairs > poly[y].part_pairs; });
+    std::vector<uint32_t> items;
+    for (int kz : {16, 8})
+        for (uint32_t most : {256u, 512u, kPolySegMax}) {
+            PolyGroup g;
+            g.first = (uint32_t)(items.size() / 2u);
+            for (uint32_t i : order) {
+                const LdsPolyShape& sh = poly[i].shape;
+                if (sh.kz != kz || sh.seg > most || (most > 256u && sh.seg <= most / 2u)) continue;
+                g.shape.kz = kz;
+                g.shape.deg = std::max(g.shape.deg, sh.deg);
+                g.shape.seg = std::max(g.shape.seg, sh.seg);
+                g.counts = g.counts || poly[i].counts;
+                const uint32_t blocks = (uint32_t)lds_tile_count(plans[i]->g, sh) * poly[i].parts;
+                for (uint32_t k = 0; k < blocks; ++k) {
+                    items.push_back(i);
+                    items.push_back(k);
+                }
+            }
+            g.n = (uint32_t)(items.size() / 2u) - g.first;
+            if (g.n) poly_groups.push_back(g);
+        }
+    poly_items.alloc(4u * items.size());
+    hip_check(hipMemcpy(poly_items.ptr, items.data(), 4u * items.size(), hipMemcpyHostToDevice), "hipMemcpy");
+}
 
 void BatchImpl::build(const bpx_batch_config& c) {
     if (c.lane_voxels != 2u && c.lane_voxels != 4u) fail(BPX_ERR_INVALID_ARGUMENT, "lane_voxels must be 2 or 4");
@@ -88,6 +180,7 @@ void BatchImpl::build(const bpx_batch_config& c) {
     std::vector<StageJob> sj(std::max<uint32_t>(n, 1));
     std::vector<uint32_t> fl(n), nt(n), ns(n);
     std::vector<char> lds(n, 0), wide(n, 0);
+    std::vector<LdsPolyArgs> pargs(std::max<uint32_t>(n, 1u));
     for (uint32_t i = 0; i < n; ++i) {
         const PlanImpl& pl = *plans[i];
         ConfocalArgs& a = args[i];
@@ -115,7 +208,20 @@ void BatchImpl::build(const bpx_batch_config& c) {
                 : wide[i] ? batch_lds_tiles(pl.g, 16)
                 : lds[i]  ? batch_lds_tiles(pl.g, kz)
                           : (two ? 4u : 1u) * a.t.count;
-        if (pl.P) {
+        if (poly[i].shape.kz) {
+            const PolyCapture& pc = poly[i];
+            uint32_t* const flag = static_cast<uint32_t*>(fmt_flags.ptr) + i;
+            sj[i] = stage_job(pl);
+            sj[i].format = sj[i].alt_format = poly_format;
+            if (pc.counts) {
+                sj[i].fmt_flag = flag;
+                sj[i].count_rows = 1;
+            }
+            pargs[i] = lds_poly_args(a, pc.shape);
+            pargs[i].part_pairs = pc.part_pairs;
+            pargs[i].parts = pc.parts > 1 ? static_cast<char*>(poly_parts.ptr) + pc.parts_offset : nullptr;
+            nt[i] = (uint32_t)lds_tile_count(pl.g, pc.shape);
+        } else if (pl.P) {
             sj[i] = stage_job(pl);
             ns[i] = two ? 0u : (stage_row_blocks(sj[i]) + kBatchStageBlocks - 1u) / kBatchStageBlocks;
         }
@@ -136,6 +242,7 @@ void BatchImpl::build(const bpx_batch_config& c) {
         }
     };
     auto push_gather = [&](uint32_t i) {
+        if (poly[i].shape.kz) return;
         const uint32_t type = lds[i] ? kBatchItemLds : kBatchItemTex;
         for (uint32_t t = 0; t < nt[i]; ++t) {
             it.push_back(i | (type << 28));
@@ -147,6 +254,7 @@ void BatchImpl::build(const bpx_batch_config& c) {
         std::vector<uint32_t> a, b;   // LDS-staged and texture-path gather items, capture order
         for (uint32_t k = 0; k < n; ++k) {
             const uint32_t i = order[k];
+            if (poly[i].shape.kz) continue;
             std::vector<uint32_t>& q = lds[i] ? a : b;
             const uint32_t type = lds[i] ? kBatchItemLds : kBatchItemTex;
             for (uint32_t t = 0; t < nt[i]; ++t) {
@@ -187,8 +295,15 @@ void BatchImpl::build(const bpx_batch_config& c) {
     // path-length tables of every capture in the prologue: each job's blocks follow the previous one's
     std::vector<StageJob> zj;
     uint64_t zb = 0, rb = 0;
-    for (uint32_t i = 0; i < n; ++i) {
-        if (!plans[i]->P) continue;
+    std::vector<uint32_t> by_kernel;
+    for (const bool first : {true, false})
+        for (uint32_t i = 0; i < n; ++i)
+            if (plans[i]->P && (poly[i].shape.kz != 0) == first) by_kernel.push_back(i);
+    for (uint32_t i : by_kernel) {
+        if (zj.size() == n_poly) {   // the others' row blocks are numbered by themselves
+            poly_row_blocks = (uint32_t)rb;
+            rb = 0;
+        }
         StageJob j = sj[i];
         j.z_first = (uint32_t)zb;
         j.s_first = (uint32_t)rb;
@@ -198,6 +313,10 @@ void BatchImpl::build(const bpx_batch_config& c) {
     }
     if (zb >= (1ull << 31) || rb >= (1ull << 31)) fail(BPX_ERR_UNSUPPORTED, "batch staging too large");
     n_zjobs = (uint32_t)zj.size();
+    if (n_zjobs == n_poly) {
+        poly_row_blocks = (uint32_t)rb;
+        rb = 0;
+    }
     z_blocks = (uint32_t)zb;
     row_blocks = (uint32_t)rb;
     std::vector<uint32_t> in(2 * std::max<uint32_t>(n, 1), 0u);
@@ -213,6 +332,22 @@ void BatchImpl::build(const bpx_batch_config& c) {
     items.alloc(8u * std::max<uint32_t>(n_items, 1));
     items_tex.alloc(8u * std::max<uint32_t>(n_tex_items, 1));
     items_wide.alloc(8u * std::max<uint32_t>(n_wide_items, 1));
+    // per row format (counts, the batch's own): the same arguments, other samples wanted
+    std::vector<LdsPolyArgs> pa(2u * pargs.size());
+    for (size_t i = 0; i < pargs.size(); ++i) {
+        ConfocalArgs &counts = pa[i].c, &own = pa[pargs.size() + i].c;
+        pa[i] = pa[pargs.size() + i] = pargs[i];
+        counts.fmt_flag = static_cast<const uint32_t*>(fmt_flags.ptr) + i;
+        if (poly[i].counts) {
+            own.fmt_flag = counts.fmt_flag;
+            counts.fmt_mask = 2u;      // all counts
+            own.fmt_mask = own.fmt_want = 2u;
+        } else {
+            counts.fmt_want = 1u;      // never
+        }
+    }
+    poly_args.alloc(sizeof(LdsPolyArgs) * pa.size());
+    hip_check(hipMemcpy(poly_args.ptr, pa.data(), sizeof(LdsPolyArgs) * pa.size(), hipMemcpyHostToDevice), "hipMemcpy");
     if (n_zjobs)
         hip_check(hipMemcpy(zjobs.ptr, zj.data(), sizeof(StageJob) * n_zjobs, hipMemcpyHostToDevice), "hipMemcpy");
     hip_check(hipMemcpy(jobs.ptr, sj.data(), sizeof(StageJob) * sj.size(), hipMemcpyHostToDevice), "hipMemcpy");
@@ -283,12 +418,33 @@ void BatchImpl::build(const bpx_batch_config& c) {
                       "fill kernel");
         }
         hip_check(launch_batch_prologue(static_cast<const StageJob*>(zjobs.ptr), n_zjobs, z_blocks, q,
-                                        static_cast<const uint32_t*>(init.ptr), n,
+                                        static_cast<const uint32_t*>(init.ptr), n, static_cast<uint32_t*>(fmt_flags.ptr),
                                         static_cast<uint64_t*>(stamps.ptr), stream),
                   "batch prologue kernel");
+        if (n_poly) {
+            if (format == kF32)
+                hip_check(launch_batch_exact16(static_cast<const StageJob*>(zjobs.ptr), n_poly, stream),
+                          "batch sample check kernel");
+            hip_check(launch_stage(static_cast<const StageJob*>(zjobs.ptr), n_poly, 0u, poly_row_blocks, stream),
+                      "batch row staging kernel");
+            BatchPolyArgs pb{};
+            pb.first_tile = static_cast<const uint32_t*>(poly_first.ptr);
+            pb.left = static_cast<uint32_t*>(poly_left.ptr);
+            pb.remaining = static_cast<uint32_t*>(remaining.ptr);
+            pb.done = q.done;
+            for (const bool counts : {true, false})
+                for (const PolyGroup& g : poly_groups) {
+                    if (counts && !g.counts) continue;
+                    pb.caps = static_cast<const LdsPolyArgs*>(poly_args.ptr) + (counts ? 0u : pargs.size());
+                    pb.items = static_cast<const uint2*>(poly_items.ptr) + g.first;
+                    hip_check(launch_batch_poly(pb, g.shape, counts ? (int)kCount : poly_format, g.n, stream),
+                              "batch gather kernel (polynomial quotients)");
+                }
+        }
         if (two) {
             // every row staged first (no waits in either queue), then both queues side by side
-            hip_check(launch_stage(static_cast<const StageJob*>(zjobs.ptr), n_zjobs, 0u, row_blocks, stream),
+            hip_check(launch_stage(static_cast<const StageJob*>(zjobs.ptr) + n_poly, n_zjobs - n_poly, 0u, row_blocks,
+                                   stream),
                       "batch row staging kernel");
             // every queue with items on its own stream: the 16 x 16 x kz one on the graph's
             // stream, the texture-path one on `side`, the 16^3 one on `side2`
@@ -423,6 +579,7 @@ bpx_status bpx_batch_create(const bpx_capture_desc* captures, uint32_t count, co
         b->staged.alloc(4u * n);
         b->remaining.alloc(4u * n);
         b->stamps.alloc(8u * (n + 1u));
+        b->choose_poly();
         b->build(bpx_batch_config{2u, 0u, 0u, 0u, 8u, 1u});
         auto h = std::make_unique<bpx_batch_s>();
         h->impl = std::move(b);
@@ -460,9 +617,12 @@ bpx_status bpx_batch_tune(bpx_batch batch, int32_t reps, bpx_batch_config* chose
         reps = std::max(reps, 1);
         bpx_batch_config best{2u, 0u, 0u, 0u, 8u, 1u};
         double best_ms = INFINITY;
+        // the configuration is that of the queues: without items it changes nothing
+        const bool queued = b.n_items || b.n_tex_items || b.n_wide_items;
         for (uint32_t launches : {1u, 2u, 3u})
             for (uint32_t k : {2u, 4u})
                 for (uint32_t kz : {8u, 16u}) {
+                    if (!queued) continue;
                     if (kz == 16u && format_complex(b.format)) continue;   // complex formats: depth 8
                     if (launches == 3u && (kz == 16u || format_complex(b.format))) continue;   // both depths
                     const int resident = batch_queue_resident_groups((int)k, (int)kz, b.format, (int)launches);
@@ -494,9 +654,10 @@ bpx_status bpx_batch_execute(bpx_batch batch, void* hip_stream) {
             hip_check(hipEventRecord(b.ready, b.stream), "hipEventRecord");
             hip_check(hipStreamWaitEvent(s, b.ready, 0), "hipStreamWaitEvent");
         }
-        hip_check(hipStreamWaitEvent(s, b.done, 0), "hipStreamWaitEvent");
+        if (b.foreign) hip_check(hipStreamWaitEvent(s, b.done, 0), "hipStreamWaitEvent");
+        b.foreign = b.foreign || s != b.stream;
         hip_check(hipGraphLaunch(b.exec, s), "hipGraphLaunch");
-        hip_check(hipEventRecord(b.done, s), "hipEventRecord");
+        if (b.foreign) hip_check(hipEventRecord(b.done, s), "hipEventRecord");
     });
 }
 

@@ -411,6 +411,19 @@ __device__ __forceinline__ float2 kahan_result(float2 sum, float2 comp) {
     return make_float2(sum.x - comp.x, sum.y - comp.y);
 }
 
+// A struct every lane reads from the same address, moved word by word into scalar registers:
+// the buffer descriptors built from it are then wave-uniform (no per-pair waterfall loops).
+template <class T>
+__device__ __forceinline__ T wave_uniform_load(const T* p) {
+    static_assert(sizeof(T) % 4 == 0, "word-sized struct");
+    T out;
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(p);
+    uint32_t* dst = reinterpret_cast<uint32_t*>(&out);
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(T) / 4); ++i) dst[i] = __builtin_amdgcn_readfirstlane(src[i]);
+    return out;
+}
+
 // Work-group index remap so that consecutive tiles land on the same XCD (dispatch places
 // work-group i on XCD i mod 8): neighbouring voxel tiles read the same transient-row
 // segments and share that XCD's L2.

@@ -135,12 +135,16 @@ struct PlanImpl {
     // integer of magnitude <= 2048; fmt_flag (one word) = 0 then, 1 otherwise
     bool rows16 = false;
     bool keep_f32 = false;               // BPX_FLAG_KEEP_F32_ROWS: rows16 never applies
-    // rows of counts (integers 0 .. 2048) gathered with integer sums by the polynomial-quotient
-    // kernel whenever every sample of the execution is one; poly.kz = 0: never
+    // the polynomial-quotient kernel, where it applies (poly.kz != 0): rows of counts (integers
+    // 0 .. 2048) with integer sums whenever every sample of the execution is one, and the other rows
     LdsPolyShape poly;
+    bool poly_counts = false;            // poly takes count rows
+    bool poly_real = false;              // poly takes the plan's own format (and exact fp16 rows)
+    int row_format = kF32;               // of the fused rows (but for count and exact fp16 rows)
     bool auto_variant = false;           // the variant was not asked for: poly applies whatever it is
-    uint32_t poly_parts = 1, poly_part_pairs = 0;
-    DeviceBuffer parts;                  // integer partial sums [poly_parts][voxels] when split
+    uint32_t poly_parts = 1, poly_part_pairs = 0;   // of count rows (and of the window path)
+    uint32_t real_parts = 1, real_part_pairs = 0;   // of the others
+    DeviceBuffer parts;                  // partial sums [parts][voxels] when split
     double tap_bound = 0, max_path = 0;  // of the approximate quotient; longest total path
     DeviceBuffer fmt_flag;
     float lz = 0;

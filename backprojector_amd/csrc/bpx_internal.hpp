@@ -11,13 +11,16 @@ enum SampleFormat : int {
     kF32 = 0, kF16 = 1, kBF16 = 2,     // real
     kC64 = 3, kCF16 = 4, kCBF16 = 5,   // complex (interleaved re, im)
     kCount = 6,                        // real integers 0 .. 2048 as 16-bit integers (fused rows only)
+    // a row's thresholds before its samples (fused rows only)
+    kC64Split = 7, kF32Split = 8,
 };
-__host__ __device__ inline bool format_complex(int f) { return f >= kC64 && f <= kCBF16; }
+__host__ __device__ constexpr bool format_complex(int f) { return (f >= kC64 && f <= kCBF16) || f == kC64Split; }
+__host__ __device__ constexpr bool format_split(int f) { return f == kC64Split || f == kF32Split; }
 inline int format_bytes(int f) {
     switch (f) {
         case kF32: return 4;
         case kF16: case kBF16: case kCount: return 2;
-        case kC64: return 8;
+        case kC64: case kC64Split: return 8;
         default: return 4;
     }
 }
@@ -66,7 +69,7 @@ struct LdsPolyArgs {
     ConfocalArgs c;
     uint32_t seg;
     uint32_t part_pairs; // pairs per work-group (a multiple of 4; >= P when not split)
-    uint32_t* parts;     // [parts][voxels] integer partial sums, or nullptr: straight to c.out
+    void* parts;         // [parts][voxels] partial sums (lds_poly_part_bytes each), or nullptr: straight to c.out
     // the tiles of a list (its length on the device; partial sums [work-groups][256 kz]); nullptr:
     // every tile of the grid
     const uint32_t* tiles;
@@ -335,10 +338,25 @@ hipError_t launch_confocal(const ConfocalArgs& a, int format, int variant, bool 
 // bound = the host's bound on the approximate quotient's error, max_path = longest total path.
 constexpr uint32_t kPolySegMax = 1024;
 constexpr double kPolyBudget = 0.24, kWindowPolyBudget = 0.18;
-LdsPolyShape lds_poly_shape(const Grid& g, float inv2, float lz, double bound, double max_path, double budget);
+LdsPolyShape lds_poly_shape(const Grid& g, float inv2, float lz, double bound, double max_path, double budget,
+                            int format);
 uint32_t lds_poly_parts(const Grid& g, const LdsPolyShape& sh, uint32_t P, uint32_t sum_bytes, uint32_t* part_pairs);
 LdsPolyArgs lds_poly_args(const ConfocalArgs& c, const LdsPolyShape& sh);
-hipError_t launch_lds_counts(const LdsPolyArgs& a, const LdsPolyShape& sh, uint32_t parts, hipStream_t s);
+// Rows of kCount, kF16, kBF16, kF32Split or kC64Split; shapes of lds_poly_shape for that format.
+hipError_t launch_lds_poly(const LdsPolyArgs& a, const LdsPolyShape& sh, int format, uint32_t parts, hipStream_t s);
+uint32_t lds_poly_part_bytes(int format);
+// The same for n items of many captures (one kz, degree and LDS segment per launch).
+struct BatchPolyArgs {
+    const LdsPolyArgs* caps;      // per capture
+    const uint2* items;           // (capture, part x tiles of the capture + tile)
+    const uint32_t* first_tile;   // per capture, in left
+    uint32_t* left;               // parts per tile still to finish (as many as it has before and after a launch)
+    uint32_t* remaining;          // tiles per capture still to finish
+    uint64_t* done;               // completion stamp per capture
+};
+hipError_t launch_batch_poly(const BatchPolyArgs& b, const LdsPolyShape& sh, int format, uint32_t n, hipStream_t s);
+// Per job the flag word of launch_exact16_check (StageJob::fmt_flag, cleared by the caller).
+hipError_t launch_batch_exact16(const StageJob* jobs, uint32_t n_jobs, hipStream_t s);
 uint64_t lds_tile_count(const Grid& g, const LdsPolyShape& sh);
 hipError_t launch_tile_lists(const TileListArgs& a, const LdsPolyShape& sh, const uint32_t* const lists[2],
                              const uint32_t n[2], uint32_t dense, hipStream_t s);
@@ -369,7 +387,7 @@ int batch_wide_resident_groups(int format);
 hipError_t launch_batch_wide(const BatchQueueArgs& b, int format, uint32_t groups, hipStream_t s);
 hipError_t launch_batch_tex(const BatchQueueArgs& b, int K, int format, uint32_t groups, hipStream_t s);
 hipError_t launch_batch_prologue(const StageJob* jobs, uint32_t n_jobs, uint32_t z_blocks, const BatchQueueArgs& b,
-                                 const uint32_t* init, uint32_t n, uint64_t* start, hipStream_t s);
+                                 const uint32_t* init, uint32_t n, uint32_t* fmt_flags, uint64_t* start, hipStream_t s);
 bool batch_lds_applies(const Grid& g, float inv2, int format, bool sep, bool flat, int kz);
 uint32_t batch_lds_tiles(const Grid& g, int kz);
 hipError_t launch_window(const WindowArgs& a, int complex_samples, hipStream_t stream);

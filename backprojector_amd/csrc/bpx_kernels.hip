@@ -190,8 +190,8 @@ __device__ __forceinline__ float padded_sample(const float* row, uint32_t i, uin
 // formats), v[2] and v[3] (re and im of the next padded index for the 16-bit complex formats).
 template <int F>
 __device__ __forceinline__ void fused_samples(const float* row, uint32_t j, uint32_t Tc, float inv_scale, float v[4]) {
-    constexpr int cplx = (F == kC64 || F == kCF16 || F == kCBF16) ? 1 : 0;
-    constexpr bool two = F != kF32 && F != kC64;   // 16-bit layouts hold two padded indices
+    constexpr int cplx = format_complex(F) ? 1 : 0;
+    constexpr bool two = F != kF32 && F != kC64 && !format_split(F);   // 16-bit layouts hold two padded indices
     v[0] = padded_sample(row, j, Tc, inv_scale, 0, cplx);
     v[1] = cplx ? padded_sample(row, j, Tc, inv_scale, 1, 1) : two ? padded_sample(row, j + 1u, Tc, inv_scale, 0, 0) : 0.0f;
     v[2] = cplx && two ? padded_sample(row, j + 1u, Tc, inv_scale, 0, 1) : 0.0f;
@@ -249,7 +249,7 @@ __device__ __forceinline__ void stage_z_entry(const StageJob& jb, uint32_t j) {
 template <int F>
 __device__ __forceinline__ void stage_row_elements(const StageJob& jb, uint32_t p) {
     constexpr int kE = (int)(kStageSpan / 256u);
-    constexpr bool cplx = F == kC64 || F == kCF16 || F == kCBF16;
+    constexpr bool cplx = format_complex(F);
     const float* row = jb.src + (size_t)p * jb.Tc * (cplx ? 2u : 1u);
     const float lw = jb.pair8[8u * p + 7u], cw = jb.pair8[8u * p + 6u];
     uint32_t lo = 0u, hi = jb.lde;
@@ -270,7 +270,14 @@ __device__ __forceinline__ void stage_row_elements(const StageJob& jb, uint32_t 
             const uint32_t j = base + threadIdx.x + 256u * (uint32_t)k;
             if (j < hi) {
                 const float S = j <= jb.Tc ? stable_threshold(lw, cw, z[k]) : 0.0f;
-                write_fused<F>(jb.dst, (uint64_t)p * jb.lde + j, v[k], S);
+                if constexpr (format_split(F)) {   // [thresholds][samples] of the row
+                    float* const r = static_cast<float*>(jb.dst) + (uint64_t)p * jb.lde * (cplx ? 3u : 2u);
+                    r[j] = S;
+                    if constexpr (cplx) reinterpret_cast<float2*>(r + jb.lde)[j] = make_float2(v[k][0], v[k][1]);
+                    else r[jb.lde + j] = v[k][0];
+                } else {
+                    write_fused<F>(jb.dst, (uint64_t)p * jb.lde + j, v[k], S);
+                }
             }
         }
     }
@@ -290,6 +297,8 @@ __device__ __forceinline__ void stage_row_block(const StageJob& jb, uint32_t p) 
         case kF16: stage_row_elements<kF16>(jb, p); break;
         case kBF16: stage_row_elements<kBF16>(jb, p); break;
         case kC64: stage_row_elements<kC64>(jb, p); break;
+        case kF32Split: stage_row_elements<kF32Split>(jb, p); break;
+        case kC64Split: stage_row_elements<kC64Split>(jb, p); break;
         case kCF16: stage_row_elements<kCF16>(jb, p); break;
         default: stage_row_elements<kCBF16>(jb, p); break;
     }
@@ -552,8 +561,7 @@ __device__ __forceinline__ uint32_t sample_flags(float x) {
 
 // Sets the bits of *flag that any sample sets: 16-byte loads over the aligned body (src 16-byte
 // aligned), single samples for the tail.
-__global__ __launch_bounds__(256) void exact16_check_kernel(const float* __restrict__ src, uint64_t n,
-                                                            uint32_t* flag) {
+__device__ __forceinline__ void exact16_check(const float* __restrict__ src, uint64_t n, uint32_t* flag) {
     uint32_t bad = 0u;
     const uint64_t n4 = n / 4u, stride = (uint64_t)gridDim.x * blockDim.x;
     const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -568,6 +576,19 @@ __global__ __launch_bounds__(256) void exact16_check_kernel(const float* __restr
     if (wave && (threadIdx.x & 63u) == 0u &&
         (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & wave) != wave)
         atomicOr(flag, wave);
+}
+__global__ __launch_bounds__(256) void exact16_check_kernel(const float* __restrict__ src, uint64_t n,
+                                                            uint32_t* flag) {
+    exact16_check(src, n, flag);
+}
+// One row of work-groups per job that has a flag.
+__global__ __launch_bounds__(256) void batch_exact16_kernel(const StageJob* __restrict__ jobs) {
+    const StageJob& jb = jobs[blockIdx.y];
+    if (jb.fmt_flag) exact16_check(jb.src, (uint64_t)jb.rows * jb.Tc, const_cast<uint32_t*>(jb.fmt_flag));
+}
+hipError_t launch_batch_exact16(const StageJob* jobs, uint32_t n_jobs, hipStream_t s) {
+    hipLaunchKernelGGL(batch_exact16_kernel, dim3(256, n_jobs), dim3(256), 0, s, jobs);
+    return hipGetLastError();
 }
 
 hipError_t launch_exact16_check(const float* src, uint64_t n, uint32_t* flag, hipStream_t stream) {
@@ -1015,19 +1036,6 @@ __global__ __launch_bounds__(NW * 64) void confocal_lds_kernel(ConfocalArgs a) {
 // count, so the launch always drains.  Each tile runs the single-capture kernels' tile body:
 // every volume is bit-identical to its own plan's.  The work-group finishing a capture's last
 // gather item stamps the device wall clock (per-capture latency).
-// A struct every lane reads from the same address, moved word by word into scalar registers:
-// the buffer descriptors built from it are then wave-uniform (no per-pair waterfall loops).
-template <class T>
-__device__ __forceinline__ T wave_uniform_load(const T* p) {
-    static_assert(sizeof(T) % 4 == 0, "word-sized struct");
-    T out;
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(p);
-    uint32_t* dst = reinterpret_cast<uint32_t*>(&out);
-#pragma unroll
-    for (int i = 0; i < (int)(sizeof(T) / 4); ++i) dst[i] = __builtin_amdgcn_readfirstlane(src[i]);
-    return out;
-}
-
 // KINDS: the item kinds the instantiation serves (bit 0 staging, bit 1 LDS-staged, bit 2 texture
 // path); an LDS-only queue compiles without the other paths and needs fewer registers.  NW:
 // waves per work-group -- 4, or 8 for an LDS-only queue of 16^3 tiles with 8 voxels per lane
@@ -1121,12 +1129,12 @@ __global__ __launch_bounds__(256) void batch_tex_kernel(BatchQueueArgs b) {
 }
 
 // Before the queue: every capture's path-length table (blocks < z_blocks, as stage_z_kernel)
-// and, in the last block, the queue reset: both heads and the error word 0, per-capture
+// and, in the last block, the queue reset: both heads, the error word and the sample flags 0, per-capture
 // counters from their initial values, completion stamps 0, the start stamp.
 __global__ __launch_bounds__(256) void batch_prologue_kernel(const StageJob* __restrict__ jobs, uint32_t n_jobs,
                                                              uint32_t z_blocks, BatchQueueArgs b,
                                                              const uint32_t* __restrict__ init, uint32_t n,
-                                                             uint64_t* start) {
+                                                             uint32_t* fmt_flags, uint64_t* start) {
     if (blockIdx.x < z_blocks) {
         const StageJob& jb = jobs[stage_job_of<true>(jobs, n_jobs, blockIdx.x)];
         const uint32_t j = (blockIdx.x - jb.z_first) * 256u + threadIdx.x;
@@ -1137,6 +1145,7 @@ __global__ __launch_bounds__(256) void batch_prologue_kernel(const StageJob* __r
         b.staged[i] = init[2u * i];
         b.remaining[i] = init[2u * i + 1u];
         b.done[i] = 0ull;
+        fmt_flags[i] = 0u;
     }
     if (threadIdx.x == 0) {
         b.next[0] = 0u;   // the queue head; the texture-path and 16^3-tile heads of the
@@ -1240,9 +1249,9 @@ hipError_t launch_batch_queue(const BatchQueueArgs& b, int K, int kz, int format
 }
 
 hipError_t launch_batch_prologue(const StageJob* jobs, uint32_t n_jobs, uint32_t z_blocks, const BatchQueueArgs& b,
-                                 const uint32_t* init, uint32_t n, uint64_t* start, hipStream_t s) {
+                                 const uint32_t* init, uint32_t n, uint32_t* fmt_flags, uint64_t* start, hipStream_t s) {
     hipLaunchKernelGGL(batch_prologue_kernel, dim3(z_blocks + 1u), dim3(256), 0, s, jobs, n_jobs, z_blocks, b, init,
-                       n, start);
+                       n, fmt_flags, start);
     return hipGetLastError();
 }
 

@@ -21,6 +21,10 @@
 #define SEL16(dst, src)                                                                         \
     "v_cndmask_b32_sdwa " dst ", " src ", " src ", vcc dst_sel:DWORD dst_unused:UNUSED_PAD "   \
     "src0_sel:WORD_0 src1_sel:WORD_1"
+// the same into the high half of dst, zero below
+#define SEL16_HIGH(dst, src)                                                                    \
+    "v_cndmask_b32_sdwa " dst ", " src ", " src ", vcc dst_sel:WORD_1 dst_unused:UNUSED_PAD "  \
+    "src0_sel:WORD_0 src1_sel:WORD_1"
 
 namespace bpx {
 
@@ -33,9 +37,27 @@ namespace {
 // that makes the next update's s; written in one chain so that the two wait states the select
 // needs after the compare (and the one the add needs after the select) hold the neighbours' adds.
 struct CountRows {
-    using acc_t = uint32_t;
+    static constexpr int kFormat = kCount;
+    using part_t = uint32_t;
     template <int KZ>
-    __device__ static __forceinline__ void column(acc_t (&acc)[KZ], const uint2 (&e)[KZ], float axy,
+    struct Acc {
+        uint32_t sum[KZ];
+        __device__ __forceinline__ void clear() {
+#pragma unroll
+            for (int r = 0; r < KZ; ++r) sum[r] = 0u;
+        }
+        __device__ __forceinline__ void end_pair(uint32_t) {}
+        __device__ __forceinline__ void finish() {}
+        __device__ __forceinline__ uint32_t part(int r) const { return sum[r]; }
+        __device__ __forceinline__ void store(const ConfocalArgs& a, size_t id, int r) const {
+            static_cast<float*>(a.out)[id] = (float)sum[r];
+        }
+    };
+    __device__ static __forceinline__ void store_sum(const ConfocalArgs& a, size_t id, uint32_t v) {
+        static_cast<float*>(a.out)[id] = (float)v;
+    }
+    template <int KZ>
+    __device__ static __forceinline__ void column(Acc<KZ>& acc, const uint2 (&e)[KZ], float axy,
                                                   const float (&dz2)[KZ]) {
         float s = axy + dz2[column_order<KZ>(0)];
         uint32_t h;
@@ -49,10 +71,202 @@ struct CountRows {
             asm("v_cmp_ge_f32_e32 vcc, %2, %3\n\t"
                 "v_add_u32_e32 %0, %0, %5\n\t"
                 "s_nop 0\n\t" SEL16("%1", "%4")
-                : "+&v"(acc[prev]), "=v"(hn) : "v"(s), "v"(e[i].x), "v"(e[i].y), "v"(h) : "vcc");
+                : "+&v"(acc.sum[prev]), "=v"(hn) : "v"(s), "v"(e[i].x), "v"(e[i].y), "v"(h) : "vcc");
             h = hn;
         }
-        acc[column_order<KZ>(KZ - 1)] += h;
+        acc.sum[column_order<KZ>(KZ - 1)] += h;
+    }
+    template <int KZ, int DEG>
+    __device__ static __forceinline__ void pair(Acc<KZ>& acc, const ColumnQuotient<KZ, DEG>& q, float axy,
+                                                const float (&dz2)[KZ], uint32_t) {
+        uint2 e[KZ];
+#pragma unroll
+        for (int i = 0; i < KZ; ++i) e[i] = lds_read8(ElemOffset<8>::of(q.at(i)));
+        __builtin_amdgcn_sched_barrier(0);
+        column<KZ>(acc, e, axy, dz2);
+    }
+};
+
+// Real and complex rows keep the sums of the other confocal kernels: fp32 partials of kahan_block
+// pairs, added to a compensated fp32 sum.  With the pairs in one part the volume is theirs bit for
+// bit; more parts add up in double.
+template <int KZ>
+struct RealAcc {
+    float sum[KZ], comp[KZ], blk[KZ];
+    uint32_t n;
+    __device__ __forceinline__ void clear() {
+        n = 0u;
+#pragma unroll
+        for (int r = 0; r < KZ; ++r) sum[r] = comp[r] = blk[r] = 0.0f;
+    }
+    __device__ __forceinline__ void flush() {
+#pragma unroll
+        for (int r = 0; r < KZ; ++r) {
+            kahan_add(sum[r], comp[r], blk[r]);
+            blk[r] = 0.0f;
+        }
+        n = 0u;
+    }
+    __device__ __forceinline__ void end_pair(uint32_t kahan_block) {
+        if (++n == kahan_block) flush();
+    }
+    __device__ __forceinline__ void finish() {
+        if (n) flush();
+    }
+    __device__ __forceinline__ double part(int r) const { return (double)sum[r] - (double)comp[r]; }
+    __device__ __forceinline__ void store(const ConfocalArgs& a, size_t id, int r) const {
+        static_cast<float*>(a.out)[id] = kahan_result(sum[r], comp[r]) * a.scale;
+    }
+};
+struct RealRowsBase {
+    using part_t = double;
+    template <int KZ>
+    using Acc = RealAcc<KZ>;
+    __device__ static __forceinline__ void store_sum(const ConfocalArgs& a, size_t id, double v) {
+        static_cast<float*>(a.out)[id] = (float)v * a.scale;
+    }
+};
+// fp32 rows, thresholds and samples apart (kF32Split): S is read first and the comparison picks the
+// address of the one sample that is needed.  Two 4-byte reads at a stride of 4 bytes an update; an
+// (S, sample) element takes an 8- and a 4-byte read at a stride of 8.  Measured at 9,216 pairs into
+// 128 x 120 x 100: 5.06 ms against 5.74.
+struct F32Rows : RealRowsBase {
+    static constexpr int kFormat = kF32Split;
+    template <int KZ, int DEG>
+    __device__ static __forceinline__ void pair(Acc<KZ>& acc, const ColumnQuotient<KZ, DEG>& q, float axy,
+                                                const float (&dz2)[KZ], uint32_t samples) {
+        uint32_t o[KZ];
+        float S[KZ], v[KZ];
+#pragma unroll
+        for (int i = 0; i < KZ; ++i) {
+            o[i] = ElemOffset<8>::of(q.at(i)) >> 1;
+            S[i] = lds_read4(o[i]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t next = samples + 4u;
+#pragma unroll
+        for (int i = 0; i < KZ; ++i) {
+            const float s = axy + dz2[column_order<KZ>(i)];
+            v[i] = lds_read4(o[i] + (s >= S[i] ? next : samples));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < KZ; ++i) {
+            const int r = column_order<KZ>(i);
+            acc.blk[r] = acc.blk[r] + v[i];
+        }
+    }
+};
+// 16-bit rows: element (S, lo | hi << 16), the chain of CountRows::column with the sum in fp32 (fp16:
+// the half is added by one mixed-precision FMA, h x 1 + sum; bf16: it lands in the high word, which
+// is its fp32 value).
+template <bool BF>
+struct Half16Rows : RealRowsBase {
+    static constexpr int kFormat = BF ? kBF16 : kF16;
+    template <int KZ, int DEG>
+    __device__ static __forceinline__ void pair(Acc<KZ>& acc, const ColumnQuotient<KZ, DEG>& q, float axy,
+                                                const float (&dz2)[KZ], uint32_t) {
+        uint2 e[KZ];
+#pragma unroll
+        for (int i = 0; i < KZ; ++i) e[i] = lds_read8(ElemOffset<8>::of(q.at(i)));
+        __builtin_amdgcn_sched_barrier(0);
+        float s = axy + dz2[column_order<KZ>(0)];
+        uint32_t h;
+        if constexpr (BF)
+            asm("v_cmp_ge_f32_e32 vcc, %1, %2\n\ts_nop 1\n\t" SEL16_HIGH("%0", "%3")
+                : "=v"(h) : "v"(s), "v"(e[0].x), "v"(e[0].y) : "vcc");
+        else
+            asm("v_cmp_ge_f32_e32 vcc, %1, %2\n\ts_nop 1\n\t" SEL16("%0", "%3")
+                : "=v"(h) : "v"(s), "v"(e[0].x), "v"(e[0].y) : "vcc");
+#pragma unroll
+        for (int i = 1; i < KZ; ++i) {
+            const int r = column_order<KZ>(i), prev = column_order<KZ>(i - 1);
+            s = axy + dz2[r];
+            uint32_t hn;
+            if constexpr (BF)
+                asm("v_cmp_ge_f32_e32 vcc, %2, %3\n\t"
+                    "v_add_f32_e32 %0, %0, %5\n\t"
+                    "s_nop 0\n\t" SEL16_HIGH("%1", "%4")
+                    : "+&v"(acc.blk[prev]), "=v"(hn) : "v"(s), "v"(e[i].x), "v"(e[i].y), "v"(h) : "vcc");
+            else
+                asm("v_cmp_ge_f32_e32 vcc, %2, %3\n\t"
+                    "v_fma_mix_f32 %0, %5, 1.0, %0 op_sel_hi:[1,0,0]\n\t"
+                    "s_nop 0\n\t" SEL16("%1", "%4")
+                    : "+&v"(acc.blk[prev]), "=v"(hn) : "v"(s), "v"(e[i].x), "v"(e[i].y), "v"(h) : "vcc");
+            h = hn;
+        }
+        constexpr int last = column_order<KZ>(KZ - 1);
+        if constexpr (BF) acc.blk[last] = acc.blk[last] + __uint_as_float(h);
+        else acc.blk[last] = acc.blk[last] + (float)__builtin_bit_cast(_Float16, (unsigned short)h);
+    }
+};
+// Complex rows, thresholds and samples apart (kC64Split): S is read first and the comparison picks
+// the address of the one sample that is needed -- 12 LDS bytes an update at full bank spread,
+// against 24 at a stride of 16 for elements that hold (re, im, S).
+struct ComplexRows {
+    static constexpr int kFormat = kC64Split;
+    struct part_t {
+        double re, im;
+        __device__ __forceinline__ part_t& operator+=(const part_t& o) {
+            re += o.re;
+            im += o.im;
+            return *this;
+        }
+    };
+    template <int KZ>
+    struct Acc {
+        RealAcc<KZ> re, im;
+        __device__ __forceinline__ void clear() {
+            re.clear();
+            im.clear();
+        }
+        __device__ __forceinline__ void end_pair(uint32_t kahan_block) {
+            if (++re.n == kahan_block) {
+                re.flush();
+                im.flush();
+            }
+        }
+        __device__ __forceinline__ void finish() {
+            if (re.n) {
+                re.flush();
+                im.flush();
+            }
+        }
+        __device__ __forceinline__ part_t part(int r) const { return {re.part(r), im.part(r)}; }
+        __device__ __forceinline__ void store(const ConfocalArgs& a, size_t id, int r) const {
+            static_cast<float2*>(a.out)[id] = make_float2(kahan_result(re.sum[r], re.comp[r]) * a.scale,
+                                                          kahan_result(im.sum[r], im.comp[r]) * a.scale);
+        }
+    };
+    __device__ static __forceinline__ void store_sum(const ConfocalArgs& a, size_t id, part_t v) {
+        static_cast<float2*>(a.out)[id] = make_float2((float)v.re * a.scale, (float)v.im * a.scale);
+    }
+    // samples: LDS address of the sample of offset 0
+    template <int KZ, int DEG>
+    __device__ static __forceinline__ void pair(Acc<KZ>& acc, const ColumnQuotient<KZ, DEG>& q, float axy,
+                                                const float (&dz2)[KZ], uint32_t samples) {
+        uint32_t o[KZ];
+        float S[KZ];
+        uint2 v[KZ];
+#pragma unroll
+        for (int i = 0; i < KZ; ++i) {
+            o[i] = ElemOffset<8>::of(q.at(i));
+            S[i] = lds_read4(o[i] >> 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t next = samples + 8u;
+#pragma unroll
+        for (int i = 0; i < KZ; ++i) {
+            const float s = axy + dz2[column_order<KZ>(i)];
+            v[i] = lds_read8(o[i] + (s >= S[i] ? next : samples));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < KZ; ++i) {
+            const int r = column_order<KZ>(i);
+            acc.re.blk[r] = acc.re.blk[r] + __uint_as_float(v[i].x);
+            acc.im.blk[r] = acc.im.blk[r] + __uint_as_float(v[i].y);
+        }
     }
 };
 
@@ -65,24 +279,31 @@ __device__ __forceinline__ uint32_t list_part_pairs(uint32_t P, uint32_t count, 
     return ((P + parts - 1u) / parts + 3u) / 4u * 4u;
 }
 
+// Work-group `block` of `blocks`: its tile's share of the pairs.  Returns the tile.
 template <class Fz, int KZ, int DEG, bool TILES>
-__global__ __launch_bounds__(256, 4) void confocal_lds_kernel_poly(LdsPolyArgs a) {
+__device__ __forceinline__ uint32_t poly_tile(const LdsPolyArgs& a, uint32_t block, uint32_t blocks, char* smem) {
     constexpr uint32_t NW = 4, PS = NW;   // waves; pairs per stage (one per wave)
     using Off = ElemOffset<8>;
-    using acc_t = typename Fz::acc_t;
-    if (!rows_wanted(a.c)) return;
-    extern __shared__ char smem[];   // [2][PS][seg] 8-byte elements, then [2][PS] pair records
-    const uint32_t slot_bytes = a.seg * 8u, lds0 = lds_offset(smem);
-    float4* const meta = reinterpret_cast<float4*>(smem + 2u * PS * slot_bytes);
+    using part_t = typename Fz::part_t;
+    constexpr bool SPLIT = format_split(Fz::kFormat);
+    constexpr uint32_t EB = Fz::kFormat == kF32Split ? 4u : 8u;   // bytes of an element (split: of its sample)
+    // smem: [2][PS][seg] elements (split: thresholds first, then as many samples), then [2][PS] pair
+    // records
+    const uint32_t slot_bytes = a.seg * EB, lds0 = lds_offset(smem);
+    const uint32_t s_bytes = SPLIT ? 2u * PS * a.seg * 4u : 0u;
+    float4* const meta = reinterpret_cast<float4*>(smem + s_bytes + 2u * PS * slot_bytes);
+    // ElemOffset's offset of the stage's first element; split: the threshold of offset o lies at o / 2,
+    // its sample at EB o / 8 + samples
+    const uint32_t origin = SPLIT ? 2u * lds0 : lds0, samples = lds0 + s_bytes - origin / 8u * EB;
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
     const Grid& g = a.c.g;
     const uint32_t n0 = g.n[0], n1 = g.n[1], n2 = g.n[2], tiles = poly_tiles(g, KZ);
     // every tile of the grid, or those of a list whose length is on the device (then the launch is
     // fixed and its work-groups are shared out here)
     const uint32_t count = TILES ? __builtin_amdgcn_readfirstlane(*a.n_tiles) : tiles;
-    const uint32_t part_pairs = TILES ? list_part_pairs(a.c.P, count, gridDim.x) : a.part_pairs;
-    const uint32_t part = count ? blockIdx.x / count : 0u, index = count ? blockIdx.x % count : 0u;
-    if (TILES && (count == 0u || part * part_pairs >= a.c.P)) return;
+    const uint32_t part_pairs = TILES ? list_part_pairs(a.c.P, count, blocks) : a.part_pairs;
+    const uint32_t part = count ? block / count : 0u, index = count ? block % count : 0u;
+    if (TILES && (count == 0u || part * part_pairs >= a.c.P)) return 0u;
     const uint32_t tile = TILES ? __builtin_amdgcn_readfirstlane(a.tiles[index]) : xcd_remap(index, tiles);
     const uint32_t p0 = part * part_pairs, p1 = min(p0 + part_pairs, a.c.P);
     const ColumnTile<KZ> t(g, tile, w, lane);
@@ -96,7 +317,7 @@ __global__ __launch_bounds__(256, 4) void confocal_lds_kernel_poly(LdsPolyArgs a
     }
     const float u = t.centre(g, a.c.lz), u2 = u * u;
     const TileBox<KZ> box(g, t, a.c.lz);
-    const uint32_t row_bytes = a.c.ldh * 8u;
+    const uint32_t row_bytes = a.c.ldh * (SPLIT ? 4u + EB : EB);
     const uint32_t nstage = (p1 - p0 + PS - 1u) / PS;
 
     // Windows and pair records, 64 stages of this wave at a time (one pair per lane): lane L holds
@@ -111,15 +332,15 @@ __global__ __launch_bounds__(256, 4) void confocal_lds_kernel_poly(LdsPolyArgs a
             const float4 pr = a.c.pairs[p];
             float smin, smax;
             box.distances(pr.x, pr.y, smin, smax);
-            // 2 elements of margin each way; the start even, so that a 16-byte load never
-            // straddles a row end
-            const int jl = ((int)__builtin_fmaf(__builtin_amdgcn_sqrtf(smin), a.c.inv2, pr.w) - 2) & ~1;
+            // 2 elements of margin each way; the start even (split: a multiple of 4), so that a
+            // 16-byte load never straddles a row end
+            const int jl = ((int)__builtin_fmaf(__builtin_amdgcn_sqrtf(smin), a.c.inv2, pr.w) - 2) & (SPLIT ? ~3 : ~1);
             const int jh = (int)__builtin_fmaf(__builtin_amdgcn_sqrtf(smax), a.c.inv2, pr.w) + 2;
             mjl = jl;
             mcnt = min(jh + 2 - jl, (int)a.seg);
             mx = pr.x;
             my = pr.y;
-            mw = pr.w + (float)(int)((((st & 1u) * PS + w) * a.seg) - (uint32_t)jl + (lds0 >> 3) + (uint32_t)Off::kBias);
+            mw = pr.w + (float)(int)((((st & 1u) * PS + w) * a.seg) - (uint32_t)jl + (origin >> 3) + (uint32_t)Off::kBias);
         }
     };
     auto stage = [&](uint32_t b) {
@@ -128,25 +349,28 @@ __global__ __launch_bounds__(256, 4) void confocal_lds_kernel_poly(LdsPolyArgs a
         const uint32_t slot = (b & 1u) * PS + w;
         const int jl = __builtin_amdgcn_readlane(mjl, sl), cnt = __builtin_amdgcn_readlane(mcnt, sl);
         if (lane == sl) meta[slot] = make_float4(mx, my, mw, 0.0f);
-        const __amdgpu_buffer_rsrc_t rr =
-            make_rsrc(static_cast<const char*>(a.c.H) + (size_t)(p0 + b * PS + w) * row_bytes, row_bytes);
-        const int vo = jl * 8 + (int)lane * 16;
-        const uint32_t base = lds0 + slot * slot_bytes;
-        for (int m = 0; m < cnt; m += 128) load_lds16(rr, base + (uint32_t)m * 8u, vo + m * 8);
+        const char* row = static_cast<const char*>(a.c.H) + (size_t)(p0 + b * PS + w) * row_bytes;
+        const uint32_t t_bytes = SPLIT ? a.c.ldh * 4u : 0u;
+        if (SPLIT) {   // seg is a multiple of 256
+            const __amdgpu_buffer_rsrc_t rt = make_rsrc(row, t_bytes);
+            const uint32_t base = lds0 + slot * a.seg * 4u;
+            for (int m = 0; m < cnt; m += 256) load_lds16(rt, base + (uint32_t)m * 4u, (jl + m) * 4 + (int)lane * 16);
+        }
+        const __amdgpu_buffer_rsrc_t rr = make_rsrc(row + t_bytes, row_bytes - t_bytes);
+        constexpr int step = 1024 / (int)EB;
+        const int vo = jl * (int)EB + (int)lane * 16;
+        const uint32_t base = lds0 + s_bytes + slot * slot_bytes;
+        for (int m = 0; m < cnt; m += step) load_lds16(rr, base + (uint32_t)m * EB, vo + m * (int)EB);
     };
 
-    acc_t acc[KZ];
-#pragma unroll
-    for (int r = 0; r < KZ; ++r) acc[r] = 0;
+    typename Fz::template Acc<KZ> acc;
+    acc.clear();
     auto pair_step = [&](const float4 m) {
         const float dx = m.x - t.vx, dy = m.y - t.vy;
         const float axy = dx * dx + dy * dy;
         const ColumnQuotient<KZ, DEG> q(axy, u, u2, a.c.inv2, a.k1, a.k2, a.k3, m.z);
-        uint2 e[KZ];
-#pragma unroll
-        for (int i = 0; i < KZ; ++i) e[i] = lds_read8(Off::of(q.at(i)));
-        __builtin_amdgcn_sched_barrier(0);
-        Fz::template column<KZ>(acc, e, axy, dz2);
+        Fz::template pair<KZ, DEG>(acc, q, axy, dz2, samples);
+        acc.end_pair(a.c.kahan_block);
     };
     if (nstage) stage(0u);
     wait_loads();
@@ -165,31 +389,85 @@ __global__ __launch_bounds__(256, 4) void confocal_lds_kernel_poly(LdsPolyArgs a
         wait_loads();
         __syncthreads();
     }
+    acc.finish();
+    part_t* const sums = static_cast<part_t*>(a.parts);
     if (TILES) {   // [work-group = part x listed tiles + index][voxel of the column][lane]
-        uint32_t* o = a.parts + (size_t)blockIdx.x * (256u * KZ) + threadIdx.x;
+        part_t* o = sums + (size_t)block * (256u * KZ) + threadIdx.x;
 #pragma unroll
-        for (int r = 0; r < KZ; ++r) o[256u * r] = acc[r];
+        for (int r = 0; r < KZ; ++r) o[256u * r] = acc.part(r);
     } else if (t.ix < n0 && t.iy < n1) {
         const size_t id = t.id(g);
-        if (a.parts) {
-            uint32_t* o = a.parts + (size_t)part * n0 * n1 * n2 + id;
+        if (sums) {
+            part_t* o = sums + (size_t)part * n0 * n1 * n2 + id;
 #pragma unroll
-            for (int r = 0; r < KZ; ++r) o[r] = acc[r];
+            for (int r = 0; r < KZ; ++r) o[r] = acc.part(r);
         } else {
-            float* o = static_cast<float*>(a.c.out) + id;
 #pragma unroll
-            for (int r = 0; r < KZ; ++r) o[r] = (float)acc[r];
+            for (int r = 0; r < KZ; ++r) acc.store(a.c, id + r, r);
         }
     }
+    return tile;
 }
 
-// The volume from the integer partial sums of every part.
+template <class Fz, int KZ, int DEG, bool TILES>
+__global__ __launch_bounds__(256, 4) void confocal_lds_kernel_poly(LdsPolyArgs a) {
+    extern __shared__ char smem[];
+    if (!rows_wanted(a.c)) return;
+    poly_tile<Fz, KZ, DEG, TILES>(a, blockIdx.x, gridDim.x, smem);
+}
+
+// Captures of many sizes: one work-group per item (capture, part x its tiles + tile).  The last
+// part of a tile to finish adds up the tile's parts, in part order (the plans' sums bit for bit),
+// and the last tile of a capture stamps its completion.  No work-group waits for another.
+template <class Fz, int KZ, int DEG>
+__global__ __launch_bounds__(256, 4) void batch_lds_kernel_poly(BatchPolyArgs b) {
+    extern __shared__ char smem[];
+    const uint2 item = b.items[blockIdx.x];
+    const uint32_t c = __builtin_amdgcn_readfirstlane(item.x), block = __builtin_amdgcn_readfirstlane(item.y);
+    const LdsPolyArgs a = wave_uniform_load(b.caps + c);
+    if (!rows_wanted(a.c)) return;
+    const uint32_t tile = poly_tile<Fz, KZ, DEG, false>(a, block, 0u, smem);
+    uint32_t* const word = reinterpret_cast<uint32_t*>(smem);   // free: the tile's last stage is done
+    __threadfence();
+    __syncthreads();
+    if (a.parts) {
+        const uint32_t parts = (a.c.P + a.part_pairs - 1u) / a.part_pairs;
+        uint32_t* const left = b.left + b.first_tile[c] + tile;
+        if (threadIdx.x == 0) *word = atomicSub(left, 1u);
+        __syncthreads();
+        if (__builtin_amdgcn_readfirstlane(*word) != 1u) return;
+        if (threadIdx.x == 0) *left = parts;   // for the next execution
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");   // the other parts, for every wave
+        const ColumnTile<KZ> t(a.c.g, tile, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63u);
+        if (t.ix < a.c.g.n[0] && t.iy < a.c.g.n[1]) {
+            using part_t = typename Fz::part_t;
+            const size_t n = (size_t)a.c.g.n[0] * a.c.g.n[1] * a.c.g.n[2];
+            const part_t* const sums = static_cast<const part_t*>(a.parts) + t.id(a.c.g);
+            part_t v[KZ];
+#pragma unroll
+            for (int r = 0; r < KZ; ++r) v[r] = sums[r];
+            for (uint32_t k = 1; k < parts; ++k)
+#pragma unroll
+                for (int r = 0; r < KZ; ++r) v[r] += sums[(size_t)k * n + r];
+#pragma unroll
+            for (int r = 0; r < KZ; ++r) Fz::store_sum(a.c, t.id(a.c.g) + r, v[r]);
+        }
+        __threadfence();
+        __syncthreads();
+    }
+    if (threadIdx.x == 0 && atomicSub(&b.remaining[c], 1u) == 1u)
+        atomicMax(reinterpret_cast<unsigned long long*>(&b.done[c]), (unsigned long long)wall_clock64());
+}
+
+// The volume from the partial sums of every part, in part order.
+template <class Fz>
 __global__ __launch_bounds__(256) void lds_parts_sum_kernel(LdsPolyArgs a, uint32_t parts, uint64_t n) {
     if (!rows_wanted(a.c)) return;
+    const typename Fz::part_t* const sums = static_cast<const typename Fz::part_t*>(a.parts);
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
-        uint32_t v = 0;
-        for (uint32_t k = 0; k < parts; ++k) v += a.parts[(size_t)k * n + i];
-        static_cast<float*>(a.c.out)[i] = (float)v;
+        typename Fz::part_t v = sums[i];
+        for (uint32_t k = 1; k < parts; ++k) v += sums[(size_t)k * n + i];
+        Fz::store_sum(a.c, i, v);
     }
 }
 
@@ -270,27 +548,61 @@ __global__ __launch_bounds__(256) void tile_store_kernel(TileListArgs a, LdsPoly
         if (bits >> r & 1u) {
             uint32_t v = 0;
             for (uint32_t k = 0; k < parts; ++k)
-                v += p.parts[((size_t)k * count + blockIdx.x) * (256u * KZ) + 256u * r + threadIdx.x];
+                v += static_cast<const uint32_t*>(p.parts)[((size_t)k * count + blockIdx.x) * (256u * KZ) + 256u * r + threadIdx.x];
             out[r] = (float)v;
         }
 }
 
-template <int KZ, int DEG, bool TILES>
+// LDS of a work-group: two stages of 4 pairs and their records.
+template <class Fz, class Kernel>
+static hipError_t poly_lds(Kernel fn, uint32_t seg, size_t* bytes) {
+    *bytes = 2u * 4u * ((size_t)seg * (Fz::kFormat == kC64Split ? 12u : 8u) + sizeof(float4));
+    if (*bytes <= 64u * 1024u) return hipSuccess;
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)*bytes);
+}
+template <class Fz, int KZ, int DEG, bool TILES>
 static hipError_t poly_launch(const LdsPolyArgs& a, uint32_t groups, hipStream_t s) {
-    const auto fn = confocal_lds_kernel_poly<CountRows, KZ, DEG, TILES>;
-    const size_t lds = 2u * 4u * ((size_t)a.seg * 8u + sizeof(float4));
-    if (lds > 64u * 1024u) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-    }
+    const auto fn = confocal_lds_kernel_poly<Fz, KZ, DEG, TILES>;
+    size_t lds = 0;
+    const hipError_t e = poly_lds<Fz>(fn, a.seg, &lds);
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(fn, dim3(groups), dim3(256), lds, s, a);
     return hipGetLastError();
 }
-template <bool TILES>
+template <class Fz, int KZ, int DEG>
+static hipError_t batch_poly_launch(const BatchPolyArgs& b, uint32_t seg, uint32_t groups, hipStream_t s) {
+    const auto fn = batch_lds_kernel_poly<Fz, KZ, DEG>;
+    size_t lds = 0;
+    const hipError_t e = poly_lds<Fz>(fn, seg, &lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(fn, dim3(groups), dim3(256), lds, s, b);
+    return hipGetLastError();
+}
+template <class Fz>
+static hipError_t batch_poly_rows(const BatchPolyArgs& b, const LdsPolyShape& sh, uint32_t n, hipStream_t s) {
+    if constexpr (Fz::kFormat != kC64Split)
+        if (sh.kz == 16)
+            return sh.deg == 2 ? batch_poly_launch<Fz, 16, 2>(b, sh.seg, n, s) : batch_poly_launch<Fz, 16, 3>(b, sh.seg, n, s);
+    if (sh.kz != 8) return hipErrorInvalidValue;
+    return sh.deg == 2 ? batch_poly_launch<Fz, 8, 2>(b, sh.seg, n, s) : batch_poly_launch<Fz, 8, 3>(b, sh.seg, n, s);
+}
+hipError_t launch_batch_poly(const BatchPolyArgs& b, const LdsPolyShape& sh, int format, uint32_t n, hipStream_t s) {
+    switch (format) {
+        case kCount: return batch_poly_rows<CountRows>(b, sh, n, s);
+        case kF32Split: return batch_poly_rows<F32Rows>(b, sh, n, s);
+        case kF16: return batch_poly_rows<Half16Rows<false>>(b, sh, n, s);
+        case kBF16: return batch_poly_rows<Half16Rows<true>>(b, sh, n, s);
+        case kC64Split: return batch_poly_rows<ComplexRows>(b, sh, n, s);
+        default: return hipErrorInvalidValue;
+    }
+}
+template <class Fz, bool TILES>
 static hipError_t poly_launch_shape(const LdsPolyArgs& a, const LdsPolyShape& sh, uint32_t groups, hipStream_t s) {
-    if (sh.kz == 16) return sh.deg == 2 ? poly_launch<16, 2, TILES>(a, groups, s) : poly_launch<16, 3, TILES>(a, groups, s);
-    return sh.deg == 2 ? poly_launch<8, 2, TILES>(a, groups, s) : poly_launch<8, 3, TILES>(a, groups, s);
+    if constexpr (Fz::kFormat != kC64Split)   // two accumulators per voxel: 8 voxels per lane
+        if (sh.kz == 16)
+            return sh.deg == 2 ? poly_launch<Fz, 16, 2, TILES>(a, groups, s) : poly_launch<Fz, 16, 3, TILES>(a, groups, s);
+    if (sh.kz != 8) return hipErrorInvalidValue;
+    return sh.deg == 2 ? poly_launch<Fz, 8, 2, TILES>(a, groups, s) : poly_launch<Fz, 8, 3, TILES>(a, groups, s);
 }
 LdsPolyArgs lds_poly_args(const ConfocalArgs& c, const LdsPolyShape& sh) {
     LdsPolyArgs a{};
@@ -302,14 +614,26 @@ LdsPolyArgs lds_poly_args(const ConfocalArgs& c, const LdsPolyShape& sh) {
     a.k3 = (float)(A * step * step * step / 2.0);
     return a;
 }
-hipError_t launch_lds_counts(const LdsPolyArgs& a, const LdsPolyShape& sh, uint32_t parts, hipStream_t s) {
-    const hipError_t e = poly_launch_shape<false>(a, sh, (uint32_t)poly_tiles(a.c.g, sh.kz) * parts, s);
+template <class Fz>
+static hipError_t launch_rows(const LdsPolyArgs& a, const LdsPolyShape& sh, uint32_t parts, hipStream_t s) {
+    const hipError_t e = poly_launch_shape<Fz, false>(a, sh, (uint32_t)poly_tiles(a.c.g, sh.kz) * parts, s);
     if (e != hipSuccess || !a.parts) return e;
     const uint64_t n = (uint64_t)a.c.g.n[0] * a.c.g.n[1] * a.c.g.n[2];
-    hipLaunchKernelGGL(lds_parts_sum_kernel, dim3((uint32_t)std::min<uint64_t>((n + 255u) / 256u, 4096u)), dim3(256), 0,
-                       s, a, parts, n);
+    hipLaunchKernelGGL(lds_parts_sum_kernel<Fz>, dim3((uint32_t)std::min<uint64_t>((n + 255u) / 256u, 4096u)), dim3(256),
+                       0, s, a, parts, n);
     return hipGetLastError();
 }
+hipError_t launch_lds_poly(const LdsPolyArgs& a, const LdsPolyShape& sh, int format, uint32_t parts, hipStream_t s) {
+    switch (format) {
+        case kCount: return launch_rows<CountRows>(a, sh, parts, s);
+        case kF32Split: return launch_rows<F32Rows>(a, sh, parts, s);
+        case kF16: return launch_rows<Half16Rows<false>>(a, sh, parts, s);
+        case kBF16: return launch_rows<Half16Rows<true>>(a, sh, parts, s);
+        case kC64Split: return launch_rows<ComplexRows>(a, sh, parts, s);
+        default: return hipErrorInvalidValue;
+    }
+}
+uint32_t lds_poly_part_bytes(int format) { return format == kCount ? 4u : format == kC64Split ? 16u : 8u; }
 
 uint64_t lds_tile_count(const Grid& g, const LdsPolyShape& sh) { return poly_tiles(g, sh.kz); }
 
@@ -333,7 +657,7 @@ hipError_t launch_lds_counts_tiles(LdsPolyArgs a, const LdsPolyShape& sh, const 
                                    uint32_t groups, hipStream_t s) {
     a.tiles = t.tiles;
     a.n_tiles = t.counts;
-    const hipError_t e = poly_launch_shape<true>(a, sh, groups, s);
+    const hipError_t e = poly_launch_shape<CountRows, true>(a, sh, groups, s);
     if (e != hipSuccess) return e;
     if (sh.kz == 16) hipLaunchKernelGGL(tile_store_kernel<16>, dim3(max_tiles), dim3(256), 0, s, t, a, groups);
     else hipLaunchKernelGGL(tile_store_kernel<8>, dim3(max_tiles), dim3(256), 0, s, t, a, groups);
@@ -349,7 +673,7 @@ hipError_t launch_lds_counts_tiles(LdsPolyArgs a, const LdsPolyShape& sh, const 
 // times (w, c0, the even part, the sum: 1/16 each), so the bound on the approximate quotient
 // (`bound`, which covers the arithmetic of its terms) and the polynomial's error must stay below
 // 1/4 together (`budget`; the window kernel's end edge rounds a fifth time: 3/16).
-LdsPolyShape lds_poly_shape(const Grid& g, float inv2, float lz, double bound, double max_path, double budget) {
+LdsPolyShape lds_poly_shape(const Grid& g, float inv2, float lz, double bound, double max_path, double budget, int format) {
     LdsPolyShape none;
     // column along z alone; coordinates whose squares and reciprocals stay normal floats
     if (g.inc[2] != 0.0f || g.inc[5] != 0.0f || g.inc[6] != 0.0f || g.inc[7] != 0.0f) return none;
@@ -358,7 +682,7 @@ LdsPolyShape lds_poly_shape(const Grid& g, float inv2, float lz, double bound, d
     const double zmin = std::min(std::fabs(za), std::fabs(zb)) * (1.0 - 1e-5);
     if (!(za * zb > 0.0) || !(zmin > 1e-12) || !(max_path < 1e12) || !(step > 0.0)) return none;
     for (int kz : {16, 8}) {
-        if (g.n[2] < (uint32_t)kz) continue;
+        if (g.n[2] < (uint32_t)kz || (kz > 8 && format == kC64Split)) continue;
         const double h = 0.5 * (kz - 1) * step;
         const double e3 = A * 0.0559 * h * h * h * h / (zmin * zmin * zmin);
         const double e2 = e3 + A * 0.0930 * h * h * h / (4.0 * zmin * zmin);
@@ -371,13 +695,20 @@ LdsPolyShape lds_poly_shape(const Grid& g, float inv2, float lz, double bound, d
                              (kz - 1.0) * std::fabs((double)g.inc[6 + k]);
             d2 += r * r;
         }
-        // as confocal_lds_fits, with one more element for the even start
-        const double need = std::ceil(std::sqrt(d2) * A * (1.0 + 1e-6)) + 9.0;
+        // as confocal_lds_fits, with up to three more elements for the aligned start
+        const double need = std::ceil(std::sqrt(d2) * A * (1.0 + 1e-6)) + 11.0;
         if (!(need <= (double)kPolySegMax)) continue;
+        // Depth 16 spreads a pair's coefficients over more updates, depth 8 pads the last slab less:
+        // per slice of z fp32 and bf16 rows take 5 to 6 % more time at depth 8, counts some 10 %
+        // (4,096 pairs into 96^3, bf16: 0.79 ms at depth 16, 0.84 at 8; 9,216 pairs into
+        // 128 x 120 x 100, fp32: 5.08 ms for 7 slabs of 16, 4.96 for 13 of 8).
+        const uint32_t pad16 = (g.n[2] + 15u) / 16u * 16u, pad8 = (g.n[2] + 7u) / 8u * 8u;
+        if (kz == 16 && format != kCount && pad16 * 10u > pad8 * 11u) continue;
         LdsPolyShape sh;
         sh.kz = kz;
         sh.deg = deg;
-        sh.seg = ((uint32_t)need + 127u) / 128u * 128u;
+        const uint32_t unit = format_split(format) ? 256u : 128u;
+        sh.seg = ((uint32_t)need + unit - 1u) / unit * unit;
         return sh;
     }
     return none;

@@ -14,6 +14,9 @@ __device__ __forceinline__ uint2 lds_read8(uint32_t off) {
     const u32x2 v = *(const __attribute__((address_space(3))) u32x2*)(uintptr_t)off;
     return make_uint2(v[0], v[1]);
 }
+__device__ __forceinline__ float lds_read4(uint32_t off) {
+    return *(const __attribute__((address_space(3))) float*)(uintptr_t)off;
+}
 __device__ __forceinline__ double lds_read_f64(uint32_t off) {
     return *(const __attribute__((address_space(3))) double*)(uintptr_t)off;
 }

@@ -161,7 +161,7 @@ PlanImpl* make_plan_octree(const CaptureIn& c, const uint32_t n[3], const float 
     hip_check(hipHostMalloc(&st->host_total, sizeof(uint32_t) * 2, hipHostMallocDefault), "hipHostMalloc");
     hip_check(hipHostMalloc(&st->host_stats, sizeof(double) * 8, hipHostMallocDefault), "hipHostMalloc");
     if (P && pl->fused && pl->sep && pl->flat && pl->kahan_block <= 4096u && P <= (1u << 20))
-        st->poly = lds_poly_shape(pl->g, pl->inv2, pl->lz, pl->tap_bound, pl->max_path, kPolyBudget);
+        st->poly = lds_poly_shape(pl->g, pl->inv2, pl->lz, pl->tap_bound, pl->max_path, kPolyBudget, kCount);
     if (st->poly.kz) {
         const uint64_t tiles = lds_tile_count(pl->g, st->poly);
         st->count_rows.alloc(pl->H.bytes);

@@ -708,6 +708,7 @@ PlanImpl* make_plan_single_tap(const CaptureIn& c, const uint32_t n[3], const fl
     pl->cplx = c.cplx;
     pl->format = c.cplx ? (o.storage == BPX_STORAGE_F16 ? kCF16 : o.storage == BPX_STORAGE_BF16 ? kCBF16 : kC64)
                         : (o.storage == BPX_STORAGE_F16 ? kF16 : o.storage == BPX_STORAGE_BF16 ? kBF16 : kF32);
+    pl->row_format = pl->format;
     pl->kahan_block = o.kahan_block;
     pl->t0 = c.t0;
     pl->dT = c.dT;
@@ -862,11 +863,11 @@ PlanImpl* make_plan_single_tap(const CaptureIn& c, const uint32_t n[3], const fl
 }
 
 int staged_format(const PlanImpl& pl) {
-    if (!pl.fmt_flag.ptr || (!pl.rows16 && !pl.poly.kz)) return pl.format;
+    if (!pl.fmt_flag.ptr || (!pl.rows16 && !pl.poly_counts)) return pl.row_format;
     plan_wait(pl);
     uint32_t flag = 3;
     hip_check(hipMemcpy(&flag, pl.fmt_flag.ptr, 4, hipMemcpyDeviceToHost), "hipMemcpy(row format)");
-    return flag == 0u && pl.poly.kz ? kCount : pl.rows16 && !(flag & 1u) ? kF16 : pl.format;
+    return flag == 0u && pl.poly_counts ? kCount : pl.rows16 && !(flag & 1u) ? kF16 : pl.row_format;
 }
 
 StageJob stage_job(const PlanImpl& pl) {
@@ -878,11 +879,11 @@ StageJob stage_job(const PlanImpl& pl) {
     j.rows = pl.P;
     j.Tc = pl.T;
     j.lde = pl.ldh;
-    j.format = pl.format;
-    j.fmt_flag = pl.rows16 || pl.poly.kz ? static_cast<const uint32_t*>(pl.fmt_flag.ptr) : nullptr;
+    j.format = pl.row_format;
+    j.fmt_flag = pl.rows16 || pl.poly_counts ? static_cast<const uint32_t*>(pl.fmt_flag.ptr) : nullptr;
     j.win = static_cast<const uint32_t*>(pl.win.ptr);
-    j.alt_format = pl.rows16 ? kF16 : pl.format;
-    j.count_rows = pl.poly.kz ? 1 : 0;
+    j.alt_format = pl.rows16 ? kF16 : pl.row_format;
+    j.count_rows = pl.poly_counts ? 1 : 0;
     j.inv_scale = 1.0f / pl.scale;
     j.t0 = pl.t0;
     j.dT = pl.dT;
@@ -909,16 +910,35 @@ void set_fused_variant(PlanImpl& pl, int variant) {
     // gives the volume of the fp32 rows bit for bit while a block of kahan_block counts stays
     // below 2^24 and the whole sum below 2^32.  For variants 7 and 8 (as the exact fp16 rows), and for
     // every confocal plan whose variant was left to the library.
+    // The other rows (fp32, 16-bit, complex64) for every confocal plan whose variant was left to the
+    // library.
     pl.poly = LdsPolyShape{};
-    if (pl.format == kF32 && !pl.keep_f32 && pl.sep && pl.flat && (pl.auto_variant || variant > kLdsVariant) &&
-        pl.kahan_block <= 4096u && pl.P <= (1u << 20))
-        pl.poly = lds_poly_shape(pl.g, pl.inv2, pl.lz, pl.tap_bound, pl.max_path, kPolyBudget);
-    if (pl.poly.kz) {
-        pl.poly_parts = lds_poly_parts(pl.g, pl.poly, pl.P, 4u, &pl.poly_part_pairs);
-        const size_t bytes = pl.poly_parts > 1 ? (size_t)pl.poly_parts * pl.g.n[0] * pl.g.n[1] * pl.g.n[2] * 4u : 0;
+    pl.poly_counts = pl.poly_real = false;
+    pl.row_format = pl.format;
+    if (!pl.keep_f32 && pl.sep && pl.flat) {
+        const bool counts = pl.format == kF32 && (pl.auto_variant || variant > kLdsVariant) && pl.kahan_block <= 4096u &&
+                            pl.P <= (1u << 20);
+        const bool real = pl.auto_variant && (!format_complex(pl.format) || pl.format == kC64);
+        const int rows = pl.format == kC64 ? (int)kC64Split : pl.format == kF32 ? (int)kF32Split : pl.format;
+        if (counts || real)
+            pl.poly = lds_poly_shape(pl.g, pl.inv2, pl.lz, pl.tap_bound, pl.max_path, kPolyBudget, real ? rows : (int)kCount);
+        pl.poly_counts = counts && pl.poly.kz;
+        pl.poly_real = real && pl.poly.kz;
+        if (pl.poly_real) pl.row_format = rows;
+        const size_t vox = (size_t)pl.g.n[0] * pl.g.n[1] * pl.g.n[2];
+        size_t bytes = 0;
+        if (pl.poly_counts) {
+            pl.poly_parts = lds_poly_parts(pl.g, pl.poly, pl.P, 4u, &pl.poly_part_pairs);
+            if (pl.poly_parts > 1) bytes = pl.poly_parts * vox * 4u;
+        }
+        if (pl.poly_real) {
+            const uint32_t b = lds_poly_part_bytes(rows);
+            pl.real_parts = lds_poly_parts(pl.g, pl.poly, pl.P, b, &pl.real_part_pairs);
+            if (pl.real_parts > 1) bytes = std::max(bytes, pl.real_parts * vox * b);
+        }
         if (bytes > pl.parts.bytes) pl.parts.alloc(bytes);
     }
-    if ((pl.rows16 || pl.poly.kz) && !pl.fmt_flag.ptr) {
+    if ((pl.rows16 || pl.poly_counts) && !pl.fmt_flag.ptr) {
         pl.fmt_flag.alloc(4);
         // fp32 until run
         hip_check(hipMemsetAsync(pl.fmt_flag.ptr, 0xff, 4, pl.stream), "hipMemsetAsync(row format)");
@@ -1010,7 +1030,7 @@ void PlanImpl::execute(hipStream_t s) {
     hip_check(hipEventRecord(ev[1], s), "hipEventRecord");
     if (path == kPathConfocal) {
         if (fused) {
-            if (rows16 || poly.kz) {
+            if (rows16 || poly_counts) {
                 hip_check(launch_fill(static_cast<float*>(fmt_flag.ptr), 1, 0.0f, s), "fill kernel");
                 hip_check(launch_exact16_check(static_cast<const float*>(raw.ptr), (uint64_t)P * T,
                                                static_cast<uint32_t*>(fmt_flag.ptr), s),
@@ -1042,27 +1062,34 @@ void PlanImpl::execute(hipStream_t s) {
         a.scale = scale;
         a.lz = lz;
         a.kahan_block = kahan_block;
-        if (rows16 || poly.kz) {
+        const auto gather = [&](int rows) {
+            const bool counts = rows == kCount;
+            if (!counts && !poly_real) {
+                hip_check(launch_confocal(a, rows, variant, sep, flat, s), "confocal gather kernel");
+                return;
+            }
+            LdsPolyArgs pa = lds_poly_args(a, poly);
+            const uint32_t n = counts ? poly_parts : real_parts;
+            pa.part_pairs = counts ? poly_part_pairs : real_part_pairs;
+            pa.parts = n > 1 ? parts.ptr : nullptr;
+            hip_check(launch_lds_poly(pa, poly, rows, n, s), "confocal gather kernel (polynomial quotients)");
+        };
+        if (rows16 || poly_counts) {
             // every instantiation launched; those the device check did not pick return at once
             a.fmt_flag = static_cast<const uint32_t*>(fmt_flag.ptr);
-            if (poly.kz) {
-                LdsPolyArgs pa = lds_poly_args(a, poly);
-                pa.c.fmt_mask = 3u;
-                pa.c.fmt_want = 0u;
-                pa.part_pairs = poly_part_pairs;
-                pa.parts = poly_parts > 1 ? static_cast<uint32_t*>(parts.ptr) : nullptr;
-                hip_check(launch_lds_counts(pa, poly, poly_parts, s), "confocal gather kernel (count rows)");
+            if (poly_counts) {
+                a.fmt_mask = 3u;
+                a.fmt_want = 0u;
+                gather(kCount);
             }
             if (rows16) {
-                a.fmt_mask = poly.kz ? 3u : 1u;
-                a.fmt_want = poly.kz ? 2u : 0u;
-                hip_check(launch_confocal(a, kF16, variant, sep, flat, s), "confocal gather kernel (fp16 rows)");
+                a.fmt_mask = poly_counts ? 3u : 1u;
+                a.fmt_want = poly_counts ? 2u : 0u;
+                gather(kF16);
             }
             a.fmt_mask = a.fmt_want = rows16 ? 1u : 2u;
-            hip_check(launch_confocal(a, format, variant, sep, flat, s), "confocal gather kernel");
-        } else {
-            hip_check(launch_confocal(a, format, variant, sep, flat, s), "confocal gather kernel");
         }
+        gather(row_format);
     } else {
         hip_check(launch_ztable(0, t0, dT, 0.0f, T + 1, static_cast<float*>(Z.ptr), s),
                   "threshold table kernel");
@@ -1132,7 +1159,7 @@ static void window_lds_setup(PlanImpl& pl, const std::vector<bpx_pair>& pr, floa
     }
     pl.lz = pr[0].laser_point[2];
     pl.inv2 = (float)(2.0 / (double)pl.dT);
-    const LdsPolyShape sh = lds_poly_shape(pl.g, pl.inv2, pl.lz, pl.tap_bound, pl.max_path, kWindowPolyBudget);
+    const LdsPolyShape sh = lds_poly_shape(pl.g, pl.inv2, pl.lz, pl.tap_bound, pl.max_path, kWindowPolyBudget, kCount);
     const double bins = (double)width / (double)pl.dT;
     if (!sh.kz || !(bins < 1024.0)) return;
     WindowLdsArgs& a = pl.wlds;

@@ -431,7 +431,8 @@ typedef struct bpx_batch_config {
     uint32_t order;        /* queue: 0 = most work first, 1 = given order, 2 = most work
                               first with texture-path tiles spread among LDS-staged ones */
     uint32_t lds_captures; /* out (get/tune): captures run as LDS-staged tiles (those whose
-                              bin windows fit the LDS segment); ignored by set_config   */
+                              bin windows fit the queue's LDS segment); ignored by
+                              set_config                                                */
     uint32_t lds_depth;    /* LDS-staged tile depth: 8 (16 x 16 x 8) or 16 (16^3); 0 = 8;
                               complex formats always use 8                              */
     uint32_t launches;     /* 1 (or 0): one persistent launch serves the rows' staging, the

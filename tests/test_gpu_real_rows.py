@@ -1,0 +1,91 @@
+"""Confocal captures that are no counts (fp32, 16-bit and complex rows): the LDS-staged kernel with
+polynomial quotients against the texture-path kernel of an explicit variant, and exact sums against
+the oracle."""
+import numpy as np
+import pytest
+
+from test_gpu_count_rows import CASES, basis, pairs_of
+
+pytestmark = pytest.mark.gpu
+f32 = np.float32
+EPS = 2.0 ** -24
+
+
+@pytest.mark.parametrize("storage,cplx", [("f32", False), ("f16", False), ("bf16", False), ("f32", True)])
+@pytest.mark.parametrize("N,size,T,dT,t0,scan", CASES)
+def test_real_rows_equal_the_texture_path(gpu, N, size, T, dT, t0, scan, storage, cplx):
+    """One part: the same sums in the same order, bit for bit.  More parts: every voxel is a sum of the
+    same non-negative samples in other groups.  A group of 32 added in turn is off by at most 31
+    roundings, its compensated sum by 2 and the end by 1, on either side: |a - b| <= 68 eps sum."""
+    pr = pairs_of(*scan)
+    rng = np.random.default_rng(N[2])
+    H = rng.gamma(0.5, 2.0, (len(pr), T)).astype(f32)
+    if cplx:
+        H = (H + 1j * rng.gamma(0.5, 2.0, H.shape)).astype(np.complex64)
+    zero, inc = basis(N, (0.03, -0.02, 0.75), size)
+    vols, parts = [], 0
+    for variant in (-1, 5):
+        with gpu.Plan(H, pr, N, zero, inc, t0, dT, variant=variant, storage=storage) as plan:
+            plan.execute()
+            plan.execute()   # partial sums are rewritten by every execution
+            name = plan.info()["kernel"]
+            assert ("degree=" in name) == (variant == -1), name
+            if variant == -1:
+                parts = int(name.split("tiles, ")[1].split()[0])
+                th = plan.thresholds()
+            else:
+                assert np.array_equal(th, plan.thresholds())
+            vols.append(plan.volume())
+    a, b = vols
+    assert np.abs(b).max() > 0
+    if parts == 1:
+        assert np.array_equal(a, b)
+    for x, y in ((a.real, b.real), (a.imag, b.imag)):
+        assert np.all(np.abs(x.astype(np.float64) - y) <= 68 * EPS * np.abs(y).astype(np.float64))
+
+
+@pytest.mark.parametrize("kahan", [1, 5, 32, 5000])
+@pytest.mark.parametrize("N,size,T,dT,t0,scan", CASES[1:4])
+def test_complex_integer_rows_equal_oracle(gpu, oracle, N, size, T, dT, t0, scan, kahan):
+    pr = pairs_of(*scan)
+    rng = np.random.default_rng(N[2])
+    re, im = (rng.integers(-60, 61, (len(pr), T)).astype(f32) for _ in range(2))
+    zero, inc = basis(N, (0.03, -0.02, 0.75), size)
+    with gpu.Plan((re + 1j * im).astype(np.complex64), pr, N, zero, inc, t0, dT, kahan_block=kahan) as plan:
+        plan.execute()
+        assert "degree=" in plan.info()["kernel"]
+        vol = plan.volume()
+    assert np.array_equal(vol.real, oracle.a1_volume_f64acc(re, pr, N, zero, inc, t0, dT).astype(f32))
+    assert np.array_equal(vol.imag, oracle.a1_volume_f64acc(im, pr, N, zero, inc, t0, dT).astype(f32))
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+def test_values_that_are_no_numbers(gpu, value):
+    """They reach the voxels that the texture path gives them to, and no other."""
+    N, T = (35, 33, 17), 2001
+    pr = pairs_of(15, 15)
+    zero, inc = basis(N, (0.03, -0.02, 0.75), (0.25, 0.22, 0.12))
+    H = np.full((len(pr), T), 0.5, f32)
+    H[::7, 100::211] = value
+    vols = []
+    for variant in (-1, 5):
+        with gpu.Plan(H, pr, N, zero, inc, 1.2, 0.001, variant=variant) as plan:
+            plan.execute()
+            vols.append(plan.volume())
+    bad = ~np.isfinite(vols[1])
+    assert 0 < bad.sum() < bad.size
+    assert np.array_equal(~np.isfinite(vols[0]), bad) and np.array_equal(vols[0][~bad], vols[1][~bad])
+
+
+def test_tune_may_keep_the_default_kernel(gpu):
+    N, T = (48, 48, 48), 2000
+    pr = pairs_of(24, 24)
+    zero, inc = basis(N, (0.03, -0.02, 0.75), (0.5, 0.5, 0.5))
+    H = np.random.default_rng(2).gamma(0.5, 2.0, (len(pr), T)).astype(f32)
+    with gpu.Plan(H, pr, N, zero, inc, 0.5, 0.002) as plan:
+        plan.execute()
+        before = plan.volume().astype(np.float64)
+        got = plan.tune(reps=2)
+        plan.execute()
+        assert plan.info()["kernel"] == got["kernel"]
+        assert np.all(np.abs(plan.volume() - before) <= 68 * EPS * before)
