@@ -3,8 +3,9 @@
 // Captures that the polynomial-quotient kernel takes (flat wall, columns along its normal; the
 // plans' rule) are gathered by it, as a plan of their own gathers them: their rows are staged
 // first (counts where a capture's samples all are), then one launch per depth and window class
-// covers the (capture, part of the pairs, tile) items of all of them.  Every item is computed
-// alike whatever the configuration below.
+// covers the (capture, part of the pairs, tile) items of all of them.  One more launch takes those
+// that a plan of their own gathers on the texture path with the pairs split.  Every item of these is
+// computed alike whatever the configuration below.
 //
 // The others: one persistent launch over a single work queue of staging items (fused rows and thresholds), LDS-staged
 // tiles (captures whose bin windows fit the LDS segment) and texture-path tiles (the rest),
@@ -35,7 +36,7 @@ struct BatchImpl {
     hipEvent_t done = nullptr, ready = nullptr;   // as PlanImpl::done / ready
     DeviceBuffer caps, flags, items, items_tex, items_wide, jobs, init, next, staged, remaining, error;
     DeviceBuffer stamps;   // uint64 [1 + captures]: batch start, then each capture's completion
-    DeviceBuffer zjobs;    // StageJob per capture with pairs, those of poly_caps first (prologue)
+    DeviceBuffer zjobs;    // StageJob per capture with pairs, those outside the queues first (prologue)
     // the captures of the polynomial-quotient kernel (shape kz != 0)
     struct PolyCapture {
         LdsPolyShape shape;
@@ -43,6 +44,15 @@ struct BatchImpl {
         bool counts = false;
         size_t parts_offset = 0;   // bytes in poly_parts
     };
+    // the captures that a plan of their own gathers on the texture path with the pairs split
+    struct SplitCapture {
+        uint32_t parts = 1, part_pairs = 0;
+        size_t parts_offset = 0;
+        Tiles tiles{};
+    };
+    std::vector<SplitCapture> split;
+    uint32_t n_split = 0, n_split_items = 0;
+    DeviceBuffer split_args, split_items;
     struct PolyGroup {             // one launch per row format
         LdsPolyShape shape;
         uint32_t first = 0, n = 0;
@@ -50,9 +60,9 @@ struct BatchImpl {
     };
     std::vector<PolyCapture> poly;
     std::vector<PolyGroup> poly_groups;
-    uint32_t n_poly = 0, poly_row_blocks = 0;
+    uint32_t n_poly = 0, staged_row_blocks = 0;
     int poly_format = kF32Split;
-    DeviceBuffer poly_args, poly_items, poly_left, poly_first, poly_parts, fmt_flags;
+    DeviceBuffer poly_args, poly_items, part_sums, sum_args, fmt_flags;
     bool foreign = false;          // executed on a caller's stream (`done` says when it ends)
     uint32_t n_zjobs = 0, z_blocks = 0, row_blocks = 0;
     uint32_t n_items = 0, n_tex_items = 0, n_wide_items = 0;
@@ -83,7 +93,8 @@ struct BatchImpl {
         if (side2) (void)hipStreamDestroy(side2);
         if (stream) (void)hipStreamDestroy(stream);
     }
-    void choose_poly();
+    void choose_kernels();
+    bool queued(uint32_t i) const { return !poly[i].shape.kz && split[i].parts <= 1u; }
     void build(const bpx_batch_config& c);
     // Waits for the batch's own stream and for its last execution on a caller's stream, then
     // checks the queue's error word.
@@ -96,42 +107,46 @@ struct BatchImpl {
     }
 };
 
-// Shapes, parts and items of the polynomial-quotient kernel: they depend on the captures alone.
-// Parts as a plan of its own has them, so that the sums are the plan's.
-void BatchImpl::choose_poly() {
+// Captures outside the queues, their parts and items: they depend on the captures alone, and are as a
+// plan of each capture's own has them, so that the sums are the plan's.
+void BatchImpl::choose_kernels() {
     const uint32_t n = (uint32_t)plans.size();
     poly.assign(std::max<uint32_t>(n, 1u), PolyCapture{});
+    split.assign(std::max<uint32_t>(n, 1u), SplitCapture{});
     fmt_flags.alloc(4u * std::max<uint32_t>(n, 1u));
-    if (format == kCF16 || format == kCBF16) return;
-    poly_format = format == kC64 ? (int)kC64Split : format == kF32 ? (int)kF32Split : format;
+    const bool takes_poly = format != kCF16 && format != kCBF16;
+    if (!takes_poly) poly_format = format;
+    else poly_format = format == kC64 ? (int)kC64Split : format == kF32 ? (int)kF32Split : format;
     const uint32_t bytes = lds_poly_part_bytes(poly_format);
-    size_t total = 0, tiles = 0;
-    std::vector<uint32_t> left, first(std::max<uint32_t>(n, 1u), 0u);
+    size_t total = 0;
     for (uint32_t i = 0; i < n; ++i) {
         const PlanImpl& pl = *plans[i];
         PolyCapture& pc = poly[i];
-        if (!pl.P || !pl.sep || !pl.flat) continue;
-        pc.shape = lds_poly_shape(pl.g, pl.inv2, pl.lz, pl.tap_bound, pl.max_path, kPolyBudget, poly_format);
-        if (!pc.shape.kz) continue;
+        if (!pl.P) continue;
+        if (takes_poly && pl.sep && pl.flat)
+            pc.shape = lds_poly_shape(pl.g, pl.inv2, pl.lz, pl.tap_bound, pl.max_path, kPolyBudget, poly_format);
+        if (!pc.shape.kz) {
+            SplitCapture& sc = split[i];
+            if (default_variant(pl) != kDefaultVariant) continue;
+            sc.tiles = make_tiles(pl.g.n, 2);
+            sc.parts = split_parts(sc.tiles, pl.P, part_unit(pl.kahan_block), &sc.part_pairs);
+            if (sc.parts <= 1u) continue;
+            ++n_split;
+            sc.parts_offset = total;
+            total += ((size_t)sc.parts * pl.g.n[0] * pl.g.n[1] * pl.g.n[2] * (cplx ? 16u : 8u) + 255u) / 256u * 256u;
+            continue;
+        }
         ++n_poly;
         pc.counts = format == kF32 && pl.kahan_block <= 4096u && pl.P <= (1u << 20);
-        pc.parts = lds_poly_parts(pl.g, pc.shape, pl.P, bytes, &pc.part_pairs);
+        pc.parts = lds_poly_parts(pl.g, pc.shape, pl.P, bytes, part_unit(pl.kahan_block), &pc.part_pairs);
         const uint64_t t = lds_tile_count(pl.g, pc.shape);
         if (t * pc.parts >= (1ull << 31)) fail(BPX_ERR_UNSUPPORTED, "batch capture too large");
         pc.parts_offset = total;
         if (pc.parts > 1)
             total += ((size_t)pc.parts * pl.g.n[0] * pl.g.n[1] * pl.g.n[2] * bytes + 255u) / 256u * 256u;
-        first[i] = (uint32_t)tiles;
-        tiles += t;
-        left.insert(left.end(), t, pc.parts);
     }
-    if (!n_poly) return;
-    if (tiles >= (1ull << 31)) fail(BPX_ERR_UNSUPPORTED, "batch too large");
-    poly_parts.alloc(total);
-    poly_left.alloc(4u * tiles);
-    poly_first.alloc(4u * first.size());
-    hip_check(hipMemcpy(poly_left.ptr, left.data(), 4u * tiles, hipMemcpyHostToDevice), "hipMemcpy");
-    hip_check(hipMemcpy(poly_first.ptr, first.data(), 4u * first.size(), hipMemcpyHostToDevice), "hipMemcpy");
+    if (!n_poly && !n_split) return;
+    part_sums.alloc(total);
     // a launch per depth and window class (LDS decides how many work-groups a CU holds), its items
     // by falling length: the short ones fill the end
     std::vector<uint32_t> order(n);
@@ -159,7 +174,25 @@ void BatchImpl::choose_poly() {
             if (g.n) poly_groups.push_back(g);
         }
     poly_items.alloc(4u * items.size());
-    hip_check(hipMemcpy(poly_items.ptr, items.data(), 4u * items.size(), hipMemcpyHostToDevice), "hipMemcpy");
+    if (!items.empty())
+        hip_check(hipMemcpy(poly_items.ptr, items.data(), 4u * items.size(), hipMemcpyHostToDevice), "hipMemcpy");
+    items.clear();
+    std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return split[x].part_pairs > split[y].part_pairs; });
+    for (uint32_t i : order)
+        for (uint32_t k = 0; split[i].parts > 1u && k < split[i].tiles.count * split[i].parts; ++k) {
+            items.push_back(i);
+            items.push_back(k);
+        }
+    n_split_items = (uint32_t)(items.size() / 2u);
+    split_items.alloc(4u * items.size());
+    if (n_split_items)
+        hip_check(hipMemcpy(split_items.ptr, items.data(), 4u * items.size(), hipMemcpyHostToDevice), "hipMemcpy");
+    std::vector<SplitPairs> sp(std::max<uint32_t>(n, 1u), SplitPairs{});
+    for (uint32_t i = 0; i < n; ++i)
+        if (split[i].parts > 1u)
+            sp[i] = {static_cast<char*>(part_sums.ptr) + split[i].parts_offset, split[i].part_pairs, 0u};
+    split_args.alloc(sizeof(SplitPairs) * sp.size());
+    hip_check(hipMemcpy(split_args.ptr, sp.data(), sizeof(SplitPairs) * sp.size(), hipMemcpyHostToDevice), "hipMemcpy");
 }
 
 void BatchImpl::build(const bpx_batch_config& c) {
@@ -219,8 +252,12 @@ void BatchImpl::build(const bpx_batch_config& c) {
             }
             pargs[i] = lds_poly_args(a, pc.shape);
             pargs[i].part_pairs = pc.part_pairs;
-            pargs[i].parts = pc.parts > 1 ? static_cast<char*>(poly_parts.ptr) + pc.parts_offset : nullptr;
-            nt[i] = (uint32_t)lds_tile_count(pl.g, pc.shape);
+            pargs[i].parts = pc.parts > 1 ? static_cast<char*>(part_sums.ptr) + pc.parts_offset : nullptr;
+            nt[i] = kBatchSumBlocks;
+        } else if (!queued(i)) {
+            a.t = split[i].tiles;
+            sj[i] = stage_job(pl);
+            nt[i] = kBatchSumBlocks;
         } else if (pl.P) {
             sj[i] = stage_job(pl);
             ns[i] = two ? 0u : (stage_row_blocks(sj[i]) + kBatchStageBlocks - 1u) / kBatchStageBlocks;
@@ -242,7 +279,7 @@ void BatchImpl::build(const bpx_batch_config& c) {
         }
     };
     auto push_gather = [&](uint32_t i) {
-        if (poly[i].shape.kz) return;
+        if (!queued(i)) return;
         const uint32_t type = lds[i] ? kBatchItemLds : kBatchItemTex;
         for (uint32_t t = 0; t < nt[i]; ++t) {
             it.push_back(i | (type << 28));
@@ -254,7 +291,7 @@ void BatchImpl::build(const bpx_batch_config& c) {
         std::vector<uint32_t> a, b;   // LDS-staged and texture-path gather items, capture order
         for (uint32_t k = 0; k < n; ++k) {
             const uint32_t i = order[k];
-            if (poly[i].shape.kz) continue;
+            if (!queued(i)) continue;
             std::vector<uint32_t>& q = lds[i] ? a : b;
             const uint32_t type = lds[i] ? kBatchItemLds : kBatchItemTex;
             for (uint32_t t = 0; t < nt[i]; ++t) {
@@ -298,10 +335,10 @@ void BatchImpl::build(const bpx_batch_config& c) {
     std::vector<uint32_t> by_kernel;
     for (const bool first : {true, false})
         for (uint32_t i = 0; i < n; ++i)
-            if (plans[i]->P && (poly[i].shape.kz != 0) == first) by_kernel.push_back(i);
+            if (plans[i]->P && queued(i) != first) by_kernel.push_back(i);
     for (uint32_t i : by_kernel) {
-        if (zj.size() == n_poly) {   // the others' row blocks are numbered by themselves
-            poly_row_blocks = (uint32_t)rb;
+        if (zj.size() == n_poly + n_split) {   // the others' row blocks are numbered by themselves
+            staged_row_blocks = (uint32_t)rb;
             rb = 0;
         }
         StageJob j = sj[i];
@@ -313,8 +350,8 @@ void BatchImpl::build(const bpx_batch_config& c) {
     }
     if (zb >= (1ull << 31) || rb >= (1ull << 31)) fail(BPX_ERR_UNSUPPORTED, "batch staging too large");
     n_zjobs = (uint32_t)zj.size();
-    if (n_zjobs == n_poly) {
-        poly_row_blocks = (uint32_t)rb;
+    if (n_zjobs == n_poly + n_split) {
+        staged_row_blocks = (uint32_t)rb;
         rb = 0;
     }
     z_blocks = (uint32_t)zb;
@@ -346,6 +383,17 @@ void BatchImpl::build(const bpx_batch_config& c) {
             counts.fmt_want = 1u;      // never
         }
     }
+    std::vector<PartsSum> sums(std::max<uint32_t>(n, 1u), PartsSum{});
+    for (uint32_t i = 0; i < n; ++i) {
+        if (!plans[i]->P || queued(i)) continue;
+        const uint32_t own = poly[i].shape.kz ? poly[i].parts : split[i].parts;
+        sums[i] = {args[i].out, static_cast<char*>(part_sums.ptr) + (poly[i].shape.kz ? poly[i].parts_offset : split[i].parts_offset),
+                   static_cast<const uint32_t*>(fmt_flags.ptr) + i,
+                   (uint64_t)args[i].g.n[0] * args[i].g.n[1] * args[i].g.n[2], poly[i].counts ? poly[i].parts : 0u, own,
+                   cplx ? 1u : 0u, args[i].scale};
+    }
+    sum_args.alloc(sizeof(PartsSum) * sums.size());
+    hip_check(hipMemcpy(sum_args.ptr, sums.data(), sizeof(PartsSum) * sums.size(), hipMemcpyHostToDevice), "hipMemcpy");
     poly_args.alloc(sizeof(LdsPolyArgs) * pa.size());
     hip_check(hipMemcpy(poly_args.ptr, pa.data(), sizeof(LdsPolyArgs) * pa.size(), hipMemcpyHostToDevice), "hipMemcpy");
     if (n_zjobs)
@@ -421,30 +469,33 @@ void BatchImpl::build(const bpx_batch_config& c) {
                                         static_cast<const uint32_t*>(init.ptr), n, static_cast<uint32_t*>(fmt_flags.ptr),
                                         static_cast<uint64_t*>(stamps.ptr), stream),
                   "batch prologue kernel");
-        if (n_poly) {
-            if (format == kF32)
-                hip_check(launch_batch_exact16(static_cast<const StageJob*>(zjobs.ptr), n_poly, stream),
+        if (n_poly + n_split) {
+            if (format == kF32 && n_poly)
+                hip_check(launch_batch_exact16(static_cast<const StageJob*>(zjobs.ptr), n_poly + n_split, stream),
                           "batch sample check kernel");
-            hip_check(launch_stage(static_cast<const StageJob*>(zjobs.ptr), n_poly, 0u, poly_row_blocks, stream),
+            hip_check(launch_stage(static_cast<const StageJob*>(zjobs.ptr), n_poly + n_split, 0u, staged_row_blocks, stream),
                       "batch row staging kernel");
-            BatchPolyArgs pb{};
-            pb.first_tile = static_cast<const uint32_t*>(poly_first.ptr);
-            pb.left = static_cast<uint32_t*>(poly_left.ptr);
-            pb.remaining = static_cast<uint32_t*>(remaining.ptr);
-            pb.done = q.done;
             for (const bool counts : {true, false})
                 for (const PolyGroup& g : poly_groups) {
                     if (counts && !g.counts) continue;
-                    pb.caps = static_cast<const LdsPolyArgs*>(poly_args.ptr) + (counts ? 0u : pargs.size());
-                    pb.items = static_cast<const uint2*>(poly_items.ptr) + g.first;
-                    hip_check(launch_batch_poly(pb, g.shape, counts ? (int)kCount : poly_format, g.n, stream),
+                    const LdsPolyArgs* caps = static_cast<const LdsPolyArgs*>(poly_args.ptr) + (counts ? 0u : pargs.size());
+                    const BatchItems b{static_cast<const uint2*>(poly_items.ptr) + g.first, g.n};
+                    hip_check(launch_batch_poly(b, caps, g.shape, counts ? (int)kCount : poly_format, stream),
                               "batch gather kernel (polynomial quotients)");
                 }
+            if (n_split_items)
+                hip_check(launch_batch_split(BatchItems{static_cast<const uint2*>(split_items.ptr), n_split_items}, q.caps,
+                                             static_cast<const SplitPairs*>(split_args.ptr), q.flags, format, stream),
+                          "batch gather kernel (pairs split)");
+            for (uint32_t i = 0; i < n; i += 32768u)
+                hip_check(launch_batch_sum_parts(static_cast<const PartsSum*>(sum_args.ptr) + i, std::min(n - i, 32768u),
+                                                 q.remaining + i, q.done + i, stream),
+                          "batch partial sums kernel");
         }
         if (two) {
             // every row staged first (no waits in either queue), then both queues side by side
-            hip_check(launch_stage(static_cast<const StageJob*>(zjobs.ptr) + n_poly, n_zjobs - n_poly, 0u, row_blocks,
-                                   stream),
+            hip_check(launch_stage(static_cast<const StageJob*>(zjobs.ptr) + n_poly + n_split,
+                                   n_zjobs - n_poly - n_split, 0u, row_blocks, stream),
                       "batch row staging kernel");
             // every queue with items on its own stream: the 16 x 16 x kz one on the graph's
             // stream, the texture-path one on `side`, the 16^3 one on `side2`
@@ -579,7 +630,7 @@ bpx_status bpx_batch_create(const bpx_capture_desc* captures, uint32_t count, co
         b->staged.alloc(4u * n);
         b->remaining.alloc(4u * n);
         b->stamps.alloc(8u * (n + 1u));
-        b->choose_poly();
+        b->choose_kernels();
         b->build(bpx_batch_config{2u, 0u, 0u, 0u, 8u, 1u});
         auto h = std::make_unique<bpx_batch_s>();
         h->impl = std::move(b);

@@ -144,6 +144,7 @@ struct PlanImpl {
     bool auto_variant = false;           // the variant was not asked for: poly applies whatever it is
     uint32_t poly_parts = 1, poly_part_pairs = 0;   // of count rows (and of the window path)
     uint32_t real_parts = 1, real_part_pairs = 0;   // of the others
+    uint32_t tex_parts = 1, tex_part_pairs = 0;     // of the texture-path kernel (default plans)
     DeviceBuffer parts;                  // partial sums [parts][voxels] when split
     double tap_bound = 0, max_path = 0;  // of the approximate quotient; longest total path
     DeviceBuffer fmt_flag;
@@ -181,6 +182,7 @@ struct PlanImpl {
 void plan_wait(const PlanImpl& pl);
 // The storage the plan's last execution staged its rows in (waits for that execution).
 int staged_format(const PlanImpl& pl);
+int default_variant(const PlanImpl& pl);
 
 void execute_octree(PlanImpl& pl, hipStream_t s);
 

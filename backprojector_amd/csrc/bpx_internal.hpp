@@ -340,21 +340,44 @@ constexpr uint32_t kPolySegMax = 1024;
 constexpr double kPolyBudget = 0.24, kWindowPolyBudget = 0.18;
 LdsPolyShape lds_poly_shape(const Grid& g, float inv2, float lz, double bound, double max_path, double budget,
                             int format);
-uint32_t lds_poly_parts(const Grid& g, const LdsPolyShape& sh, uint32_t P, uint32_t sum_bytes, uint32_t* part_pairs);
+uint32_t lds_poly_parts(const Grid& g, const LdsPolyShape& sh, uint32_t P, uint32_t sum_bytes, uint32_t unit,
+                        uint32_t* part_pairs);
+uint32_t part_unit(uint32_t kahan_block);   // a multiple of 4
 LdsPolyArgs lds_poly_args(const ConfocalArgs& c, const LdsPolyShape& sh);
 // Rows of kCount, kF16, kBF16, kF32Split or kC64Split; shapes of lds_poly_shape for that format.
 hipError_t launch_lds_poly(const LdsPolyArgs& a, const LdsPolyShape& sh, int format, uint32_t parts, hipStream_t s);
 uint32_t lds_poly_part_bytes(int format);
-// The same for n items of many captures (one kz, degree and LDS segment per launch).
-struct BatchPolyArgs {
-    const LdsPolyArgs* caps;      // per capture
-    const uint2* items;           // (capture, part x tiles of the capture + tile)
-    const uint32_t* first_tile;   // per capture, in left
-    uint32_t* left;               // parts per tile still to finish (as many as it has before and after a launch)
-    uint32_t* remaining;          // tiles per capture still to finish
-    uint64_t* done;               // completion stamp per capture
+// Items (capture, part x tiles of the capture + tile) of many captures.
+struct BatchItems {
+    const uint2* items;
+    uint32_t n;
 };
-hipError_t launch_batch_poly(const BatchPolyArgs& b, const LdsPolyShape& sh, int format, uint32_t n, hipStream_t s);
+// The same for items of captures with one kz, degree and LDS segment; caps: per capture.
+hipError_t launch_batch_poly(const BatchItems& b, const LdsPolyArgs* caps, const LdsPolyShape& sh, int format,
+                             hipStream_t s);
+// A complex partial sum.
+struct ComplexSum {
+    double re, im;
+    __host__ __device__ ComplexSum& operator+=(const ComplexSum& o) {
+        re += o.re;
+        im += o.im;
+        return *this;
+    }
+};
+// Adds up partial sums [parts][n]: uint32_t where *fmt_flag is 0 and count_parts is not, else double or
+// ComplexSum.  Parts of 1 (or 0): nothing to do.
+struct PartsSum {
+    void* out;
+    const void* sums;
+    const uint32_t* fmt_flag;
+    uint64_t n;
+    uint32_t count_parts, real_parts, cplx;
+    float scale;
+};
+hipError_t launch_sum_parts(const PartsSum& d, hipStream_t s);
+constexpr uint32_t kBatchSumBlocks = 64;   // work-groups per capture
+// n captures (out nullptr: none); remaining[c] counts kBatchSumBlocks down, then done[c] is stamped.
+hipError_t launch_batch_sum_parts(const PartsSum* d, uint32_t n, uint32_t* remaining, uint64_t* done, hipStream_t s);
 // Per job the flag word of launch_exact16_check (StageJob::fmt_flag, cleared by the caller).
 hipError_t launch_batch_exact16(const StageJob* jobs, uint32_t n_jobs, hipStream_t s);
 uint64_t lds_tile_count(const Grid& g, const LdsPolyShape& sh);
@@ -362,6 +385,16 @@ hipError_t launch_tile_lists(const TileListArgs& a, const LdsPolyShape& sh, cons
                              const uint32_t n[2], uint32_t dense, hipStream_t s);
 hipError_t launch_lds_counts_tiles(LdsPolyArgs a, const LdsPolyShape& sh, const TileListArgs& t, uint32_t max_tiles,
                                    uint32_t groups, hipStream_t s);
+// The texture-path kernel with the pairs split over work-groups (2 voxels per lane, fused rows).
+struct SplitPairs {
+    void* parts;            // [parts][voxels] partial sums, double (complex: two)
+    uint32_t part_pairs, pad;
+};
+uint32_t split_parts(const Tiles& t, uint32_t P, uint32_t unit, uint32_t* part_pairs);
+hipError_t launch_split(const ConfocalArgs& a, const SplitPairs& sp, int format, uint32_t parts, bool sep, bool flat,
+                        hipStream_t s);
+hipError_t launch_batch_split(const BatchItems& b, const ConfocalArgs* caps, const SplitPairs* split,
+                              const uint32_t* flags, int format, hipStream_t s);
 hipError_t launch_grid(const GridArgs& a, int format, int variant, hipStream_t stream);
 hipError_t launch_pairs(const PairsArgs& a, int format, int variant, hipStream_t stream);
 // The LDS-staged kernel: arguments with seg a multiple of 256 and at least 256, every leg's squared

@@ -686,10 +686,19 @@ struct FusedSource {
     }
 };
 
+template <class T>
+using part_of = std::conditional_t<std::is_same<T, float>::value, double, ComplexSum>;
+__device__ __forceinline__ double kahan_part(float sum, float comp) { return (double)sum - (double)comp; }
+__device__ __forceinline__ ComplexSum kahan_part(float2 sum, float2 comp) {
+    return {kahan_part(sum.x, comp.x), kahan_part(sum.y, comp.y)};
+}
+
 // Wave quarter w of one 8 x 8 x 4K tile of a confocal capture (the body of the gather
-// kernels; no work-group barrier, so a wave can run it alone).
-template <class Src, int K, bool SEP, bool FLAT>
-__device__ __forceinline__ void confocal_tile(const ConfocalArgs& a, uint32_t tile, uint32_t w) {
+// kernels; no work-group barrier, so a wave can run it alone).  PART: pairs p .. p_end - 1 only,
+// their partial sums to parts[voxel].
+template <class Src, int K, bool SEP, bool FLAT, bool PART = false>
+__device__ __forceinline__ void confocal_tile(const ConfocalArgs& a, uint32_t tile, uint32_t w, uint32_t p = 0,
+                                              uint32_t p_end = 0, void* parts = nullptr) {
     using acc_t = typename Src::acc_t;
     const LaneVoxels lv = lane_voxels_of(a.t, K, tile, w);
     const uint32_t cx = min(lv.ix, a.g.n[0] - 1u), cy = min(lv.iy, a.g.n[1] - 1u);
@@ -722,9 +731,9 @@ __device__ __forceinline__ void confocal_tile(const ConfocalArgs& a, uint32_t ti
         acc_zero(comp[r]);
         acc_zero(blk[r]);
     }
-    uint32_t p = 0;
-    while (p < a.P) {
-        const uint32_t pend = min(p + a.kahan_block, a.P);
+    if (!PART) p_end = a.P;
+    while (p < p_end) {
+        const uint32_t pend = p_end - p > a.kahan_block ? p + a.kahan_block : p_end;
         for (; p < pend; ++p) {
             const float4 pr = a.pairs[p];
             src.set_pair(p);
@@ -763,10 +772,40 @@ __device__ __forceinline__ void confocal_tile(const ConfocalArgs& a, uint32_t ti
             const uint32_t iz = lv.iz0 + 4u * r;
             if (iz < a.g.n[2]) {
                 const size_t id = ((size_t)lv.ix * a.g.n[1] + lv.iy) * a.g.n[2] + iz;
-                store_voxel(a.out, id, scaled(kahan_result(sum[r], comp[r]), a.scale));
+                if constexpr (PART) static_cast<part_of<acc_t>*>(parts)[id] = kahan_part(sum[r], comp[r]);
+                else store_voxel(a.out, id, scaled(kahan_result(sum[r], comp[r]), a.scale));
             }
         }
     }
+}
+
+// The pairs split over work-groups, for volumes whose tiles alone leave most of the chip idle:
+// work-group part x tiles + tile.
+template <class Src, int K, bool SEP, bool FLAT>
+__global__ __launch_bounds__(256) void confocal_split_kernel(ConfocalArgs a, SplitPairs sp) {
+    const uint32_t part = blockIdx.x / a.t.count, tile = blockIdx.x % a.t.count;
+    const uint32_t p0 = part * sp.part_pairs, p1 = min(p0 + sp.part_pairs, a.P);
+    const size_t n = (size_t)a.g.n[0] * a.g.n[1] * a.g.n[2];
+    using part_t = part_of<typename Src::acc_t>;
+    confocal_tile<Src, K, SEP, FLAT, true>(a, tile, threadIdx.x >> 6, p0, p1, static_cast<part_t*>(sp.parts) + part * n);
+}
+// The same for captures of many sizes: an item (capture, part x its tiles + tile) per work-group.
+template <class Src, int K>
+__global__ __launch_bounds__(256) void batch_split_kernel(BatchItems b, const ConfocalArgs* __restrict__ caps,
+                                                          const SplitPairs* __restrict__ split,
+                                                          const uint32_t* __restrict__ flags) {
+    const uint2 item = b.items[blockIdx.x];
+    const uint32_t c = __builtin_amdgcn_readfirstlane(item.x), block = __builtin_amdgcn_readfirstlane(item.y);
+    const ConfocalArgs a = wave_uniform_load(caps + c);
+    const SplitPairs sp = wave_uniform_load(split + c);
+    const uint32_t part = block / a.t.count, tile = block % a.t.count, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t p0 = part * sp.part_pairs, p1 = min(p0 + sp.part_pairs, a.P);
+    const size_t n = (size_t)a.g.n[0] * a.g.n[1] * a.g.n[2];
+    void* const out = static_cast<part_of<typename Src::acc_t>*>(sp.parts) + part * n;
+    const uint32_t f = __builtin_amdgcn_readfirstlane(flags[c]);
+    if (f == 3u) confocal_tile<Src, K, true, true, true>(a, tile, w, p0, p1, out);
+    else if (f == 1u) confocal_tile<Src, K, true, false, true>(a, tile, w, p0, p1, out);
+    else confocal_tile<Src, K, false, false, true>(a, tile, w, p0, p1, out);
 }
 
 template <class Src, int K, bool SEP, bool FLAT>
@@ -1604,6 +1643,58 @@ static hipError_t confocal_dispatch(const ConfocalArgs& a, int variant, bool sep
         case 8: return confocal_dispatch_k<Src, 8>(a, sep, flat, s);
         case 2: return confocal_dispatch_k<Src, 2>(a, sep, flat, s);
         default: return confocal_dispatch_k<Src, 4>(a, sep, flat, s);
+    }
+}
+
+template <class T>
+struct TypeOf {
+    using type = T;
+};
+// The texture-path kernel of default plans (2 voxels per lane) with the pairs split; fused rows.
+uint32_t split_parts(const Tiles& t, uint32_t P, uint32_t unit, uint32_t* part_pairs) {
+    // Towards 2,048 work-groups (8 on each of 256 CUs) while each keeps 64 pairs: one part of the
+    // 64 tiles of 31^3 leaves three of four CUs without work.  16 uneven captures of 12.0e9 updates
+    // in one batch, 7 of them here: 17.5 ms unsplit, 9.0 split.
+    const uint32_t parts = std::max(1u, std::min((2048u + t.count - 1u) / std::max(t.count, 1u), P / 64u));
+    *part_pairs = ((P + parts - 1u) / parts + unit - 1u) / unit * unit;
+    return std::max(1u, (P + *part_pairs - 1u) / *part_pairs);
+}
+template <class Src>
+static hipError_t split_launch(const ConfocalArgs& a, const SplitPairs& sp, uint32_t parts, bool sep, bool flat,
+                               hipStream_t s) {
+    const dim3 grid(a.t.count * parts), block(256);
+    if (sep && flat) hipLaunchKernelGGL((confocal_split_kernel<Src, 2, true, true>), grid, block, 0, s, a, sp);
+    else if (sep) hipLaunchKernelGGL((confocal_split_kernel<Src, 2, true, false>), grid, block, 0, s, a, sp);
+    else hipLaunchKernelGGL((confocal_split_kernel<Src, 2, false, false>), grid, block, 0, s, a, sp);
+    return hipGetLastError();
+}
+hipError_t launch_split(const ConfocalArgs& a, const SplitPairs& sp, int format, uint32_t parts, bool sep, bool flat,
+                        hipStream_t s) {
+    switch (format) {
+        case kF32: return split_launch<FusedSource<FusedF32>>(a, sp, parts, sep, flat, s);
+        case kF16: return split_launch<FusedSource<FusedH16<false>>>(a, sp, parts, sep, flat, s);
+        case kBF16: return split_launch<FusedSource<FusedH16<true>>>(a, sp, parts, sep, flat, s);
+        case kC64: return split_launch<FusedSource<FusedC64>>(a, sp, parts, sep, flat, s);
+        case kCF16: return split_launch<FusedSource<FusedC16<false>>>(a, sp, parts, sep, flat, s);
+        case kCBF16: return split_launch<FusedSource<FusedC16<true>>>(a, sp, parts, sep, flat, s);
+        default: return hipErrorInvalidValue;
+    }
+}
+hipError_t launch_batch_split(const BatchItems& b, const ConfocalArgs* caps, const SplitPairs* split,
+                              const uint32_t* flags, int format, hipStream_t s) {
+    const auto launch = [&](auto src) {
+        hipLaunchKernelGGL((batch_split_kernel<typename decltype(src)::type, 2>), dim3(b.n), dim3(256), 0, s, b, caps, split,
+                           flags);
+        return hipGetLastError();
+    };
+    switch (format) {
+        case kF32: return launch(TypeOf<FusedSource<FusedF32>>{});
+        case kF16: return launch(TypeOf<FusedSource<FusedH16<false>>>{});
+        case kBF16: return launch(TypeOf<FusedSource<FusedH16<true>>>{});
+        case kC64: return launch(TypeOf<FusedSource<FusedC64>>{});
+        case kCF16: return launch(TypeOf<FusedSource<FusedC16<false>>>{});
+        case kCBF16: return launch(TypeOf<FusedSource<FusedC16<true>>>{});
+        default: return hipErrorInvalidValue;
     }
 }
 

@@ -53,9 +53,6 @@ struct CountRows {
             static_cast<float*>(a.out)[id] = (float)sum[r];
         }
     };
-    __device__ static __forceinline__ void store_sum(const ConfocalArgs& a, size_t id, uint32_t v) {
-        static_cast<float*>(a.out)[id] = (float)v;
-    }
     template <int KZ>
     __device__ static __forceinline__ void column(Acc<KZ>& acc, const uint2 (&e)[KZ], float axy,
                                                   const float (&dz2)[KZ]) {
@@ -122,9 +119,6 @@ struct RealRowsBase {
     using part_t = double;
     template <int KZ>
     using Acc = RealAcc<KZ>;
-    __device__ static __forceinline__ void store_sum(const ConfocalArgs& a, size_t id, double v) {
-        static_cast<float*>(a.out)[id] = (float)v * a.scale;
-    }
 };
 // fp32 rows, thresholds and samples apart (kF32Split): S is read first and the comparison picks the
 // address of the one sample that is needed.  Two 4-byte reads at a stride of 4 bytes an update; an
@@ -205,14 +199,7 @@ struct Half16Rows : RealRowsBase {
 // against 24 at a stride of 16 for elements that hold (re, im, S).
 struct ComplexRows {
     static constexpr int kFormat = kC64Split;
-    struct part_t {
-        double re, im;
-        __device__ __forceinline__ part_t& operator+=(const part_t& o) {
-            re += o.re;
-            im += o.im;
-            return *this;
-        }
-    };
+    using part_t = ComplexSum;
     template <int KZ>
     struct Acc {
         RealAcc<KZ> re, im;
@@ -238,9 +225,6 @@ struct ComplexRows {
                                                           kahan_result(im.sum[r], im.comp[r]) * a.scale);
         }
     };
-    __device__ static __forceinline__ void store_sum(const ConfocalArgs& a, size_t id, part_t v) {
-        static_cast<float2*>(a.out)[id] = make_float2((float)v.re * a.scale, (float)v.im * a.scale);
-    }
     // samples: LDS address of the sample of offset 0
     template <int KZ, int DEG>
     __device__ static __forceinline__ void pair(Acc<KZ>& acc, const ColumnQuotient<KZ, DEG>& q, float axy,
@@ -416,59 +400,52 @@ __global__ __launch_bounds__(256, 4) void confocal_lds_kernel_poly(LdsPolyArgs a
     poly_tile<Fz, KZ, DEG, TILES>(a, blockIdx.x, gridDim.x, smem);
 }
 
-// Captures of many sizes: one work-group per item (capture, part x its tiles + tile).  The last
-// part of a tile to finish adds up the tile's parts, in part order (the plans' sums bit for bit),
-// and the last tile of a capture stamps its completion.  No work-group waits for another.
+// Captures of many sizes: one work-group per item (capture, part x its tiles + tile).
 template <class Fz, int KZ, int DEG>
-__global__ __launch_bounds__(256, 4) void batch_lds_kernel_poly(BatchPolyArgs b) {
+__global__ __launch_bounds__(256, 4) void batch_lds_kernel_poly(BatchItems b, const LdsPolyArgs* __restrict__ caps) {
     extern __shared__ char smem[];
     const uint2 item = b.items[blockIdx.x];
     const uint32_t c = __builtin_amdgcn_readfirstlane(item.x), block = __builtin_amdgcn_readfirstlane(item.y);
-    const LdsPolyArgs a = wave_uniform_load(b.caps + c);
+    const LdsPolyArgs a = wave_uniform_load(caps + c);
     if (!rows_wanted(a.c)) return;
-    const uint32_t tile = poly_tile<Fz, KZ, DEG, false>(a, block, 0u, smem);
-    uint32_t* const word = reinterpret_cast<uint32_t*>(smem);   // free: the tile's last stage is done
-    __threadfence();
-    __syncthreads();
-    if (a.parts) {
-        const uint32_t parts = (a.c.P + a.part_pairs - 1u) / a.part_pairs;
-        uint32_t* const left = b.left + b.first_tile[c] + tile;
-        if (threadIdx.x == 0) *word = atomicSub(left, 1u);
-        __syncthreads();
-        if (__builtin_amdgcn_readfirstlane(*word) != 1u) return;
-        if (threadIdx.x == 0) *left = parts;   // for the next execution
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");   // the other parts, for every wave
-        const ColumnTile<KZ> t(a.c.g, tile, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63u);
-        if (t.ix < a.c.g.n[0] && t.iy < a.c.g.n[1]) {
-            using part_t = typename Fz::part_t;
-            const size_t n = (size_t)a.c.g.n[0] * a.c.g.n[1] * a.c.g.n[2];
-            const part_t* const sums = static_cast<const part_t*>(a.parts) + t.id(a.c.g);
-            part_t v[KZ];
-#pragma unroll
-            for (int r = 0; r < KZ; ++r) v[r] = sums[r];
-            for (uint32_t k = 1; k < parts; ++k)
-#pragma unroll
-                for (int r = 0; r < KZ; ++r) v[r] += sums[(size_t)k * n + r];
-#pragma unroll
-            for (int r = 0; r < KZ; ++r) Fz::store_sum(a.c, t.id(a.c.g) + r, v[r]);
-        }
-        __threadfence();
-        __syncthreads();
-    }
-    if (threadIdx.x == 0 && atomicSub(&b.remaining[c], 1u) == 1u)
-        atomicMax(reinterpret_cast<unsigned long long*>(&b.done[c]), (unsigned long long)wall_clock64());
+    poly_tile<Fz, KZ, DEG, false>(a, block, 0u, smem);
 }
 
-// The volume from the partial sums of every part, in part order.
-template <class Fz>
-__global__ __launch_bounds__(256) void lds_parts_sum_kernel(LdsPolyArgs a, uint32_t parts, uint64_t n) {
-    if (!rows_wanted(a.c)) return;
-    const typename Fz::part_t* const sums = static_cast<const typename Fz::part_t*>(a.parts);
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
-        typename Fz::part_t v = sums[i];
-        for (uint32_t k = 1; k < parts; ++k) v += sums[(size_t)k * n + i];
-        Fz::store_sum(a.c, i, v);
+// The volume from the partial sums of its parts, in part order; a launch of its own, which costs less
+// than having the last work-group of a tile add them up: the fences that this takes write back a
+// whole L2 per work-group (1,961 pairs into 45 x 61 x 38: 0.20 ms against 0.10 with this kernel).
+template <class T>
+__device__ __forceinline__ T parts_at(const PartsSum& d, uint32_t parts, uint64_t i) {
+    const T* const sums = static_cast<const T*>(d.sums) + i;
+    T v = sums[0];
+#pragma unroll 8
+    for (uint32_t k = 1; k < parts; ++k) v += sums[(uint64_t)k * d.n];
+    return v;
+}
+__device__ __forceinline__ void sum_parts(const PartsSum& d, uint32_t block, uint32_t blocks) {
+    const bool counts = d.count_parts && __builtin_amdgcn_readfirstlane(*d.fmt_flag) == 0u;
+    const uint32_t parts = counts ? d.count_parts : d.real_parts;
+    if (parts <= 1u) return;   // written by the gather
+    for (uint64_t i = (uint64_t)block * 256u + threadIdx.x; i < d.n; i += (uint64_t)blocks * 256u) {
+        if (counts) static_cast<float*>(d.out)[i] = (float)parts_at<uint32_t>(d, parts, i);
+        else if (!d.cplx) static_cast<float*>(d.out)[i] = (float)parts_at<double>(d, parts, i) * d.scale;
+        else {
+            const ComplexSum v = parts_at<ComplexSum>(d, parts, i);
+            static_cast<float2*>(d.out)[i] = make_float2((float)v.re * d.scale, (float)v.im * d.scale);
+        }
     }
+}
+__global__ __launch_bounds__(256) void sum_parts_kernel(PartsSum d) { sum_parts(d, blockIdx.x, gridDim.x); }
+// Captures of many sizes, a row of work-groups each; the last of a row stamps its capture's completion.
+__global__ __launch_bounds__(256) void batch_sum_parts_kernel(const PartsSum* __restrict__ d, uint32_t* remaining,
+                                                              uint64_t* done) {
+    const uint32_t c = blockIdx.y;
+    const PartsSum s = wave_uniform_load(d + c);
+    if (!s.out) return;
+    sum_parts(s, blockIdx.x, gridDim.x);
+    __syncthreads();
+    if (threadIdx.x == 0 && atomicSub(&remaining[c], 1u) == 1u)
+        atomicMax(reinterpret_cast<unsigned long long*>(&done[c]), (unsigned long long)wall_clock64());
 }
 
 // Voxel (x, y, z) in the tiles of the kernel above: tile, lane of its column and place in it.
@@ -569,33 +546,6 @@ static hipError_t poly_launch(const LdsPolyArgs& a, uint32_t groups, hipStream_t
     hipLaunchKernelGGL(fn, dim3(groups), dim3(256), lds, s, a);
     return hipGetLastError();
 }
-template <class Fz, int KZ, int DEG>
-static hipError_t batch_poly_launch(const BatchPolyArgs& b, uint32_t seg, uint32_t groups, hipStream_t s) {
-    const auto fn = batch_lds_kernel_poly<Fz, KZ, DEG>;
-    size_t lds = 0;
-    const hipError_t e = poly_lds<Fz>(fn, seg, &lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(fn, dim3(groups), dim3(256), lds, s, b);
-    return hipGetLastError();
-}
-template <class Fz>
-static hipError_t batch_poly_rows(const BatchPolyArgs& b, const LdsPolyShape& sh, uint32_t n, hipStream_t s) {
-    if constexpr (Fz::kFormat != kC64Split)
-        if (sh.kz == 16)
-            return sh.deg == 2 ? batch_poly_launch<Fz, 16, 2>(b, sh.seg, n, s) : batch_poly_launch<Fz, 16, 3>(b, sh.seg, n, s);
-    if (sh.kz != 8) return hipErrorInvalidValue;
-    return sh.deg == 2 ? batch_poly_launch<Fz, 8, 2>(b, sh.seg, n, s) : batch_poly_launch<Fz, 8, 3>(b, sh.seg, n, s);
-}
-hipError_t launch_batch_poly(const BatchPolyArgs& b, const LdsPolyShape& sh, int format, uint32_t n, hipStream_t s) {
-    switch (format) {
-        case kCount: return batch_poly_rows<CountRows>(b, sh, n, s);
-        case kF32Split: return batch_poly_rows<F32Rows>(b, sh, n, s);
-        case kF16: return batch_poly_rows<Half16Rows<false>>(b, sh, n, s);
-        case kBF16: return batch_poly_rows<Half16Rows<true>>(b, sh, n, s);
-        case kC64Split: return batch_poly_rows<ComplexRows>(b, sh, n, s);
-        default: return hipErrorInvalidValue;
-    }
-}
 template <class Fz, bool TILES>
 static hipError_t poly_launch_shape(const LdsPolyArgs& a, const LdsPolyShape& sh, uint32_t groups, hipStream_t s) {
     if constexpr (Fz::kFormat != kC64Split)   // two accumulators per voxel: 8 voxels per lane
@@ -603,6 +553,44 @@ static hipError_t poly_launch_shape(const LdsPolyArgs& a, const LdsPolyShape& sh
             return sh.deg == 2 ? poly_launch<Fz, 16, 2, TILES>(a, groups, s) : poly_launch<Fz, 16, 3, TILES>(a, groups, s);
     if (sh.kz != 8) return hipErrorInvalidValue;
     return sh.deg == 2 ? poly_launch<Fz, 8, 2, TILES>(a, groups, s) : poly_launch<Fz, 8, 3, TILES>(a, groups, s);
+}
+template <class Fz, int KZ, int DEG>
+static hipError_t batch_poly_launch(const BatchItems& b, const LdsPolyArgs* caps, uint32_t seg, hipStream_t s) {
+    const auto fn = batch_lds_kernel_poly<Fz, KZ, DEG>;
+    size_t lds = 0;
+    const hipError_t e = poly_lds<Fz>(fn, seg, &lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(fn, dim3(b.n), dim3(256), lds, s, b, caps);
+    return hipGetLastError();
+}
+template <class Fz>
+static hipError_t batch_poly_rows(const BatchItems& b, const LdsPolyArgs* caps, const LdsPolyShape& sh, hipStream_t s) {
+    if constexpr (Fz::kFormat != kC64Split)
+        if (sh.kz == 16)
+            return sh.deg == 2 ? batch_poly_launch<Fz, 16, 2>(b, caps, sh.seg, s) : batch_poly_launch<Fz, 16, 3>(b, caps, sh.seg, s);
+    if (sh.kz != 8) return hipErrorInvalidValue;
+    return sh.deg == 2 ? batch_poly_launch<Fz, 8, 2>(b, caps, sh.seg, s) : batch_poly_launch<Fz, 8, 3>(b, caps, sh.seg, s);
+}
+hipError_t launch_batch_poly(const BatchItems& b, const LdsPolyArgs* caps, const LdsPolyShape& sh, int format,
+                             hipStream_t s) {
+    switch (format) {
+        case kCount: return batch_poly_rows<CountRows>(b, caps, sh, s);
+        case kF32Split: return batch_poly_rows<F32Rows>(b, caps, sh, s);
+        case kF16: return batch_poly_rows<Half16Rows<false>>(b, caps, sh, s);
+        case kBF16: return batch_poly_rows<Half16Rows<true>>(b, caps, sh, s);
+        case kC64Split: return batch_poly_rows<ComplexRows>(b, caps, sh, s);
+        default: return hipErrorInvalidValue;
+    }
+}
+hipError_t launch_sum_parts(const PartsSum& d, hipStream_t s) {
+    const uint32_t blocks = (uint32_t)std::max<uint64_t>(1u, std::min<uint64_t>((d.n + 255u) / 256u, 4096u));
+    hipLaunchKernelGGL(sum_parts_kernel, dim3(blocks), dim3(256), 0, s, d);
+    return hipGetLastError();
+}
+hipError_t launch_batch_sum_parts(const PartsSum* d, uint32_t n, uint32_t* remaining, uint64_t* done, hipStream_t s) {
+    if (n > 65535u) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(batch_sum_parts_kernel, dim3(kBatchSumBlocks, n), dim3(256), 0, s, d, remaining, done);
+    return hipGetLastError();
 }
 LdsPolyArgs lds_poly_args(const ConfocalArgs& c, const LdsPolyShape& sh) {
     LdsPolyArgs a{};
@@ -614,26 +602,24 @@ LdsPolyArgs lds_poly_args(const ConfocalArgs& c, const LdsPolyShape& sh) {
     a.k3 = (float)(A * step * step * step / 2.0);
     return a;
 }
-template <class Fz>
-static hipError_t launch_rows(const LdsPolyArgs& a, const LdsPolyShape& sh, uint32_t parts, hipStream_t s) {
-    const hipError_t e = poly_launch_shape<Fz, false>(a, sh, (uint32_t)poly_tiles(a.c.g, sh.kz) * parts, s);
-    if (e != hipSuccess || !a.parts) return e;
-    const uint64_t n = (uint64_t)a.c.g.n[0] * a.c.g.n[1] * a.c.g.n[2];
-    hipLaunchKernelGGL(lds_parts_sum_kernel<Fz>, dim3((uint32_t)std::min<uint64_t>((n + 255u) / 256u, 4096u)), dim3(256),
-                       0, s, a, parts, n);
-    return hipGetLastError();
-}
 hipError_t launch_lds_poly(const LdsPolyArgs& a, const LdsPolyShape& sh, int format, uint32_t parts, hipStream_t s) {
+    const uint32_t groups = (uint32_t)poly_tiles(a.c.g, sh.kz) * parts;
     switch (format) {
-        case kCount: return launch_rows<CountRows>(a, sh, parts, s);
-        case kF32Split: return launch_rows<F32Rows>(a, sh, parts, s);
-        case kF16: return launch_rows<Half16Rows<false>>(a, sh, parts, s);
-        case kBF16: return launch_rows<Half16Rows<true>>(a, sh, parts, s);
-        case kC64Split: return launch_rows<ComplexRows>(a, sh, parts, s);
+        case kCount: return poly_launch_shape<CountRows, false>(a, sh, groups, s);
+        case kF32Split: return poly_launch_shape<F32Rows, false>(a, sh, groups, s);
+        case kF16: return poly_launch_shape<Half16Rows<false>, false>(a, sh, groups, s);
+        case kBF16: return poly_launch_shape<Half16Rows<true>, false>(a, sh, groups, s);
+        case kC64Split: return poly_launch_shape<ComplexRows, false>(a, sh, groups, s);
         default: return hipErrorInvalidValue;
     }
 }
 uint32_t lds_poly_part_bytes(int format) { return format == kCount ? 4u : format == kC64Split ? 16u : 8u; }
+
+// Parts of rows summed in compensated blocks hold whole blocks where those are short: the blocks, and
+// so the error within them, are those of one part.
+uint32_t part_unit(uint32_t kahan_block) {
+    return kahan_block > 128u ? 4u : kahan_block % 4u == 0u ? kahan_block : kahan_block % 2u ? kahan_block * 4u : kahan_block * 2u;
+}
 
 uint64_t lds_tile_count(const Grid& g, const LdsPolyShape& sh) { return poly_tiles(g, sh.kz); }
 
@@ -720,12 +706,14 @@ LdsPolyShape lds_poly_shape(const Grid& g, float inv2, float lz, double bound, d
 // tiles) 8.65 ms in 1 part, 6.85 in 2, 6.42 in 4, 6.08 in 8, 6.11 in 16 -- more rounds of resident
 // work-groups even out the last one; 1,961 pairs into 45 x 61 x 38 (60 tiles) 0.107 ms in 9 parts,
 // 0.082 in 18, 0.087 in 61.
-uint32_t lds_poly_parts(const Grid& g, const LdsPolyShape& sh, uint32_t P, uint32_t sum_bytes, uint32_t* part_pairs) {
+// Parts are of whole blocks of `unit` pairs.
+uint32_t lds_poly_parts(const Grid& g, const LdsPolyShape& sh, uint32_t P, uint32_t sum_bytes, uint32_t unit,
+                        uint32_t* part_pairs) {
     const uint64_t tiles = poly_tiles(g, sh.kz), vox = (uint64_t)g.n[0] * g.n[1] * g.n[2];
     uint64_t parts = std::max(std::min<uint64_t>((4096u + tiles - 1u) / tiles, P / 128u),
                               std::min<uint64_t>((1024u + tiles - 1u) / tiles, P / 32u));
     parts = std::max<uint64_t>(1u, std::min<uint64_t>(parts, (64ull << 20) / (sum_bytes * vox)));
-    *part_pairs = (uint32_t)(((P + parts - 1u) / parts + 3u) / 4u * 4u);
+    *part_pairs = (uint32_t)(((P + parts - 1u) / parts + unit - 1u) / unit * unit);
     return std::max(1u, (P + *part_pairs - 1u) / *part_pairs);
 }
 

@@ -687,6 +687,26 @@ static void paths_lds_setup(PlanImpl& pl, const std::vector<bpx_pair>& pr, const
     pl.paths = a;
 }
 
+// Default confocal kernel where the polynomial-quotient kernel does not apply: the LDS-staged one where
+// it does (separable grid, flat wall, short bin windows) and has enough tiles to fill the GPU.  Real
+// formats: 16^3 tiles of 256 lanes (16 voxels per lane) from 1,024 tiles, 16^3 tiles of 512 lanes (8
+// per lane) from 512; else, and for complex formats, 16 x 16 x 8 tiles of 256 lanes from 512.
+// Measured at 16,384 pairs (gather ms, the three shapes in that order, texture path last): 256^3
+// 81.7 / 85.8 / 96.7 / 141; 128^3 16.1 / 12.8 / 14.4 / 20.0; 112^3 - / 13.2 / 12.1 / 19.4; 96^3 - / -
+// / 10.2 / 10.0.
+int default_variant(const PlanImpl& pl) {
+    const uint32_t* n = pl.g.n;
+    if (!pl.fused || !pl.sep || !pl.flat) return kDefaultVariant;
+    const uint32_t seg = lds_seg_elems(pl.format);
+    const uint64_t t16 = (uint64_t)((n[0] + 15) / 16) * ((n[1] + 15) / 16) * ((n[2] + 15) / 16);
+    const uint64_t t8 = (uint64_t)((n[0] + 15) / 16) * ((n[1] + 15) / 16) * ((n[2] + 7) / 8);
+    const bool cplx = pl.format == kCF16 || pl.format == kCBF16;   // two accumulators per voxel
+    const bool fits16 = confocal_lds_fits(pl.g.inc, pl.inv2, 16, seg), fits8 = confocal_lds_fits(pl.g.inc, pl.inv2, 8, seg);
+    if (!cplx && t16 >= kLdsDeepTiles && fits16) return kLdsVariant;
+    if (!cplx && t16 >= kLdsMinTiles && fits16) return kLdsVariant + 2;
+    return t8 >= kLdsMinTiles && fits8 ? kLdsVariant + 1 : kDefaultVariant;
+}
+
 PlanImpl* make_plan_single_tap(const CaptureIn& c, const uint32_t n[3], const float zero[3],
                                const float inc[9], const bpx_options* opt) {
     validate_common(c, n);
@@ -804,23 +824,7 @@ PlanImpl* make_plan_single_tap(const CaptureIn& c, const uint32_t n[3], const fl
         pl->lz = pr[0].laser_point[2];
         pl->sep = inc[6] == 0.0f && inc[7] == 0.0f;
         if (!pl->sep) pl->flat = false;
-        // Default kernel: the LDS-staged one where it applies (separable grid, flat wall, short
-        // bin windows) and has enough tiles to fill the GPU.  Real formats: 16^3 tiles of 256
-        // lanes (16 voxels per lane) from 1,024 tiles, 16^3 tiles of 512 lanes (8 per lane)
-        // from 512; else, and for complex formats, 16 x 16 x 8 tiles of 256 lanes from 512.
-        // Measured at 16,384 pairs (gather ms, the three shapes in that order, texture path
-        // last): 256^3 81.7 / 85.8 / 96.7 / 141; 128^3 16.1 / 12.8 / 14.4 / 20.0; 112^3 - /
-        // 13.2 / 12.1 / 19.4; 96^3 - / - / 10.2 / 10.0.
-        const uint32_t seg = lds_seg_elems(pl->format);
-        if (o.variant < 0 && pl->fused && pl->sep && pl->flat) {
-            const uint64_t t16 = (uint64_t)((n[0] + 15) / 16) * ((n[1] + 15) / 16) * ((n[2] + 15) / 16);
-            const uint64_t t8 = (uint64_t)((n[0] + 15) / 16) * ((n[1] + 15) / 16) * ((n[2] + 7) / 8);
-            const bool cplx = pl->format == kCF16 || pl->format == kCBF16;   // two accumulators per voxel
-            const bool fits16 = confocal_lds_fits(inc, pl->inv2, 16, seg), fits8 = confocal_lds_fits(inc, pl->inv2, 8, seg);
-            if (!cplx && t16 >= kLdsDeepTiles && fits16) pl->variant = kLdsVariant;
-            else if (!cplx && t16 >= kLdsMinTiles && fits16) pl->variant = kLdsVariant + 2;
-            else if (t8 >= kLdsMinTiles && fits8) pl->variant = kLdsVariant + 1;
-        }
+        if (o.variant < 0) pl->variant = default_variant(*pl);
         pl->keep_f32 = (o.flags & BPX_FLAG_KEEP_F32_ROWS) != 0;
         pl->auto_variant = o.variant < 0;
         if (pl->fused) {
@@ -928,15 +932,21 @@ void set_fused_variant(PlanImpl& pl, int variant) {
         const size_t vox = (size_t)pl.g.n[0] * pl.g.n[1] * pl.g.n[2];
         size_t bytes = 0;
         if (pl.poly_counts) {
-            pl.poly_parts = lds_poly_parts(pl.g, pl.poly, pl.P, 4u, &pl.poly_part_pairs);
+            pl.poly_parts = lds_poly_parts(pl.g, pl.poly, pl.P, 4u, 4u, &pl.poly_part_pairs);
             if (pl.poly_parts > 1) bytes = pl.poly_parts * vox * 4u;
         }
         if (pl.poly_real) {
             const uint32_t b = lds_poly_part_bytes(rows);
-            pl.real_parts = lds_poly_parts(pl.g, pl.poly, pl.P, b, &pl.real_part_pairs);
+            pl.real_parts = lds_poly_parts(pl.g, pl.poly, pl.P, b, part_unit(pl.kahan_block), &pl.real_part_pairs);
             if (pl.real_parts > 1) bytes = std::max(bytes, pl.real_parts * vox * b);
         }
         if (bytes > pl.parts.bytes) pl.parts.alloc(bytes);
+    }
+    pl.tex_parts = 1;
+    if (pl.auto_variant && !pl.poly_real && !pl.lds_tiles && variant == kDefaultVariant) {
+        pl.tex_parts = split_parts(pl.tiles, pl.P, part_unit(pl.kahan_block), &pl.tex_part_pairs);
+        const size_t bytes = (size_t)pl.tex_parts * pl.g.n[0] * pl.g.n[1] * pl.g.n[2] * (pl.cplx ? 16u : 8u);
+        if (pl.tex_parts > 1 && bytes > pl.parts.bytes) pl.parts.alloc(bytes);
     }
     if ((pl.rows16 || pl.poly_counts) && !pl.fmt_flag.ptr) {
         pl.fmt_flag.alloc(4);
@@ -1064,6 +1074,11 @@ void PlanImpl::execute(hipStream_t s) {
         a.kahan_block = kahan_block;
         const auto gather = [&](int rows) {
             const bool counts = rows == kCount;
+            if (tex_parts > 1) {
+                hip_check(launch_split(a, SplitPairs{parts.ptr, tex_part_pairs, 0u}, rows, tex_parts, sep, flat, s),
+                          "confocal gather kernel (pairs split)");
+                return;
+            }
             if (!counts && !poly_real) {
                 hip_check(launch_confocal(a, rows, variant, sep, flat, s), "confocal gather kernel");
                 return;
@@ -1090,6 +1105,11 @@ void PlanImpl::execute(hipStream_t s) {
             a.fmt_mask = a.fmt_want = rows16 ? 1u : 2u;
         }
         gather(row_format);
+        const uint32_t count_parts = poly_counts ? poly_parts : 0u, own_parts = poly_real ? real_parts : tex_parts;
+        if (count_parts > 1u || own_parts > 1u)
+            hip_check(launch_sum_parts(PartsSum{vol.ptr, parts.ptr, static_cast<const uint32_t*>(fmt_flag.ptr), nvox,
+                                                count_parts, own_parts, cplx ? 1u : 0u, scale}, s),
+                      "partial sums kernel");
     } else {
         hip_check(launch_ztable(0, t0, dT, 0.0f, T + 1, static_cast<float*>(Z.ptr), s),
                   "threshold table kernel");
@@ -1197,7 +1217,7 @@ static void window_lds_setup(PlanImpl& pl, const std::vector<bpx_pair>& pr, floa
     pl.ldh = a.ldp;
     // double sums: a split changes their last bits only; half the parts of the integer kernel
     pl.poly = sh;
-    pl.poly_parts = lds_poly_parts(pl.g, sh, pl.P, 8u, &a.part_pairs);
+    pl.poly_parts = lds_poly_parts(pl.g, sh, pl.P, 8u, 4u, &a.part_pairs);
     if (pl.poly_parts > 1) pl.parts.alloc((size_t)pl.poly_parts * pl.g.n[0] * pl.g.n[1] * pl.g.n[2] * 8u);
 }
 

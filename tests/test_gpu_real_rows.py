@@ -89,3 +89,39 @@ def test_tune_may_keep_the_default_kernel(gpu):
         plan.execute()
         assert plan.info()["kernel"] == got["kernel"]
         assert np.all(np.abs(plan.volume() - before) <= 68 * EPS * before)
+
+
+# coarse grids and long time axes, whose tiles' bin windows or column polynomials are out of the LDS
+# kernel's range: non-round volumes, one voxel, a wall that is not flat, a rotated basis
+SPLIT_CASES = [((9, 7, 5), False, False), ((24, 24, 24), False, False), ((1, 1, 1), False, False),
+               ((16, 8, 9), True, False), ((11, 17, 8), False, True)]
+
+
+@pytest.mark.parametrize("storage,cplx", [("f32", False), ("bf16", False), ("f32", True), ("f16", True)])
+@pytest.mark.parametrize("N,tilted,rotated", SPLIT_CASES)
+def test_split_pairs_equal_the_whole(gpu, N, tilted, rotated, storage, cplx):
+    """Pairs split over work-groups on the texture path, against the unsplit kernel of the explicit
+    variant; tolerance as above."""
+    pr = pairs_of(31, 33)
+    if tilted:
+        pr["laser_point"][:, 2] = np.linspace(0, 0.05, len(pr)).astype(f32)
+        pr["camera_point"] = pr["laser_point"]
+    T, dT = 3000, 0.0012
+    rng = np.random.default_rng(N[0])
+    H = rng.gamma(0.5, 2.0, (len(pr), T)).astype(f32)
+    if cplx:
+        H = (H + 1j * rng.gamma(0.5, 2.0, H.shape)).astype(np.complex64)
+    zero, inc = basis(N, (0.03, -0.02, 0.75), (0.8, 0.8, 0.6))
+    if rotated:
+        inc = inc + np.array([0, 0, 0.004, 0, 0, 0.002, -0.004, 0.001, 0], f32)
+    vols = []
+    for variant in (-1, 5):
+        with gpu.Plan(H, pr, N, zero, inc, 0.8, dT, variant=variant, storage=storage) as plan:
+            plan.execute()
+            plan.execute()
+            assert plan.info()["kernel"].startswith("confocal_kernel"), plan.info()
+            vols.append(plan.volume())
+    a, b = vols
+    assert np.abs(b).min() > 0
+    for x, y in ((a.real, b.real), (a.imag, b.imag)):
+        assert np.all(np.abs(x.astype(np.float64) - y) <= 68 * EPS * np.abs(y).astype(np.float64))
