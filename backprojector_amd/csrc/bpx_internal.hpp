@@ -74,6 +74,8 @@ struct LdsPolyArgs {
     // every tile of the grid
     const uint32_t* tiles;
     const uint32_t* n_tiles;
+    const uint32_t* fill;   // TileListArgs::fill; quarters below `dense` are left out
+    uint32_t dense;
     float k1, k2, k3;    // Taylor coefficients' constants: -inv2 step, inv2 step^2 / 2, inv2 step^3 / 2
 };
 // Fine-voxel lists sorted into tiles of that kernel (octree): the voxels of well-filled tiles are
@@ -81,10 +83,10 @@ struct LdsPolyArgs {
 struct TileListArgs {
     Grid g;
     uint32_t* mask;      // 16 bits per tile column, [tiles][256] (cleared by the caller)
-    uint32_t* fill;      // listed voxels per tile (cleared)
+    uint32_t* fill;      // listed voxels per quarter of a tile, a wave's 8 x 8 columns (cleared)
     uint32_t* counts;    // [0] listed tiles, [1] other voxels (cleared)
-    uint32_t* tiles;     // the well-filled tiles
-    uint32_t* rest;      // packed voxels of the others
+    uint32_t* tiles;     // the tiles with a well-filled quarter
+    uint32_t* rest;      // packed voxels of the other quarters
 };
 
 // Factorised exhaustive-grid kernel parameters (threshold table in path-length space).
@@ -384,7 +386,7 @@ uint64_t lds_tile_count(const Grid& g, const LdsPolyShape& sh);
 hipError_t launch_tile_lists(const TileListArgs& a, const LdsPolyShape& sh, const uint32_t* const lists[2],
                              const uint32_t n[2], uint32_t dense, hipStream_t s);
 hipError_t launch_lds_counts_tiles(LdsPolyArgs a, const LdsPolyShape& sh, const TileListArgs& t, uint32_t max_tiles,
-                                   uint32_t groups, hipStream_t s);
+                                   uint32_t dense, uint32_t groups, hipStream_t s);
 // The texture-path kernel with the pairs split over work-groups (2 voxels per lane, fused rows).
 struct SplitPairs {
     void* parts;            // [parts][voxels] partial sums, double (complex: two)

@@ -290,7 +290,8 @@ __device__ __forceinline__ uint32_t poly_tile(const LdsPolyArgs& a, uint32_t blo
     if (TILES && (count == 0u || part * part_pairs >= a.c.P)) return 0u;
     const uint32_t tile = TILES ? __builtin_amdgcn_readfirstlane(a.tiles[index]) : xcd_remap(index, tiles);
     const uint32_t p0 = part * part_pairs, p1 = min(p0 + part_pairs, a.c.P);
-    const ColumnTile<KZ> t(g, tile, w, lane);
+    ColumnTile<KZ> t(g, tile, w, lane);
+    if (TILES) t.idle = t.idle || __builtin_amdgcn_readfirstlane(a.fill[4u * tile + w]) < a.dense;
     float dz2[KZ];   // uniform
 #pragma unroll
     for (int r = 0; r < KZ; ++r) {
@@ -362,7 +363,7 @@ __device__ __forceinline__ uint32_t poly_tile(const LdsPolyArgs& a, uint32_t blo
     for (uint32_t b = 0; b < nstage; ++b) {
         if (b + 1u < nstage) stage(b + 1u);
         const float4* mb = meta + (b & 1u) * PS;
-        const uint32_t np = min(PS, p1 - p0 - b * PS);
+        const uint32_t np = t.idle ? 0u : min(PS, p1 - p0 - b * PS);
         float4 m = mb[0];
 #pragma unroll 1
         for (uint32_t i = 0; i < np; ++i) {
@@ -463,35 +464,39 @@ __device__ __forceinline__ TileVoxel tile_voxel(const Grid& g, uint32_t x, uint3
     return t;
 }
 
-// Marks the listed voxels: one bit per voxel (16 per column of a tile) and the number per tile.
-// Lists follow the octree's blocks, so a wave's voxels share few tiles; the counters are updated
-// once per (wave, tile).
+// Marks the listed voxels: one bit per voxel (16 per column of a tile) and the number per quarter of a
+// tile.  Lists follow the octree's blocks, so a wave's voxels share few quarters; the counters are
+// updated once per (wave, quarter).
 template <int KZ>
 __global__ __launch_bounds__(256) void tile_mark_kernel(TileListArgs a, const uint32_t* __restrict__ voxels, uint32_t n) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    TileVoxel t{0xffffffffu, 0u, 0u};
+    TileVoxel t{0u, 0u, 0u};
+    uint32_t q = 0xffffffffu;   // quarter
     if (i < n) {
         const uint32_t v = voxels[i];
         t = tile_voxel<KZ>(a.g, v & 1023u, (v >> 10) & 1023u, v >> 20);
+        q = 4u * t.tile + (t.lane >> 6);
         const uint32_t col = t.tile * 256u + t.lane;
         atomicOr(&a.mask[col >> 1], 1u << (t.r + 16u * (col & 1u)));
     }
     bool left = i < n;
     while (__ballot(left) != 0ull) {
         const uint32_t first = (uint32_t)__builtin_ctzll(__ballot(left));
-        const uint32_t tile = __builtin_amdgcn_readlane(t.tile, first);
-        const bool mine = left && t.tile == tile;
+        const uint32_t quarter = __builtin_amdgcn_readlane(q, first);
+        const bool mine = left && q == quarter;
         const uint64_t m = __ballot(mine);
-        if ((threadIdx.x & 63u) == first) atomicAdd(&a.fill[tile], (uint32_t)__builtin_popcountll(m));
+        if ((threadIdx.x & 63u) == first) atomicAdd(&a.fill[quarter], (uint32_t)__builtin_popcountll(m));
         left = left && !mine;
     }
 }
-// Tiles with at least `dense` listed voxels, in any order (each is computed by itself).
+// Tiles with a quarter of at least `dense` listed voxels, in any order (each is computed by itself).
 __global__ __launch_bounds__(256) void tile_pick_kernel(TileListArgs a, uint32_t tiles, uint32_t dense) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < tiles && a.fill[i] >= dense) a.tiles[atomicAdd(&a.counts[0], 1u)] = i;
+    if (i >= tiles) return;
+    const uint4 f = reinterpret_cast<const uint4*>(a.fill)[i];
+    if (max(max(f.x, f.y), max(f.z, f.w)) >= dense) a.tiles[atomicAdd(&a.counts[0], 1u)] = i;
 }
-// The listed voxels of the other tiles, 64 neighbours of the list at a time.
+// The listed voxels of the other quarters, 64 neighbours of the list at a time.
 template <int KZ>
 __global__ __launch_bounds__(256) void tile_rest_kernel(TileListArgs a, const uint32_t* __restrict__ voxels, uint32_t n,
                                                         uint32_t dense) {
@@ -500,7 +505,8 @@ __global__ __launch_bounds__(256) void tile_rest_kernel(TileListArgs a, const ui
     bool rest = false;
     if (i < n) {
         v = voxels[i];
-        rest = a.fill[tile_voxel<KZ>(a.g, v & 1023u, (v >> 10) & 1023u, v >> 20).tile] < dense;
+        const TileVoxel t = tile_voxel<KZ>(a.g, v & 1023u, (v >> 10) & 1023u, v >> 20);
+        rest = a.fill[4u * t.tile + (t.lane >> 6)] < dense;
     }
     const uint64_t m = __ballot(rest);
     uint32_t base = 0;
@@ -508,7 +514,8 @@ __global__ __launch_bounds__(256) void tile_rest_kernel(TileListArgs a, const ui
     base = __builtin_amdgcn_readfirstlane(base);
     if (rest) a.rest[base + (uint32_t)__builtin_popcountll(m & ((1ull << lane) - 1ull))] = v;
 }
-// Volume values of the marked voxels of the listed tiles from their integer partial sums.
+// Volume values of the marked voxels of the listed tiles' well-filled quarters from their integer
+// partial sums.
 template <int KZ>
 __global__ __launch_bounds__(256) void tile_store_kernel(TileListArgs a, LdsPolyArgs p, uint32_t groups) {
     const uint32_t count = a.counts[0];
@@ -516,7 +523,7 @@ __global__ __launch_bounds__(256) void tile_store_kernel(TileListArgs a, LdsPoly
     const uint32_t part_pairs = list_part_pairs(p.c.P, count, groups), parts = (p.c.P + part_pairs - 1u) / part_pairs;
     const uint32_t tile = a.tiles[blockIdx.x], col = tile * 256u + threadIdx.x;
     const uint32_t bits = a.mask[col >> 1] >> (16u * (col & 1u)) & 0xffffu;
-    if (!bits) return;
+    if (!bits || a.fill[4u * tile + (threadIdx.x >> 6)] < p.dense) return;
     const uint32_t ntz = (a.g.n[2] + KZ - 1u) / KZ, nty = (a.g.n[1] + 15u) / 16u;
     const uint32_t tz = tile % ntz, ty = tile / ntz % nty, tx = tile / ntz / nty, w = threadIdx.x >> 6;
     const uint32_t ix = tx * 16u + (w & 1u) * 8u + (threadIdx.x & 7u), iy = ty * 16u + (w >> 1) * 8u + ((threadIdx.x >> 3) & 7u);
@@ -640,7 +647,9 @@ hipError_t launch_tile_lists(const TileListArgs& a, const LdsPolyShape& sh, cons
     return sh.kz == 16 ? tile_lists<16>(a, lists, n, dense, s) : tile_lists<8>(a, lists, n, dense, s);
 }
 hipError_t launch_lds_counts_tiles(LdsPolyArgs a, const LdsPolyShape& sh, const TileListArgs& t, uint32_t max_tiles,
-                                   uint32_t groups, hipStream_t s) {
+                                   uint32_t dense, uint32_t groups, hipStream_t s) {
+    a.fill = t.fill;
+    a.dense = dense;
     a.tiles = t.tiles;
     a.n_tiles = t.counts;
     const hipError_t e = poly_launch_shape<CountRows, true>(a, sh, groups, s);

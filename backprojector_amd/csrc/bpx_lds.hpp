@@ -49,6 +49,9 @@ template <int KZ>
 struct ColumnTile {
     uint32_t tx, ty, ix, iy, iz0, cx, cy;
     float vx, vy;
+    // The wave's 8 x 8 columns all lie past the grid (uniform): it stages with the others and skips
+    // the updates, which leaves its issue slots to them.
+    bool idle;
     __device__ __forceinline__ ColumnTile(const Grid& g, uint32_t tile, uint32_t w, uint32_t lane) {
         const uint32_t ntz = (g.n[2] + KZ - 1u) / KZ, nty = (g.n[1] + 15u) / 16u;
         const uint32_t tz = tile % ntz, txy = tile / ntz;
@@ -56,6 +59,7 @@ struct ColumnTile {
         tx = txy / nty;
         ix = tx * 16u + (w & 1u) * 8u + (lane & 7u);
         iy = ty * 16u + (w >> 1) * 8u + (lane >> 3);
+        idle = tx * 16u + (w & 1u) * 8u >= g.n[0] || ty * 16u + (w >> 1) * 8u >= g.n[1];
         iz0 = min(tz * KZ, g.n[2] - KZ);   // the last slab reaches back over its neighbour
         cx = min(ix, g.n[0] - 1u);
         cy = min(iy, g.n[1] - 1u);

@@ -168,7 +168,7 @@ PlanImpl* make_plan_octree(const CaptureIn& c, const uint32_t n[3], const float 
         hip_check(hipMemset(st->count_rows.ptr, 0, pl->H.bytes), "hipMemset(count rows)");
         st->count_flag.alloc(4);
         st->tile_mask.alloc(tiles * 512u);
-        st->tile_fill.alloc(4u * tiles);
+        st->tile_fill.alloc(16u * tiles);
         st->tile_list.alloc(4u * tiles);
         st->tile_counts.alloc(8);
         StageJob job = stage_job(*pl);
@@ -222,15 +222,17 @@ static void build_winmax(PlanImpl& pl, uint32_t P, const uint32_t* rows, hipStre
     }
 }
 
-// The fine voxels of a capture of counts (n of the fine list, n_fb of the fallback list): tiles
-// with at least 3 listed voxels in 10 are computed whole from the count rows and stored where
-// listed, the other voxels one by one.  The tile kernel runs 6e12 updates/s, the gather of
-// listed voxels 1.75e12: a tile is the cheaper from 29 % on.
+// The fine voxels of a capture of counts (n of the fine list, n_fb of the fallback list): quarters of
+// tiles (8 x 8 columns, a wave) with at least 3 listed voxels in 10 are computed whole from the count
+// rows and stored where listed, the other voxels one by one beside them.  Alone, a quarter is the
+// cheaper from 29 % on (6e12 updates/s against 1.75e12).  Learned 256^3 executions, ms: one with its
+// volume, whole tiles from 30 % 14.6 to 15.3, quarters from 20 / 30 / 45 / 60 % 13.1 / 12.9 / 12.7 / 12.8;
+// three others alone, quarters from 30 / 40 / 50 % 12.4, 13.8, 15.4 / 13.1, 14.7, 16.1 / 13.7, 15.5, 17.7.
 static void gather_tiles(PlanImpl& pl, const OctFineArgs& fine, uint32_t n, uint32_t n_fb, hipStream_t s) {
     OctreeState& st = *pl.oct;
     const uint32_t total = n + n_fb;
     if (!total) return;
-    const uint32_t cells = 256u * (uint32_t)st.poly.kz, dense = cells * 3u / 10u;
+    const uint32_t cells = 256u * (uint32_t)st.poly.kz, dense = cells / 4u * 3u / 10u;
     const uint64_t tiles = lds_tile_count(pl.g, st.poly);
     TileListArgs t{};
     t.g = pl.g;
@@ -240,7 +242,7 @@ static void gather_tiles(PlanImpl& pl, const OctFineArgs& fine, uint32_t n, uint
     t.tiles = static_cast<uint32_t*>(st.tile_list.ptr);
     t.rest = static_cast<uint32_t*>(st.flags.ptr);   // the child flags are done with
     hip_check(launch_fill(static_cast<float*>(st.tile_mask.ptr), tiles * 128u, 0.0f, s), "fill kernel");
-    hip_check(launch_fill(static_cast<float*>(st.tile_fill.ptr), tiles, 0.0f, s), "fill kernel");
+    hip_check(launch_fill(static_cast<float*>(st.tile_fill.ptr), 4u * tiles, 0.0f, s), "fill kernel");
     hip_check(launch_fill(static_cast<float*>(st.tile_counts.ptr), 2, 0.0f, s), "fill kernel");
     const uint32_t* lists[2] = {static_cast<const uint32_t*>(st.fine_list.ptr),
                                 static_cast<const uint32_t*>(st.fb_voxels.ptr)};
@@ -255,7 +257,7 @@ static void gather_tiles(PlanImpl& pl, const OctFineArgs& fine, uint32_t n, uint
     f.n_dev = t.counts + 1;
     f.E = st.count_rows.ptr;
     hip_check(launch_oct_fine_counts(f, st.side), "octree fine kernel (count rows)");
-    // at most total / dense such tiles; 4,096 work-groups share them out in parts of the pairs
+    // at most total / dense tiles with such a quarter; 4,096 work-groups share them out in parts of the pairs
     const uint32_t max_tiles = (uint32_t)std::min<uint64_t>(tiles, total / dense);
     if (max_tiles) {
         const uint32_t groups = std::max(max_tiles, 4096u);
@@ -276,7 +278,7 @@ static void gather_tiles(PlanImpl& pl, const OctFineArgs& fine, uint32_t n, uint
         c.lz = pl.lz;
         LdsPolyArgs a = lds_poly_args(c, st.poly);
         a.parts = static_cast<uint32_t*>(st.tile_parts.ptr);
-        hip_check(launch_lds_counts_tiles(a, st.poly, t, max_tiles, groups, s), "octree tile gather kernel");
+        hip_check(launch_lds_counts_tiles(a, st.poly, t, max_tiles, dense, groups, s), "octree tile gather kernel");
     }
 }
 

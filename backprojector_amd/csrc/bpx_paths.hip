@@ -190,7 +190,7 @@ __global__ __launch_bounds__(256, GRID ? 2 : 3) void paths_lds_kernel(PathsLdsAr
         const uint32_t sl = (b & 1u) * CS;
         if constexpr (GRID) {
             const uint32_t chunk = b / lasers, l = first + b % lasers;
-            if (b % lasers == 0u) {
+            if (b % lasers == 0u && !t.idle) {
 #pragma unroll
                 for (uint32_t c = 0; c < CS; ++c) {
                     const float4 sp = a.spads[min(chunk * CS + c, a.C - 1u)];
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(256, GRID ? 2 : 3) void paths_lds_kernel(PathsLdsAr
                 const float z = lp.z - vz[r];
                 d1[r] = lp.w + exact_root(xy + z * z);
             }
-            const uint32_t n = min(CS, a.C - chunk * CS);
+            const uint32_t n = t.idle ? 0u : min(CS, a.C - chunk * CS);
 #pragma unroll
             for (uint32_t c = 0; c < CS; ++c)
                 if (const int2 m = win[sl + c]; c < n && __builtin_amdgcn_readfirstlane(m.y) != kNoWindow) {
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(256, GRID ? 2 : 3) void paths_lds_kernel(PathsLdsAr
                 }
             settle(n);
         } else {
-            const uint32_t n = min(CS, end - first - b * CS);
+            const uint32_t n = t.idle ? 0u : min(CS, end - first - b * CS);
 #pragma unroll 1
             for (uint32_t c = 0; c < n; ++c) {
                 const int2 m = win[sl + c];

@@ -202,7 +202,7 @@ __global__ __launch_bounds__(256, 3) void window_lds_kernel(WindowLdsArgs a) {
     for (uint32_t b = 0; b < nstage; ++b) {
         if (b + 1u < nstage) stage(b + 1u);
         const float4* mb = meta + (b & 1u) * PS;
-        const uint32_t np = min(PS, p1 - p0 - b * PS);
+        const uint32_t np = t.idle ? 0u : min(PS, p1 - p0 - b * PS);
 #pragma unroll 1
         for (uint32_t i = 0; i < np; ++i) {
             const float4 m = mb[i];
