@@ -259,9 +259,10 @@ bpx_status bpx_plan_execute(bpx_plan plan, void* hip_stream) {
             hip_check(hipEventRecord(pl.ready, pl.stream), "hipEventRecord");
             hip_check(hipStreamWaitEvent(s, pl.ready, 0), "hipStreamWaitEvent");
         }
-        hip_check(hipStreamWaitEvent(s, pl.done, 0), "hipStreamWaitEvent");
+        if (pl.foreign) hip_check(hipStreamWaitEvent(s, pl.done, 0), "hipStreamWaitEvent");
+        pl.foreign = pl.foreign || s != pl.stream;   // its own stream keeps its executions in order
         pl.execute(s);
-        hip_check(hipEventRecord(pl.done, s), "hipEventRecord");
+        if (pl.foreign) hip_check(hipEventRecord(pl.done, s), "hipEventRecord");
     });
 }
 
@@ -392,6 +393,11 @@ bpx_status bpx_plan_benchmark(bpx_plan plan, int32_t warmup, int32_t iterations,
         if (!plan || !out || iterations <= 0 || warmup < 0) fail(BPX_ERR_INVALID_ARGUMENT, "bad arguments");
         PlanImpl& pl = *plan->impl;
         plan_wait(pl);
+        struct Timed {
+            bool& on;
+            explicit Timed(bool& b) : on(b) { on = true; }
+            ~Timed() { on = false; }
+        } timed(pl.timed);
         for (int i = 0; i < warmup; ++i) pl.execute(pl.stream);
         hip_check(hipStreamSynchronize(pl.stream), "hipStreamSynchronize");
         double table_ms = 0, gather_ms = 0;
@@ -481,7 +487,7 @@ bpx_status bpx_plan_tune(bpx_plan plan, int32_t reps, int32_t* variant) {
 void bpx_plan_destroy(bpx_plan plan) {
     if (!plan) return;
     (void)hipStreamSynchronize(plan->impl->stream);
-    if (plan->impl->done) (void)hipEventSynchronize(plan->impl->done);
+    if (plan->impl->foreign) (void)hipEventSynchronize(plan->impl->done);
     delete plan;
 }
 

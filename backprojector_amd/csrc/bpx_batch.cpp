@@ -641,7 +641,7 @@ bpx_status bpx_batch_create(const bpx_capture_desc* captures, uint32_t count, co
 void bpx_batch_destroy(bpx_batch batch) {
     if (!batch) return;
     (void)hipStreamSynchronize(batch->impl->stream);
-    if (batch->impl->done) (void)hipEventSynchronize(batch->impl->done);
+    if (batch->impl->foreign) (void)hipEventSynchronize(batch->impl->done);
     delete batch;
 }
 

@@ -171,7 +171,10 @@ struct PlanImpl {
     uint32_t rows_in = 0;                // rows of the capture the plan was made from
     uint32_t stage_zb = 0, stage_sb = 0; // its blocks in the two staging passes
     hipEvent_t ev[8] = {};
-    hipEvent_t done = nullptr;           // recorded after each bpx_plan_execute, on its stream
+    bool timed = false;                  // executions record ev[0] .. ev[3]
+    // recorded after each bpx_plan_execute, on its stream, from the first one on a caller's stream on
+    hipEvent_t done = nullptr;
+    bool foreign = false;
     hipEvent_t ready = nullptr;          // work queued on the plan's own stream (caller-stream runs)
     std::unique_ptr<OctreeState> oct;
     ~PlanImpl();

@@ -311,6 +311,7 @@ struct StageJob {
     float inv_scale, t0, dT;
     uint32_t z_first, s_first;
     int32_t alt_format, count_rows;
+    uint32_t clear_flag;        // the first pass sets *fmt_flag to 0
     uint32_t skip_mask;         // nothing is staged while *fmt_flag has one of these bits
 };
 // raw[r][c] = src[map[r]][from + c - cfrom] for c in [cfrom, cfrom + ncopy), else 0

@@ -310,6 +310,7 @@ __global__ __launch_bounds__(256) void stage_z_kernel(const StageJob* __restrict
         const StageJob& jb = jobs[stage_job_of<true>(jobs, n_jobs, blk)];
         const uint32_t j = (blk - jb.z_first) * 256u + threadIdx.x;
         if (j <= jb.Tc) stage_z_entry(jb, j);
+        if (jb.clear_flag && j == 0u) *const_cast<uint32_t*>(jb.fmt_flag) = 0u;
     }
 }
 

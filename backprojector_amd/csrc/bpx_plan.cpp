@@ -603,7 +603,7 @@ static void make_events(PlanImpl& pl) {
 
 void plan_wait(const PlanImpl& pl) {
     hip_check(hipStreamSynchronize(pl.stream), "hipStreamSynchronize");
-    if (pl.done) hip_check(hipEventSynchronize(pl.done), "hipEventSynchronize");
+    if (pl.foreign) hip_check(hipEventSynchronize(pl.done), "hipEventSynchronize");
 }
 
 // Exhaustive-grid structure: p = l*C + c with laser data depending only on l and camera
@@ -888,6 +888,7 @@ StageJob stage_job(const PlanImpl& pl) {
     j.win = static_cast<const uint32_t*>(pl.win.ptr);
     j.alt_format = pl.rows16 ? kF16 : pl.row_format;
     j.count_rows = pl.poly_counts ? 1 : 0;
+    j.clear_flag = j.fmt_flag ? 1u : 0u;
     j.inv_scale = 1.0f / pl.scale;
     j.t0 = pl.t0;
     j.dT = pl.dT;
@@ -970,15 +971,19 @@ void PlanImpl::execute(hipStream_t s) {
         return;
     }
     const size_t nvox = (size_t)g.n[0] * g.n[1] * g.n[2];
+    // a recorded event costs the GPU about as much as a small kernel's launch
+    const auto mark = [&](int k) {
+        if (timed) hip_check(hipEventRecord(ev[k], s), "hipEventRecord");
+    };
     if (path == kPathWindow) {
         if (P == 0 || T < 2) {
             hip_check(hipMemsetAsync(vol.ptr, 0, nvox * (cplx ? 8 : 4), s), "hipMemsetAsync");
             return;
         }
-        hip_check(hipEventRecord(ev[0], s), "hipEventRecord");
+        mark(0);
         hip_check(launch_prefix(static_cast<const float*>(raw.ptr), P, T, cplx ? 1 : 0, H.ptr, ldh, s),
                   "prefix kernel");
-        hip_check(hipEventRecord(ev[1], s), "hipEventRecord");
+        mark(1);
         hip_check(launch_ztable(1, t0, dT, half_width, T, static_cast<float*>(Z.ptr), s), "window table (start)");
         hip_check(launch_ztable(2, t0, dT, half_width, T, static_cast<float*>(Z2.ptr), s), "window table (end)");
         if (poly.kz) {
@@ -994,12 +999,12 @@ void PlanImpl::execute(hipStream_t s) {
             a.parts = poly_parts > 1 ? static_cast<double*>(parts.ptr) : nullptr;
             hip_check(launch_window_tables(a, static_cast<double*>(win_lo.ptr), static_cast<double*>(win_hi.ptr), s),
                       "window threshold kernel");
-            hip_check(hipEventRecord(ev[2], s), "hipEventRecord");
+            mark(2);
             hip_check(launch_window_lds(a, poly, poly_parts, s), "window gather kernel (LDS-staged)");
-            hip_check(hipEventRecord(ev[3], s), "hipEventRecord");
+            mark(3);
             return;
         }
-        hip_check(hipEventRecord(ev[2], s), "hipEventRecord");
+        mark(2);
         WindowArgs a{};
         a.PS = H.ptr;
         a.pairs = static_cast<const float*>(pair8.ptr);
@@ -1018,16 +1023,16 @@ void PlanImpl::execute(hipStream_t s) {
         a.c1_hi = c1_hi;
         a.confocal = all_confocal ? 1u : 0u;
         hip_check(launch_window(a, cplx ? 1 : 0, s), "window gather kernel");
-        hip_check(hipEventRecord(ev[3], s), "hipEventRecord");
+        mark(3);
         return;
     }
     if (P == 0) {
         hip_check(hipMemsetAsync(vol.ptr, 0, nvox * (cplx ? 8 : 4), s), "hipMemsetAsync");
         return;
     }
-    // events: ev[0] | split-layout row padding | ev[1] | tables (fused: all staging) | ev[2] |
+    // marks: ev[0] | split-layout row padding | ev[1] | tables (fused: all staging) | ev[2] |
     // gather | ev[3]
-    hip_check(hipEventRecord(ev[0], s), "hipEventRecord");
+    mark(0);
     if (paths.seg) {
         if (format != kF32)
             hip_check(launch_quantise_rows(static_cast<const float*>(raw.ptr), (uint64_t)P * T, format, 1.0f / scale,
@@ -1037,16 +1042,16 @@ void PlanImpl::execute(hipStream_t s) {
         hip_check(launch_pad_rows(static_cast<const float*>(raw.ptr), P, T, T, H.ptr, ldh, format,
                                   1.0f / scale, s),
                   "row staging kernel");
-    hip_check(hipEventRecord(ev[1], s), "hipEventRecord");
+    mark(1);
     if (path == kPathConfocal) {
         if (fused) {
-            if (rows16 || poly_counts) {
-                hip_check(launch_fill(static_cast<float*>(fmt_flag.ptr), 1, 0.0f, s), "fill kernel");
+            const StageJob* const job = static_cast<const StageJob*>(stage.ptr);
+            hip_check(launch_stage(job, 1u, stage_zb, 0u, s), "path-length table kernel");   // clears the flag
+            if (rows16 || poly_counts)
                 hip_check(launch_exact16_check(static_cast<const float*>(raw.ptr), (uint64_t)P * T,
                                                static_cast<uint32_t*>(fmt_flag.ptr), s),
                           "exact fp16 check kernel");
-            }
-            stage_rows(*this, s);
+            hip_check(launch_stage(job, 1u, 0u, stage_sb, s), "row staging kernel");
         } else {
             hip_check(launch_ztable(0, t0, dT, 0.0f, T + 1, static_cast<float*>(Z.ptr), s),
                       "path-length table kernel");
@@ -1054,7 +1059,7 @@ void PlanImpl::execute(hipStream_t s) {
                                     static_cast<float*>(S.ptr), lds, 1u, 0u, s),
                       "threshold table kernel");
         }
-        hip_check(hipEventRecord(ev[2], s), "hipEventRecord");
+        mark(2);
         ConfocalArgs a{};
         a.H = H.ptr;
         a.S = static_cast<const float*>(S.ptr);
@@ -1113,7 +1118,7 @@ void PlanImpl::execute(hipStream_t s) {
     } else {
         hip_check(launch_ztable(0, t0, dT, 0.0f, T + 1, static_cast<float*>(Z.ptr), s),
                   "threshold table kernel");
-        hip_check(hipEventRecord(ev[2], s), "hipEventRecord");
+        mark(2);
         if (paths.seg) {
             PathsLdsArgs a = paths;
             a.rows = static_cast<const float*>(format == kF32 ? raw.ptr : H.ptr);
@@ -1164,7 +1169,7 @@ void PlanImpl::execute(hipStream_t s) {
             hip_check(launch_pairs(a, format, variant, s), "pairs gather kernel");
         }
     }
-    hip_check(hipEventRecord(ev[3], s), "hipEventRecord");
+    mark(3);
 }
 
 // The LDS-staged window kernel where it applies: real samples, confocal pairs on a flat wall, bin

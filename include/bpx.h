@@ -408,11 +408,12 @@ void bpx_plan_destroy(bpx_plan plan);
 bpx_status bpx_copy_benchmark(uint64_t bytes, int32_t iterations, double* mean_ms);
 
 /* ------------------------------------------------------------------ batched uneven captures
- * Many confocal fp32 captures of different sizes reconstructed by ONE persistent work-queue
- * launch over (capture, tile) items; the per-batch sequence (staging of every capture, queue
- * reset, gather) is a hipGraph replayed by bpx_batch_execute.  Each volume is bit-identical to
- * bpx_backprojection of that capture alone.  No reference counterpart: the reference runs one
- * capture per call_cuda_backprojection (backproject_cuda.cu:370-500); a batch is that call
+ * Many confocal captures of different sizes reconstructed by a few launches over (capture, part of
+ * its pairs, tile) items, and persistent work queues for the captures that the item kernels do not
+ * take; the per-batch sequence (staging of every capture, gathers, partial sums) is a hipGraph
+ * replayed by bpx_batch_execute.  Each volume is bit-identical to bpx_backprojection of that capture
+ * alone.  No reference counterpart: the reference runs one capture per call_cuda_backprojection
+ * (backproject_cuda.cu:370-500); a batch is that call
  * applied to each capture. */
 typedef struct bpx_capture_desc {
     const float* transient_chunk;   /* as bpx_backprojection */
