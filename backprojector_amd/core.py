@@ -382,7 +382,7 @@ class Net:
 
 
 class Batch:
-    """Many confocal captures reconstructed by one persistent work-queue launch replayed from a
+    """Many confocal captures reconstructed by a few launches over items of all of them, replayed from a
     hipGraph (no reference counterpart; each volume equals backprojection() of that capture
     alone with the same storage).  captures: iterable of (transient_chunk, pairs,
     voxels_per_side, volume_zero_pos, voxel_inc, t0, deltaT); storage "f32", "f16" or "bf16"

@@ -468,7 +468,8 @@ bpx_status bpx_batch_execute(bpx_batch batch, void* hip_stream);
 bpx_status bpx_batch_synchronize(bpx_batch batch);
 bpx_status bpx_batch_read_volume(bpx_batch batch, uint32_t index, float* voxel_volume);
 /* Completion time of each capture in the last execution, ms after the batch's queue reset
- * (device wall clock stamped when a capture's last tile finishes). */
+ * (device wall clock stamped when its volume is complete: with a queue's last tile of it, else as its
+ * partial sums are added up, after the gathers of every capture). */
 bpx_status bpx_batch_latencies(bpx_batch batch, double* ms);
 bpx_status bpx_batch_benchmark(bpx_batch batch, int32_t warmup, int32_t iterations, bpx_batch_timing* out);
 void bpx_batch_destroy(bpx_batch batch);
