@@ -154,12 +154,12 @@ void BatchImpl::choose_kernels() {
     std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return poly[x].part_pairs > poly[y].part_pairs; });
     std::vector<uint32_t> items;
     for (int kz : {16, 8})
-        for (uint32_t most : {256u, 512u, kPolySegMax}) {
+        for (uint32_t most = 128u; most <= kPolySegMax; most += 128u) {
             PolyGroup g;
             g.first = (uint32_t)(items.size() / 2u);
             for (uint32_t i : order) {
                 const LdsPolyShape& sh = poly[i].shape;
-                if (sh.kz != kz || sh.seg > most || (most > 256u && sh.seg <= most / 2u)) continue;
+                if (sh.kz != kz || (sh.seg + 127u) / 128u * 128u != most) continue;
                 g.shape.kz = kz;
                 g.shape.deg = std::max(g.shape.deg, sh.deg);
                 g.shape.seg = std::max(g.shape.seg, sh.seg);
