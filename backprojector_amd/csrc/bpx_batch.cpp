@@ -2,9 +2,10 @@
 //
 // Captures that the polynomial-quotient kernel takes (flat wall, columns along its normal; the
 // plans' rule) are gathered by it, as a plan of their own gathers them: their rows are staged
-// first (counts where a capture's samples all are), then one launch per depth and window class
+// first (counts where a capture's samples all are), then one launch per depth and window length
 // covers the (capture, part of the pairs, tile) items of all of them.  One more launch takes those
-// that a plan of their own gathers on the texture path with the pairs split.  Every item of these is
+// that a plan of their own gathers on the texture path with the pairs split, beside the others on a
+// side stream (64 captures of 1.2e11 updates: 31.0 ms in turn, 30.0 so).  Every item of these is
 // computed alike whatever the configuration below.
 //
 // The others: one persistent launch over a single work queue of staging items (fused rows and thresholds), LDS-staged
@@ -147,7 +148,7 @@ void BatchImpl::choose_kernels() {
     }
     if (!n_poly && !n_split) return;
     part_sums.alloc(total);
-    // a launch per depth and window class (LDS decides how many work-groups a CU holds), its items
+    // a launch per depth and window length (LDS decides how many work-groups a CU holds), its items
     // by falling length: the short ones fill the end
     std::vector<uint32_t> order(n);
     std::iota(order.begin(), order.end(), 0u);
@@ -475,6 +476,18 @@ void BatchImpl::build(const bpx_batch_config& c) {
                           "batch sample check kernel");
             hip_check(launch_stage(static_cast<const StageJob*>(zjobs.ptr), n_poly + n_split, 0u, staged_row_blocks, stream),
                       "batch row staging kernel");
+            // the split captures' scattered gathers beside the LDS gathers: they load other units
+            const bool beside = n_split_items && !poly_groups.empty();
+            if (beside) {
+                hip_check(hipEventRecord(fork, stream), "hipEventRecord");
+                hip_check(hipStreamWaitEvent(side, fork, 0), "hipStreamWaitEvent");
+                side_joined = true;
+            }
+            if (n_split_items)
+                hip_check(launch_batch_split(BatchItems{static_cast<const uint2*>(split_items.ptr), n_split_items}, q.caps,
+                                             static_cast<const SplitPairs*>(split_args.ptr), q.flags, format,
+                                             beside ? side : stream),
+                          "batch gather kernel (pairs split)");
             for (const bool counts : {true, false})
                 for (const PolyGroup& g : poly_groups) {
                     if (counts && !g.counts) continue;
@@ -483,10 +496,11 @@ void BatchImpl::build(const bpx_batch_config& c) {
                     hip_check(launch_batch_poly(b, caps, g.shape, counts ? (int)kCount : poly_format, stream),
                               "batch gather kernel (polynomial quotients)");
                 }
-            if (n_split_items)
-                hip_check(launch_batch_split(BatchItems{static_cast<const uint2*>(split_items.ptr), n_split_items}, q.caps,
-                                             static_cast<const SplitPairs*>(split_args.ptr), q.flags, format, stream),
-                          "batch gather kernel (pairs split)");
+            if (beside) {
+                hip_check(hipEventRecord(join, side), "hipEventRecord");
+                hip_check(hipStreamWaitEvent(stream, join, 0), "hipStreamWaitEvent");
+                side_joined = false;
+            }
             for (uint32_t i = 0; i < n; i += 32768u)
                 hip_check(launch_batch_sum_parts(static_cast<const PartsSum*>(sum_args.ptr) + i, std::min(n - i, 32768u),
                                                  q.remaining + i, q.done + i, stream),
