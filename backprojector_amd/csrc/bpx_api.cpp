@@ -253,16 +253,8 @@ bpx_status bpx_plan_execute(bpx_plan plan, void* hip_stream) {
         if (!plan) fail(BPX_ERR_INVALID_ARGUMENT, "NULL plan");
         PlanImpl& pl = *plan->impl;
         const hipStream_t s = hip_stream ? (hipStream_t)hip_stream : pl.stream;
-        // Executions of one plan share its buffers: order this one after the work queued on the
-        // plan's own stream and after the previous execution, whichever stream that used.
-        if (s != pl.stream) {
-            hip_check(hipEventRecord(pl.ready, pl.stream), "hipEventRecord");
-            hip_check(hipStreamWaitEvent(s, pl.ready, 0), "hipStreamWaitEvent");
-        }
-        if (pl.foreign) hip_check(hipStreamWaitEvent(s, pl.done, 0), "hipStreamWaitEvent");
-        pl.foreign = pl.foreign || s != pl.stream;   // its own stream keeps its executions in order
-        pl.execute(s);
-        if (pl.foreign) hip_check(hipEventRecord(pl.done, s), "hipEventRecord");
+        // executions of one plan share its buffers: one after the other, whichever streams they use
+        run_on_stream(s, pl.stream, pl.ready, pl.done, [&] { pl.execute(s); });
     });
 }
 
@@ -487,7 +479,6 @@ bpx_status bpx_plan_tune(bpx_plan plan, int32_t reps, int32_t* variant) {
 void bpx_plan_destroy(bpx_plan plan) {
     if (!plan) return;
     (void)hipStreamSynchronize(plan->impl->stream);
-    if (plan->impl->foreign) (void)hipEventSynchronize(plan->impl->done);
     delete plan;
 }
 

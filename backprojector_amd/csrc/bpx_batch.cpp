@@ -34,7 +34,7 @@ struct BatchImpl {
     std::vector<uint64_t> updates;   // voxel-pair updates per capture
     hipStream_t stream = nullptr;
     hipEvent_t ev[2] = {};
-    hipEvent_t done = nullptr, ready = nullptr;   // as PlanImpl::done / ready
+    hipEvent_t ready = nullptr, done = nullptr;   // of run_on_stream
     DeviceBuffer caps, flags, items, items_tex, items_wide, jobs, init, next, staged, remaining, error;
     DeviceBuffer stamps;   // uint64 [1 + captures]: batch start, then each capture's completion
     DeviceBuffer zjobs;    // StageJob per capture with pairs, those outside the queues first (prologue)
@@ -64,7 +64,6 @@ struct BatchImpl {
     uint32_t n_poly = 0, staged_row_blocks = 0;
     int poly_format = kF32Split;
     DeviceBuffer poly_args, poly_items, part_sums, sum_args, fmt_flags;
-    bool foreign = false;          // executed on a caller's stream (`done` says when it ends)
     uint32_t n_zjobs = 0, z_blocks = 0, row_blocks = 0;
     uint32_t n_items = 0, n_tex_items = 0, n_wide_items = 0;
     uint32_t tex_groups = 0, wide_groups = 0;
@@ -97,11 +96,9 @@ struct BatchImpl {
     void choose_kernels();
     bool queued(uint32_t i) const { return !poly[i].shape.kz && split[i].parts <= 1u; }
     void build(const bpx_batch_config& c);
-    // Waits for the batch's own stream and for its last execution on a caller's stream, then
-    // checks the queue's error word.
+    // Waits for every execution, then checks the queue's error word.
     void wait() const {
         hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
-        if (foreign) hip_check(hipEventSynchronize(done), "hipEventSynchronize");
         uint32_t e = 0;
         hip_check(hipMemcpy(&e, error.ptr, 4, hipMemcpyDeviceToHost), "hipMemcpy(error word)");
         if (e) fail(BPX_ERR_DEVICE, "batch queue: a capture's staging did not finish in time");
@@ -655,7 +652,6 @@ bpx_status bpx_batch_create(const bpx_capture_desc* captures, uint32_t count, co
 void bpx_batch_destroy(bpx_batch batch) {
     if (!batch) return;
     (void)hipStreamSynchronize(batch->impl->stream);
-    if (batch->impl->foreign) (void)hipEventSynchronize(batch->impl->done);
     delete batch;
 }
 
@@ -714,15 +710,7 @@ bpx_status bpx_batch_execute(bpx_batch batch, void* hip_stream) {
         if (!batch) fail(BPX_ERR_INVALID_ARGUMENT, "NULL batch");
         BatchImpl& b = *batch->impl;
         const hipStream_t s = hip_stream ? (hipStream_t)hip_stream : b.stream;
-        // one set of buffers: after the work on the batch's stream and the previous execution
-        if (s != b.stream) {
-            hip_check(hipEventRecord(b.ready, b.stream), "hipEventRecord");
-            hip_check(hipStreamWaitEvent(s, b.ready, 0), "hipStreamWaitEvent");
-        }
-        if (b.foreign) hip_check(hipStreamWaitEvent(s, b.done, 0), "hipStreamWaitEvent");
-        b.foreign = b.foreign || s != b.stream;
-        hip_check(hipGraphLaunch(b.exec, s), "hipGraphLaunch");
-        if (b.foreign) hip_check(hipEventRecord(b.done, s), "hipEventRecord");
+        run_on_stream(s, b.stream, b.ready, b.done, [&] { hip_check(hipGraphLaunch(b.exec, s), "hipGraphLaunch"); });
     });
 }
 

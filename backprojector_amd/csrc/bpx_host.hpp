@@ -172,16 +172,41 @@ struct PlanImpl {
     uint32_t stage_zb = 0, stage_sb = 0; // its blocks in the two staging passes
     hipEvent_t ev[8] = {};
     bool timed = false;                  // executions record ev[0] .. ev[3]
-    // recorded after each bpx_plan_execute, on its stream, from the first one on a caller's stream on
-    hipEvent_t done = nullptr;
-    bool foreign = false;
-    hipEvent_t ready = nullptr;          // work queued on the plan's own stream (caller-stream runs)
+    hipEvent_t ready = nullptr, done = nullptr;   // of run_on_stream
     std::unique_ptr<OctreeState> oct;
     ~PlanImpl();
     void execute(hipStream_t s);
 };
 
-// Waits for the plan's own stream and for its last execution on a caller's stream.
+// Queues f's work on s, a caller's stream or the object's own.  On a caller's stream it comes after
+// everything queued on `own`, and what is queued on `own` later comes after it, so the own stream stands
+// for every execution: the host waits for that one alone, never for an event recorded on a stream that
+// its owner may have destroyed by then.  While s is being captured nothing is ordered: the work runs
+// when the graph is launched, and the caller orders that.
+template <class F>
+void run_on_stream(hipStream_t s, hipStream_t own, hipEvent_t ready, hipEvent_t done, F&& f) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (s != own) hip_check(hipStreamIsCapturing(s, &capture), "hipStreamIsCapturing");
+    if (s == own || capture != hipStreamCaptureStatusNone) {
+        f();
+        return;
+    }
+    hip_check(hipEventRecord(ready, own), "hipEventRecord");
+    hip_check(hipStreamWaitEvent(s, ready, 0), "hipStreamWaitEvent");
+    const auto join = [&] {
+        const hipError_t e = hipEventRecord(done, s);
+        return e == hipSuccess ? hipStreamWaitEvent(own, done, 0) : e;
+    };
+    try {
+        f();
+    } catch (...) {
+        (void)join();   // what was queued before the error
+        throw;
+    }
+    hip_check(join(), "hipStreamWaitEvent");
+}
+
+// Waits for every execution of the plan (run_on_stream).
 void plan_wait(const PlanImpl& pl);
 // The storage the plan's last execution staged its rows in (waits for that execution).
 int staged_format(const PlanImpl& pl);

@@ -161,6 +161,7 @@ void give_stream(hipStream_t s) {
 }
 
 PlanImpl::~PlanImpl() {
+    oct.reset();   // its events were recorded on `stream`: before that is given back
     for (auto& e : ev)
         if (e) (void)hipEventDestroy(e);
     if (done) (void)hipEventDestroy(done);
@@ -603,7 +604,6 @@ static void make_events(PlanImpl& pl) {
 
 void plan_wait(const PlanImpl& pl) {
     hip_check(hipStreamSynchronize(pl.stream), "hipStreamSynchronize");
-    if (pl.foreign) hip_check(hipEventSynchronize(pl.done), "hipEventSynchronize");
 }
 
 // Exhaustive-grid structure: p = l*C + c with laser data depending only on l and camera
