@@ -365,19 +365,22 @@ constexpr size_t kRingChunk = 2u << 20;
 constexpr size_t kRingBytes = 32u << 20;
 constexpr size_t kStagedDown = 16u << 20;   // from here on an array goes through the ring
 constexpr size_t kStagedUp = 64u << 20;
-std::mutex g_ring_mutex;
-char* g_ring = nullptr;
-hipEvent_t g_ring_ev[kRingBytes / kRingChunk] = {};
-
-void ensure_ring() {
-    if (!g_ring) {
-        void* p = nullptr;
-        hip_check(hipHostMalloc(&p, kRingBytes, hipHostMallocDefault), "hipHostMalloc");
-        g_ring = static_cast<char*>(p);
+// One a direction, so that neither waits for the other's transfers; used by whoever holds the mutex.
+struct Ring {
+    std::mutex mutex;
+    char* at = nullptr;
+    hipEvent_t ev[kRingBytes / kRingChunk] = {};
+    void ensure() {
+        if (!at) {
+            void* p = nullptr;
+            hip_check(hipHostMalloc(&p, kRingBytes, hipHostMallocDefault), "hipHostMalloc");
+            at = static_cast<char*>(p);
+        }
+        for (auto& e : ev)
+            if (!e) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
     }
-    for (auto& e : g_ring_ev)
-        if (!e) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
-}
+};
+Ring g_up, g_down;
 
 // f(chunk, offset, bytes) for every chunk of an array, on up to `most` threads that take the chunks
 // in turn; the first error any of them met.
@@ -426,15 +429,15 @@ void upload_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
         hip_check(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice), "hipMemcpy(upload)");
         return;
     }
-    std::lock_guard<std::mutex> lock(g_ring_mutex);
-    ensure_ring();
+    std::lock_guard<std::mutex> lock(g_up.mutex);
+    g_up.ensure();
     // The ring in two halves: threads fill one while the other one's copies run.
     constexpr size_t half = kRingBytes / 2;
     hipError_t e = hipSuccess;
     uint32_t round = 0;
     for (size_t base = 0; base < bytes && e == hipSuccess; base += half, ++round) {
-        char* at = g_ring + (round & 1u) * half;
-        hipEvent_t ev = g_ring_ev[round & 1u];
+        char* at = g_up.at + (round & 1u) * half;
+        hipEvent_t ev = g_up.ev[round & 1u];
         if (round >= 2) e = hipEventSynchronize(ev);   // this half's previous copies are done
         if (e == hipSuccess)
             e = for_chunks(std::min(half, bytes - base), 4, [&](uint32_t, size_t off, size_t n) {
@@ -455,21 +458,21 @@ void download_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
         return;
     }
     hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");   // other transfers may use the ring meanwhile
-    std::lock_guard<std::mutex> lock(g_ring_mutex);
-    ensure_ring();
+    std::lock_guard<std::mutex> lock(g_down.mutex);
+    g_down.ensure();
     for (size_t base = 0; base < bytes; base += kRingBytes) {
         const size_t part = std::min(bytes - base, kRingBytes);
         const char* from = static_cast<const char*>(src) + base;
         char* to = static_cast<char*>(dst) + base;
         hipError_t e = hipSuccess;
         for (size_t off = 0, b = 0; off < part && e == hipSuccess; off += kRingChunk, ++b) {
-            e = hipMemcpyAsync(g_ring + off, from + off, std::min(kRingChunk, part - off), hipMemcpyDeviceToHost, s);
-            if (e == hipSuccess) e = hipEventRecord(g_ring_ev[b], s);
+            e = hipMemcpyAsync(g_down.at + off, from + off, std::min(kRingChunk, part - off), hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess) e = hipEventRecord(g_down.ev[b], s);
         }
         if (e == hipSuccess)
             e = for_chunks(part, 8, [&](uint32_t k, size_t off, size_t n) {
-                const hipError_t w = hipEventSynchronize(g_ring_ev[k]);
-                if (w == hipSuccess) std::memcpy(to + off, g_ring + off, n);
+                const hipError_t w = hipEventSynchronize(g_down.ev[k]);
+                if (w == hipSuccess) std::memcpy(to + off, g_down.at + off, n);
                 return w;
             });
         const hipError_t done = hipStreamSynchronize(s);

@@ -136,3 +136,42 @@ def test_transient_from_pinned_memory(gpu, oracle):
     del pinned
     assert hip.hipHostFree(p) == 0
     assert np.array_equal(got, oracle.a1_volume_f64acc(H, pr, N, zero, inc, 0.5, 4.0 / 16389).astype(f32))
+
+
+def test_transfers_of_several_threads(gpu, oracle):
+    """Volumes out of and a transient into the library from several threads at once: one thread has the
+    staging chunks of a direction, the others wait for them."""
+    N = (256, 255, 97)   # 24 MiB, no round number of chunks
+    zero, inc = basis(N, (0.0, 0.0, 0.9), (0.5, 0.5, 0.5))
+    plans, refs = [], []
+    for k in range(3):
+        H, pr = capture((3, 2), 700, k)
+        plans.append(gpu.Plan(H, pr, N, zero, inc, 0.5, 0.005))
+        plans[-1].execute()
+        refs.append(oracle.a1_volume_f64acc(H, pr, N, zero, inc, 0.5, 0.005).astype(f32))
+    H, pr = capture((32, 32), 16389, 9)
+    small = (5, 4, 3)
+    grid = basis(small, (0.0, 0.0, 0.9), (0.5, 0.5, 0.5))
+    up = oracle.a1_volume_f64acc(H, pr, small, *grid, 0.5, 4.0 / 16389).astype(f32)
+    bad = []
+
+    def down(k):
+        for r in range(6):
+            if not np.array_equal(plans[k].volume(), refs[k]):
+                bad.append((k, r))
+
+    def upload():
+        for r in range(4):
+            with gpu.Plan(H, pr, small, *grid, 0.5, 4.0 / 16389) as plan:
+                plan.execute()
+                if not np.array_equal(plan.volume(), up):
+                    bad.append(("up", r))
+
+    threads = [threading.Thread(target=down, args=(k,)) for k in range(3)] + [threading.Thread(target=upload)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for p in plans:
+        p.close()
+    assert not bad
