@@ -4,6 +4,7 @@
 #include <cmath>
 #include <cstring>
 #include <limits>
+#include <map>
 #include <memory>
 #include <mutex>
 #include <system_error>
@@ -367,20 +368,26 @@ constexpr size_t kStagedDown = 16u << 20;   // from here on an array goes throug
 constexpr size_t kStagedUp = 64u << 20;
 // One a direction, so that neither waits for the other's transfers; used by whoever holds the mutex.
 struct Ring {
+    struct Events {
+        hipEvent_t of[kRingBytes / kRingChunk] = {};
+    };
     std::mutex mutex;
     char* at = nullptr;
-    hipEvent_t ev[kRingBytes / kRingChunk] = {};
-    void ensure() {
+    std::map<int, Events> events;
+    // The chunks and the current device's events (an event can be recorded on its own device alone).
+    hipEvent_t* ensure() {
         if (!at) {
             void* p = nullptr;
-            hip_check(hipHostMalloc(&p, kRingBytes, hipHostMallocDefault), "hipHostMalloc");
+            hip_check(hipHostMalloc(&p, kRingBytes, hipHostMallocPortable), "hipHostMalloc");
             at = static_cast<char*>(p);
         }
-        for (auto& e : ev)
+        Events& ev = events[current_device()];
+        for (auto& e : ev.of)
             if (!e) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+        return ev.of;
     }
 };
-Ring g_up, g_down;
+Ring &g_up = *new Ring, &g_down = *new Ring;   // never destroyed, as the pool
 
 // f(chunk, offset, bytes) for every chunk of an array, on up to `most` threads that take the chunks
 // in turn; the first error any of them met.
@@ -430,14 +437,14 @@ void upload_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
         return;
     }
     std::lock_guard<std::mutex> lock(g_up.mutex);
-    g_up.ensure();
+    hipEvent_t* const events = g_up.ensure();
     // The ring in two halves: threads fill one while the other one's copies run.
     constexpr size_t half = kRingBytes / 2;
     hipError_t e = hipSuccess;
     uint32_t round = 0;
     for (size_t base = 0; base < bytes && e == hipSuccess; base += half, ++round) {
         char* at = g_up.at + (round & 1u) * half;
-        hipEvent_t ev = g_up.ev[round & 1u];
+        hipEvent_t ev = events[round & 1u];
         if (round >= 2) e = hipEventSynchronize(ev);   // this half's previous copies are done
         if (e == hipSuccess)
             e = for_chunks(std::min(half, bytes - base), 4, [&](uint32_t, size_t off, size_t n) {
@@ -459,7 +466,7 @@ void download_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
     }
     hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");   // other transfers may use the ring meanwhile
     std::lock_guard<std::mutex> lock(g_down.mutex);
-    g_down.ensure();
+    hipEvent_t* const events = g_down.ensure();
     for (size_t base = 0; base < bytes; base += kRingBytes) {
         const size_t part = std::min(bytes - base, kRingBytes);
         const char* from = static_cast<const char*>(src) + base;
@@ -467,11 +474,11 @@ void download_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
         hipError_t e = hipSuccess;
         for (size_t off = 0, b = 0; off < part && e == hipSuccess; off += kRingChunk, ++b) {
             e = hipMemcpyAsync(g_down.at + off, from + off, std::min(kRingChunk, part - off), hipMemcpyDeviceToHost, s);
-            if (e == hipSuccess) e = hipEventRecord(g_down.ev[b], s);
+            if (e == hipSuccess) e = hipEventRecord(events[b], s);
         }
         if (e == hipSuccess)
             e = for_chunks(part, 8, [&](uint32_t k, size_t off, size_t n) {
-                const hipError_t w = hipEventSynchronize(g_down.ev[k]);
+                const hipError_t w = hipEventSynchronize(events[k]);
                 if (w == hipSuccess) std::memcpy(to + off, g_down.at + off, n);
                 return w;
             });

@@ -175,3 +175,18 @@ def test_transfers_of_several_threads(gpu, oracle):
     for p in plans:
         p.close()
     assert not bad
+
+
+def test_transfers_on_a_second_device(gpu, oracle):
+    """The staging chunks serve every device of the process, each with its own events."""
+    import torch
+    if torch.cuda.device_count() < 2:
+        pytest.skip("needs two GPUs")
+    N = (256, 255, 97)
+    zero, inc = basis(N, (0.0, 0.0, 0.9), (0.5, 0.5, 0.5))
+    H, pr = capture((32, 32), 16389, 5)
+    ref = oracle.a1_volume_f64acc(H, pr, N, zero, inc, 0.5, 4.0 / 16389).astype(f32)
+    for device in (0, 1, 0):
+        with torch.cuda.device(device), gpu.Plan(H, pr, N, zero, inc, 0.5, 4.0 / 16389) as plan:
+            plan.execute()
+            assert np.array_equal(plan.volume(), ref), device
