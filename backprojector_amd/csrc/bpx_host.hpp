@@ -62,6 +62,7 @@ struct DeviceBuffer {
         std::swap(device, o.device);
     }
     void alloc(size_t n);
+    bool try_alloc(size_t n);   // false (and empty) where the device's memory does not suffice
     void release();
     ~DeviceBuffer() { release(); }
 };

@@ -54,6 +54,7 @@ size_t block_size(size_t n) {
 // kPooledTicks allocations; the caller frees them outside the lock.
 std::vector<void*> evict(Pool& p, size_t room) {
     std::vector<void*> out;
+    out.reserve(p.blocks.size());   // nothing below throws: the list and its total stay in step
     size_t n = 0;
     while (n < p.blocks.size() && (p.bytes > room || p.ticks - p.blocks[n].tick > kPooledTicks)) {
         out.push_back(p.blocks[n].ptr);
@@ -66,9 +67,14 @@ std::vector<void*> evict(Pool& p, size_t room) {
 }  // namespace
 
 void DeviceBuffer::alloc(size_t n) {
+    if (!try_alloc(n))
+        fail(BPX_ERR_OUT_OF_MEMORY, "hipMalloc(" + std::to_string(n) + " bytes) failed: " +
+                                        hipGetErrorString(hipErrorOutOfMemory));
+}
+bool DeviceBuffer::try_alloc(size_t n) {
     release();
     if (n == 0) n = 256;
-    const size_t want = block_size(n);
+    size_t want = block_size(n);
     Pool& p = pool();
     device = current_device();
     {
@@ -97,15 +103,22 @@ void DeviceBuffer::alloc(size_t n) {
             }
             for (void* b : all) (void)hipFree(b);
             e = hipMalloc(&ptr, want);
+            if (e == hipErrorOutOfMemory) {   // without the rounding for reuse
+                (void)hipGetLastError();
+                want = (n + 255u) / 256u * 256u;
+                e = hipMalloc(&ptr, want);
+            }
         }
         if (e != hipSuccess) {
             ptr = nullptr;
-            fail(BPX_ERR_OUT_OF_MEMORY, "hipMalloc(" + std::to_string(n) + " bytes) failed: " +
-                                            hipGetErrorString(e));
+            (void)hipGetLastError();   // or the next launch would report it
+            if (e == hipErrorOutOfMemory) return false;
+            fail(BPX_ERR_OUT_OF_MEMORY, "hipMalloc(" + std::to_string(n) + " bytes) failed: " + hipGetErrorString(e));
         }
         cap = want;
     }
     bytes = n;
+    return true;
 }
 void DeviceBuffer::release() {
     if (ptr) {
