@@ -1207,7 +1207,8 @@ void PlanImpl::execute(hipStream_t s) {
 }
 
 // The LDS-staged window kernel where it applies: real samples, confocal pairs on a flat wall, bin
-// windows and threshold tables that fit.  Sets the row pitch of the prefix sums.
+// windows and threshold tables that fit, in LDS and in the device's memory.  Allocates the prefix sums
+// then (H) and sets their row pitch; the general kernel's are the caller's.
 static void window_lds_setup(PlanImpl& pl, const std::vector<bpx_pair>& pr, float width) {
     bool flat = true;
     for (const auto& p : pr) flat = flat && p.laser_point[2] == pr[0].laser_point[2];
@@ -1249,15 +1250,18 @@ static void window_lds_setup(PlanImpl& pl, const std::vector<bpx_pair>& pr, floa
         p4[4 * p + 3] = (float)(((double)pr[p].laser_wall + (double)pr[p].camera_wall - (double)pl.half_width -
                                  (double)pl.t0) / (double)pl.dT + 1.0);
     }
-    pl.pair4.alloc(sizeof(float) * p4.size());
-    hip_check(hipMemcpy(pl.pair4.ptr, p4.data(), sizeof(float) * p4.size(), hipMemcpyHostToDevice), "hipMemcpy(pairs)");
-    pl.win_lo.alloc((size_t)pl.P * a.pitch * 8u);
-    pl.win_hi.alloc((size_t)pl.P * a.pitch * 8u);
-    pl.ldh = a.ldp;
-    // double sums: a split changes their last bits only; half the parts of the integer kernel
-    pl.poly = sh;
+    // double sums: a split changes their last bits only
     pl.poly_parts = lds_poly_parts(pl.g, sh, pl.P, 8u, 4u, &a.part_pairs);
-    if (pl.poly_parts > 1) pl.parts.alloc((size_t)pl.poly_parts * pl.g.n[0] * pl.g.n[1] * pl.g.n[2] * 8u);
+    const size_t sums = pl.poly_parts > 1 ? (size_t)pl.poly_parts * pl.g.n[0] * pl.g.n[1] * pl.g.n[2] * 8u : 0u;
+    const size_t table = (size_t)pl.P * a.pitch * 8u;
+    if (!pl.pair4.try_alloc(sizeof(float) * p4.size()) || !pl.win_lo.try_alloc(table) || !pl.win_hi.try_alloc(table) ||
+        (sums && !pl.parts.try_alloc(sums)) || !pl.H.try_alloc((size_t)pl.P * a.ldp * 8u)) {
+        for (DeviceBuffer* b : {&pl.pair4, &pl.win_lo, &pl.win_hi, &pl.parts, &pl.H}) b->release();
+        return;
+    }
+    hip_check(hipMemcpy(pl.pair4.ptr, p4.data(), sizeof(float) * p4.size(), hipMemcpyHostToDevice), "hipMemcpy(pairs)");
+    pl.ldh = a.ldp;
+    pl.poly = sh;
 }
 
 PlanImpl* make_plan_window(const CaptureIn& c, const uint32_t n[3], const float vpos[3],
@@ -1312,8 +1316,6 @@ PlanImpl* make_plan_window(const CaptureIn& c, const uint32_t n[3], const float 
     if (pl->P == 0 || c.T < 2) return pl.release();
     stage_raw(*pl, c, idx);
     pl->ldh = round_up(c.T, 32);
-    window_lds_setup(*pl, pr, width);
-    pl->H.alloc((size_t)pl->P * pl->ldh * (c.cplx ? 16 : 8));
     pl->Z.alloc(sizeof(float) * c.T);
     pl->Z2.alloc(sizeof(float) * c.T);
     std::vector<float> p8((size_t)pl->P * 8);
@@ -1321,6 +1323,8 @@ PlanImpl* make_plan_window(const CaptureIn& c, const uint32_t n[3], const float 
     pl->pair8.alloc(sizeof(float) * p8.size());
     hip_check(hipMemcpy(pl->pair8.ptr, p8.data(), sizeof(float) * p8.size(), hipMemcpyHostToDevice),
               "hipMemcpy(pairs)");
+    window_lds_setup(*pl, pr, width);
+    if (!pl->poly.kz) pl->H.alloc((size_t)pl->P * pl->ldh * (c.cplx ? 16 : 8));
     return pl.release();
 }
 

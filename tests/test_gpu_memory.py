@@ -40,3 +40,37 @@ def test_failed_allocation_leaves_no_error(gpu, oracle):
     finally:
         for p in held:
             p.close()
+
+
+@contextmanager
+def memory_left(n):
+    """All of the device's free memory but n bytes taken."""
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    hip.hipMemGetInfo.argtypes = [ctypes.POINTER(ctypes.c_size_t)] * 2
+    hip.hipMalloc.argtypes = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t]
+    hip.hipFree.argtypes = [ctypes.c_void_p]
+    free, total, p = ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_void_p()
+    assert hip.hipDeviceSynchronize() == 0 and hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    assert free.value > n and hip.hipMalloc(ctypes.byref(p), free.value - n) == 0
+    try:
+        yield
+    finally:
+        assert hip.hipFree(p) == 0
+
+
+def long_rows(scan, T):
+    pr = pairs_of(*scan)
+    rows = np.random.default_rng(T).integers(0, 9, (64, T)).astype(f32)
+    return np.tile(rows, (len(pr) // 64, 1)), pr
+
+
+def test_window_tables_that_do_not_fit(gpu):
+    """8,192 rows of 16,384 bins: 0.5 GiB of samples and 1 of prefix sums for the general kernel, 2 more for
+    the LDS-staged one's tables."""
+    T, N = 16384, (32, 32, 32)
+    H, pr = long_rows((128, 64), T)
+    args = (H, pr, N, (0.0, 0.0, 0.8), (0.15, 0.15, 0.15), 0.0, 4.0 / T)
+    ref = gpu.window_backprojection(*args)
+    assert ref.max() > 0
+    with memory_left(5 << 29):
+        assert np.array_equal(gpu.window_backprojection(*args), ref)
