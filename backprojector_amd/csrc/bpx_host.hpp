@@ -100,7 +100,8 @@ struct OctreeState {
     uint32_t coarse_P = 0;                // pairs the coarse levels used in the last execution
     std::vector<uint32_t> fallback_voxels;  // fine voxels added by the fallback, per level
     // Captures of counts: the fine voxels of well-filled 16 x 16 x kz tiles are gathered tile by
-    // tile with integer sums (LdsPolyShape; kz 0: never), from count rows beside the fp32 ones
+    // tile with integer sums (LdsPolyShape; kz 0: never), from count rows beside the fp32 ones (kept
+    // where every sample was a count when the plan was made)
     LdsPolyShape poly;
     DeviceBuffer count_rows, count_job, count_flag;
     DeviceBuffer tile_mask, tile_fill, tile_counts, tile_list, tile_parts;

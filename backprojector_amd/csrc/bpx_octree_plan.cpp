@@ -98,6 +98,28 @@ static void build_pair_subset(PlanImpl& pl, uint32_t s) {
     st.sub_stride = s;
 }
 
+// Memory of the count rows and their tile lists: where every sample is a count (the plan keeps its rows;
+// each execution looks again), and where it can be had.  The count rows are as large as the fp32 ones.
+static bool count_buffers(const PlanImpl& pl, OctreeState& st) {
+    st.count_flag.alloc(4);
+    uint32_t* const flag = static_cast<uint32_t*>(st.count_flag.ptr);
+    uint32_t found = 0;
+    hip_check(launch_fill(reinterpret_cast<float*>(flag), 1, 0.0f, pl.stream), "fill kernel");
+    hip_check(launch_exact16_check(static_cast<const float*>(pl.raw.ptr), (uint64_t)pl.P * pl.T, flag, pl.stream),
+              "count check kernel");
+    hip_check(hipStreamSynchronize(pl.stream), "hipStreamSynchronize");
+    hip_check(hipMemcpy(&found, flag, 4, hipMemcpyDeviceToHost), "hipMemcpy(row format)");
+    if (found) return false;
+    const uint64_t tiles = lds_tile_count(pl.g, st.poly);
+    if (!st.count_rows.try_alloc(pl.H.bytes) || !st.tile_mask.try_alloc(tiles * 512u) || !st.tile_fill.try_alloc(16u * tiles) ||
+        !st.tile_list.try_alloc(4u * tiles) || !st.tile_counts.try_alloc(8)) {
+        for (DeviceBuffer* b : {&st.count_rows, &st.tile_mask, &st.tile_fill, &st.tile_list, &st.tile_counts}) b->release();
+        return false;
+    }
+    hip_check(hipMemset(st.count_rows.ptr, 0, pl.H.bytes), "hipMemset(count rows)");
+    return true;
+}
+
 PlanImpl* make_plan_octree(const CaptureIn& c, const uint32_t n[3], const float zero[3],
                            const float inc[9], const bpx_octree_options* oo) {
     bpx_octree_options o{4u, 0.25f, 0.5f, 0u, {}, 0.0f, {}, 1u};
@@ -162,15 +184,8 @@ PlanImpl* make_plan_octree(const CaptureIn& c, const uint32_t n[3], const float 
     hip_check(hipHostMalloc(&st->host_stats, sizeof(double) * 8, hipHostMallocDefault), "hipHostMalloc");
     if (P && pl->fused && pl->sep && pl->flat && pl->kahan_block <= 4096u && P <= (1u << 20))
         st->poly = lds_poly_shape(pl->g, pl->inv2, pl->lz, pl->tap_bound, pl->max_path, kPolyBudget, kCount);
+    if (st->poly.kz && !count_buffers(*pl, *st)) st->poly = LdsPolyShape{};
     if (st->poly.kz) {
-        const uint64_t tiles = lds_tile_count(pl->g, st->poly);
-        st->count_rows.alloc(pl->H.bytes);
-        hip_check(hipMemset(st->count_rows.ptr, 0, pl->H.bytes), "hipMemset(count rows)");
-        st->count_flag.alloc(4);
-        st->tile_mask.alloc(tiles * 512u);
-        st->tile_fill.alloc(16u * tiles);
-        st->tile_list.alloc(4u * tiles);
-        st->tile_counts.alloc(8);
         StageJob job = stage_job(*pl);
         job.dst = st->count_rows.ptr;
         job.fmt_flag = static_cast<const uint32_t*>(st->count_flag.ptr);

@@ -74,3 +74,41 @@ def test_window_tables_that_do_not_fit(gpu):
     assert ref.max() > 0
     with memory_left(5 << 29):
         assert np.array_equal(gpu.window_backprojection(*args), ref)
+
+
+def octree_args(samples):
+    """16,384 rows of 8,192 bins: 0.5 GiB of samples, 1 GiB of fused rows."""
+    T, N = 8192, (32, 32, 32)
+    H, pr = long_rows((128, 128), T)
+    if samples == "real":
+        H += f32(0.25)
+    return (H, pr, N, *basis(N, (0.0, 0.0, 0.8), (0.2, 0.2, 0.2)), 0.0, 4.0 / T)
+
+
+def memory_of(make):
+    """(object, bytes of device memory that making it took)."""
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    free, after, total = ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipDeviceSynchronize() == 0 and hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    obj = make()
+    assert hip.hipDeviceSynchronize() == 0 and hip.hipMemGetInfo(ctypes.byref(after), ctypes.byref(total)) == 0
+    return obj, free.value - after.value
+
+
+def test_octree_count_rows_only_where_they_serve(gpu):
+    """Real samples take no count rows (as large as the fused rows, 1 GiB); counts that find no room for
+    them give the volume of those that do."""
+    counts, real = octree_args("counts"), octree_args("real")
+    rows = 8 * counts[0].size
+    plan, with_rows = memory_of(lambda: gpu.Plan.octree(*counts, levels=2))
+    with plan:
+        plan.execute()
+        ref = plan.volume()
+        other, without = memory_of(lambda: gpu.Plan.octree(*real, levels=2))
+        other.close()
+    # blocks released by earlier plans, at most 0.5 GiB, may serve either
+    assert without < with_rows - rows // 2, (with_rows, without)
+    with memory_left(without + (3 << 27)):
+        with gpu.Plan.octree(*counts, levels=2) as plan:
+            plan.execute()
+            assert np.array_equal(plan.volume(), ref)
