@@ -243,12 +243,19 @@ static void build_winmax(PlanImpl& pl, uint32_t P, const uint32_t* rows, hipStre
 // cheaper from 29 % on (6e12 updates/s against 1.75e12).  Learned 256^3 executions, ms: one with its
 // volume, whole tiles from 30 % 14.6 to 15.3, quarters from 20 / 30 / 45 / 60 % 13.1 / 12.9 / 12.7 / 12.8;
 // three others alone, quarters from 30 / 40 / 50 % 12.4, 13.8, 15.4 / 13.1, 14.7, 16.1 / 13.7, 15.5, 17.7.
-static void gather_tiles(PlanImpl& pl, const OctFineArgs& fine, uint32_t n, uint32_t n_fb, hipStream_t s) {
+// False, with nothing queued, where the device's memory does not suffice for the tiles' partial sums.
+static bool gather_tiles(PlanImpl& pl, const OctFineArgs& fine, uint32_t n, uint32_t n_fb, hipStream_t s) {
     OctreeState& st = *pl.oct;
     const uint32_t total = n + n_fb;
-    if (!total) return;
+    if (!total) return true;
     const uint32_t cells = 256u * (uint32_t)st.poly.kz, dense = cells / 4u * 3u / 10u;
     const uint64_t tiles = lds_tile_count(pl.g, st.poly);
+    // at most total / dense tiles with such a quarter; 4,096 work-groups share them out in parts of the pairs
+    const uint32_t max_tiles = (uint32_t)std::min<uint64_t>(tiles, total / dense), groups = std::max(max_tiles, 4096u);
+    if (max_tiles && st.tile_parts.bytes < (size_t)groups * cells * 4u) {
+        hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");   // nothing else uses the old one
+        if (!st.tile_parts.try_alloc((size_t)groups * cells * 4u)) return false;
+    }
     TileListArgs t{};
     t.g = pl.g;
     t.mask = static_cast<uint32_t*>(st.tile_mask.ptr);
@@ -272,14 +279,7 @@ static void gather_tiles(PlanImpl& pl, const OctFineArgs& fine, uint32_t n, uint
     f.n_dev = t.counts + 1;
     f.E = st.count_rows.ptr;
     hip_check(launch_oct_fine_counts(f, st.side), "octree fine kernel (count rows)");
-    // at most total / dense tiles with such a quarter; 4,096 work-groups share them out in parts of the pairs
-    const uint32_t max_tiles = (uint32_t)std::min<uint64_t>(tiles, total / dense);
     if (max_tiles) {
-        const uint32_t groups = std::max(max_tiles, 4096u);
-        if (!st.tile_parts.ptr || st.tile_parts.bytes < (size_t)groups * cells * 4u) {
-            hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");   // nothing else uses the old one
-            st.tile_parts.alloc((size_t)groups * cells * 4u);
-        }
         ConfocalArgs c{};
         c.H = st.count_rows.ptr;
         c.pairs = static_cast<const float4*>(pl.pair4.ptr);
@@ -295,6 +295,7 @@ static void gather_tiles(PlanImpl& pl, const OctFineArgs& fine, uint32_t n, uint
         a.parts = static_cast<uint32_t*>(st.tile_parts.ptr);
         hip_check(launch_lds_counts_tiles(a, st.poly, t, max_tiles, dense, groups, s), "octree tile gather kernel");
     }
+    return true;
 }
 
 void execute_octree(PlanImpl& pl, hipStream_t s) {
@@ -454,14 +455,18 @@ void execute_octree(PlanImpl& pl, hipStream_t s) {
     if ((uint64_t)n + fb_total > nvox) fail(BPX_ERR_DEVICE, "octree fine list overflow");
     st.level_active[st.L] = st.bounds_only ? 0u : n + (uint32_t)fb_total;
     hip_check(hipEventRecord(pl.ev[2], s), "hipEventRecord");
-    if (!st.bounds_only && counts) {
-        gather_tiles(pl, fine, n, (uint32_t)fb_total, s);
+    if (!st.bounds_only && counts && gather_tiles(pl, fine, n, (uint32_t)fb_total, s)) {
         side_used = n + fb_total != 0;
     } else if (!st.bounds_only) {
         OctFineArgs f = fine;
         f.voxels = static_cast<const uint32_t*>(st.fine_list.ptr);
         f.n = n;
         hip_check(launch_oct_fine(f, s), "octree fine kernel");
+        if (counts && fb_total) {   // without the tiles' memory: the fallback voxels were left for them
+            f.voxels = fb_voxels;
+            f.n = (uint32_t)fb_total;
+            hip_check(launch_oct_fine(f, s), "octree fine kernel (fallback voxels)");
+        }
     }
     if (side_used) {
         hip_check(hipEventRecord(st.join, st.side), "hipEventRecord");

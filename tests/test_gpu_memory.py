@@ -112,3 +112,20 @@ def test_octree_count_rows_only_where_they_serve(gpu):
         with gpu.Plan.octree(*counts, levels=2) as plan:
             plan.execute()
             assert np.array_equal(plan.volume(), ref)
+
+
+def test_octree_tile_sums_that_do_not_fit(gpu):
+    """1024 x 1024 x 512 voxels, every one listed: 131,072 tiles take 2 GiB of partial sums at the first
+    execution; without them the voxels are gathered one by one."""
+    H, pr = capture((8, 8), 1200)
+    N = (1024, 1024, 512)
+    args = (H, pr, N, *basis(N, (0.0, 0.0, 0.8), (0.5, 0.5, 0.25)), 0.5, 0.0025)
+    with gpu.Plan.octree(*args, levels=2, threshold=0.0) as plan:
+        plan.execute()
+        ref = plan.volume()
+    assert ref.max() > 0
+    with gpu.Plan.octree(*args, levels=2, threshold=0.0) as plan, memory_left(1 << 30):
+        plan.execute()
+        assert np.array_equal(plan.volume(), ref)
+        plan.execute()
+        assert np.array_equal(plan.volume(), ref)
