@@ -337,7 +337,8 @@ bpx_status bpx_plan_info(bpx_plan plan, int32_t* path, int32_t* lane_voxels, uin
         if (!plan) fail(BPX_ERR_INVALID_ARGUMENT, "NULL plan");
         const PlanImpl& pl = *plan->impl;
         if (path) *path = pl.path;
-        if (lane_voxels) *lane_voxels = pl.lds_tiles ? lds_shape(pl.variant, pl.format).kz : pl.K;
+        if (lane_voxels)
+            *lane_voxels = pl.poly_real ? pl.poly.kz : pl.paths.seg ? 8 : pl.lds_tiles ? lds_shape(pl.variant, pl.format).kz : pl.K;
         if (pairs_used) *pairs_used = pl.P;
         if (Tc) *Tc = pl.T;
         if (scale) *scale = pl.scale;
@@ -357,12 +358,19 @@ bpx_status bpx_plan_kernel_name(bpx_plan plan, char* out, uint64_t capacity) {
         if (!plan || !out || capacity == 0) fail(BPX_ERR_INVALID_ARGUMENT, "NULL argument");
         const PlanImpl& pl = *plan->impl;
         std::string name;
-        const bool counts = pl.poly_counts && staged_format(pl) == kCount;
-        if (counts || pl.poly_real) {
-            const uint32_t parts = counts ? pl.poly_parts : pl.real_parts;
-            name = (counts ? "confocal_lds_kernel_poly<KZ=" : "confocal_lds_kernel<KZ=") + std::to_string(pl.poly.kz) +
+        const int rows = pl.poly_counts || pl.poly_real ? staged_format(pl) : pl.format;
+        if (rows == kCount || pl.poly_real) {
+            const uint32_t parts = rows == kCount ? pl.poly_parts : pl.real_parts;
+            const char* kernel = rows == kCount    ? "confocal_lds_kernel_poly<CountRows"
+                                 : rows == kF16    ? "confocal_lds_kernel_column<Half16Rows<false>"
+                                 : rows == kBF16   ? "confocal_lds_kernel_column<Half16Rows<true>"
+                                 : format_complex(rows) ? "confocal_lds_kernel_column<ComplexRows"
+                                                   : "confocal_lds_kernel_column<F32Rows";
+            name = std::string(kernel) + ", KZ=" + std::to_string(pl.poly.kz) +
                    ", degree=" + std::to_string(pl.poly.deg) + "> (16x16x" + std::to_string(pl.poly.kz) + " tiles, " +
                    std::to_string(parts) + (parts > 1 ? " pair parts)" : " pair part)");
+        } else if (pl.tex_parts > 1) {
+            name = "confocal_kernel_split<K=2> (8x8x8 tiles, " + std::to_string(pl.tex_parts) + " pair parts)";
         } else if (pl.paths.seg) {
             name = std::string("paths_lds_kernel<") + (pl.paths.L ? "grid" : "pairs") + "> (16x16x8 tiles, " +
                    std::to_string(pl.paths_parts) + (pl.paths_parts > 1 ? " parts)" : " part)");

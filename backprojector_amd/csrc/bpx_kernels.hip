@@ -824,7 +824,7 @@ __device__ __forceinline__ void confocal_tile(const ConfocalArgs& a, uint32_t ti
 // The pairs split over work-groups, for volumes whose tiles alone leave most of the chip idle:
 // work-group part x tiles + tile.
 template <class Src, int K, bool SEP, bool FLAT>
-__global__ __launch_bounds__(256) void confocal_split_kernel(ConfocalArgs a, SplitPairs sp) {
+__global__ __launch_bounds__(256) void confocal_kernel_split(ConfocalArgs a, SplitPairs sp) {
     const uint32_t part = blockIdx.x / a.t.count, tile = blockIdx.x % a.t.count;
     const uint32_t p0 = part * sp.part_pairs, p1 = min(p0 + sp.part_pairs, a.P);
     const size_t n = (size_t)a.g.n[0] * a.g.n[1] * a.g.n[2];
@@ -1705,9 +1705,9 @@ template <class Src>
 static hipError_t split_launch(const ConfocalArgs& a, const SplitPairs& sp, uint32_t parts, bool sep, bool flat,
                                hipStream_t s) {
     const dim3 grid(a.t.count * parts), block(256);
-    if (sep && flat) hipLaunchKernelGGL((confocal_split_kernel<Src, 2, true, true>), grid, block, 0, s, a, sp);
-    else if (sep) hipLaunchKernelGGL((confocal_split_kernel<Src, 2, true, false>), grid, block, 0, s, a, sp);
-    else hipLaunchKernelGGL((confocal_split_kernel<Src, 2, false, false>), grid, block, 0, s, a, sp);
+    if (sep && flat) hipLaunchKernelGGL((confocal_kernel_split<Src, 2, true, true>), grid, block, 0, s, a, sp);
+    else if (sep) hipLaunchKernelGGL((confocal_kernel_split<Src, 2, true, false>), grid, block, 0, s, a, sp);
+    else hipLaunchKernelGGL((confocal_kernel_split<Src, 2, false, false>), grid, block, 0, s, a, sp);
     return hipGetLastError();
 }
 hipError_t launch_split(const ConfocalArgs& a, const SplitPairs& sp, int format, uint32_t parts, bool sep, bool flat,

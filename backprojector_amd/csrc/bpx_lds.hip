@@ -382,11 +382,19 @@ __device__ __forceinline__ uint32_t poly_tile(const LdsPolyArgs& a, uint32_t blo
     return tile;
 }
 
+// Count rows.
 template <class Fz, int KZ, int DEG, bool TILES>
 __global__ __launch_bounds__(256, 4) void confocal_lds_kernel_poly(LdsPolyArgs a) {
     extern __shared__ char smem[];
     if (!rows_wanted(a.c)) return;
     poly_tile<Fz, KZ, DEG, TILES>(a, blockIdx.x, gridDim.x, smem);
+}
+// The other rows.
+template <class Fz, int KZ, int DEG>
+__global__ __launch_bounds__(256, 4) void confocal_lds_kernel_column(LdsPolyArgs a) {
+    extern __shared__ char smem[];
+    if (!rows_wanted(a.c)) return;
+    poly_tile<Fz, KZ, DEG, false>(a, blockIdx.x, gridDim.x, smem);
 }
 
 // Captures of many sizes: one work-group per item (capture, part x its tiles + tile).
@@ -534,7 +542,10 @@ static hipError_t poly_lds(Kernel fn, uint32_t seg, size_t* bytes) {
 }
 template <class Fz, int KZ, int DEG, bool TILES>
 static hipError_t poly_launch(const LdsPolyArgs& a, uint32_t groups, hipStream_t s) {
-    const auto fn = confocal_lds_kernel_poly<Fz, KZ, DEG, TILES>;
+    const auto fn = [] {
+        if constexpr (Fz::kFormat == kCount) return confocal_lds_kernel_poly<Fz, KZ, DEG, TILES>;
+        else return confocal_lds_kernel_column<Fz, KZ, DEG>;
+    }();
     size_t lds = 0;
     const hipError_t e = poly_lds<Fz>(fn, a.seg, &lds);
     if (e != hipSuccess) return e;

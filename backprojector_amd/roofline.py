@@ -148,7 +148,7 @@ def find_kernel(counts: dict, name: str):
 def signature(kernel: str) -> str:
     """`void bpx::confocal_lds_kernel<bpx::FusedF32, 8, 8>(bpx::ConfocalArgs)` ->
     `confocal_lds_kernel<FusedF32, 8, 8>`."""
-    k = kernel.replace("void ", "").replace("bpx::", "")
+    k = kernel.replace("void ", "").replace("bpx::", "").replace("(anonymous namespace)::", "")
     depth, end = 0, len(k)
     for i, ch in enumerate(k):
         if ch == "<":

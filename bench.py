@@ -337,6 +337,12 @@ def device_kernel(info, storage, cplx):
     """Signature prefix (roofline.signature form) of the gather kernel a plan launches."""
     import re
     k = info["kernel"]
+    m = re.match(r"(confocal_lds_kernel_(?:poly|column)<.*), KZ=(\d+), degree=(\d+)>", k)
+    if m:
+        return f"{m.group(1)}, {m.group(2)}, {m.group(3)}"
+    m = re.match(r"(paths_lds_kernel|confocal_kernel_split)<(\w+)", k)
+    if m:
+        return {"grid": "paths_lds_kernel<true", "pairs": "paths_lds_kernel<false"}.get(m.group(2), m.group(1))
     m = re.match(r"confocal_lds_kernel<KZ=(\d+), waves=(\d+)>", k)
     if m:
         fz = {("f32", False): "FusedF32", ("f16", False): "FusedH16<false>", ("bf16", False): "FusedH16<true>",

@@ -362,16 +362,18 @@ bpx_status bpx_plan_synchronize(bpx_plan plan);
 /* Copies the device volume to host (float or interleaved complex). */
 bpx_status bpx_plan_read_volume(bpx_plan plan, float* voxel_volume);
 /* Describes the plan: kernel path (0 confocal, 1 grid, 2 pairs), voxels per lane (the tile
- * depth, 8 or 16, for the LDS-staged kernel), number of
+ * depth, 8 or 16, for the LDS-staged kernels), number of
  * pairs used, chunk length, per-capture scale. */
 bpx_status bpx_plan_info(bpx_plan plan, int32_t* path, int32_t* lane_voxels, uint32_t* pairs_used,
                          uint32_t* Tc, float* scale);
-/* Name of the gather kernel an execution of the plan launches, with its tile shape (for
- * profiles and reports), as a NUL-terminated string of at most `capacity` bytes.  No reference
- * counterpart (the reference has one kernel per path). */
+/* Name of the gather kernel that the plan's last execution launched (as profiles show it: the kernel's
+ * function and, where they follow from the samples, its rows), with its tile shape and the number of
+ * parts that the pairs are split into, as a NUL-terminated string of at most `capacity` bytes.  No
+ * reference counterpart (the reference has one kernel per path). */
 bpx_status bpx_plan_kernel_name(bpx_plan plan, char* out, uint64_t capacity);
 /* The row storage (bpx_storage) the plan's last execution staged its samples in: F16 when an
- * F32 plan's samples were all exact in fp16 (see BPX_FLAG_KEEP_F32_ROWS), else the plan's own.
+ * F32 plan's samples were all held exactly in 16 bits, as fp16 values or as integer counts 0 .. 2048
+ * (see BPX_FLAG_KEEP_F32_ROWS; bpx_plan_kernel_name tells the two apart), else the plan's own.
  * Waits for that execution.  No reference counterpart. */
 bpx_status bpx_plan_row_storage(bpx_plan plan, uint32_t* storage);
 

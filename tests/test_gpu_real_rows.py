@@ -125,3 +125,36 @@ def test_split_pairs_equal_the_whole(gpu, N, tilted, rotated, storage, cplx):
     assert np.abs(b).min() > 0
     for x, y in ((a.real, b.real), (a.imag, b.imag)):
         assert np.all(np.abs(x.astype(np.float64) - y) <= 68 * EPS * np.abs(y).astype(np.float64))
+
+
+@pytest.mark.parametrize("storage,cplx,rows", [("f32", False, "F32Rows"), ("f16", False, "Half16Rows<false>"),
+                                               ("bf16", False, "Half16Rows<true>"), ("f32", True, "ComplexRows")])
+def test_reported_kernel_names_its_rows(gpu, storage, cplx, rows):
+    N, size, T, dT, t0, scan = CASES[1]
+    pr = pairs_of(*scan)
+    H = np.random.default_rng(1).gamma(0.5, 2.0, (len(pr), T)).astype(np.complex64 if cplx else f32)
+    grid = basis(N, (0.03, -0.02, 0.75), size)
+    with gpu.Plan(H, pr, N, *grid, t0, dT, storage=storage) as plan:
+        plan.execute()
+        info = plan.info()
+    kz = int(info["kernel"].split("KZ=")[1].split(",")[0])
+    assert info["kernel"].startswith(f"confocal_lds_kernel_column<{rows}, KZ=") and info["lane_voxels"] == kz, info
+
+
+@pytest.mark.parametrize("N,tilted,rotated", SPLIT_CASES)
+def test_split_pairs_are_reported(gpu, N, tilted, rotated):
+    """The plans of the test above: more than one part, and none with an explicit variant."""
+    pr = pairs_of(31, 33)
+    if tilted:
+        pr["laser_point"][:, 2] = np.linspace(0, 0.05, len(pr)).astype(f32)
+        pr["camera_point"] = pr["laser_point"]
+    zero, inc = basis(N, (0.03, -0.02, 0.75), (0.8, 0.8, 0.6))
+    if rotated:
+        inc = inc + np.array([0, 0, 0.004, 0, 0, 0.002, -0.004, 0.001, 0], f32)
+    H = np.random.default_rng(1).gamma(0.5, 2.0, (len(pr), 3000)).astype(f32)
+    for variant in (-1, 5):
+        with gpu.Plan(H, pr, N, zero, inc, 0.8, 0.0012, variant=variant) as plan:
+            plan.execute()
+            name = plan.info()["kernel"]
+        assert name.startswith("confocal_kernel_split<") == (variant == -1), name
+        assert variant == 5 or int(name.split("tiles, ")[1].split()[0]) > 1, name
