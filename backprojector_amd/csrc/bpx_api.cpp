@@ -441,7 +441,7 @@ bpx_status bpx_plan_tune(bpx_plan plan, int32_t reps, int32_t* variant) {
             float best_ms = INFINITY;
             try {
                 // the plan as it is (its default kernel, which no variant names), then each variant
-                const bool own = initial_auto && pl.poly_real;
+                const bool own = initial_auto && (pl.poly_real || pl.tex_parts > 1);
                 bool keep = own;
                 for (int v = own ? 2 : 3; v < variant_count(); ++v) {
                     if (v > 2) {

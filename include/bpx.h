@@ -398,10 +398,10 @@ bpx_status bpx_plan_benchmark(bpx_plan plan, int32_t warmup, int32_t iterations,
  * occupancy-only launch policy of backproject_cuda.cu:406): executes the plan once plus `reps`
  * times in every gather variant 3-8 that applies to it (the texture-path shapes of 4, 8 and 2
  * voxels per lane; the LDS-staged tile shapes whose bin windows fit) on its own stream and keeps
- * the fastest; every variant gives the same volume bit for bit.  A plan whose default kernel for real
- * rows is no variant is timed as it is first (it adds partial sums in double, so real volumes differ
- * from the variants' in the last bits) and keeps that kernel if nothing beats it.  *variant (may be
- * NULL) receives the chosen one; other plans keep theirs. */
+ * the fastest; every variant gives the same volume bit for bit.  A plan whose default kernel is no
+ * variant (polynomial quotients, pairs split over work-groups) is timed as it is first (it adds partial
+ * sums in double, so real volumes differ from the variants' in the last bits) and keeps that kernel if
+ * nothing beats it.  *variant (may be NULL) receives the chosen one; other plans keep theirs. */
 bpx_status bpx_plan_tune(bpx_plan plan, int32_t reps, int32_t* variant);
 void bpx_plan_destroy(bpx_plan plan);
 

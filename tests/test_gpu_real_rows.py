@@ -158,3 +158,19 @@ def test_split_pairs_are_reported(gpu, N, tilted, rotated):
             name = plan.info()["kernel"]
         assert name.startswith("confocal_kernel_split<") == (variant == -1), name
         assert variant == 5 or int(name.split("tiles, ")[1].split()[0]) > 1, name
+
+
+def test_tune_may_keep_split_pairs(gpu):
+    """27 tiles for 256 CUs: no kernel that leaves the pairs whole comes near the split default, so a tuned
+    plan runs it still, and its volume is the untuned plan's bit for bit."""
+    pr = pairs_of(61, 67)
+    N, grid = (24, 24, 24), basis((24, 24, 24), (0.03, -0.02, 0.75), (0.8, 0.8, 0.6))
+    H = np.random.default_rng(2).gamma(0.5, 2.0, (len(pr), 3000)).astype(f32)
+    with gpu.Plan(H, pr, N, *grid, 0.8, 0.0012) as plan:
+        plan.execute()
+        ref, name = plan.volume(), plan.info()["kernel"]
+        assert name.startswith("confocal_kernel_split<")
+        got = plan.tune(reps=4)
+        assert got["kernel"] == name, got
+        plan.execute()
+        assert plan.info()["kernel"] == name and np.array_equal(plan.volume(), ref)
