@@ -56,8 +56,9 @@ __device__ __forceinline__ void box_range(const float bmin[3], const float bmax[
 
 // GRID: pair p = l C + c; a part takes a range of lasers and, 8 SPADs at a time, walks its lasers with
 // the 8 SPAD legs of its voxels in registers.  Otherwise a part takes a range of pairs, both legs per
-// update.  A stage is 8 pairs, two copied by each wave, double-buffered.
-template <bool GRID, int KZ>
+// update.  A stage is 8 pairs, two copied by each wave, double-buffered.  FINE: compensated adds within a
+// grid's stages, for blocks of fewer than 8 pairs.
+template <bool GRID, int KZ, bool FINE>
 __global__ __launch_bounds__(256, GRID ? 2 : 3) void paths_lds_kernel(PathsLdsArgs a) {
     constexpr uint32_t CS = 8;
     constexpr int kNoWindow = (int)0x80000000;
@@ -222,8 +223,9 @@ __global__ __launch_bounds__(256, GRID ? 2 : 3) void paths_lds_kernel(PathsLdsAr
                         total[r] = total[r] + cw[c];
                     }
                     taps(total, m);
+                    if (FINE) settle(1u);
                 }
-            settle(n);
+            if (!FINE) settle(n);
         } else {
             const uint32_t n = t.idle ? 0u : min(CS, end - first - b * CS);
 #pragma unroll 1
@@ -294,9 +296,9 @@ size_t paths_lds_bytes(const PathsLdsArgs& a) {
     return 4u * ((size_t)((a.Tc + 1u + 63u) / 64u * 64u) + 17u * (size_t)a.seg);
 }
 
-template <bool GRID>
+template <bool GRID, bool FINE>
 static hipError_t paths_launch(const PathsLdsArgs& a, uint32_t parts, hipStream_t s) {
-    const auto fn = paths_lds_kernel<GRID, 8>;
+    const auto fn = paths_lds_kernel<GRID, 8, FINE>;
     const size_t lds = paths_lds_bytes(a);
     if (lds > 64u * 1024u) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
@@ -311,7 +313,8 @@ static hipError_t paths_launch(const PathsLdsArgs& a, uint32_t parts, hipStream_
     return hipGetLastError();
 }
 hipError_t launch_paths_lds(const PathsLdsArgs& a, uint32_t parts, hipStream_t s) {
-    return a.L ? paths_launch<true>(a, parts, s) : paths_launch<false>(a, parts, s);
+    if (!a.L) return paths_launch<false, false>(a, parts, s);
+    return a.kahan_block < 8u ? paths_launch<true, true>(a, parts, s) : paths_launch<true, false>(a, parts, s);
 }
 
 }  // namespace bpx

@@ -72,7 +72,9 @@ typedef enum bpx_semantics {
 /* Options of the extended entry points; a NULL pointer means all defaults. */
 typedef struct bpx_options {
     uint32_t storage;     /* bpx_storage (default F32)                                       */
-    uint32_t kahan_block; /* pairs summed plainly between compensated adds (0 -> 32)          */
+    uint32_t kahan_block; /* pairs summed plainly between compensated adds (0 -> 32; exhaustive
+                             grids end a block of 8 or more with a stage of up to 8 pairs, at
+                             most 7 late)                                                     */
     uint32_t flags;       /* BPX_FLAG_*                                                       */
     int32_t variant;      /* gather-kernel variant: -1 default (the LDS-staged kernel where it
                              applies: fp32 real samples, separable grid, flat wall, short bin

@@ -103,3 +103,23 @@ def test_paths_that_keep_the_general_kernels(gpu, oracle):
             vol = plan.volume()
         ref = oracle.a1_volume_f64acc(H, pr, N, zero, inc, 2.0, dT).astype(f32)
         assert np.array_equal(vol.real if cplx else vol, ref), (N, v, cplx)
+
+
+@pytest.mark.parametrize("variant", [-1, 2])
+@pytest.mark.parametrize("kahan", [1, 2])
+@pytest.mark.parametrize("nl,nc", [(9, 4), (7, 5)])
+def test_grid_blocks_shorter_than_a_stage(gpu, oracle, nl, nc, kahan, variant):
+    """Every sample 1.6000018: 8 of them summed plainly are 2.5 units (of 2^-24, relative) off, 1 or 2 are
+    exact.  Blocks of 1 or 2 leave the compensated sum's n 2^-48 and the final rounding, at most 1 unit;
+    blocks of 8 would end 1.8 to 2.9 off."""
+    pr = grid_pairs(oracle, nl, nc)
+    N, T = (32, 20, 16), 2500
+    zero, inc = basis(N, (0.05, -0.02, 0.75), (0.5, 0.4, 0.3))
+    H = np.full((len(pr), T), 1.6000018, f32)
+    exact = oracle.a1_volume_f64acc(H, pr, N, zero, inc, 0.0, 0.004)
+    assert np.allclose(exact, len(pr) * float(H[0, 0]), rtol=1e-12)
+    with gpu.Plan(H, pr, N, zero, inc, 0.0, 0.004, kahan_block=kahan, variant=variant) as plan:
+        plan.execute()
+        assert plan.info()["path"] == "grid" and plan.info()["kernel"].startswith("paths_lds") == (variant < 0)
+        vol = plan.volume().astype(np.float64)
+    assert np.abs(vol / exact - 1).max() <= 1.1 * 2.0 ** -24

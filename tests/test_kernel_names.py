@@ -20,8 +20,8 @@ NAMES = {
         "void bpx::confocal_lds_kernel_column<bpx::(anonymous namespace)::ComplexRows, 8, 2>(bpx::LdsPolyArgs)",
     "confocal_kernel_split<K=2> (8x8x8 tiles, 12 pair parts)":
         "void bpx::confocal_kernel_split<bpx::FusedSource<bpx::FusedF32>, 2, true, true>(bpx::ConfocalArgs, bpx::SplitPairs)",
-    "paths_lds_kernel<grid> (16x16x8 tiles, 4 parts)": "void bpx::paths_lds_kernel<true, 8>(bpx::PathsLdsArgs)",
-    "paths_lds_kernel<pairs> (16x16x8 tiles, 4 parts)": "void bpx::paths_lds_kernel<false, 8>(bpx::PathsLdsArgs)",
+    "paths_lds_kernel<grid> (16x16x8 tiles, 4 parts)": "void bpx::paths_lds_kernel<true, 8, false>(bpx::PathsLdsArgs)",
+    "paths_lds_kernel<pairs> (16x16x8 tiles, 4 parts)": "void bpx::paths_lds_kernel<false, 8, false>(bpx::PathsLdsArgs)",
     "confocal_lds_kernel<KZ=8, waves=4> (16x16x8 tiles)":
         "void bpx::confocal_lds_kernel<bpx::FusedF32, 8, 4>(bpx::ConfocalArgs)",
 }
