@@ -29,6 +29,8 @@
 
 namespace bpx {
 
+constexpr size_t kPartSums = 4ull << 30;   // partial sums of a batch, at most
+
 struct BatchImpl {
     std::vector<std::unique_ptr<PlanImpl>> plans;
     std::vector<uint64_t> updates;   // voxel-pair updates per capture
@@ -43,16 +45,18 @@ struct BatchImpl {
         LdsPolyShape shape;
         uint32_t parts = 1, part_pairs = 0;
         bool counts = false;
-        size_t parts_offset = 0;   // bytes in poly_parts
+        size_t parts_offset = 0;   // bytes in part_sums
+        uint32_t wave = 0;
     };
     // the captures that a plan of their own gathers on the texture path with the pairs split
     struct SplitCapture {
         uint32_t parts = 1, part_pairs = 0;
         size_t parts_offset = 0;
+        uint32_t wave = 0;
         Tiles tiles{};
     };
     std::vector<SplitCapture> split;
-    uint32_t n_split = 0, n_split_items = 0;
+    uint32_t n_split = 0;
     DeviceBuffer split_args, split_items;
     struct PolyGroup {             // one launch per row format
         LdsPolyShape shape;
@@ -60,7 +64,12 @@ struct BatchImpl {
         bool counts = false;       // some capture of it may hold counts
     };
     std::vector<PolyCapture> poly;
-    std::vector<PolyGroup> poly_groups;
+    // Captures whose partial sums are in part_sums together; the waves follow each other.
+    struct Wave {
+        std::vector<PolyGroup> groups;
+        uint32_t split_first = 0, split_n = 0;   // of split_items
+    };
+    std::vector<Wave> waves;
     uint32_t n_poly = 0, staged_row_blocks = 0;
     int poly_format = kF32Split;
     DeviceBuffer poly_args, poly_items, part_sums, sum_args, fmt_flags;
@@ -116,7 +125,7 @@ void BatchImpl::choose_kernels() {
     if (!takes_poly) poly_format = format;
     else poly_format = format == kC64 ? (int)kC64Split : format == kF32 ? (int)kF32Split : format;
     const uint32_t bytes = lds_poly_part_bytes(poly_format);
-    size_t total = 0;
+    std::vector<size_t> need(n, 0);   // partial sums of each
     for (uint32_t i = 0; i < n; ++i) {
         const PlanImpl& pl = *plans[i];
         PolyCapture& pc = poly[i];
@@ -130,8 +139,7 @@ void BatchImpl::choose_kernels() {
             sc.parts = split_parts(sc.tiles, pl.P, part_unit(pl.kahan_block), &sc.part_pairs);
             if (sc.parts <= 1u) continue;
             ++n_split;
-            sc.parts_offset = total;
-            total += ((size_t)sc.parts * pl.g.n[0] * pl.g.n[1] * pl.g.n[2] * (cplx ? 16u : 8u) + 255u) / 256u * 256u;
+            need[i] = ((size_t)sc.parts * pl.g.n[0] * pl.g.n[1] * pl.g.n[2] * (cplx ? 16u : 8u) + 255u) / 256u * 256u;
             continue;
         }
         ++n_poly;
@@ -139,51 +147,71 @@ void BatchImpl::choose_kernels() {
         pc.parts = lds_poly_parts(pl.g, pc.shape, pl.P, bytes, part_unit(pl.kahan_block), &pc.part_pairs);
         const uint64_t t = lds_tile_count(pl.g, pc.shape);
         if (t * pc.parts >= (1ull << 31)) fail(BPX_ERR_UNSUPPORTED, "batch capture too large");
-        pc.parts_offset = total;
-        if (pc.parts > 1)
-            total += ((size_t)pc.parts * pl.g.n[0] * pl.g.n[1] * pl.g.n[2] * bytes + 255u) / 256u * 256u;
+        if (pc.parts > 1) need[i] = ((size_t)pc.parts * pl.g.n[0] * pl.g.n[1] * pl.g.n[2] * bytes + 255u) / 256u * 256u;
     }
     if (!n_poly && !n_split) return;
-    part_sums.alloc(total);
+    // The partial sums of a capture take up to 64 MiB.  Captures whose sums fit kPartSums together
+    // are gathered in one wave; where memory is short, in smaller ones, one after the other.
+    uint32_t n_waves = 0;
+    for (size_t room = kPartSums;; room /= 4u) {
+        size_t used = 0, most = 0;
+        n_waves = 1u;
+        for (uint32_t i = 0; i < n; ++i) {
+            if (used + need[i] > room && used) {
+                ++n_waves;
+                used = 0;
+            }
+            poly[i].wave = split[i].wave = n_waves - 1u;
+            poly[i].parts_offset = split[i].parts_offset = used;
+            used += need[i];
+            most = std::max(most, used);
+        }
+        if (room > (64u << 20) ? part_sums.try_alloc(most) : (part_sums.alloc(most), true)) break;
+    }
+    waves.assign(n_waves, Wave{});
     // a launch per depth and window length (LDS decides how many work-groups a CU holds), its items
     // by falling length: the short ones fill the end
     std::vector<uint32_t> order(n);
     std::iota(order.begin(), order.end(), 0u);
     std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return poly[x].part_pairs > poly[y].part_pairs; });
     std::vector<uint32_t> items;
-    for (int kz : {16, 8})
-        for (uint32_t most = 128u; most <= kPolySegMax; most += 128u) {
-            PolyGroup g;
-            g.first = (uint32_t)(items.size() / 2u);
-            for (uint32_t i : order) {
-                const LdsPolyShape& sh = poly[i].shape;
-                if (sh.kz != kz || (sh.seg + 127u) / 128u * 128u != most) continue;
-                g.shape.kz = kz;
-                g.shape.deg = std::max(g.shape.deg, sh.deg);
-                g.shape.seg = std::max(g.shape.seg, sh.seg);
-                g.counts = g.counts || poly[i].counts;
-                const uint32_t blocks = (uint32_t)lds_tile_count(plans[i]->g, sh) * poly[i].parts;
-                for (uint32_t k = 0; k < blocks; ++k) {
-                    items.push_back(i);
-                    items.push_back(k);
+    for (uint32_t wave = 0; wave < n_waves; ++wave)
+        for (int kz : {16, 8})
+            for (uint32_t most = 128u; most <= kPolySegMax; most += 128u) {
+                PolyGroup g;
+                g.first = (uint32_t)(items.size() / 2u);
+                for (uint32_t i : order) {
+                    const LdsPolyShape& sh = poly[i].shape;
+                    if (poly[i].wave != wave || sh.kz != kz || (sh.seg + 127u) / 128u * 128u != most) continue;
+                    g.shape.kz = kz;
+                    g.shape.deg = std::max(g.shape.deg, sh.deg);
+                    g.shape.seg = std::max(g.shape.seg, sh.seg);
+                    g.counts = g.counts || poly[i].counts;
+                    const uint32_t blocks = (uint32_t)lds_tile_count(plans[i]->g, sh) * poly[i].parts;
+                    for (uint32_t k = 0; k < blocks; ++k) {
+                        items.push_back(i);
+                        items.push_back(k);
+                    }
                 }
+                g.n = (uint32_t)(items.size() / 2u) - g.first;
+                if (g.n) waves[wave].groups.push_back(g);
             }
-            g.n = (uint32_t)(items.size() / 2u) - g.first;
-            if (g.n) poly_groups.push_back(g);
-        }
     poly_items.alloc(4u * items.size());
     if (!items.empty())
         hip_check(hipMemcpy(poly_items.ptr, items.data(), 4u * items.size(), hipMemcpyHostToDevice), "hipMemcpy");
     items.clear();
     std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return split[x].part_pairs > split[y].part_pairs; });
-    for (uint32_t i : order)
-        for (uint32_t k = 0; split[i].parts > 1u && k < split[i].tiles.count * split[i].parts; ++k) {
-            items.push_back(i);
-            items.push_back(k);
-        }
-    n_split_items = (uint32_t)(items.size() / 2u);
+    for (uint32_t wave = 0; wave < n_waves; ++wave) {
+        waves[wave].split_first = (uint32_t)(items.size() / 2u);
+        for (uint32_t i : order)
+            for (uint32_t k = 0; split[i].wave == wave && split[i].parts > 1u && k < split[i].tiles.count * split[i].parts; ++k) {
+                items.push_back(i);
+                items.push_back(k);
+            }
+        waves[wave].split_n = (uint32_t)(items.size() / 2u) - waves[wave].split_first;
+    }
     split_items.alloc(4u * items.size());
-    if (n_split_items)
+    if (!items.empty())
         hip_check(hipMemcpy(split_items.ptr, items.data(), 4u * items.size(), hipMemcpyHostToDevice), "hipMemcpy");
     std::vector<SplitPairs> sp(std::max<uint32_t>(n, 1u), SplitPairs{});
     for (uint32_t i = 0; i < n; ++i)
@@ -381,11 +409,11 @@ void BatchImpl::build(const bpx_batch_config& c) {
             counts.fmt_want = 1u;      // never
         }
     }
-    std::vector<PartsSum> sums(std::max<uint32_t>(n, 1u), PartsSum{});
+    std::vector<PartsSum> sums(std::max<size_t>(n * waves.size(), 1u), PartsSum{});   // of each wave, its captures'
     for (uint32_t i = 0; i < n; ++i) {
         if (!plans[i]->P || queued(i)) continue;
         const uint32_t own = poly[i].shape.kz ? poly[i].parts : split[i].parts;
-        sums[i] = {args[i].out, static_cast<char*>(part_sums.ptr) + (poly[i].shape.kz ? poly[i].parts_offset : split[i].parts_offset),
+        sums[(size_t)poly[i].wave * n + i] = {args[i].out, static_cast<char*>(part_sums.ptr) + (poly[i].shape.kz ? poly[i].parts_offset : split[i].parts_offset),
                    static_cast<const uint32_t*>(fmt_flags.ptr) + i,
                    (uint64_t)args[i].g.n[0] * args[i].g.n[1] * args[i].g.n[2], poly[i].counts ? poly[i].parts : 0u, own,
                    cplx ? 1u : 0u, args[i].scale};
@@ -473,35 +501,38 @@ void BatchImpl::build(const bpx_batch_config& c) {
                           "batch sample check kernel");
             hip_check(launch_stage(static_cast<const StageJob*>(zjobs.ptr), n_poly + n_split, 0u, staged_row_blocks, stream),
                       "batch row staging kernel");
-            // the split captures' scattered gathers beside the LDS gathers: they load other units
-            const bool beside = n_split_items && !poly_groups.empty();
-            if (beside) {
-                hip_check(hipEventRecord(fork, stream), "hipEventRecord");
-                hip_check(hipStreamWaitEvent(side, fork, 0), "hipStreamWaitEvent");
-                side_joined = true;
-            }
-            if (n_split_items)
-                hip_check(launch_batch_split(BatchItems{static_cast<const uint2*>(split_items.ptr), n_split_items}, q.caps,
-                                             static_cast<const SplitPairs*>(split_args.ptr), q.flags, format,
-                                             beside ? side : stream),
-                          "batch gather kernel (pairs split)");
-            for (const bool counts : {true, false})
-                for (const PolyGroup& g : poly_groups) {
-                    if (counts && !g.counts) continue;
-                    const LdsPolyArgs* caps = static_cast<const LdsPolyArgs*>(poly_args.ptr) + (counts ? 0u : pargs.size());
-                    const BatchItems b{static_cast<const uint2*>(poly_items.ptr) + g.first, g.n};
-                    hip_check(launch_batch_poly(b, caps, g.shape, counts ? (int)kCount : poly_format, stream),
-                              "batch gather kernel (polynomial quotients)");
+            for (size_t k = 0; k < waves.size(); ++k) {
+                const Wave& wave = waves[k];
+                // the split captures' scattered gathers beside the LDS gathers: they load other units
+                const bool beside = wave.split_n && !wave.groups.empty();
+                if (beside) {
+                    hip_check(hipEventRecord(fork, stream), "hipEventRecord");
+                    hip_check(hipStreamWaitEvent(side, fork, 0), "hipStreamWaitEvent");
+                    side_joined = true;
                 }
-            if (beside) {
-                hip_check(hipEventRecord(join, side), "hipEventRecord");
-                hip_check(hipStreamWaitEvent(stream, join, 0), "hipStreamWaitEvent");
-                side_joined = false;
+                if (wave.split_n)
+                    hip_check(launch_batch_split(
+                                  BatchItems{static_cast<const uint2*>(split_items.ptr) + wave.split_first, wave.split_n}, q.caps,
+                                  static_cast<const SplitPairs*>(split_args.ptr), q.flags, format, beside ? side : stream),
+                              "batch gather kernel (pairs split)");
+                for (const bool counts : {true, false})
+                    for (const PolyGroup& g : wave.groups) {
+                        if (counts && !g.counts) continue;
+                        const LdsPolyArgs* caps = static_cast<const LdsPolyArgs*>(poly_args.ptr) + (counts ? 0u : pargs.size());
+                        const BatchItems b{static_cast<const uint2*>(poly_items.ptr) + g.first, g.n};
+                        hip_check(launch_batch_poly(b, caps, g.shape, counts ? (int)kCount : poly_format, stream),
+                                  "batch gather kernel (polynomial quotients)");
+                    }
+                if (beside) {
+                    hip_check(hipEventRecord(join, side), "hipEventRecord");
+                    hip_check(hipStreamWaitEvent(stream, join, 0), "hipStreamWaitEvent");
+                    side_joined = false;
+                }
+                for (uint32_t i = 0; i < n; i += 32768u)
+                    hip_check(launch_batch_sum_parts(static_cast<const PartsSum*>(sum_args.ptr) + k * n + i,
+                                                     std::min(n - i, 32768u), q.remaining + i, q.done + i, stream),
+                              "batch partial sums kernel");
             }
-            for (uint32_t i = 0; i < n; i += 32768u)
-                hip_check(launch_batch_sum_parts(static_cast<const PartsSum*>(sum_args.ptr) + i, std::min(n - i, 32768u),
-                                                 q.remaining + i, q.done + i, stream),
-                          "batch partial sums kernel");
         }
         if (two) {
             // every row staged first (no waits in either queue), then both queues side by side

@@ -2,7 +2,7 @@
 along; what a faster kernel would need beside its general form is given up instead.  Counts, so every
 volume must EQUAL the oracle's exactly accumulated one."""
 import ctypes
-from contextlib import contextmanager
+from contextlib import contextmanager, nullcontext
 
 import numpy as np
 import pytest
@@ -129,3 +129,32 @@ def test_octree_tile_sums_that_do_not_fit(gpu):
         assert np.array_equal(plan.volume(), ref)
         plan.execute()
         assert np.array_equal(plan.volume(), ref)
+
+
+def test_batch_sums_that_do_not_fit(gpu):
+    """70 captures of 64 MiB of partial sums each: at most 4 GiB at a time, and where they do not fit
+    either, in smaller waves.  Every volume is its own plan's bit for bit."""
+    N, T = (64, 64, 64), 300
+    grid = basis(N, (0.0, 0.0, 0.7), (0.4, 0.4, 0.4))
+    kinds = []
+    for k in range(5):
+        H, pr = capture((64, 64), T, k)
+        kinds.append(((H + f32(0.25) if k % 2 else H), pr, N, *grid, 1.0, 0.006))
+    refs = []
+    for a in kinds:
+        with gpu.Plan(*a) as plan:
+            plan.execute()
+            refs.append(plan.volume())
+            assert int(plan.info()["kernel"].split("tiles, ")[1].split()[0]) >= 32
+    args = [kinds[i % 5] for i in range(70)]
+    b, taken = memory_of(lambda: gpu.Batch(args))
+    rows = len(args) * (T * 4096 * 4 + 8 * 4096 * 384 + 4 * 64 ** 3)
+    assert taken < rows + (4 << 30) + (256 << 20), taken
+    for room in (None, 5 << 29):
+        with memory_left(room) if room else nullcontext(), b or gpu.Batch(args) as batch:
+            for rep in range(2):
+                batch.execute()
+                for i in range(0, 70, 3):
+                    assert np.array_equal(batch.volume(i), refs[i % 5]), (room, rep, i)
+            assert np.all(batch.latencies() > 0)
+        b = None
