@@ -432,14 +432,16 @@ typedef struct bpx_capture_desc {
     float voxel_inc[9];
     float t0, deltaT;
 } bpx_capture_desc;
+/* The configuration of the queues: it concerns the captures that the item launches do not take (groups
+ * reads 1 where the first queue is empty). */
 typedef struct bpx_batch_config {
     uint32_t lane_voxels;  /* voxels per lane: 2 or 4                                   */
     uint32_t groups;       /* persistent work-groups (0 = all that are resident at once) */
     uint32_t order;        /* queue: 0 = most work first, 1 = given order, 2 = most work
                               first with texture-path tiles spread among LDS-staged ones */
-    uint32_t lds_captures; /* out (get/tune): captures run as LDS-staged tiles (those whose
-                              bin windows fit the queue's LDS segment); ignored by
-                              set_config                                                */
+    uint32_t lds_captures; /* out (get/tune): captures whose bin windows fit the queues' LDS
+                              segment, those that the item launches take (and never a
+                              queue) among them; ignored by set_config                 */
     uint32_t lds_depth;    /* LDS-staged tile depth: 8 (16 x 16 x 8) or 16 (16^3); 0 = 8;
                               complex formats always use 8                              */
     uint32_t launches;     /* 1 (or 0): one persistent launch serves the rows' staging, the

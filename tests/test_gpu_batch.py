@@ -254,3 +254,108 @@ def test_c4_64_uneven_captures(gpu, oracle):
             ref = oracle.a1_voxels_f64acc(H, pr, vox, zero, inc, t0, dT)
             got = b.volume(i)[vox[:, 0], vox[:, 1], vox[:, 2]]
             assert ref.max() > 0 and np.array_equal(got.astype(np.float64), ref), i
+
+
+# ------------------------------------------------------------------ captures outside the queues
+def _plan_volumes(gpu, caps, storage="f32"):
+    out = []
+    for c in caps:
+        with gpu.Plan(*c, storage=storage) as plan:
+            plan.execute()
+            out.append((plan.volume(), plan.info()["kernel"]))
+    return out
+
+
+def _poly_captures(samples):
+    """The geometries of the polynomial-quotient gather's own tests: columns of 8 and 16, several window
+    lengths, one part of the pairs and many.  samples: one kind per capture, in turn."""
+    from test_gpu_count_rows import CASES, basis, pairs_of
+    caps = []
+    for i, (N, size, T, dT, t0, scan) in enumerate(CASES):
+        pr, rng = pairs_of(*scan), np.random.default_rng(i)
+        H = rng.integers(0, 60, (len(pr), T)).astype(f32)
+        kind = samples[i % len(samples)]
+        if kind == "real":
+            H = rng.gamma(0.5, 2.0, H.shape).astype(f32)
+        elif kind == "negative":
+            H[len(pr) // 2, T // 2] = -3
+        elif kind == "complex":
+            H = (rng.gamma(0.5, 2.0, H.shape) - 1j * rng.gamma(0.5, 2.0, H.shape)).astype(np.complex64)
+        caps.append((H, pr, N, *basis(N, (0.03, -0.02, 0.75), size), t0, dT))
+    return caps
+
+
+@pytest.mark.parametrize("samples,storage", [(("real",), "f32"), (("counts", "real", "negative"), "f32"),
+                                             (("negative", "counts", "real"), "f32"), (("real",), "f16"), (("real",), "bf16"),
+                                             (("complex",), "f32")])
+def test_batch_of_polynomial_captures(gpu, samples, storage):
+    """Each capture's rows are chosen by its own samples; every volume is its own plan's bit for bit."""
+    caps = _poly_captures(samples)
+    alone = _plan_volumes(gpu, caps, storage)
+    names = [n for _, n in alone]
+    assert all(n.startswith("confocal_lds_kernel_") for n in names), names
+    parts = [int(n.split("tiles, ")[1].split()[0]) for n in names]
+    assert min(parts) == 1 and max(parts) > 4, names
+    if samples[0] != "complex":
+        assert {n.split("KZ=")[1].split(",")[0] for n in names} == {"8", "16"}
+    if len(samples) > 1:
+        assert any("CountRows" in n for n in names) and any("F32Rows" in n for n in names)
+    with gpu.Batch(caps, storage=storage) as b:
+        assert b.config()["groups"] == 1      # nothing queued
+        for rep in range(3):
+            b.execute()
+            for i, (ref, _) in enumerate(alone):
+                assert np.array_equal(b.volume(i), ref), (rep, i)
+        assert np.all(b.latencies() > 0)
+
+
+QUEUE_CONFIGS = [dict(lane_voxels=k, groups=g, order=o, lds_depth=d, launches=l)
+                 for k, g, o, d, l in [(2, 0, 0, 8, 1), (4, 7, 1, 8, 1), (2, 0, 2, 16, 1), (4, 3, 2, 16, 1), (2, 0, 0, 8, 2), (4, 5, 1, 16, 2),
+                                       (2, 0, 0, 8, 3), (4, 2, 1, 8, 3)]]
+
+
+def _queued_captures(cplx=False):
+    """Volumes that reach the wall, from too few pairs to split: LDS-staged tiles of 16^3, of 16 x 16 x 8 and
+    texture-path tiles of the queues, among captures outside them."""
+    from test_gpu_count_rows import basis, pairs_of
+    # volume, size, centre's z, bin width, scan
+    spec = [((40, 33, 35), (0.2, 0.2, 0.2), 0.05, 0.002, (9, 8)), ((24, 20, 18), (0.3, 0.3, 0.2), 0.05, 0.004, (7, 6)),
+            ((20, 22, 9), (1.5, 1.5, 0.5), 0.1, 0.0015, (5, 9)), ((17, 16, 31), (0.3, 0.3, 0.3), 0.75, 0.001, (20, 21)),
+            ((33, 17, 40), (0.15, 0.1, 0.2), 0.02, 0.003, (11, 11)), ((9, 7, 5), (0.8, 0.8, 0.6), 0.75, 0.0012, (31, 33))]
+    caps = []
+    for i, (N, size, z, dT, scan) in enumerate(spec):
+        pr, T = pairs_of(*scan), 1400
+        H = np.random.default_rng(i).gamma(0.5, 2.0, (len(pr), T)).astype(f32)
+        if cplx:
+            H = (H - 0.5j * H[:, ::-1]).astype(np.complex64)
+        caps.append((H, pr, N, *basis(N, (0.03, -0.02, z), size), 0.9 if z < 0.5 else 1.8, dT))
+    return caps
+
+
+@pytest.mark.parametrize("storage,cplx", [("f32", False), ("bf16", False), ("f32", True), ("f16", True)])
+def test_batch_queues(gpu, storage, cplx):
+    caps = _queued_captures(cplx)
+    alone = _plan_volumes(gpu, caps, storage)
+    assert all(np.abs(v).max() > 0 for v, _ in alone)
+    assert sum(n.startswith("confocal_kernel<") for _, n in alone) >= 4, [n for _, n in alone]
+    groups = {}
+    with gpu.Batch(caps, storage=storage) as b:
+        for cfg in QUEUE_CONFIGS:
+            if cplx and (cfg["launches"] == 3 or cfg["lds_depth"] == 16):
+                continue
+            b.set_config(**cfg)
+            got = b.config()
+            groups[cfg["launches"], cfg["groups"], cfg["lds_depth"]] = got["groups"]
+            for rep in range(2):
+                b.execute()
+                for i, (ref, _) in enumerate(alone):
+                    assert np.array_equal(b.volume(i), ref), (cfg, rep, i)
+            assert np.all(b.latencies() > 0)
+        tuned = b.tune(reps=1)
+        b.execute()
+        for i, (ref, _) in enumerate(alone):
+            assert np.array_equal(b.volume(i), ref), (tuned, i)
+    # groups 0: as many as the queue has items, here; three launches take the 16^3 tiles out of it
+    assert groups[1, 0, 8] > groups[2, 0, 8] > 1, groups
+    if not cplx:
+        assert groups[3, 0, 8] < groups[2, 0, 8], groups
