@@ -141,7 +141,7 @@ _lib = None
 
 # Every symbol include/bpx.h declares (checked by the CPU test suite).
 EXPORTED = [
-    "bpx_last_error", "bpx_version", "bpx_abi_version", "bpx_device_count", "bpx_row_windows",
+    "bpx_last_error", "bpx_version", "bpx_abi_version", "bpx_device_count", "bpx_release_memory", "bpx_row_windows",
     "bpx_backprojection", "bpx_complex_backprojection", "bpx_backprojection_ex", "bpx_backprojection_noalloc",
     "bpx_window_backprojection", "bpx_phasor_pulse", "bpx_nlos_backproject", "bpx_nlos_phasor", "bpx_nlos_phasor_multi",
     "bpx_nlos_phasor_output",
@@ -172,6 +172,7 @@ def lib():
     L.bpx_version.restype = ctypes.c_char_p
     L.bpx_abi_version.restype = ctypes.c_int
     L.bpx_device_count.restype = ctypes.c_int
+    L.bpx_release_memory.argtypes = [ctypes.POINTER(u64)]
     for name in ("bpx_backprojection", "bpx_complex_backprojection"):
         getattr(L, name).argtypes = [c_p, u64, u32, c_p, u32, c_p, c_p, c_p, c_p, f32, f32]
     L.bpx_backprojection_ex.argtypes = [c_p, u64, u32, c_p, u32, c_p, c_p, c_p, c_p, f32, f32,

@@ -109,6 +109,14 @@ def phasor_pulse(transient_data, wavelength, deltaT, times=4, sigma=0.0):
     return out
 
 
+def release_memory():
+    """Gives the device memory back that the library keeps for reuse (at most 512 MiB of destroyed plans'
+    blocks); returns its bytes."""
+    n = ctypes.c_uint64()
+    check(lib().bpx_release_memory(ctypes.byref(n)))
+    return int(n.value)
+
+
 def row_windows(pairs, voxels_per_side, volume_zero_pos, voxel_inc, t0, deltaT, Tc):
     """[P][2] uint32 element windows [lo, hi) of the fused rows that a confocal plan of this
     geometry stages at each execution (no reference counterpart; host only, no device call)."""

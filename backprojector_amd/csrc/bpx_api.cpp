@@ -90,6 +90,12 @@ const char* bpx_last_error(void) { return g_error.c_str(); }
 const char* bpx_version(void) { return "bpx 0.1.0 (gfx950)"; }
 int bpx_abi_version(void) { return BPX_ABI_VERSION; }
 int bpx_device_count(void) { return find_device() >= 0 ? 1 : 0; }
+bpx_status bpx_release_memory(uint64_t* bytes) {
+    return guarded([&] {
+        const size_t n = release_pooled();
+        if (bytes) *bytes = n;
+    });
+}
 
 bpx_status bpx_backprojection_ex(const float* transient_chunk, uint64_t transient_size, uint32_t T,
                                  const bpx_pair* scanned_pairs, uint32_t num_pairs,

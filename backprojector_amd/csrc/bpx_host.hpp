@@ -67,6 +67,9 @@ struct DeviceBuffer {
     ~DeviceBuffer() { release(); }
 };
 
+// Gives back every block that is kept for later allocations; their bytes.
+size_t release_pooled();
+
 struct PlanImpl;
 
 // Octree refinement state (bpx_octree.hip kernels, bpx_octree_plan.cpp orchestration).

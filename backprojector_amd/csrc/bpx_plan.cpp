@@ -142,6 +142,19 @@ void DeviceBuffer::release() {
     bytes = cap = 0;
 }
 
+size_t release_pooled() {
+    Pool& p = pool();
+    std::vector<void*> all;
+    size_t bytes = 0;
+    {
+        std::lock_guard<std::mutex> lock(p.mutex);
+        bytes = p.bytes;
+        all = evict(p, 0);
+    }
+    for (void* b : all) (void)hipFree(b);
+    return bytes;
+}
+
 hipStream_t take_stream() {
     const int device = current_device();
     {

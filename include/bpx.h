@@ -109,6 +109,12 @@ const char* bpx_version(void);
 int bpx_abi_version(void);
 /* Number of usable gfx950 devices (0 when none); never fails. */
 int bpx_device_count(void);
+/* Gives the device memory back that the library keeps for reuse: blocks of up to 256 MiB of destroyed
+ * plans and batches, at most 512 MiB in all, none for longer than 256 allocations; they are also given
+ * back before an allocation of the library fails, but another allocator in the process cannot have them.
+ * *bytes (may be NULL) receives their size.  Pinned host memory of up to 68 MiB (staging of transfers
+ * and tables) stays until the process ends.  No reference counterpart. */
+bpx_status bpx_release_memory(uint64_t* bytes);
 /* The per-pair element windows [lo, hi) of the fused rows that a confocal plan of this
  * geometry stages at each execution: every element a gather kernel can read for the pair and
  * any voxel of the grid (element j of a row holds bin j - 1's sample and bin j's threshold).

@@ -158,3 +158,22 @@ def test_batch_sums_that_do_not_fit(gpu):
                     assert np.array_equal(batch.volume(i), refs[i % 5]), (room, rep, i)
             assert np.all(batch.latencies() > 0)
         b = None
+
+
+def test_kept_blocks_can_be_given_back(gpu, oracle):
+    """What destroyed plans leave with the library is bounded, and a call returns it to the device."""
+    H, pr = capture((64, 64), 2000)
+    N = (128, 128, 128)
+    args = (H, pr, N, *basis(N, (0.0, 0.0, 0.7), (0.4, 0.4, 0.4)), 0.5, 0.003)
+    gpu.release_memory()
+    assert gpu.release_memory() == 0
+    with gpu.Plan(*args) as plan:
+        plan.execute()
+        ref = plan.volume()
+    kept = []
+    _, taken = memory_of(lambda: kept.append(gpu.release_memory()))
+    assert 100 << 20 < kept[0] <= 512 << 20
+    assert -taken >= kept[0] // 2 and gpu.release_memory() == 0
+    with gpu.Plan(*args) as plan:
+        plan.execute()
+        assert np.array_equal(plan.volume(), ref)
