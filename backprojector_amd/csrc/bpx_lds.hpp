@@ -36,7 +36,7 @@ __device__ __forceinline__ double uniform_f64(double x) {
 // before the current stage's gathers.)
 __device__ __forceinline__ void load_lds16(__amdgpu_buffer_rsrc_t r, uint32_t lds_base, int off) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                 :: "s"(lds_base), "v"(off), "s"(r) : "memory");
+                 :: "s"(lds_base), "v"(off), "s"(r) : "m0", "memory");
 }
 __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
