@@ -8,7 +8,8 @@
 // The gather is the arbitrary-pair kernel reading the caller's unpadded rows directly
 // (pairs_kernel, RAW): both legs of the path with the exact square root, the bin decided
 // against the capture's path-length thresholds, the same per-update values and Kahan blocks of
-// 32 pairs in pair order as the table-driven kernels, so the volume equals bpx_backprojection's.
+// 32 pairs in pair order as the table-driven kernels, so for confocal captures the volume is variant 5's
+// bit for bit (the default kernels may split the pairs, and differ in the last bits where sums round).
 #include <hip/hip_runtime.h>
 
 #include <cmath>

@@ -76,12 +76,18 @@ typedef struct bpx_options {
                              grids end a block of 8 or more with a stage of up to 8 pairs, at
                              most 7 late)                                                     */
     uint32_t flags;       /* BPX_FLAG_*                                                       */
-    int32_t variant;      /* gather-kernel variant: -1 default (the LDS-staged kernel where it
-                             applies: fp32 real samples, separable grid, flat wall, short bin
-                             windows; else 5); 0-2 split tables, 3-5 fused rows with 4, 8, 2
-                             voxels per lane; 6 / 7 / 8 LDS-staged 16^3 tiles of 256 lanes,
-                             16x16x8 of 256, 16^3 of 512                                    */
+    int32_t variant;      /* gather-kernel variant: -1 default (below); 0-2 split tables, 3-5
+                             fused rows with 4, 8, 2 voxels per lane; 6 / 7 / 8 LDS-staged
+                             16^3 tiles of 256 lanes, 16x16x8 of 256, 16^3 of 512           */
 } bpx_options;
+/* Default kernels.  Confocal captures on a flat wall with voxel columns along its normal: the LDS-staged
+ * gather with polynomial quotients, where its bin windows and column polynomials fit (counts, fp32,
+ * 16-bit real and complex64 rows).  Other confocal captures: the LDS-staged tiles of variants 6-8 where
+ * they apply and fill the GPU, else 5.  Exhaustive grids and pair lists of real samples: LDS-staged
+ * paths, where their windows fit.  The first, the last and 5 split the pairs where the volume's tiles
+ * alone would leave the GPU idle: every part is summed as kahan_block says, the parts are added in double
+ * and rounded once.  Sums that are exact in any order (integers below 2^24, as those of counts) are the
+ * same from every kernel, others agree within the sums' rounding. */
 
 /* Drop the last P mod min(256, P) pairs exactly as the reference launcher does
  * (backproject_cuda.cu:150, 418); off by default (every pair is used). */
@@ -96,11 +102,12 @@ typedef struct bpx_options {
 /* bpx_batch_create: every capture's transient_chunk holds interleaved complex samples
  * (transient_size counts complex elements) and every volume is complex (2 floats per voxel). */
 #define BPX_FLAG_COMPLEX_SAMPLES 0x4u
-/* F32 storage on the LDS-staged confocal kernel: when every sample of an execution is an
- * integer of magnitude <= 2048 (photon counts, as captures hold), the rows are staged as fp16,
- * which holds those values exactly, and the gather reads half the LDS bytes per lookup; the
- * volume is the fp32 rows' bit for bit.  Each execution checks its samples on the device.
- * This flag keeps fp32 rows always (no reference counterpart: an internal layout choice). */
+/* F32 storage of confocal captures: when every sample of an execution is a count (an integer 0 .. 2048)
+ * the polynomial-quotient gather stages the rows as 16-bit integers and sums them as integers; the
+ * LDS-staged tiles of 8 voxels per lane stage integers of magnitude <= 2048 as fp16, which holds them
+ * exactly.  The volume is the fp32 rows' bit for bit either way, and each execution checks its samples on
+ * the device.  This flag keeps fp32 rows always, and with them the kernels of the explicit variants (no
+ * reference counterpart: an internal layout choice). */
 #define BPX_FLAG_KEEP_F32_ROWS 0x8u
 
 /* ------------------------------------------------------------------ diagnostics */
@@ -154,7 +161,9 @@ bpx_status bpx_backprojection_ex(const float* transient_chunk, uint64_t transien
 /* No counterpart in the reference.  For callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): the volume of
  * bpx_backprojection (fp32 samples, every pair used) computed on caller-owned DEVICE buffers,
- * with no hipMalloc / hipFree / allocating library call.  The library's working tables live in
+ * with no hipMalloc / hipFree / allocating library call.  Blocks of 32 pairs in pair order: for confocal
+ * captures variant 5's volume bit for bit, and the default's within the rounding of its sums (equal for
+ * counts).  The library's working tables live in
  * one fixed device array of BPX_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends.
  *   transient_chunk: device pointer, [num_pairs][T] fp32 samples (transient_size = num_pairs * T)
  *   scanned_pairs:   HOST array (copied into the fixed array; finite values only)
