@@ -404,7 +404,7 @@ struct Ring {
     hipEvent_t* ensure() {
         if (!at) {
             void* p = nullptr;
-            hip_check(hipHostMalloc(&p, kRingBytes, hipHostMallocPortable), "hipHostMalloc");
+            hip_check(hipHostMalloc(&p, kRingBytes, hipHostMallocDefault), "hipHostMalloc");
             at = static_cast<char*>(p);
         }
         Events& ev = events[current_device()];
