@@ -159,11 +159,11 @@ struct PlanImpl {
     // window path
     float vpos[3]{}, vsize_in[3]{}, wzero[3]{}, wvs[3]{}, half_width = 0, c1_lo = 0, c1_hi = 0;
     bool all_confocal = false;
-    // the LDS-staged window kernel (poly.kz != 0): its arguments but for the buffers
     // the LDS-staged kernel of non-confocal captures (paths.seg != 0): its arguments but for the
     // buffers, parts and whether it applies
     PathsLdsArgs paths{};
     uint32_t paths_parts = 1;
+    // the LDS-staged window kernel (poly.kz != 0): its arguments but for the buffers
     WindowLdsArgs wlds{};
     DeviceBuffer win_lo, win_hi;         // threshold tables [P][pitch], double
     DeviceBuffer raw, H, S, Z, Z2, pair8, pair4, lasers, spads, vol;

@@ -695,7 +695,9 @@ LdsPolyShape lds_poly_shape(const Grid& g, float inv2, float lz, double bound, d
         // Depth 16 spreads a pair's coefficients over more updates, depth 8 pads the last slab less:
         // per slice of z fp32 and bf16 rows take 5 to 6 % more time at depth 8, counts some 10 %
         // (4,096 pairs into 96^3, bf16: 0.79 ms at depth 16, 0.84 at 8; 9,216 pairs into
-        // 128 x 120 x 100, fp32: 5.08 ms for 7 slabs of 16, 4.96 for 13 of 8).
+        // 128 x 120 x 100, fp32: 5.08 ms for 7 slabs of 16, 4.96 for 13 of 8).  The line at 10 %
+        // padding is the counts'; for the rows that it serves (counts keep depth 16) the two sides
+        // are level near 6 %, so up to 4 % are given away between 11 and 17 slabs of 8.
         const uint32_t pad16 = (g.n[2] + 15u) / 16u * 16u, pad8 = (g.n[2] + 7u) / 8u * 8u;
         if (kz == 16 && format != kCount && pad16 * 10u > pad8 * 11u) continue;
         LdsPolyShape sh;

@@ -11,8 +11,12 @@ rooflines they place it against.
   instruction issue, transcendental (sqrt) rate, HBM bandwidth -- and the binding one.
 
 MI355X figures: 256 CUs x 4 SIMDs x 16 lanes at 2.4 GHz = 3.93e13 VALU lane-instructions/s
-(non-packed); transcendental instructions (v_sqrt_f32) issue at a quarter of that, 9.83e12/s;
-HBM3E 8 TB/s.
+(non-packed); transcendental instructions (v_sqrt_f32) nominally issue at a quarter of that, 9.83e12/s;
+HBM3E 8 TB/s.  The fractions are of these nominal rates, which some instructions beat (measured with 8
+independent chains a lane on 4,096 work-groups): plain fp32 adds, multiplies and v_fmamk_f32 6.5e13 to
+6.7e13/s, 32-bit integer adds, ands and shifts 5.5e13 to 5.9e13, v_sqrt_f32 1.95e13; v_fma_f32 and compares
+stay at 3.7e13 to 3.8e13.  A kernel of the faster ones can pass a nominal fraction of 1; `frac_of_fastest`
+is its fraction of the rate that no kernel exceeds.
 """
 from __future__ import annotations
 
@@ -28,6 +32,7 @@ import sys
 import tempfile
 
 VALU_LANE_OPS_PER_S = 256 * 4 * 16 * 2.4e9
+VALU_FASTEST_PER_S = 6.7e13
 TRANS_LANE_OPS_PER_S = VALU_LANE_OPS_PER_S / 4
 HBM_BYTES_PER_S = 8.0e12
 
@@ -201,7 +206,8 @@ def kernel_roofline(c: dict, kernel_ms: float, algorithmic_bytes: float = None):
     if "SQ_INSTS_VALU" in c:
         a = c["SQ_INSTS_VALU"] * 64 / t
         out["valu"] = {"achieved": a, "peak": VALU_LANE_OPS_PER_S, "unit": "VALU lane-instructions/s",
-                       "frac": a / VALU_LANE_OPS_PER_S, "instructions_per_dispatch": c["SQ_INSTS_VALU"]}
+                       "frac": a / VALU_LANE_OPS_PER_S, "frac_of_fastest": a / VALU_FASTEST_PER_S,
+                       "instructions_per_dispatch": c["SQ_INSTS_VALU"]}
         frac["valu"] = a / VALU_LANE_OPS_PER_S
     if "VALUBusy" in c:
         out["valu_busy"] = c["VALUBusy"] / 100.0

@@ -131,7 +131,8 @@ def octree_rooflines(ctx):
         return None
     out = {}
     for name in ("oct_bound_kernel<1", "oct_bound_kernel<2", "oct_fine_kernel<1", "oct_fine_kernel<2",
-                 "oct_tile_kernel", "winmax_fused_kernel", "conv3_fwd_kernel"):
+                 "oct_fine_count_kernel", "confocal_lds_kernel_poly<CountRows, 16, 2, true>", "winmax_fused_kernel",
+                 "conv3_fwd_kernel"):
         r = roofline_of(ctx["counters"], name, None, None, ctx["fingerprint"], pick="max")
         if r is not None:
             out[name] = r
@@ -139,8 +140,8 @@ def octree_rooflines(ctx):
 
 
 def batch_comparison(bp, count, seed=1004, serial=True, ctx=None):
-    """Uneven confocal captures: one persistent work-queue launch (autotuned, hipGraph replay)
-    against one plan execution per capture."""
+    """Uneven confocal captures: one batch (autotuned, hipGraph replay) against one plan execution per
+    capture."""
     from backprojector_amd import proposals, scenes
     t_r = time.perf_counter()
     caps = scenes.batch_captures(count, seed)
@@ -155,7 +156,7 @@ def batch_comparison(bp, count, seed=1004, serial=True, ctx=None):
            "updates": t["updates"], "batch_ms": t["per_exec_ms"], "updates_per_s": t["updates_per_s"],
            "latency_ms_p50": float(np.percentile(lat, 50)), "latency_ms_p99": float(np.percentile(lat, 99)),
            "config": cfg}
-    for st in ("bf16",):   # 16-bit rows (per-capture scale): half the row memory, same queue
+    for st in ("bf16",):   # 16-bit rows (per-capture scale): half the row memory, the same launches
         with bp.Batch(args, storage=st) as b:
             c16 = b.tune(reps=2)
             t16 = b.benchmark(1, 5)
@@ -168,13 +169,14 @@ def batch_comparison(bp, count, seed=1004, serial=True, ctx=None):
         out["one_launch_per_capture_ms"] = ms
         out["speedup_vs_one_launch_per_capture"] = ms / t["per_exec_ms"]
     if ctx is not None and ctx.get("counters"):
-        # the persistent queue kernel of the chosen configuration, and the prologue
+        # the item launches, then the persistent queue kernel of the chosen configuration and the prologue
         k, d = cfg["lane_voxels"], cfg["lds_depth"]
         if cfg["launches"] == 1:
             queue = f"batch_queue_kernel<FusedF32, FusedSource<FusedF32>, {k}, {d}, 7, 4>"
         else:   # the LDS-staged tiles' queue (its voxels per lane are the LDS tile's)
             queue = f"batch_queue_kernel<FusedF32, FusedSource<FusedF32>, 2, {d}, 2, 4>"
-        names = [queue, "batch_prologue_kernel"]
+        names = ["batch_lds_kernel_poly<CountRows, 16", "batch_lds_kernel_poly<CountRows, 8", "batch_split_kernel",
+                 queue, "batch_prologue_kernel"]
         if cfg["launches"] == 3:   # the 512-lane 16^3-tile queue
             names.append("batch_queue_kernel<FusedF32, FusedSource<FusedF32>, 2, 8, 2, 8>")
         if cfg["launches"] >= 2:
@@ -248,7 +250,7 @@ def config_measurements(bp, cap, reps=5, ctx=None):
                                  "updates": upd, "updates_per_s": upd / (wms * 1e-3)}
     if ctx is not None:   # kernel time: its duration under the counter passes
         out["confocal_128cube_cpu_path_semantics"]["roofline"] = roofline_of(
-            ctx["counters"], "window_kernel", None, None, ctx["fingerprint"])
+            ctx["counters"], "window_lds_kernel", None, None, ctx["fingerprint"])
     cplx = bp.phasor_pulse(pre["chunk"], 0.004, cap.deltaT)
     if ctx is not None:   # the complex FIR filter (one-shot call; kernel time under the counter passes)
         out["phasor_fir_4mm"] = {"workload": "phasor FIR (4 mm) of the 128x128 x Tc chunk, complex64 out",
@@ -550,7 +552,8 @@ def main():
                 "achieved": rl_block[rl_block["bound"]]["achieved"], "peak": rl_block[rl_block["bound"]]["peak"],
                 "unit": rl_block[rl_block["bound"]]["unit"], "frac": rl_block["frac"],
                 "traffic": rl_block.get("hbm", {}).get("traffic_bytes"),
-                "valu_frac": rl_block["valu"]["frac"], "valu_busy": rl_block.get("valu_busy"),
+                "valu_frac": rl_block["valu"]["frac"], "valu_frac_of_fastest": rl_block["valu"]["frac_of_fastest"],
+                "valu_busy": rl_block.get("valu_busy"),
                 "sqrt_frac": rl_block.get("sqrt", {}).get("frac"), "hbm_frac": rl_block.get("hbm", {}).get("frac"),
                 "lds_bank_conflict_frac": rl_block.get("lds_bank_conflict_frac"),
                 "valu_instructions_per_update": rl_block["valu"]["instructions_per_dispatch"] * 64 / updates,
