@@ -563,7 +563,8 @@ def main():
                 "counters_source": rl_block["counters_source"], "stale": rl_block["stale"],
                 "counters_per_dispatch": rl_block["counters_per_dispatch"],
                 "note": "bound = the roofline with the largest fraction; VALU: SQ_INSTS_VALU x 64 lanes / kernel "
-                        "time against 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz; sqrt: SQ_INSTS_VALU_TRANS_F32 x 64 "
+                        "time against 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz (nominal; plain adds beat it, "
+                        "valu_frac_of_fastest is of 6.7e13/s); sqrt: SQ_INSTS_VALU_TRANS_F32 x 64 "
                         "against a quarter of that; HBM: (FETCH_SIZE x 2.000 + WRITE_SIZE) KiB (copy-kernel "
                         "calibration) against 8 TB/s.  effective_gather_GBps = 4 B per update / kernel time "
                         "(each staged sample is read from LDS for every voxel of a tile, so it exceeds HBM)"}
