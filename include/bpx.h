@@ -180,7 +180,9 @@ bpx_status bpx_backprojection_noalloc(const float* transient_chunk, uint64_t tra
                                       float t0, float deltaT, void* hip_stream);
 
 /* CPU-path semantics on the GPU: the grid is given as the reference CPU path takes it
- * (volume_position = centre, volume_size), spacing size/N, voxel-diagonal window. */
+ * (volume_position = centre, volume_size), spacing size/N, voxel-diagonal window.  Confocal captures of
+ * real samples take device memory for threshold tables (16 bytes a pair and bin, 16 GiB at most); without
+ * it a slower kernel that needs none runs. */
 bpx_status bpx_window_backprojection(const float* transient_chunk, uint64_t transient_size,
                                      uint32_t T, const bpx_pair* scanned_pairs,
                                      uint32_t num_pairs, float* voxel_volume,

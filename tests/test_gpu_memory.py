@@ -132,8 +132,8 @@ def test_octree_tile_sums_that_do_not_fit(gpu):
 
 
 def test_batch_sums_that_do_not_fit(gpu):
-    """70 captures of 64 MiB of partial sums each: at most 4 GiB at a time, and where they do not fit
-    either, in smaller waves.  Every volume is its own plan's bit for bit."""
+    """70 captures of 64 MiB of partial sums each, split texture-path captures among them: at most 4 GiB at a
+    time, and where they do not fit either, in smaller waves.  Every volume is its own plan's bit for bit."""
     N, T = (64, 64, 64), 300
     grid = basis(N, (0.0, 0.0, 0.7), (0.4, 0.4, 0.4))
     kinds = []
@@ -146,16 +146,22 @@ def test_batch_sums_that_do_not_fit(gpu):
             plan.execute()
             refs.append(plan.volume())
             assert int(plan.info()["kernel"].split("tiles, ")[1].split()[0]) >= 32
-    args = [kinds[i % 5] for i in range(70)]
+    H, pr = capture((31, 33), 2000, 9)
+    kinds.append((H, pr, (24, 24, 24), *basis((24, 24, 24), (0.0, 0.0, 0.7), (0.8, 0.8, 0.6)), 0.5, 0.0015))
+    with gpu.Plan(*kinds[-1]) as plan:
+        plan.execute()
+        refs.append(plan.volume())
+        assert plan.info()["kernel"].startswith("confocal_kernel_split<")
+    args = [kinds[i % 6] for i in range(84)]
     b, taken = memory_of(lambda: gpu.Batch(args))
-    rows = len(args) * (T * 4096 * 4 + 8 * 4096 * 384 + 4 * 64 ** 3)
+    rows = 70 * (T * 4096 * 4 + 8 * 4096 * 384 + 4 * 64 ** 3) + 14 * 12 * H.size
     assert taken < rows + (4 << 30) + (256 << 20), taken
     for room in (None, 5 << 29):
         with memory_left(room) if room else nullcontext(), b or gpu.Batch(args) as batch:
             for rep in range(2):
                 batch.execute()
-                for i in range(0, 70, 3):
-                    assert np.array_equal(batch.volume(i), refs[i % 5]), (room, rep, i)
+                for i in range(84):
+                    assert np.array_equal(batch.volume(i), refs[i % 6]), (room, rep, i)
             assert np.all(batch.latencies() > 0)
         b = None
 
